@@ -17,20 +17,25 @@
 // lu from checkpoints (the two-sided scheme of the forward SW solver).  Per (column, g-point)
 // the inputs are read twice; no per-layer state is stored.
 //
-// Shortwave.  The forward is the two-sided adding solver of the SW solver kernel, per column and
-// g-point, with layers j counted from the top: the direct beam dir_{j+1} = dir_j Tn_j with layer
-// sources SU_j = Rdir_j dir_j, SD_j = Tdir_j dir_j; top-down D_{j+1} = SD + T (D + Ru SU) e1,
-// Ru_{j+1} = R + T^2 Ru e1, e1 = 1/(1 - R Ru); bottom-up A_j = R + T^2 A' e2,
-// S_j = SU + T (S' + A' SD) e2, e2 = 1/(1 - R A') (A' = A_{j+1}); fluxes dn = (D + Ru S)/(1 - Ru A),
-// up = A dn + S, total down dn + dir.  The adjoint stores these states (in the build's precision, per column,
-// g-point and level, in a scratch buffer sized by the caller's g-point range), then runs the
-// reverse of the bottom-up recursion top-down and the reverse of the top-down recursion and the
-// direct beam bottom-up.  The layer Jacobian d(R, T, Rdir, Tdir, Tn)/d(tau, w0, g) comes from the
-// FP64 layer formulas evaluated on dual numbers.
+// Shortwave.  With layers j counted from the top, the direct beam dir_{j+1} = dir_j Tn_j and the layer
+// sources SU_j = Rdir_j dir_j, SD_j = Tdir_j dir_j, the diffuse fluxes solve
+//     dn_{j+1} = T_j dn_j + R_j up_{j+1} + SD_j,      dn_0 = inc_dif
+//     up_j     = T_j up_{j+1} + R_j dn_j + SU_j,      up_n = A_s dn_n + alb_dir dir_n.
+// For cotangents c^u, c^d of up and dn, the multipliers lam_{j+1}, mu_j of these equations solve
+//     mu_{j+1} = T_j mu_j + R_j lam_{j+1} + c^u_{j+1},   mu_0 = c^u_0
+//     lam_j    = T_j lam_{j+1} + R_j mu_j + c^d_j,       lam_n = A_s mu_n + c^d_n:
+// the same two-stream problem with mu in the place of dn, lam of up and the cotangents as sources.
+// So one pair of adding recursions (R_up above, albedo A below) serves both, with two sources each:
+// top-down dn = D + R_up up and mu = E + R_up lam, bottom-up up = A dn + S and lam = A mu + F.  A
+// top-down sweep stores R_up, D, E and dir at every level; a bottom-up sweep carries A, S, F and the
+// beam's adjoint, forms dn, up, mu and lam at each level from both sides, and with them the layer's
+// cotangents (gR = lam_{j+1} up_{j+1} + mu_j dn_j, gT = lam_{j+1} dn_j + mu_j up_{j+1}, gSU = mu_j,
+// gSD = lam_{j+1}), which it carries through the layer formulas in reverse mode.  Everything is FP64
+// but the inputs, the stored level states and the outputs.
 #include <algorithm>
 
 #include "common.h"
-#include "two_stream.h"
+#include "solver_math.h"
 
 namespace rrtmgp_hip
 {
@@ -284,15 +289,8 @@ int lw_adjoint(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t n
 }
 // ---------------------------------------------------------------------------------------------
 // Shortwave adjoint: one (column, g-point) per thread, 64 columns x 4 g-points per work-group.
-// State store per (column, g-point): the layer properties R, T, Rdir, Tdir, Tn and the level
-// states D, Ru, dir, A, S and the reverse sweep's adjoints lA, lS, all in the build's precision.
-// The recursions carry them in FP64; the stored values are the FP64 ones rounded, and every
-// sweep computes in FP64 from what it reads.  The four sweeps are four kernels: they communicate
-// through the store only, and the three light ones then run at the occupancy their own registers
-// allow instead of that of the dual-number sweep.
 constexpr int SWA_GPTS = 4;
-constexpr int SWA_NL = 5;    // stored layer properties
-constexpr int SWA_NV = 7;    // stored level states
+constexpr int SWA_NS = 4;    // stored level states: R_up, D, E, dir
 
 template<typename Real>
 struct SwAdjArgs
@@ -300,201 +298,260 @@ struct SwAdjArgs
     int64_t ncol, nlay, ngpt;
     int top_at_1;
     const Real *tau, *ssa, *gasy, *mu0, *alb_dir, *alb_dif, *inc_dir, *inc_dif, *a_up, *a_dn, *a_dir;
-    Real *sl, *sv, *d_tau, *d_ssa, *d_g, *d_alb_dir, *d_alb_dif;
+    Real *st, *d_tau, *d_ssa, *d_g, *d_alb_dir, *d_alb_dif;
 };
 
-// Indexing of one thread's (column, g-point).  Layer properties: 0 R, 1 T, 2 Rdir, 3 Tdir, 4 Tn.
-// Level states: 0 D, 1 Ru, 2 dir, 3 A, 4 S, 5 lA, 6 lS (adjoints of A and S at the level, from
-// the top-down reverse sweep; slot n of 5 and 6 holds the sweep's final values).
-template<typename Real>
-struct SwAdjAt
+// 1/x to within a rounding: the approximation and two Newton steps.
+__device__ __forceinline__ double rcp_full(double x)
 {
-    const SwAdjArgs<Real>& a;
-    int64_t icol, igpt, n, nlev, c2, lb;
-    __device__ SwAdjAt(const SwAdjArgs<Real>& args, int64_t ic, int64_t ig)
-        : a(args), icol(ic), igpt(ig), n(args.nlay), nlev(args.nlay + 1), c2(ic + args.ncol * ig),
-          lb(ic + args.ncol * args.nlay * ig) {}
-    __device__ int64_t lay(int64_t j) const { return lb + a.ncol * (a.top_at_1 ? j : n - 1 - j); }
-    __device__ int64_t lev(int64_t j) const { return icol + a.ncol * (a.top_at_1 ? j : n - j); }
-    __device__ Real& L(int q, int64_t jj) const { return a.sl[((int64_t(q) * nlev + jj) * a.ngpt + igpt) * a.ncol + icol]; }
-    __device__ Real& V(int q, int64_t jj) const { return a.sv[((int64_t(q) * nlev + jj) * a.ngpt + igpt) * a.ncol + icol]; }
+    const double r = rcp_f64(x);
+    return fma(r, fma(-x, r, 1.), r);
+}
 
-    // Flux cotangents at level j: gradients with respect to D, Ru, A, S.
-    __device__ void level_partials(int64_t jj, double D, double Ru, double A, double S, double& gD, double& gRu,
-                                   double& gA, double& gS) const
+// The two-stream layer (F90:1043-1104 with the clamp of rte_solver_kernels.cu:581-583) and what its
+// reverse mode reads again.  The direct-beam terms are written with G = (e^{-k tau} - Tn) / (1 - k mu0),
+// in which the reference's factor 1 / (1 - (k mu0)^2) cancels to 1 / (1 + k mu0) identically (see
+// sw_layer_fp32): no term grows as k mu0 approaches 1.  With x = (1 - k mu0) tau / mu0 and
+// chi = ((1 - e^{-x}) / x - 1) / x,
+//     G = e^{-k tau} (tau / mu0) (1 + x chi),   dG/dk = tau e^{-k tau} (tau / mu0) chi,
+//     dG/dtau = (e^{-k tau} - G) / mu0;
+// chi comes from its series for |x| < 1/4 (truncation < 1e-16); elsewhere G and dG/dk are difference
+// quotients, which lose less than 1 / x^2 there.
+struct SwLayerAdj
+{
+    double R, T, Rd, Td, Tn;                                            // the layer's properties
+    double w0, om, g, k, g1, g2, g3, g4, a1, a2, e1, c2, RT, r, P, Q, G, dGdk, rd, td, b;
+
+    __device__ __forceinline__ void eval(double tau, double w0_, double g_, double mu0, double inv_mu0)
     {
-        const double au = double(a.a_up[lev(jj)]), adn = double(a.a_dn[lev(jj)]);
-        const double q = D + Ru * S, den = 1. / (1. - Ru * A), dn = q * den;
-        const double gdn = adn + au * A;
-        gD = gdn * den;
-        gRu = gdn * (S * den + q * A * den * den);
-        gA = gdn * q * Ru * den * den + au * dn;
-        gS = gdn * Ru * den + au;
+        w0 = w0_; g = g_;
+        om = 1. - w0;
+        g1 = 2. - w0 * (1.25 + .75 * g);
+        g2 = .75 * w0 * (1. - g);
+        g3 = .5 - .75 * mu0 * g;
+        g4 = 1. - g3;
+        a1 = g1 * g4 + g2 * g3;
+        a2 = g1 * g3 + g2 * g4;
+        k = sqrt(fmax(2. * om * (g1 + g2), Limits<double>::k_min));     // gamma1 - gamma2 = 2 (1 - w0)
+        e1 = exp(-tau * k);
+        const double y = tau * inv_mu0;
+        Tn = exp(-y);
+        c2 = 1. - e1 * e1;
+        const double km = k * mu0, ek = 1. - km, x = y * ek;
+        if (fabs(x) < .25)
+        {
+            double c = 1. / 479001600.;                                 // 1/12!, alternating down to 1/2!
+            c = 1. / 39916800. - x * c;
+            c = 1. / 3628800. - x * c;
+            c = 1. / 362880. - x * c;
+            c = 1. / 40320. - x * c;
+            c = 1. / 5040. - x * c;
+            c = 1. / 720. - x * c;
+            c = 1. / 120. - x * c;
+            c = 1. / 24. - x * c;
+            c = 1. / 6. - x * c;
+            c = .5 - x * c;                                             // -chi
+            const double ey = e1 * y;
+            G = ey * (1. - x * c);
+            dGdk = -tau * ey * c;
+        }
+        else
+        {
+            const double iek = rcp_full(ek);
+            G = (e1 - Tn) * iek;
+            dGdk = (mu0 * G - tau * e1) * iek;
+        }
+        const double d0 = k * (2. - c2) + g1 * c2, opk = 1. + km;
+        const double q = rcp_full(d0 * opk);
+        RT = q * opk;
+        r = q * d0;                                                     // 1 / (1 + k mu0)
+        R = RT * g2 * c2;
+        T = 2. * RT * k * e1;
+        P = (a2 + k * g3) * c2 + 2. * k * (g3 - a2 * mu0) * e1 * G;
+        Q = (a1 - k * g4) * c2 * Tn - 2. * k * (g4 + a1 * mu0) * G;
+        const double s = w0 * RT * r;
+        rd = s * P;
+        td = -s * Q;
+        b = 1. - Tn;
+        Rd = fmax(fmin(rd, b), Limits<double>::eps);
+        Td = fmax(fmin(td, b - Rd), Limits<double>::eps);
+    }
+
+    // Cotangents of (tau, w0, g) for those of (R, T, Rd, Td, Tn).  max and min pass the cotangent of the
+    // operand they picked.
+    __device__ __forceinline__ void reverse(double tau, double mu0, double inv_mu0, double gR, double gT, double gRd,
+                                            double gTd, double gTn, double& g_tau, double& g_w0, double& g_g) const
+    {
+        const double eps = Limits<double>::eps;
+        const double m2 = fmin(td, b - Rd), m1 = fmin(rd, b);
+        double g_td = 0.;
+        if (m2 >= eps)
+        {
+            if (td <= b - Rd) g_td = gTd;
+            else { gTn -= gTd; gRd -= gTd; }
+        }
+        double g_rd = 0.;
+        if (m1 >= eps)
+        {
+            if (rd <= b) g_rd = gRd;
+            else gTn -= gRd;
+        }
+        const double wr = w0 * r, s = wr * RT, km = k * mu0;
+        const double g_s = g_rd * P - g_td * Q, gP = s * g_rd, gQ = -s * g_td;
+        const double eG = 2. * e1 * G, g3a = g3 - a2 * mu0, g4a = g4 + a1 * mu0, c2T = c2 * Tn, G2 = 2. * G;
+        double g_k = gP * (g3 * c2 + g3a * eG) - gQ * (g4 * c2T + g4a * G2);
+        double g_c2 = gP * (a2 + k * g3) + gQ * (a1 - k * g4) * Tn;
+        const double g_e1G = 2. * k * g3a * gP;
+        const double g_G = g_e1G * e1 - 2. * k * g4a * gQ;
+        double g_e1 = g_e1G * G;
+        gTn += gQ * (a1 - k * g4) * c2;
+        const double g_a1 = gQ * (c2T - km * G2), g_a2 = gP * (c2 - km * eG);
+        double g_g3 = gP * k * (c2 + eG);
+        const double g_g4 = -gQ * k * (c2T + G2);
+        // s = w0 RT r, R = RT gamma2 c2, T = 2 RT k e1, RT = 1 / (k (2 - c2) + gamma1 c2).
+        g_k -= g_s * s * mu0 * r;
+        const double ke = 2. * k * e1;
+        const double g_RT = g_s * wr + gR * g2 * c2 + gT * ke;
+        const double g_d0 = -g_RT * RT * RT;
+        g_c2 += gR * RT * g2 + g_d0 * (g1 - k);
+        g_k += 2. * gT * RT * e1 + g_d0 * (2. - c2) + g_G * dGdk;
+        g_e1 += 2. * (gT * RT * k - e1 * g_c2);
+        double g_g1 = g_d0 * c2, g_g2 = gR * RT * c2;
+        const double ge = g_e1 * e1;
+        g_k -= ge * tau;
+        g_tau = g_G * (e1 - G) * inv_mu0 - ge * k - gTn * Tn * inv_mu0;
+        const double q = 2. * om * (g1 + g2);
+        const double g_kk = q >= Limits<double>::k_min ? g_k * rcp_full(k) : 0.;        // k^2 = q = 2 om (gamma1 + gamma2)
+        const double g_q = g_kk * om;
+        g_w0 = g_s * RT * r - g_kk * (g1 + g2);
+        g_g1 += g_a1 * g4 + g_a2 * g3 + g_q;
+        g_g2 += g_a1 * g3 + g_a2 * g4 + g_q;
+        g_g3 += g_a1 * g2 + g_a2 * g1 - (g_g4 + g_a1 * g1 + g_a2 * g2);
+        g_w0 += .75 * (1. - g) * g_g2 - (1.25 + .75 * g) * g_g1;
+        g_g = -.75 * (w0 * (g_g1 + g_g2) + mu0 * g_g3);
     }
 };
 
-// Contributions of the bottom-up recursion's adjoint at layer j to the layer's R, T, SU, SD
-// cotangents, from the adjoints lA, lS of A_j, S_j.
-__device__ __forceinline__ void bottom_up_partials(double lA, double lS, double R, double T, double SD, double A1,
-                                                   double S1, double& gR, double& gT, double& gSU, double& gSD)
-{
-    const double e2 = 1. / (1. - R * A1);
-    const double w = S1 + A1 * SD;
-    gR = lA * (1. + T * T * A1 * A1 * e2 * e2) + lS * T * w * A1 * e2 * e2;
-    gT = lA * 2. * T * A1 * e2 + lS * w * e2;
-    gSU = lS;
-    gSD = lS * T * A1 * e2;
-}
-
+// One thread's place: offsets of its (column, g-point) in the layer arrays, the cotangents and the
+// level-state store (state q of level j at st[((4 j + q) ngpt + igpt) ncol + icol], j from the top).
 template<typename Real>
-__device__ __forceinline__ bool sw_adj_thread(const SwAdjArgs<Real>& a, int64_t& icol, int64_t& igpt)
+struct SwAdjAt
 {
-    icol = int64_t(blockIdx.x) * ADJ_COLS + threadIdx.x;
-    igpt = int64_t(blockIdx.y) * SWA_GPTS + threadIdx.y;
-    return icol < a.ncol && igpt < a.ngpt;
-}
+    int64_t icol, c2, lay0, dlay, lev0, dlev, st0, dst, dq;
+    bool in;
+    __device__ explicit SwAdjAt(const SwAdjArgs<Real>& a)
+    {
+        icol = int64_t(blockIdx.x) * ADJ_COLS + threadIdx.x;
+        const int64_t igpt = int64_t(blockIdx.y) * SWA_GPTS + threadIdx.y;
+        in = icol < a.ncol && igpt < a.ngpt;
+        c2 = icol + a.ncol * igpt;
+        lay0 = icol + a.ncol * a.nlay * igpt + (a.top_at_1 ? 0 : a.ncol * (a.nlay - 1));   // top layer
+        dlay = a.top_at_1 ? a.ncol : -a.ncol;
+        lev0 = icol + (a.top_at_1 ? 0 : a.ncol * a.nlay);                                  // top level
+        dlev = dlay;
+        dq = a.ncol * a.ngpt;
+        st0 = c2;
+        dst = SWA_NS * dq;
+    }
+};
 
-// Sweep 1, forward top-down: layer properties, direct beam, column above each level.
+// Sweep down: the column above each level, for the fluxes (D) and for the multipliers (E).
 template<typename Real>
 __global__ __launch_bounds__(ADJ_COLS * SWA_GPTS)
 void sw_adjoint_down_kernel(SwAdjArgs<Real> a)
 {
-    int64_t icol, igpt;
-    if (!sw_adj_thread(a, icol, igpt)) return;
-    const SwAdjAt<Real> t(a, icol, igpt);
-    const double m0 = double(a.mu0[icol]);
+    const SwAdjAt<Real> t(a);
+    if (!t.in) return;
+    const int64_t n = a.nlay;
+    const double m0 = double(a.mu0[t.icol]), im0 = 1. / m0;
     double dir = double(a.inc_dir[t.c2]) * m0, D = a.inc_dif ? double(a.inc_dif[t.c2]) : 0., Ru = 0.;
-    for (int64_t jj = 0; jj < t.n; ++jj)
+    double E = double(a.a_up[t.lev0]);
+    Real* st = a.st + t.st0;
+    int64_t l = t.lay0, v = t.lev0;
+    // The next layer's inputs are requested before this layer's chain starts.
+    Real nt = a.tau[l], nw = a.ssa[l], ng = a.gasy[l], ncd = a.a_dn[v], ncu = a.a_up[v + t.dlev];
+    for (int64_t j = 0; j < n; ++j)
     {
-        t.V(0, jj) = Real(D); t.V(1, jj) = Real(Ru); t.V(2, jj) = Real(dir);
-        const int64_t l = t.lay(jj);
-        double R, T, Rd, Td, Tn;
-        sw_two_stream_t<double>(double(a.tau[l]), double(a.ssa[l]), double(a.gasy[l]), m0, R, T, Rd, Td, Tn);
-        // The stored (build-precision) values are the ones every later sweep uses.
-        t.L(0, jj) = Real(R); t.L(1, jj) = Real(T); t.L(2, jj) = Real(Rd); t.L(3, jj) = Real(Td); t.L(4, jj) = Real(Tn);
-        R = double(Real(R)); T = double(Real(T)); Rd = double(Real(Rd)); Td = double(Real(Td));
-        Tn = double(Real(Tn));
-        const double SU = Rd * dir, SD = Td * dir;
-        const double e1 = 1. / (1. - R * Ru);
-        D = SD + T * (D + Ru * SU) * e1;
-        Ru = R + T * T * Ru * e1;
-        dir *= Tn;
+        const double tau = double(nt), w0 = double(nw), g = double(ng), cd = double(ncd), cu = double(ncu);
+        l += t.dlay; v += t.dlev;
+        if (j + 1 < n)
+        {
+            nt = a.tau[l]; nw = a.ssa[l]; ng = a.gasy[l]; ncd = a.a_dn[v]; ncu = a.a_up[v + t.dlev];
+        }
+        st[0] = Real(Ru); st[t.dq] = Real(D); st[2 * t.dq] = Real(E); st[3 * t.dq] = Real(dir);
+        st += t.dst;
+        SwLayerAdj L;
+        L.eval(tau, w0, g, m0, im0);
+        const double Te = L.T * rcp_full(1. - L.R * Ru);
+        D = L.Td * dir + Te * (D + Ru * L.Rd * dir);
+        E = cu + Te * (E + Ru * cd);
+        Ru = L.R + L.T * Te * Ru;
+        dir *= L.Tn;
     }
-    t.V(0, t.n) = Real(D); t.V(1, t.n) = Real(Ru); t.V(2, t.n) = Real(dir);
+    st[0] = Real(Ru); st[t.dq] = Real(D); st[2 * t.dq] = Real(E); st[3 * t.dq] = Real(dir);
 }
 
-// Sweep 2, forward bottom-up: column below each level.
+// Sweep up: the column below each level, the fluxes and multipliers of the level, the layer's gradients.
+// Bound by its FP64 arithmetic (153 VGPRs, 3 wavefronts per SIMD) next to 10 values of traffic a layer.
+// The pair of sweeps takes 3.4 + 5.4 ms for the 14 bands of 16384 columns x 128 layers in FP32; the four
+// it replaced (two forward and two reverse recursions through 12 stored states a level, the layer
+// Jacobian on forward-mode dual numbers) took 22.9 ms.
 template<typename Real>
 __global__ __launch_bounds__(ADJ_COLS * SWA_GPTS)
 void sw_adjoint_up_kernel(SwAdjArgs<Real> a)
 {
-    int64_t icol, igpt;
-    if (!sw_adj_thread(a, icol, igpt)) return;
-    const SwAdjAt<Real> t(a, icol, igpt);
-    double A = double(a.alb_dif[t.c2]), S = double(t.V(2, t.n)) * double(a.alb_dir[t.c2]);
-    t.V(3, t.n) = Real(A); t.V(4, t.n) = Real(S);
-    for (int64_t jj = t.n - 1; jj >= 0; --jj)
+    const SwAdjAt<Real> t(a);
+    if (!t.in) return;
+    const int64_t n = a.nlay;
+    const double m0 = double(a.mu0[t.icol]), im0 = 1. / m0;
+    const Real* st = a.st + t.st0 + n * t.dst;
+    int64_t l = t.lay0 + (n - 1) * t.dlay, v = t.lev0 + n * t.dlev;
+    double A, S, F, up, lam, ldir, cu;
     {
-        const double R = double(t.L(0, jj)), T = double(t.L(1, jj)), dir = double(t.V(2, jj));
-        const double SU = double(t.L(2, jj)) * dir, SD = double(t.L(3, jj)) * dir;
-        const double e2 = 1. / (1. - R * A);
-        S = SU + T * (S + A * SD) * e2;
-        A = R + T * T * A * e2;
-        t.V(3, jj) = Real(A); t.V(4, jj) = Real(S);
+        const double ad = double(a.alb_dir[t.c2]);
+        const double Ru = double(st[0]), D = double(st[t.dq]), E = double(st[2 * t.dq]), dir = double(st[3 * t.dq]);
+        const double cd = double(a.a_dn[v]);
+        cu = double(a.a_up[v]);
+        A = double(a.alb_dif[t.c2]);
+        S = dir * ad;
+        F = cd;
+        const double den = rcp_full(1. - Ru * A);
+        const double dn = (D + Ru * S) * den, mu = (E + Ru * F) * den;
+        up = A * dn + S;
+        lam = A * mu + F;
+        ldir = cd + double(a.a_dir[v]) + mu * ad;
+        a.d_alb_dif[t.c2] = Real(mu * dn);
+        a.d_alb_dir[t.c2] = Real(mu * dir);
     }
-}
-
-// Sweep 3: reverse of the bottom-up recursion, top-down; albedo gradients.
-template<typename Real>
-__global__ __launch_bounds__(ADJ_COLS * SWA_GPTS)
-void sw_adjoint_rev_down_kernel(SwAdjArgs<Real> a)
-{
-    int64_t icol, igpt;
-    if (!sw_adj_thread(a, icol, igpt)) return;
-    const SwAdjAt<Real> t(a, icol, igpt);
-    const int64_t n = t.n;
-    double lA = 0., lS = 0.;
-    double A = double(t.V(3, 0)), S = double(t.V(4, 0));
-    for (int64_t jj = 0; jj <= n; ++jj)
+    st -= t.dst; v -= t.dlev;
+    Real nt = a.tau[l], nw = a.ssa[l], ng = a.gasy[l], ncd = a.a_dn[v], ncu = a.a_up[v], ncr = a.a_dir[v];
+    Real nR = st[0], nD = st[t.dq], nE = st[2 * t.dq], ndir = st[3 * t.dq];
+    for (int64_t j = n - 1; j >= 0; --j)
     {
-        double gD, gRu, gA, gS;
-        t.level_partials(jj, double(t.V(0, jj)), double(t.V(1, jj)), A, S, gD, gRu, gA, gS);
-        lA += gA; lS += gS;
-        if (jj == n) break;
-        t.V(5, jj) = Real(lA); t.V(6, jj) = Real(lS);
-        const double R = double(t.L(0, jj)), T = double(t.L(1, jj)), dir = double(t.V(2, jj));
-        const double SD = double(t.L(3, jj)) * dir;
-        const double A1 = double(t.V(3, jj + 1)), S1 = double(t.V(4, jj + 1));
-        const double e2 = 1. / (1. - R * A1);
-        const double w = S1 + A1 * SD;
-        const double nA = lA * T * T * e2 * e2 + lS * T * e2 * (SD + w * R * e2);
-        lS = lS * T * e2;
-        lA = nA;
-        A = A1; S = S1;
-    }
-    t.V(5, n) = Real(lA); t.V(6, n) = Real(lS);
-    a.d_alb_dif[t.c2] = Real(lA);
-    a.d_alb_dir[t.c2] = Real(lS * double(t.V(2, n)));
-}
-
-// Sweep 4: reverse of the top-down recursion and the direct beam, bottom-up; layer gradients.
-template<typename Real>
-__global__ __launch_bounds__(ADJ_COLS * SWA_GPTS)
-void sw_adjoint_rev_up_kernel(SwAdjArgs<Real> a)
-{
-    int64_t icol, igpt;
-    if (!sw_adj_thread(a, icol, igpt)) return;
-    const SwAdjAt<Real> t(a, icol, igpt);
-    const int64_t n = t.n;
-    const double m0 = double(a.mu0[icol]);
-    const double ad = double(a.alb_dir[t.c2]);
-    double lD, lRu, ldir;
-    double A1 = double(t.V(3, n)), S1 = double(t.V(4, n));
-    {
-        double gD, gRu, gA, gS;
-        t.level_partials(n, double(t.V(0, n)), double(t.V(1, n)), A1, S1, gD, gRu, gA, gS);
-        lD = gD; lRu = gRu;
-        ldir = double(a.a_dn[t.lev(n)]) + double(a.a_dir[t.lev(n)]) + double(t.V(6, n)) * ad;
-    }
-    for (int64_t jj = n - 1; jj >= 0; --jj)
-    {
-        // Layer properties and their Jacobian by forward mode on (tau, w0, g); the values are
-        // rounded to the stored precision, as the earlier sweeps used them.
-        const int64_t l = t.lay(jj);
-        Dual3 oR, oT, oRd, oTd, oTn;
-        sw_two_stream_t<Dual3>(mk(double(a.tau[l]), 1., 0., 0.), mk(double(a.ssa[l]), 0., 1., 0.),
-                               mk(double(a.gasy[l]), 0., 0., 1.), m0, oR, oT, oRd, oTd, oTn);
-        const double R = double(Real(oR.v)), T = double(Real(oT.v)), Rd = double(Real(oRd.v));
-        const double Td = double(Real(oTd.v)), Tn = double(Real(oTn.v));
-        const double D = double(t.V(0, jj)), Ru = double(t.V(1, jj)), dir = double(t.V(2, jj));
-        const double SU = Rd * dir, SD = Td * dir;
-        // A_j, S_j rebuilt from A_{j+1}, S_{j+1} exactly as the bottom-up forward sweep formed them.
-        const double e2f = 1. / (1. - R * A1);
-        const double S = SU + T * (S1 + A1 * SD) * e2f;
-        const double A = R + T * T * A1 * e2f;
-        double bR, bT, bSU, bSD;
-        bottom_up_partials(double(t.V(5, jj)), double(t.V(6, jj)), R, T, SD, A1, S1, bR, bT, bSU, bSD);
-        const double e1 = 1. / (1. - R * Ru);
-        const double v = D + Ru * SU;
-        const double gSD = bSD + lD;
-        const double gSU = bSU + lD * T * Ru * e1;
-        const double gT = bT + lD * v * e1 + lRu * 2. * T * Ru * e1;
-        const double gR = bR + lD * T * v * Ru * e1 * e1 + lRu * (1. + T * T * Ru * Ru * e1 * e1);
-        const double gRd = gSU * dir, gTd = gSD * dir, gTn = ldir * dir;
-        const double nD = lD * T * e1;
-        const double nRu = lD * (T * SU * e1 + T * v * R * e1 * e1) + lRu * T * T * e1 * e1;
-        const double ndir = ldir * Tn + gSU * Rd + gSD * Td;
-        double g3[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-            g3[c] = gR * oR.d[c] + gT * oT.d[c] + gRd * oRd.d[c] + gTd * oTd.d[c] + gTn * oTn.d[c];
-        a.d_tau[l] = Real(g3[0]); a.d_ssa[l] = Real(g3[1]); a.d_g[l] = Real(g3[2]);
-        double gD, gRu, gA, gS;
-        t.level_partials(jj, D, Ru, A, S, gD, gRu, gA, gS);
-        lD = nD + gD;
-        lRu = nRu + gRu;
-        ldir = ndir + double(a.a_dn[t.lev(jj)]) + double(a.a_dir[t.lev(jj)]);
-        A1 = A; S1 = S;
+        const double tau = double(nt), w0 = double(nw), g = double(ng), cd = double(ncd), cr = double(ncr);
+        const double cu0 = double(ncu), Ru = double(nR), D = double(nD), E = double(nE), dir = double(ndir);
+        const int64_t lo = l;
+        l -= t.dlay; v -= t.dlev; st -= t.dst;
+        if (j > 0)
+        {
+            nt = a.tau[l]; nw = a.ssa[l]; ng = a.gasy[l]; ncd = a.a_dn[v]; ncu = a.a_up[v]; ncr = a.a_dir[v];
+            nR = st[0]; nD = st[t.dq]; nE = st[2 * t.dq]; ndir = st[3 * t.dq];
+        }
+        SwLayerAdj L;
+        L.eval(tau, w0, g, m0, im0);
+        const double Te = L.T * rcp_full(1. - L.R * A);
+        S = L.Rd * dir + Te * (S + A * L.Td * dir);
+        F = cd + Te * (F + A * cu);
+        A = L.R + L.T * Te * A;
+        const double den = rcp_full(1. - Ru * A);
+        const double dn = (D + Ru * S) * den, mu = (E + Ru * F) * den;
+        double gt, gw, gg;
+        L.reverse(tau, m0, im0, lam * up + mu * dn, lam * dn + mu * up, mu * dir, lam * dir, ldir * dir, gt, gw, gg);
+        a.d_tau[lo] = Real(gt); a.d_ssa[lo] = Real(gw); a.d_g[lo] = Real(gg);
+        ldir = cd + cr + mu * L.Rd + lam * L.Td + ldir * L.Tn;
+        up = A * dn + S;
+        lam = A * mu + F;
+        cu = cu0;
     }
 }
 
@@ -509,17 +566,10 @@ int sw_adjoint(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Rea
         !d_ssa || !d_g || !d_alb_dir || !d_alb_dif)
         return arg_error("sw_adjoint: NULL array");
     hipStream_t s = as_stream(stream);
-    const size_t per = size_t((nlay + 1) * ngpt * ncol);
-    Real* sl = nullptr;
-    Real* sv = nullptr;
-    RRTMGP_TRY(scratch_alloc(&sl, SWA_NL * per, s));
-    if (int rc0 = scratch_alloc(&sv, SWA_NV * per, s); rc0 != RRTMGP_OK)
-    {
-        scratch_free(sl, s);
-        return rc0;
-    }
+    Real* st = nullptr;
+    RRTMGP_TRY(scratch_alloc(&st, SWA_NS * size_t((nlay + 1) * ngpt * ncol), s));
     const SwAdjArgs<Real> args{ncol, nlay, ngpt, top_at_1, tau, ssa, g, mu0, alb_dir, alb_dif, inc_dir, inc_dif,
-                               a_up, a_dn, a_dir, sl, sv, d_tau, d_ssa, d_g, d_alb_dir, d_alb_dif};
+                               a_up, a_dn, a_dir, st, d_tau, d_ssa, d_g, d_alb_dir, d_alb_dif};
     const dim3 grid(grid1(ncol, ADJ_COLS), grid1(ngpt, SWA_GPTS));
     const dim3 block(ADJ_COLS, SWA_GPTS);
     int rc = RRTMGP_OK;
@@ -534,20 +584,7 @@ int sw_adjoint(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Rea
         hipLaunchKernelGGL(sw_adjoint_up_kernel<Real>, grid, block, 0, s, args);
         rc = check_hip(hipGetLastError(), "sw_adjoint_up_kernel");
     }
-    if (rc == RRTMGP_OK)
-    {
-        RRTMGP_TIMED("sw_adjoint_rev_down_kernel", s);
-        hipLaunchKernelGGL(sw_adjoint_rev_down_kernel<Real>, grid, block, 0, s, args);
-        rc = check_hip(hipGetLastError(), "sw_adjoint_rev_down_kernel");
-    }
-    if (rc == RRTMGP_OK)
-    {
-        RRTMGP_TIMED("sw_adjoint_rev_up_kernel", s);
-        hipLaunchKernelGGL(sw_adjoint_rev_up_kernel<Real>, grid, block, 0, s, args);
-        rc = check_hip(hipGetLastError(), "sw_adjoint_rev_up_kernel");
-    }
-    scratch_free(sv, s);
-    scratch_free(sl, s);
+    scratch_free(st, s);
     return rc;
 }
 

@@ -394,13 +394,6 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
 }
 
 // ---------------------------------------------------------------------------------------------
-// Shortwave two-stream layer properties in FP64 (sw_two_stream_t of two_stream.h).
-__device__ __forceinline__ void sw_two_stream(double tau, double w0, double g, double mu0, double& Rdif,
-                                              double& Tdif, double& Rdir, double& Tdir, double& Tnoscat)
-{
-    sw_two_stream_t<double>(tau, w0, g, mu0, Rdif, Tdif, Rdir, Tdir, Tnoscat);
-}
-
 // One layer of the top-down sweep: diffuse R/T, the direct-beam sources and transmittance, in
 // the precision St of the adding states.  ab = 1 - R - T (diffuse absorptance) and omTn = 1 - Tn
 // are only read by the heating-rate variant (dead code otherwise).
