@@ -593,6 +593,49 @@ RRTMGP_DECLARE_BOTH(RRTMGP_DECL_SW_ADJOINT)
         T* d_plev, void* stream);
 RRTMGP_DECLARE_BOTH(RRTMGP_DECL_GO_ADJOINT)
 
+/* The adjoint drivers' band-range forms (band_count bands from the 0-based band_start; g-point  */
+/* arrays hold those bands' g-points, counted from the first one).                              */
+/* gas_optics_lw_bands_factored: rrtmgp_hip_gas_optics_lw_factored_* for the range.             */
+/* lw_adjoint_factored: reverse mode of the factored longwave solver for one angle (secant,      */
+/* weight); band_lims_gpt (2, nbnd) host, 1-based within the range; sfc_emis points at the       */
+/* range's first band of an (emis_nbnd, ncol) array.  Writes the cotangents of tau and the       */
+/* Planck fractions (ncol, nlay, ngpt), of sfc_src and the emissivity (ncol, ngpt), and those of  */
+/* the band Planck functions at the layer, its level ilay (lo) and ilay+1 (hi), summed over each  */
+/* group of up to 16 consecutive g-points of a band: (ncol, nlay, groups).                       */
+/* sw_adjoint_gases: rrtmgp_hip_sw_solver_2stream_adjoint_* with the cotangents of tau, ssa and   */
+/* g carried on to the gases' absorption and Rayleigh optical depths (any band cloud held fixed). */
+/* gas_optics_{lw,sw}_adjoint_bands: rrtmgp_hip_gas_optics_{lw,sw}_adjoint_* for the range, from   */
+/* those cotangents.                                                                             */
+#define RRTMGP_DECL_ADJ_BANDS(S, T)                                                            \
+    int rrtmgp_hip_gas_optics_lw_bands_factored_##S(const rrtmgp_kdist_dev* kd,                \
+        int64_t band_start, int64_t band_count, int64_t ncol, int64_t nlay, const T* play,     \
+        const T* tlay, const T* tlev, const T* tsfc, const T* col_dry,                         \
+        const rrtmgp_gas_vmr* gases, int sfc_lay, const T* cloud_tau, T* tau, T* planck_frac,  \
+        T* band_lay_src, T* band_lev_src, T* sfc_src, T* sfc_src_jac, void* stream);           \
+    int rrtmgp_hip_lw_adjoint_factored_##S(int64_t ncol, int64_t nlay, int64_t ngpt,           \
+        int top_at_1, double secant, double weight, const T* tau, const T* planck_frac,        \
+        const T* band_lay_src, const T* band_lev_src, int64_t nbnd, const int* band_lims_gpt,  \
+        const T* sfc_emis, int64_t emis_nbnd, const T* sfc_src, const T* bb_up_cot,            \
+        const T* bb_dn_cot, T* d_tau, T* d_planck_frac, T* d_lay_src, T* d_lev_src_lo,         \
+        T* d_lev_src_hi, T* d_sfc_src, T* d_sfc_emis, void* stream);                           \
+    int rrtmgp_hip_sw_adjoint_gases_##S(int64_t ncol, int64_t nlay, int64_t ngpt,              \
+        int top_at_1, const T* tau, const T* ssa, const T* g, const T* mu0,                    \
+        const T* sfc_alb_dir, const T* sfc_alb_dif, const T* inc_flux_dir,                     \
+        const T* inc_flux_dif, const T* bb_up_cot, const T* bb_dn_cot, const T* bb_dir_cot,    \
+        T* d_tau_abs, T* d_tau_ray, T* d_sfc_alb_dir, T* d_sfc_alb_dif, void* stream);         \
+    int rrtmgp_hip_gas_optics_lw_adjoint_bands_##S(const rrtmgp_kdist_dev* kd,                 \
+        int64_t band_start, int64_t band_count, int64_t ncol, int64_t nlay, const T* play,     \
+        const T* tlay, const T* tlev, const T* tsfc, const T* col_dry,                         \
+        const rrtmgp_gas_vmr* gases, int sfc_lay, const T* g_tau, const T* g_planck_frac,      \
+        const T* g_lay_src, const T* g_lev_src_lo, const T* g_lev_src_hi, const T* g_sfc_src,  \
+        T* d_col_gas, T* d_tlay, T* d_lnp_lay, T* d_tlev_lo, T* d_tlev_hi, T* d_tsfc,          \
+        void* stream);                                                                          \
+    int rrtmgp_hip_gas_optics_sw_adjoint_bands_##S(const rrtmgp_kdist_dev* kd,                 \
+        int64_t band_start, int64_t band_count, int64_t ncol, int64_t nlay, const T* play,     \
+        const T* tlay, const T* col_dry, const rrtmgp_gas_vmr* gases, const T* g_tau_abs,      \
+        const T* g_tau_ray, T* d_col_gas, T* d_tlay, T* d_lnp_lay, void* stream);
+RRTMGP_DECLARE_BOTH(RRTMGP_DECL_ADJ_BANDS)
+
 /* Assembly steps of the adjoint driver.  col_chain: from d_col_gas (ncol, nlay, ngas+2) to    */
 /* d_vmr (ncol, nlay, ngas, overwritten; gases in the descriptor's order) and d_col_dry        */
 /* (ncol, nlay, overwritten; slot ngas+1).  levels: d_tlev (ncol, nlev) from the per-layer     */

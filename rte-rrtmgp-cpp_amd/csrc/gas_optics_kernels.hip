@@ -13,8 +13,7 @@
 //      the 4 lanes of a pair read one contiguous 64-byte segment; results -> LDS;
 //   3. lane = column, wavefront = g-point row: finishing arithmetic and 256-byte coalesced
 //      stores in the reference layout (ncol, nlay, ngpt).
-// LDS rows are padded to 68 floats (conflict-free for both lane layouts).  Work-groups of one
-// chunk are consecutive and kept on one XCD, so that XCD's L2 holds the chunk's table slice.
+// Work-groups of neighbouring tiles are kept on one XCD, whose L2 then holds the table slices they share.
 #include <algorithm>
 #include <memory>
 #include <vector>
@@ -26,7 +25,6 @@ namespace rrtmgp_hip
 constexpr int GO_THREADS = 256;   // work-group: 4 wavefronts
 constexpr int GO_COLS = 64;       // columns of a work-group's layer
 constexpr int GO_GPTS = 16;       // g-points per chunk: the lanes of one pair
-constexpr int GO_ROW = 68;        // LDS row length (64 columns + padding)
 
 // Unpadded (g-point row, column) LDS tiles of the forward kernels: column c of row r sits at
 // c ^ 16 * (r / 4 % 4), so phase 2's stores (four rows gq + e, 16 columns each, per instruction)
@@ -384,14 +382,6 @@ __device__ __forceinline__ void stage_gases(const Gases<Real>& g, int ngas, GasR
         sg[i] = GasRef<Real>{g.p[i], g.scol[i], g.slay[i]};
 }
 
-template<typename Real>
-__device__ __forceinline__ Real col_lds(const GasRef<Real>* sg, int gas, int64_t icol, int64_t ilay, Real col_dry)
-{
-    if (gas == 0) return col_dry;
-    const GasRef<Real>& r = sg[gas - 1];
-    return r.p[icol * r.scol + ilay * r.slay] * col_dry;
-}
-
 // State of one (column, layer) pair for one band, computed once per pair (phase 1 of the fused
 // kernels) and read from LDS by the four lanes that share the pair (phase 2).
 template<typename Real>
@@ -408,24 +398,9 @@ struct PairState
     Real aux[5];         // LW: B(T_lay), B(T_lev above), B(T_lev below), B(T_sfc), B(T_sfc + 1); SW: col_ray
 };
 
-// The per-(column, layer) inputs of phase 1, read from memory ...
-template<typename Real>
-struct PairInGlobal
-{
-    const GasRef<Real>* sg;
-    int64_t icol, ilay, ncol;
-    const Real *play, *tlay, *tlev, *tsfc, *col_dry;
-    __device__ Real p() const { return play[icol + ncol * ilay]; }
-    __device__ Real t() const { return tlay[icol + ncol * ilay]; }
-    __device__ Real cd() const { return col_dry[icol + ncol * ilay]; }
-    __device__ Real col(int gas, Real cdv) const { return col_lds(sg, gas, icol, ilay, cdv); }
-    __device__ Real t_hi() const { return tlev[icol + ncol * (ilay + 1)]; }
-    __device__ Real t_lo() const { return tlev[icol + ncol * ilay]; }
-    __device__ Real t_sfc() const { return tsfc[icol]; }
-};
-
-// ... or from the work-group's LDS rows, filled by all its threads at once (one memory round trip
-// instead of the dependent loads of one wavefront) and read by every chunk of the work-group:
+// The per-(column, layer) inputs of phase 1, from the work-group's LDS rows, filled by all its threads
+// at once (one memory round trip instead of the dependent loads of one wavefront) and read by every
+// chunk of the work-group:
 // row 0 p, 1 T, 2 col_dry, 3 .. 3 + ngas - 1 the vmr of gases 1 .. ngas, then (longwave) T of the
 // level below and above and T_sfc.
 constexpr int GO_IN_FIXED = 3;
@@ -491,9 +466,8 @@ __device__ __forceinline__ void stage_pair_inputs(const GasRef<Real>* sg, int ng
 }
 
 // Phase 1 for one pair (lane = column), in parts: the interpolation state of the major gathers
-// (ps_major), the minor scalings of slots q0, q0 + dq, ... (ps_minor), and the band Planck values
-// (LW) or the Rayleigh column (SW) (ps_aux).  pair_state_in runs them all; the fused forward
-// kernels share them out over their four wavefronts (pair_state_split).
+// (ps_major) and the minor scalings of slots q0, q0 + dq, ... (ps_minor); pair_state_split shares them
+// and the band Planck values (LW) or the Rayleigh column (SW) out over the four wavefronts.
 template<typename Real, typename In>
 __device__ __forceinline__ void ps_major(const Kd<Real>& k, const GoBand& bd, const CL<Real>& c, const In& in, Real cd,
                                          PairState<Real>& st)
@@ -537,38 +511,6 @@ __device__ __forceinline__ void ps_minor(const Kd<Real>& k, const GoBand& bd, in
         }
         st.scaling[q] = sc;
     }
-}
-
-template<typename Real, bool LW, typename In>
-__device__ __forceinline__ void ps_aux(const Kd<Real>& k, int ibnd, const In& in, Real tv, Real cd, bool at_sfc,
-                                       PairState<Real>& st)
-{
-    if constexpr (LW)
-    {
-        const Real* tab = k.totplnk + int64_t(ibnd) * k.nplanck;
-        st.aux[0] = interpolate1D(tv, k.temp_ref_min, k.totplnk_delta, k.nplanck, tab);
-        st.aux[1] = interpolate1D(in.t_hi(), k.temp_ref_min, k.totplnk_delta, k.nplanck, tab);
-        st.aux[2] = interpolate1D(in.t_lo(), k.temp_ref_min, k.totplnk_delta, k.nplanck, tab);
-        if (at_sfc)
-        {
-            const Real ts = in.t_sfc();
-            st.aux[3] = interpolate1D(ts, k.temp_ref_min, k.totplnk_delta, k.nplanck, tab);
-            st.aux[4] = interpolate1D(ts + Real(1), k.temp_ref_min, k.totplnk_delta, k.nplanck, tab);
-        }
-    }
-    else
-        st.aux[0] = in.col(k.idx_h2o, cd) + cd;
-}
-
-template<typename Real, bool LW, typename In>
-__device__ __forceinline__ void pair_state_in(const Kd<Real>& k, const GoBand& bd, int ibnd, const In& in,
-                                              bool at_sfc, PairState<Real>& st)
-{
-    const Real pv = in.p(), tv = in.t(), cd = in.cd();
-    const CL<Real> c = interp_cl(k, pv, tv);
-    ps_major(k, bd, c, in, cd, st);
-    ps_minor(k, bd, c.itropo, in, pv, tv, cd, 0, 1, st);
-    ps_aux<Real, LW>(k, ibnd, in, tv, cd, at_sfc, st);
 }
 
 // Band-independent state of a column, computed once per work-group by the fused kernels and kept
@@ -637,18 +579,8 @@ __device__ __forceinline__ void pair_state_split(const Kd<Real>& k, const GoBand
     else
     {
         ps_minor(k, bd, c.itropo, in, pv, tv, cd, w - 1, 3, st);
-        if (w == 1) ps_aux<Real, false>(k, ibnd, in, tv, cd, false, st);
+        if (w == 1) st.aux[0] = in.col(k.idx_h2o, cd) + cd;                          // Rayleigh column
     }
-}
-
-template<typename Real, bool LW>
-__device__ __forceinline__ void pair_state(const Kd<Real>& k, const GasRef<Real>* sg, const GoBand& bd, int ibnd,
-                                           int64_t icol, int64_t ilay, int64_t ncol, const Real* play,
-                                           const Real* tlay, const Real* tlev, const Real* tsfc,
-                                           const Real* col_dry_a, bool at_sfc, PairState<Real>& st)
-{
-    const PairInGlobal<Real> in{sg, icol, ilay, ncol, play, tlay, tlev, tsfc, col_dry_a};
-    pair_state_in<Real, LW>(k, bd, ibnd, in, at_sfc, st);
 }
 
 // Entries i..i+3 of a band-packed table (quads are 4-element aligned).  The table base is
@@ -1052,52 +984,102 @@ void gas_optics_sw_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t nlay,
 }
 
 // ---------------------------------------------------------------------------------------------
-// Gas-optics adjoint.  For one band, given the cotangents of the band's fused outputs, adds the
+// Gas-optics adjoint.  Given the cotangents of the fused outputs of the launch's bands, adds the
 // gradients with respect to the per-(column, layer) inputs: the column amounts col_gas
 // (gas 0 = dry air), T_lay, ln p_lay and, in the longwave, T_lev at the layer's two levels and
 // T_sfc.  Per g-point the outputs are linear in the table values with the pair's weights:
 //   tau_abs = sum_i col_mix_i sum_c fmajor_ic K_icg + sum_q scaling_q sum_ie fminor_ie Km_qieg
 //   pfrac   = sum_ic fmajor_ic P_icg,    tau_ray = col_ray sum_ie fminor_ie Kr_ieg,
-// so phase 2 accumulates, per pair, the gradients of those weights over the band's g-points
-// (one quad of g-points per lane, reduced over the pair's four lanes); phase 3 carries them
-// through the interpolation (ftemp, fpress, eta -> fmajor/fminor, col_mix), the minor scalings and
-// the Planck interpolation by hand.  The integer indices are piecewise constant.
+// so all the gradients of the weights follow from the dot products over the band's g-points of a
+// cotangent with each table node.  A work-group takes one
+// (64-column tile, layer) and runs the launch's bands in the forward kernels' phases: the inputs are
+// staged once; per band the pair states (phase 1, spread over the wavefronts), per 16-g-point chunk the
+// dot products (phase 2, lane = (pair, quad of g-points), one table node live at a time), and the chain
+// through the interpolation (ftemp, fpress, eta -> fmajor/fminor, col_mix), the minor scalings and the
+// Planck interpolation (phase 3, lane = column, the parts on different wavefronts, each adding into
+// gradient rows of its own in LDS).  Phase 3 of a band and phase 1 of the next share a barrier interval.
+// The rows are summed, in a fixed order, and added to memory once per launch.  The integer indices are
+// piecewise constant.
 
+// The cotangents a launch is given.
+enum GaMode
+{
+    GA_LW3,        // tau, lay_src, lev_src_inc, lev_src_dec, sfc_src
+    GA_LWF,        // tau, Planck fraction, sfc_src; band Planck values at the layer and its two levels
+    GA_SW3,        // tau, ssa, g after the optional band cloud add_to
+    GA_SW2         // absorption and Rayleigh optical depths
+};
+
+// Rows of s_acc: the cotangents of a pair's weights for one band.
 constexpr int GA_CM = 0, GA_FM = 2, GA_SC = 10, GA_FN = 18, GA_X = 22, GA_N = 26;
 
-// Derivative of interpolate1D with respect to val.
 template<typename Real>
-__device__ __forceinline__ Real interpolate1D_slope(Real val, Real offset, Real delta, int len, const Real* table)
+struct GaCot
 {
-    const Real val0 = (val - offset) / delta;
-    const int idx = min(len - 1, max(1, int(val0) + 1));
-    return (table[idx] - table[idx - 1]) / delta;
+    const Real *a, *b, *c, *d, *s;            // GaMode's g-point arrays (ncol, nlay, g-points), s (ncol, g-points)
+    const Real *blay, *blo, *bhi;             // GA_LWF: (ncol, nlay, 16-g-point groups), sums over the group
+    const Real *ctau, *cssa, *cg;             // GA_SW3: band cloud properties (ncol, nlay, nbnd) or NULL
+};
+
+template<typename Real>
+struct GaOut { Real *d_col, *d_tlay, *d_lnp, *d_tlev_lo, *d_tlev_hi, *d_tsfc; };
+
+// Sum over the four lanes of a pair (lanes 4p .. 4p+3 of a wavefront), on the DPP quad permutations.
+__device__ __forceinline__ float quad_perm(float v, int sel)
+{
+    const int i = __float_as_int(v);
+    return __int_as_float(sel == 1 ? __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, true)
+                                   : __builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double quad_perm(double v, int sel)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return sel == 1 ? __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, 0xB1, 0xF, 0xF, true),
+                                       __builtin_amdgcn_update_dpp(0, lo, 0xB1, 0xF, 0xF, true))
+                    : __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, 0x4E, 0xF, 0xF, true),
+                                       __builtin_amdgcn_update_dpp(0, lo, 0x4E, 0xF, 0xF, true));
+}
+template<typename Real>
+__device__ __forceinline__ Real quad_sum(Real v)
+{
+    v += quad_perm(v, 1);
+    return v + quad_perm(v, 2);
 }
 
-// Phase 3: the gradients of one pair's weights (acc) carried to the inputs.
-template<typename Real, bool LW>
-__device__ __forceinline__ void pair_state_backward(const Kd<Real>& k, const GasRef<Real>* sg, const GoBand& bd,
-                                                    int ibnd, int64_t icol, int64_t ilay, int64_t ncol, int64_t ncl,
-                                                    const Real* play, const Real* tlay, const Real* tlev,
-                                                    const Real* tsfc, const Real* col_dry_a, bool at_sfc,
-                                                    const Real* acc, Real* d_col, Real* d_tlay, Real* d_lnp,
-                                                    Real* d_tlev_lo, Real* d_tlev_hi, Real* d_tsfc)
+template<typename Real>
+__device__ __forceinline__ Real dot4(const Real (&a)[4], const Real (&b)[4])
 {
-    const int64_t idx = icol + ncol * ilay;
-    const Real pv = play[idx], tv = tlay[idx], cd = col_dry_a[idx];
-    const CL<Real> c = interp_cl(k, pv, tv);
-    const int s = c.itropo;
-    const int gas1 = bd.gas[s][0], gas2 = bd.gas[s][1];
-    const Real c1 = col_lds(sg, gas1, icol, ilay, cd), c2 = col_lds(sg, gas2, icol, ilay, cd);
-    auto dcol = [&](int gas, Real v) { d_col[idx + ncl * gas] += v; };
-    // g_dry: the derivative with respect to col_dry at fixed volume mixing ratios, times col_dry.
-    // Every column the gas optics reads is a vmr times col_dry, and each quantity formed from
-    // them is homogeneous in col_dry: col_mix, the minor scalings and col_ray of degree 1, eta and
-    // the scaling fraction X of degree 0.  So g_dry = sum over the degree-1 quantities of their
-    // cotangent times their value; the eta and X paths, whose per-gas terms cancel exactly in
-    // the sum over gases but not in rounded arithmetic, do not enter.
-    Real g_dry = Real(0);
-    Real g_ftemp = Real(0), g_fp = Real(0), g_c1 = Real(0), g_c2 = Real(0);
+    return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
+}
+
+// One wavefront's gradient rows of the 64 columns in LDS: the column amounts (0 = dry air, 1 .. ngas the
+// gases, ngas + 1 the derivative with respect to col_dry at fixed mixing ratios, times col_dry), then T, ln p.
+template<typename Real>
+struct GaRows
+{
+    Real* r;
+    int lane, ngas;
+    __device__ void col(int gas, Real v) const { r[gas * GO_COLS + lane] += v; }
+    __device__ void dry(Real v) const { r[(ngas + 1) * GO_COLS + lane] += v; }
+    __device__ void t(Real v) const { r[(ngas + 2) * GO_COLS + lane] += v; }
+    __device__ void lnp(Real v) const { r[(ngas + 3) * GO_COLS + lane] += v; }
+};
+
+inline __host__ __device__ constexpr int ga_rows(int ngas) { return ngas + 4; }
+
+// Phase 3, the major species: the cotangents of col_mix, fmajor and fminor carried to the two gases, T and
+// ln p.  The derivative at fixed mixing ratios: every column the gas optics reads is a vmr times col_dry,
+// and each quantity formed from them is homogeneous in col_dry: col_mix, the minor scalings and col_ray of
+// degree 1, eta and the scaling fraction X of degree 0.  So it is the sum over the degree-1 quantities of
+// their cotangent times their value; the eta and X paths, whose per-gas terms cancel exactly in the sum
+// over gases but not in rounded arithmetic, do not enter.
+template<typename Real, typename In>
+__device__ __forceinline__ void ga_major_back(const Kd<Real>& k, const GoBand& bd, const CL<Real>& c, const In& in,
+                                              Real cd, const Real* acc, const GaRows<Real>& out)
+{
+    const int s = c.itropo, gas1 = bd.gas[s][0], gas2 = bd.gas[s][1];
+    const Real c1 = in.col(gas1, cd), c2 = in.col(gas2, cd);
+    Real g_ftemp = Real(0), g_fp = Real(0), g_c1 = Real(0), g_c2 = Real(0), g_dry = Real(0);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
     {
@@ -1132,326 +1114,413 @@ __device__ __forceinline__ void pair_state_backward(const Kd<Real>& k, const Gas
             g_c2 -= g_eta * eta * r * icm;
         }
     }
-    dcol(gas1, g_c1);
-    dcol(gas2, g_c2);
-    Real g_t = g_ftemp / k.temp_ref_delta;
-    Real g_lnp = g_fp / k.press_ref_log_delta;
-    // Minor scalings (.cu:388-420): sc = col(gas) [P F], P = 0.01 p / T, F = X or 1 - X with
-    // X = col(scal) / (col_dry + col(h2o)).
+    out.col(gas1, g_c1);
+    out.col(gas2, g_c2);
+    out.dry(g_dry);
+    out.t(g_ftemp / k.temp_ref_delta);
+    out.lnp(g_fp / k.press_ref_log_delta);
+}
+
+// Phase 3, the minor scalings of slots q0, q0 + dq, ... (.cu:388-420): sc = col(gas) [P F], P = 0.01 p / T,
+// F = X or 1 - X with X = col(scal) / (col_dry + col(h2o)).
+template<typename Real, typename In>
+__device__ __forceinline__ void ga_minor_back(const Kd<Real>& k, const GoBand& bd, int s, const In& in, Real pv, Real tv,
+                                              Real cd, const Real* acc, int q0, int dq, const GaRows<Real>& out)
+{
     const int nq = bd.nq[s];
-    for (int q = 0; q < nq; ++q)
+    const Real P = Real(0.01) * pv / tv;
+    Real g_dry = Real(0), g_PP = Real(0);
+    for (int q = q0; q < nq; q += dq)
     {
         const GoMinor md = bd.minor[s][q];
         const Real g_sc = acc[GA_SC + q];
-        const Real base = col_lds(sg, md.gas, icol, ilay, cd);
+        const Real base = in.col(md.gas, cd);
         if (!md.dens)
         {
-            dcol(md.gas, g_sc);
+            out.col(md.gas, g_sc);
             g_dry += g_sc * base;
             continue;
         }
-        const Real P = Real(0.01) * pv / tv;
         Real F = Real(1), X = Real(0), den = Real(1);
         if (md.scal_gas > 0)
         {
-            den = cd + col_lds(sg, k.idx_h2o, icol, ilay, cd);
-            X = col_lds(sg, md.scal_gas, icol, ilay, cd) / den;
+            den = cd + in.col(k.idx_h2o, cd);
+            X = in.col(md.scal_gas, cd) / den;
             F = md.compl_ ? Real(1) - X : X;
         }
-        dcol(md.gas, g_sc * P * F);
-        g_dry += g_sc * base * P * F;
-        const Real g_P = g_sc * base * F;
-        g_lnp += g_P * P;
-        g_t -= g_P * P / tv;
+        out.col(md.gas, g_sc * P * F);
+        const Real v = g_sc * base * P * F;
+        g_dry += v;
+        g_PP += v;
         if (md.scal_gas > 0)
         {
             const Real g_X = (md.compl_ ? -g_sc : g_sc) * base * P;
-            dcol(md.scal_gas, g_X / den);
-            dcol(0, -g_X * X / den);
-            dcol(k.idx_h2o, -g_X * X / den);
+            out.col(md.scal_gas, g_X / den);
+            out.col(0, -g_X * X / den);
+            out.col(k.idx_h2o, -g_X * X / den);
         }
     }
-    if constexpr (LW)
-    {
-        const Real* tab = k.totplnk + int64_t(ibnd) * k.nplanck;
-        g_t += acc[GA_X + 0] * interpolate1D_slope(tv, k.temp_ref_min, k.totplnk_delta, k.nplanck, tab);
-        d_tlev_hi[idx] += acc[GA_X + 1] * interpolate1D_slope(tlev[icol + ncol * (ilay + 1)], k.temp_ref_min,
-                                                              k.totplnk_delta, k.nplanck, tab);
-        d_tlev_lo[idx] += acc[GA_X + 2] * interpolate1D_slope(tlev[idx], k.temp_ref_min, k.totplnk_delta,
-                                                              k.nplanck, tab);
-        if (at_sfc)
-            d_tsfc[icol] += acc[GA_X + 3] * interpolate1D_slope(tsfc[icol], k.temp_ref_min, k.totplnk_delta,
-                                                                k.nplanck, tab);
-    }
-    else
-    {
-        dcol(k.idx_h2o, acc[GA_X]);      // col_ray = col(h2o) + col_dry
-        dcol(0, acc[GA_X]);
-        g_dry += acc[GA_X] * (col_lds(sg, k.idx_h2o, icol, ilay, cd) + cd);
-    }
-    dcol(k.ngas + 1, g_dry / cd);
-    d_tlay[idx] += g_t;
-    d_lnp[idx] += g_lnp;
+    out.dry(g_dry);
+    out.t(-g_PP / tv);
+    out.lnp(g_PP);
 }
 
-// Sum over the four lanes of a pair (lanes 4p .. 4p+3 of a wavefront).
-__device__ __forceinline__ float quad_sum(float v)
+// Slope of a Planck table at a position of interp1d_pos.
+template<typename Real>
+__device__ __forceinline__ Real interp1d_slope(const Real* table, int idx, Real delta)
 {
-    v += __shfl_xor(v, 1);
-    return v + __shfl_xor(v, 2);
-}
-__device__ __forceinline__ double quad_sum(double v)
-{
-    v += __shfl_xor(v, 1);
-    return v + __shfl_xor(v, 2);
+    return (table[idx] - table[idx - 1]) / delta;
 }
 
-// One band; a work-group takes 64 columns of one layer and loops over the band's 16-g-point
-// chunks.  LW cotangents: ga (tau), gb (lay_src), gc (lev_src_inc), gd (lev_src_dec) of
-// (ncol, nlay, ngb) and gs (sfc_src, (ncol, ngb)); SW: ga (tau), gb (ssa), gc (g).
-template<typename Real, bool LW>
-__global__ __launch_bounds__(GO_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 3 : 1)))
-void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t nlay, int ibnd,
+template<typename Real, int MODE>
+constexpr int ga_arrays() { return MODE == GA_LW3 ? 4 : MODE == GA_SW3 ? 3 : 2; }
+
+// At 16384 columns x 128 layers in FP32 both spectral ranges take 14.5 ms (two shortwave and four longwave
+// bands a launch); with one band a launch, phases 1 and 3 on one wavefront reading and writing memory, and
+// every table node of a pair live at once they took 25.5 ms.
+template<typename Real, int MODE>
+__global__ __launch_bounds__(GO_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 4 : 2)))
+void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t nlay, GoGrid grid,
                                const Real* __restrict__ play, const Real* __restrict__ tlay,
                                const Real* __restrict__ tlev, const Real* __restrict__ tsfc,
-                               const Real* __restrict__ col_dry_a, int sfc_lay,
-                               const Real* __restrict__ ctau_a, const Real* __restrict__ cssa_a,
-                               const Real* __restrict__ cg_a,
-                               const Real* __restrict__ ga, const Real* __restrict__ gb,
-                               const Real* __restrict__ gc, const Real* __restrict__ gd,
-                               const Real* __restrict__ gs,
-                               Real* __restrict__ d_col, Real* __restrict__ d_tlay, Real* __restrict__ d_lnp,
-                               Real* __restrict__ d_tlev_lo, Real* __restrict__ d_tlev_hi, Real* __restrict__ d_tsfc)
+                               const Real* __restrict__ col_dry_a, int sfc_lay, GaCot<Real> ct, GaOut<Real> out)
 {
     static_assert(GO_GPTS == 16 && GO_THREADS == 4 * GO_COLS, "lane layout of phase 2");
+    constexpr bool LW = MODE == GA_LW3 || MODE == GA_LWF;
+    constexpr int NA = ga_arrays<Real, MODE>();
     __shared__ PairState<Real> sst[GO_COLS];
-    __shared__ Real s_g[5][GO_GPTS][GO_ROW];
+    __shared__ __align__(16) Real s_g[NA][GO_GPTS][GO_COLS];
     __shared__ Real s_acc[GO_COLS][GA_N + 1];
-    __shared__ Real s_cl[3][GO_COLS];
-    __shared__ Real s_sc[GO_MAXM][GO_THREADS];      // per lane: cotangent sums of the minor scalings
-    __shared__ GasRef<Real> sg[RRTMGP_MAX_GAS];
-    const int64_t ncoltiles = (ncol + GO_COLS - 1) / GO_COLS;
-    const int64_t u = xcd_remap(blockIdx.x, ncoltiles * nlay);
-    if (u >= ncoltiles * nlay) return;                     // uniform over the work-group
-    const int64_t ilay = u / ncoltiles, col0 = (u % ncoltiles) * GO_COLS;
-    const GoBand& bd = k.bands[ibnd];
-    const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int64_t ncl = ncol * nlay;
+    __shared__ ColState<Real, LW> s_cs;
+    __shared__ Real s_lev[LW ? 3 : 1][GO_COLS];              // LW: gradients of T_lev below, above, T_sfc
+    // The gas pointers are read by the input staging only: they share the cotangents' LDS.
+    static_assert(sizeof(GasRef<Real>) * RRTMGP_MAX_GAS <= sizeof(Real) * GO_GPTS * GO_COLS, "sg in s_g");
+    GasRef<Real>* const sg = reinterpret_cast<GasRef<Real>*>(&s_g[0][0][0]);
+    extern __shared__ __align__(16) unsigned char go_dyn[];
+    Real* const s_in = reinterpret_cast<Real*>(go_dyn);                        // input rows, then gradient rows
+    Real* const s_d = s_in + go_in_rows<LW>(k.ngas) * GO_COLS;
+    const int64_t u = xcd_remap(blockIdx.x, grid.ntl);
+    if (u >= grid.ntl) return;                               // uniform over the work-group
+    const GoTl tl = go_tl(grid, u);
+    if (!tl.ok) return;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const int64_t ilay = tl.ilay, ncl = ncol * nlay;
     const bool at_sfc = LW && (ilay == sfc_lay - 1);
 
     if (threadIdx.x == 0) stage_gases(g, k.ngas, sg);
+    for (int e = threadIdx.x; e < 4 * ga_rows(k.ngas) * GO_COLS; e += GO_THREADS) s_d[e] = Real(0);
+    if (LW && w < 3) s_lev[w][lane] = Real(0);
     __syncthreads();
-    if (w == 0)
-    {
-        const int64_t icol = col0 + lane;
-        if (icol < ncol)
-        {
-            pair_state<Real, LW>(k, sg, bd, ibnd, icol, ilay, ncol, play, tlay, tlev, tsfc, col_dry_a, at_sfc,
-                                 sst[lane]);
-            if (!LW)
-            {
-                const int64_t ib = icol + ncol * ilay + ncl * ibnd;
-                s_cl[0][lane] = ctau_a ? ctau_a[ib] : Real(0);
-                s_cl[1][lane] = ctau_a ? cssa_a[ib] : Real(0);
-                s_cl[2][lane] = ctau_a ? cg_a[ib] : Real(0);
-            }
-        }
-        else
-            sst[lane].flags = 0;
-    }
+    stage_pair_inputs<Real, LW>(sg, k.ngas, tl.col0, ilay, ncol, nlay, play, tlay, tlev, tsfc, col_dry_a, s_in);
+    __syncthreads();
+    col_state<Real, LW>(k, PairInLds<Real>{s_in, lane, k.ngas}, w, lane, s_cs);
+    __syncthreads();
 
-    const int pi = w * 16 + lane / 4;                  // pair of phase 2
-    const int gq = 4 * (lane % 4);                     // first g-point of the lane's quad in a chunk
-    Real acc[GA_N];
-#pragma unroll
-    for (int a = 0; a < GA_N; ++a) acc[a] = Real(0);
-#pragma unroll
-    for (int q = 0; q < GO_MAXM; ++q) s_sc[q][threadIdx.x] = Real(0);
-    const Real eps2 = Real(2 * prop_eps);
-    const Real op_eps = Real(3) * Limits<Real>::tiny;
-
-    for (int c0 = 0; c0 < bd.ng; c0 += GO_GPTS)
-    {
-        const int ncg = min(bd.ng - c0, GO_GPTS);
-        __syncthreads();                               // previous chunk's LDS reads are done
-        {
-            const int64_t icol = col0 + lane;
-            for (int row = w; row < ncg; row += GO_THREADS / 64)
-            {
-                Real v0 = Real(0), v1 = Real(0), v2 = Real(0), v3 = Real(0), v4 = Real(0);
-                if (icol < ncol)
-                {
-                    const int64_t o = icol + ncol * ilay + ncl * (c0 + row);
-                    v0 = ga[o]; v1 = gb[o]; v2 = gc[o];
-                    if (LW)
-                    {
-                        v3 = gd[o];
-                        if (at_sfc) v4 = gs[icol + ncol * (c0 + row)];
-                    }
-                }
-                s_g[0][row][lane] = v0; s_g[1][row][lane] = v1; s_g[2][row][lane] = v2;
-                s_g[3][row][lane] = v3; s_g[4][row][lane] = v4;
-            }
-        }
-        __syncthreads();
-        const PairState<Real>& st = sst[pi];
-        if (!((st.flags & 1) && gq < ncg)) continue;
-        const uint32_t gl = uint32_t(c0 + gq);
-        const uint32_t gp = bd.gp, sE = uint32_t(k.npres + 1) * gp, sP = gp;
-        const uint32_t kb = uint32_t(bd.koff) + gl;
-        Real K[2][4][4];
+    Real fm[2][4], cm[2], fn[2][2], x[4];                    // the lane's sums of the band's weight cotangents
+    auto clear = [&] {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
         {
-            const uint32_t o = kb + uint32_t(st.om[i]);
-            load4(k.kmajor_p, o, K[i][0]); load4(k.kmajor_p, o + sE, K[i][1]);
-            load4(k.kmajor_p, o + sP, K[i][2]); load4(k.kmajor_p, o + sP + sE, K[i][3]);
-        }
-        // Forward values per g-point that the cotangents need.
-        Real gabs[4], gray[4];
-        Real kr[2][2][4];
-        if (!LW)
-        {
-            const uint32_t rb = uint32_t(bd.roff) + gl;
-            load4(k.krayl_p, rb + uint32_t(st.ry[0]), kr[0][0]); load4(k.krayl_p, rb + uint32_t(st.ry[0]) + gp, kr[0][1]);
-            load4(k.krayl_p, rb + uint32_t(st.ry[1]), kr[1][0]); load4(k.krayl_p, rb + uint32_t(st.ry[1]) + gp, kr[1][1]);
-            Real tabs[4];
-            absorption4(k, bd, st, gl, tabs);
-            const Real t2 = s_cl[0][pi], s2 = s_cl[1][pi], g2 = s_cl[2][pi];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int c = 0; c < 4; ++c) fm[i][c] = Real(0);
+            cm[i] = Real(0);
+            fn[i][0] = Real(0); fn[i][1] = Real(0); x[2 * i] = Real(0); x[2 * i + 1] = Real(0);
+        }
+    };
+    clear();
+    int back = -1;                                           // band whose phase 3 is due
+    int group = 0;                                           // its first g-point group
+    const int nchunk = grid.nbnd * int(grid.cpb);
+    for (int cb = 0; cb <= nchunk; ++cb)
+    {
+        const int ibnd = grid.b0 + cb / int(grid.cpb);
+        const int c0 = GO_GPTS * (cb % int(grid.cpb));
+        const int ncg = cb < nchunk ? min(k.bands[ibnd].ng - c0, GO_GPTS) : 0;
+        if (cb < nchunk && ncg <= 0) continue;               // uniform: an empty chunk of a short band
+        // The lane index is made anew in every iteration: the many LDS and memory addresses formed from it
+        // would otherwise be hoisted out of the loop and spill (47 registers of the longwave kernel).
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int64_t icol = tl.col0 + ln, idx = icol + ncol * ilay;
+        const bool valid = icol < ncol;
+        const PairInLds<Real> in{s_in, ln, k.ngas};
+        const int pi = w * 16 + ln / 4;                      // pair of phase 2
+        const int gq = 4 * (ln % 4);                         // first g-point of the lane's quad in a chunk
+
+        if (back >= 0)                                       // phase 3 of the band just finished
+        {
+            const GoBand& bd = k.bands[back];
+            const GaRows<Real> rows{s_d + w * ga_rows(k.ngas) * GO_COLS, ln, k.ngas};
+            const Real pv = in.p(), tv = in.t(), cd = in.cd();
+            const CL<Real> c{s_cs.ci[0][ln], s_cs.ci[1][ln], s_cs.ci[2][ln], s_cs.cf[0][ln], s_cs.cf[1][ln]};
+            const Real* acc = s_acc[ln];
+            if (w == 0) ga_major_back(k, bd, c, in, cd, acc, rows);
+            else if (w == 1) ga_minor_back(k, bd, c.itropo, in, pv, tv, cd, acc, 0, 2, rows);
+            else if (w == 3) ga_minor_back(k, bd, c.itropo, in, pv, tv, cd, acc, 1, 2, rows);
+            else if constexpr (LW)
             {
-                const Real tray = (st.fminor[0][0] * kr[0][0][e] + st.fminor[0][1] * kr[0][1][e] +
-                                   st.fminor[1][0] * kr[1][0][e] + st.fminor[1][1] * kr[1][1][e]) * st.aux[0];
-                const Real tt = tabs[e] + tray;
-                const Real ss = (tt > eps2) ? tray / tt : Real(0);
-                const Real tau12 = tt + t2;
-                const Real tauscat = tt * ss + t2 * s2;
-                const Real gout = (t2 * s2 * g2) / max(tauscat, op_eps);
-                const Real ssa = tauscat / max(op_eps, tau12);
-                const Real gto = s_g[0][gq + e][pi], gwo = s_g[1][gq + e][pi], ggo = s_g[2][gq + e][pi];
-                const Real g_ts = (tau12 > op_eps ? gwo / tau12 : Real(0)) -
-                                  (tauscat > op_eps ? ggo * gout / tauscat : Real(0));
-                const Real g_t12 = gto - (tau12 > op_eps ? gwo * ssa / tau12 : Real(0));
-                gabs[e] = g_t12;
-                gray[e] = g_t12 + (tt > eps2 ? g_ts : Real(0));
-            }
-        }
-        else
-        {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { gabs[e] = s_g[0][gq + e][pi]; gray[e] = Real(0); }
-        }
-        // Major terms.
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-        {
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-            {
-                Real sk = Real(0);
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
+                const Real* tab = k.totplnk + int64_t(back) * k.nplanck;
+                Real xl = acc[GA_X], xh = acc[GA_X + 1], xo = acc[GA_X + 2];
+                if constexpr (MODE == GA_LWF)
                 {
-                    sk += st.fmajor[i][c] * K[i][c][e];
-                    acc[GA_FM + 4 * i + c] += gabs[e] * st.col_mix[i] * K[i][c][e];
-                }
-                acc[GA_CM + i] += gabs[e] * sk;
-            }
-            if (!LW)
-            {
-                Real sr = Real(0);
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int c = 0; c < 2; ++c)
+                    xl = Real(0); xh = Real(0); xo = Real(0);
+                    for (int q = 0; q < bd.ng; q += GO_GPTS)
                     {
-                        sr += st.fminor[i][c] * kr[i][c][e];
-                        acc[GA_FN + 2 * i + c] += gray[e] * st.aux[0] * kr[i][c][e];
+                        const int64_t ob = idx + ncl * (group + q / GO_GPTS);
+                        if (!valid) break;
+                        xl += ct.blay[ob]; xh += ct.bhi[ob]; xo += ct.blo[ob];
                     }
-                acc[GA_X] += gray[e] * sr;
+                }
+                rows.t(xl * interp1d_slope(tab, s_cs.ci[3][ln], k.totplnk_delta));
+                s_lev[1][ln] += xh * interp1d_slope(tab, s_cs.ci[4][ln], k.totplnk_delta);
+                s_lev[0][ln] += xo * interp1d_slope(tab, s_cs.ci[5][ln], k.totplnk_delta);
+                if (at_sfc)
+                {
+                    int is;
+                    Real fs;
+                    interp1d_pos(in.t_sfc(), k.temp_ref_min, k.totplnk_delta, k.nplanck, is, fs);
+                    s_lev[2][ln] += acc[GA_X + 3] * interp1d_slope(tab, is, k.totplnk_delta);
+                }
             }
+            else
+            {
+                const Real xr = acc[GA_X], ray = in.col(k.idx_h2o, cd) + cd;
+                rows.col(k.idx_h2o, xr);                     // col_ray = col(h2o) + col_dry
+                rows.col(0, xr);
+                rows.dry(xr * ray);
+            }
+            group += (bd.ng + GO_GPTS - 1) / GO_GPTS;
+            back = -1;
+            clear();                                         // here: the sums need no registers in phase 3
         }
-        // Planck-fraction terms (LW), after the major table values are dead: the two table slabs
-        // are never live together.
-        if constexpr (LW)
+        if (cb == nchunk) break;
+
+        const GoBand& bd = k.bands[ibnd];
+        const int gbase = bd.g0 - k.bands[grid.b0].g0 + c0;
+        if (c0 == 0)                                         // phase 1; padding columns repeat the last one
+            pair_state_split<Real, LW>(k, bd, ibnd, in, s_cs, ln, at_sfc, sst[ln], w);
+        // The chunk's cotangents; zero for padding columns and rows.
         {
-            __builtin_amdgcn_sched_barrier(0);
-            Real P[2][4][4];
+            const Real* const src[4] = {ct.a, ct.b, ct.c, ct.d};
+#pragma unroll
+            for (int a = 0; a < NA; ++a)
+#pragma unroll
+                for (int r4 = 0; r4 < GO_GPTS / 4; ++r4)
+                {
+                    const int row = w + 4 * r4;
+                    s_g[a][row][go_swz(row, ln)] = (valid && row < ncg) ? src[a][idx + ncl * (gbase + row)] : Real(0);
+                }
+        }
+        __syncthreads();
+
+        // Phase 2.  Lanes past the chunk's g-points run on its first quad with zero cotangents, so the
+        // lanes of a pair stay together.
+        {
+            const PairState<Real>& st = sst[pi];
+            const bool on = gq < ncg;
+            const uint32_t gl = uint32_t(c0 + (on ? gq : 0));
+            const uint32_t gp = bd.gp, sE = uint32_t(k.npres + 1) * gp, sP = gp;
+            auto cot = [&](int a, int e) { return s_g[a][gq + e][go_swz(gq + e, pi)]; };
+            Real gabs[4], gray[4];
+            if constexpr (MODE == GA_SW3)
+            {
+                // Back through the combine rule and the cloud add_to, from the forward optical depths.
+                const Real eps2 = Real(2 * prop_eps), op_eps = Real(3) * Limits<Real>::tiny;
+                Real tabs[4], tr[4];
+                absorption4(k, bd, st, gl, tabs);
+                rayleigh4(k, bd, st, gl, tr);
+                Real t2 = Real(0), s2 = Real(0), g2 = Real(0);
+                if (ct.ctau && tl.col0 + pi < ncol)
+                {
+                    const int64_t ib = tl.col0 + pi + ncol * ilay + ncl * ibnd;
+                    t2 = ct.ctau[ib]; s2 = ct.cssa[ib]; g2 = ct.cg[ib];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const Real tt = tabs[e] + tr[e];
+                    const Real ss = (tt > eps2) ? tr[e] / tt : Real(0);
+                    const Real tau12 = tt + t2;
+                    const Real tauscat = tt * ss + t2 * s2;
+                    const Real gout = (t2 * s2 * g2) / max(tauscat, op_eps);
+                    const Real ssa = tauscat / max(op_eps, tau12);
+                    const Real gto = cot(0, e), gwo = cot(1, e), ggo = cot(2, e);
+                    const Real g_ts = (tau12 > op_eps ? gwo / tau12 : Real(0)) -
+                                      (tauscat > op_eps ? ggo * gout / tauscat : Real(0));
+                    gabs[e] = gto - (tau12 > op_eps ? gwo * ssa / tau12 : Real(0));
+                    gray[e] = gabs[e] + (tt > eps2 ? g_ts : Real(0));
+                }
+            }
+            else
+            {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { gabs[e] = cot(0, e); gray[e] = MODE == GA_SW2 ? cot(1, e) : Real(0); }
+            }
+            // Major absorption.
+            const uint32_t kb = uint32_t(bd.koff) + gl;
 #pragma unroll
             for (int i = 0; i < 2; ++i)
             {
                 const uint32_t o = kb + uint32_t(st.om[i]);
-                load4(k.planck_frac_p, o, P[i][0]); load4(k.planck_frac_p, o + sE, P[i][1]);
-                load4(k.planck_frac_p, o + sP, P[i][2]); load4(k.planck_frac_p, o + sP + sE, P[i][3]);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-            {
-                Real pf = Real(0);
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) pf += st.fmajor[i][c] * P[i][c][e];
-                const Real gl_ = s_g[1][gq + e][pi], gi_ = s_g[2][gq + e][pi], gd_ = s_g[3][gq + e][pi];
-                const Real gs_ = at_sfc ? s_g[4][gq + e][pi] : Real(0);
-                const Real gpf = gl_ * st.aux[0] + gi_ * st.aux[1] + gd_ * st.aux[2] +
-                                 (at_sfc ? gs_ * st.aux[3] : Real(0));
-                acc[GA_X + 0] += gl_ * pf; acc[GA_X + 1] += gi_ * pf;
-                acc[GA_X + 2] += gd_ * pf; acc[GA_X + 3] += gs_ * pf;
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[GA_FM + 4 * i + c] += gpf * P[i][c][e];
+                Real n0[4], n1[4], n2[4], n3[4];
+                load4(k.kmajor_p, o, n0); load4(k.kmajor_p, o + sE, n1);
+                load4(k.kmajor_p, o + sP, n2); load4(k.kmajor_p, o + sP + sE, n3);
+                const Real d0 = dot4(gabs, n0), d1 = dot4(gabs, n1), d2 = dot4(gabs, n2), d3 = dot4(gabs, n3);
+                cm[i] += st.fmajor[i][0] * d0 + st.fmajor[i][1] * d1 + st.fmajor[i][2] * d2 + st.fmajor[i][3] * d3;
+                const Real mix = st.col_mix[i];
+                fm[i][0] += mix * d0; fm[i][1] += mix * d1; fm[i][2] += mix * d2; fm[i][3] += mix * d3;
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        // Minor terms, one slot at a time (a rolled loop keeps one slot's table values live); the
-        // slot's scaling cotangent goes to the lane's LDS slot.
-        const int nslot = bd.nslot;
-        const uint32_t sQ = uint32_t(nslot) * gp;
-        const uint32_t mb = uint32_t(bd.moff) + gl;
-#pragma unroll 1
-        for (int q = 0; q < nslot; ++q)
-        {
-            Real km[2][2][4];
-            const uint32_t o0 = mb + uint32_t(st.mn[0]) + uint32_t(q) * gp;
-            const uint32_t o1 = mb + uint32_t(st.mn[1]) + uint32_t(q) * gp;
-            load4(k.kminor_p, o0, km[0][0]); load4(k.kminor_p, o0 + sQ, km[0][1]);
-            load4(k.kminor_p, o1, km[1][0]); load4(k.kminor_p, o1 + sQ, km[1][1]);
-            const Real scq = st.scaling[q];
-            Real tq = Real(0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
+            if constexpr (LW)
             {
-                Real sm = Real(0);
+                // Planck fractions: their cotangent, and (GA_LW3) the band Planck values'.
+                Real gpf[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    gpf[e] = MODE == GA_LWF ? cot(1, e)
+                                            : cot(1, e) * st.aux[0] + cot(2, e) * st.aux[1] + cot(3, e) * st.aux[2];
+                auto node = [&](int i, int c, Real (&n)[4]) {
+                    load4(k.planck_frac_p, kb + uint32_t(st.om[i]) + (c & 1 ? sE : 0u) + (c & 2 ? sP : 0u), n);
+                };
+                if (at_sfc)
+                {
+                    // The surface source of the lowest layer (one layer of the launch: rolled loops).
+                    Real gs[4], xs = Real(0);
+                    const int64_t sc = tl.col0 + pi;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                    {
+                        gs[e] = (sc < ncol && gq + e < ncg) ? ct.s[sc + ncol * (gbase + gq + e)] : Real(0);
+                        gpf[e] += gs[e] * st.aux[3];
+                    }
+#pragma unroll 1
+                    for (int ic = 0; ic < 8; ++ic)
+                    {
+                        Real n[4];
+                        node(ic >> 2, ic & 3, n);
+                        xs += st.fmajor[ic >> 2][ic & 3] * dot4(gs, n);
+                    }
+                    x[3] += xs;
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                    {
+                        Real n[4];
+                        node(i, c, n);
+                        fm[i][c] += dot4(gpf, n);
+                        if constexpr (MODE == GA_LW3)
+                        {
+#pragma unroll
+                            for (int q = 0; q < 3; ++q)
+                            {
+                                const Real gb[4] = {cot(q + 1, 0), cot(q + 1, 1), cot(q + 1, 2), cot(q + 1, 3)};
+                                x[q] += st.fmajor[i][c] * dot4(gb, n);
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            else
+            {
+                const uint32_t rb = uint32_t(bd.roff) + gl;
+                const Real ray = st.aux[0];
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int c = 0; c < 2; ++c)
                     {
-                        sm += st.fminor[i][c] * km[i][c][e];
-                        acc[GA_FN + 2 * i + c] += gabs[e] * scq * km[i][c][e];
+                        Real n[4];
+                        load4(k.krayl_p, rb + uint32_t(st.ry[i]) + (c ? gp : 0u), n);
+                        const Real d = dot4(gray, n);
+                        x[0] += st.fminor[i][c] * d;
+                        fn[i][c] += ray * d;
                     }
-                tq += gabs[e] * sm;
             }
-            s_sc[q][threadIdx.x] += tq;
-        }
-    }
-    // Sum over the pair's four lanes; the first lane of each pair stores the pair's totals.
+            __builtin_amdgcn_sched_barrier(0);
+            // Minor absorption, one slot at a time; the first lane of the pair keeps the slot's sum.
+            const int nslot = bd.nslot;
+            const uint32_t sQ = uint32_t(nslot) * gp;
+            const uint32_t mb = uint32_t(bd.moff) + gl;
+#pragma unroll 1
+            for (int q = 0; q < nslot; ++q)
+            {
+                Real n0[4], n1[4], n2[4], n3[4];
+                const uint32_t o0 = mb + uint32_t(st.mn[0]) + uint32_t(q) * gp;
+                const uint32_t o1 = mb + uint32_t(st.mn[1]) + uint32_t(q) * gp;
+                load4(k.kminor_p, o0, n0); load4(k.kminor_p, o0 + sQ, n1);
+                load4(k.kminor_p, o1, n2); load4(k.kminor_p, o1 + sQ, n3);
+                const Real d0 = dot4(gabs, n0), d1 = dot4(gabs, n1), d2 = dot4(gabs, n2), d3 = dot4(gabs, n3);
+                const Real sc = st.scaling[q];
+                fn[0][0] += sc * d0; fn[0][1] += sc * d1; fn[1][0] += sc * d2; fn[1][1] += sc * d3;
+                const Real tq = quad_sum(st.fminor[0][0] * d0 + st.fminor[0][1] * d1 + st.fminor[1][0] * d2 +
+                                         st.fminor[1][1] * d3);
+                if (ln % 4 == 0) s_acc[pi][GA_SC + q] = c0 == 0 ? tq : s_acc[pi][GA_SC + q] + tq;
+            }
+            if (c0 + GO_GPTS >= bd.ng)
+            {
+                // The band's last chunk: the pair's totals.
 #pragma unroll
-    for (int a = 0; a < GA_N; ++a)
-    {
-        const Real v = quad_sum(a >= GA_SC && a < GA_SC + GO_MAXM ? s_sc[a - GA_SC][threadIdx.x] : acc[a]);
-        if (lane % 4 == 0) s_acc[pi][a] = v;
+                for (int i = 0; i < 2; ++i)
+                {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                    {
+                        const Real f = quad_sum(fm[i][c]);
+                        if (ln % 4 == 0) s_acc[pi][GA_FM + 4 * i + c] = f;
+                    }
+                    const Real m = quad_sum(cm[i]);
+                    const Real f0 = quad_sum(fn[i][0]), f1 = quad_sum(fn[i][1]);
+                    if (ln % 4 == 0)
+                    {
+                        s_acc[pi][GA_CM + i] = m;
+                        s_acc[pi][GA_FN + 2 * i] = f0;
+                        s_acc[pi][GA_FN + 2 * i + 1] = f1;
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                {
+                    if (!LW && q > 0) break;
+                    const Real v = quad_sum(x[q]);
+                    if (ln % 4 == 0) s_acc[pi][GA_X + q] = v;
+                }
+                back = ibnd;
+            }
+        }
+        __syncthreads();
     }
     __syncthreads();
-    if (w == 0)
+
+    // The wavefronts' rows summed and added to memory.
+    const int64_t icol = tl.col0 + lane, idx = icol + ncol * ilay;
+    const Real cd = s_in[2 * GO_COLS + lane];
+    const int nr = ga_rows(k.ngas);
+    auto total = [&](int r) {
+        Real v = Real(0);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v += s_d[(p * nr + r) * GO_COLS + lane];
+        return v;
+    };
+    if (icol >= ncol) return;
+    for (int r = w; r < k.ngas + 2; r += 4)
     {
-        const int64_t icol = col0 + lane;
-        if (icol < ncol)
-            pair_state_backward<Real, LW>(k, sg, bd, ibnd, icol, ilay, ncol, ncl, play, tlay, tlev, tsfc, col_dry_a,
-                                          at_sfc, s_acc[lane], d_col, d_tlay, d_lnp, d_tlev_lo, d_tlev_hi, d_tsfc);
+        const Real v = total(r);
+        out.d_col[idx + ncl * r] += r == k.ngas + 1 ? v / cd : v;
+    }
+    if (w == 0) out.d_tlay[idx] += total(k.ngas + 2);
+    else if (w == 1) out.d_lnp[idx] += total(k.ngas + 3);
+    if constexpr (LW)
+    {
+        if (w == 2)
+        {
+            out.d_tlev_lo[idx] += s_lev[0][lane];
+            out.d_tlev_hi[idx] += s_lev[1][lane];
+        }
+        else if (w == 3 && at_sfc) out.d_tsfc[icol] += s_lev[2][lane];
     }
 }
 
@@ -1949,37 +2018,32 @@ int gas_optics_sw(const rrtmgp_kdist_dev* kd, int64_t b0, int64_t nb, int64_t nc
     return RRTMGP_OK;
 }
 
-template<typename Real>
-int gas_optics_adjoint(const rrtmgp_kdist_dev* kd, bool lw, int64_t band, int64_t ncol, int64_t nlay,
+template<typename Real, int MODE>
+int gas_optics_adjoint(const rrtmgp_kdist_dev* kd, int64_t b0, int64_t nb, int64_t ncol, int64_t nlay,
                        const Real* play, const Real* tlay, const Real* tlev, const Real* tsfc, const Real* col_dry,
-                       const rrtmgp_gas_vmr* gases, int sfc_lay, const Real* ctau, const Real* cssa, const Real* cg,
-                       const Real* ga, const Real* gb, const Real* gc, const Real* gd, const Real* gs, Real* d_col,
-                       Real* d_tlay, Real* d_lnp, Real* d_tlev_lo, Real* d_tlev_hi, Real* d_tsfc, void* stream)
+                       const rrtmgp_gas_vmr* gases, int sfc_lay, const GaCot<Real>& ct, const GaOut<Real>& out,
+                       void* stream)
 {
-    RRTMGP_TRY(check_kd_fused(kd, lw));
+    constexpr bool LW = MODE == GA_LW3 || MODE == GA_LWF;
+    RRTMGP_TRY(check_kd_fused(kd, LW));
     if (ncol <= 0 || nlay <= 0) return arg_error("gas_optics_adjoint: ncol and nlay must be positive");
-    if (band < 0 || band >= kd->nbnd) return arg_error("gas_optics_adjoint: band outside the k-distribution");
-    if (!play || !tlay || !col_dry || !ga || !gb || !gc || !d_col || !d_tlay || !d_lnp)
+    if (b0 < 0 || nb < 1 || b0 + nb > kd->nbnd) return arg_error("gas_optics_adjoint: band outside the k-distribution");
+    if (!play || !tlay || !col_dry || !ct.a || !ct.b || !out.d_col || !out.d_tlay || !out.d_lnp ||
+        ((MODE == GA_LW3 || MODE == GA_SW3) && !ct.c))
         return arg_error("gas_optics_adjoint: NULL array");
-    if (lw && (!tlev || !tsfc || !gd || !gs || !d_tlev_lo || !d_tlev_hi || !d_tsfc || (sfc_lay != 1 && sfc_lay != nlay)))
+    if (LW && (!tlev || !tsfc || !ct.s || !out.d_tlev_lo || !out.d_tlev_hi || !out.d_tsfc ||
+               (MODE == GA_LW3 ? !ct.d : (!ct.blay || !ct.blo || !ct.bhi)) || (sfc_lay != 1 && sfc_lay != nlay)))
         return arg_error("gas_optics_adjoint: longwave arrays missing or sfc_lay not 1 or nlay");
-    if (!lw && ctau && (!cssa || !cg)) return arg_error("gas_optics_adjoint: cloud ssa/g missing");
+    if (MODE == GA_SW3 && ct.ctau && (!ct.cssa || !ct.cg)) return arg_error("gas_optics_adjoint: cloud ssa/g missing");
     Gases<Real> g;
     RRTMGP_TRY(make_gases(gases, kd->ngas, ncol, nlay, g));
     const Kd<Real> k = make_kd<Real>(*kd);
-    const int64_t nunits = ((ncol + GO_COLS - 1) / GO_COLS) * nlay;
-    if (nunits >= (int64_t(1) << 31)) return arg_error("gas_optics_adjoint: too many column tiles x layers");
+    const GoGrid grid = make_go_grid(ncol, nlay, b0, nb, kd->max_band_gpts);
+    if (grid.ntl >= (int64_t(1) << 31)) return arg_error("gas_optics_adjoint: too many column tiles x layers");
+    const size_t dyn = size_t(go_in_rows<LW>(kd->ngas) + 4 * ga_rows(kd->ngas)) * GO_COLS * sizeof(Real);
     RRTMGP_TIMED("gas_optics_adjoint_kernel", as_stream(stream));
-    if (lw)
-        hipLaunchKernelGGL((gas_optics_adjoint_kernel<Real, true>), dim3(xcd_grid(nunits)), dim3(GO_THREADS), 0,
-                           as_stream(stream), k, g, ncol, nlay, int(band), play, tlay, tlev, tsfc, col_dry, sfc_lay,
-                           nullptr, nullptr, nullptr, ga, gb, gc, gd, gs, d_col, d_tlay, d_lnp, d_tlev_lo,
-                           d_tlev_hi, d_tsfc);
-    else
-        hipLaunchKernelGGL((gas_optics_adjoint_kernel<Real, false>), dim3(xcd_grid(nunits)), dim3(GO_THREADS), 0,
-                           as_stream(stream), k, g, ncol, nlay, int(band), play, tlay, nullptr, nullptr, col_dry, 1,
-                           ctau, cssa, cg, ga, gb, gc, nullptr, nullptr, d_col, d_tlay, d_lnp, nullptr, nullptr,
-                           nullptr);
+    hipLaunchKernelGGL((gas_optics_adjoint_kernel<Real, MODE>), dim3(xcd_grid(grid.ntl)), dim3(GO_THREADS), dyn,
+                       as_stream(stream), k, g, ncol, nlay, grid, play, tlay, tlev, tsfc, col_dry, sfc_lay, ct, out);
     RRTMGP_LAUNCHED("gas_optics_adjoint_kernel");
     return RRTMGP_OK;
 }
@@ -2208,20 +2272,63 @@ extern "C" int rrtmgp_hip_gas_optics_lw_adjoint_##S(const rrtmgp_kdist_dev* kd, 
     const T* g_lev_src_inc, const T* g_lev_src_dec, const T* g_sfc_src, T* d_col_gas, T* d_tlay,     \
     T* d_lnp_lay, T* d_tlev_lo, T* d_tlev_hi, T* d_tsfc, void* stream)                               \
 {                                                                                                    \
-    return gas_optics_adjoint<T>(kd, true, band, ncol, nlay, play, tlay, tlev, tsfc, col_dry, gases, \
-                                 sfc_lay, nullptr, nullptr, nullptr, g_tau, g_lay_src, g_lev_src_inc,\
-                                 g_lev_src_dec, g_sfc_src, d_col_gas, d_tlay, d_lnp_lay, d_tlev_lo,  \
-                                 d_tlev_hi, d_tsfc, stream);                                         \
+    GaCot<T> ct{};                                                                                   \
+    ct.a = g_tau; ct.b = g_lay_src; ct.c = g_lev_src_inc; ct.d = g_lev_src_dec; ct.s = g_sfc_src;    \
+    return gas_optics_adjoint<T, GA_LW3>(kd, band, 1, ncol, nlay, play, tlay, tlev, tsfc, col_dry,   \
+                                         gases, sfc_lay, ct,                                         \
+                                         {d_col_gas, d_tlay, d_lnp_lay, d_tlev_lo, d_tlev_hi, d_tsfc}, \
+                                         stream);                                                    \
 }                                                                                                    \
 extern "C" int rrtmgp_hip_gas_optics_sw_adjoint_##S(const rrtmgp_kdist_dev* kd, int64_t band,       \
     int64_t ncol, int64_t nlay, const T* play, const T* tlay, const T* col_dry,                      \
     const rrtmgp_gas_vmr* gases, const T* cloud_tau, const T* cloud_ssa, const T* cloud_g,           \
     const T* g_tau, const T* g_ssa, const T* g_g, T* d_col_gas, T* d_tlay, T* d_lnp_lay, void* stream)\
 {                                                                                                    \
-    return gas_optics_adjoint<T>(kd, false, band, ncol, nlay, play, tlay, nullptr, nullptr, col_dry, \
-                                 gases, 1, cloud_tau, cloud_ssa, cloud_g, g_tau, g_ssa, g_g, nullptr, \
-                                 nullptr, d_col_gas, d_tlay, d_lnp_lay, nullptr, nullptr, nullptr,   \
-                                 stream);                                                            \
+    GaCot<T> ct{};                                                                                   \
+    ct.a = g_tau; ct.b = g_ssa; ct.c = g_g; ct.ctau = cloud_tau; ct.cssa = cloud_ssa; ct.cg = cloud_g; \
+    return gas_optics_adjoint<T, GA_SW3>(kd, band, 1, ncol, nlay, play, tlay, nullptr, nullptr,      \
+                                         col_dry, gases, 1, ct,                                      \
+                                         {d_col_gas, d_tlay, d_lnp_lay, nullptr, nullptr, nullptr},  \
+                                         stream);                                                    \
+}                                                                                                    \
+extern "C" int rrtmgp_hip_gas_optics_lw_bands_factored_##S(const rrtmgp_kdist_dev* kd,              \
+    int64_t band_start, int64_t band_count, int64_t ncol, int64_t nlay, const T* play,               \
+    const T* tlay, const T* tlev, const T* tsfc, const T* col_dry, const rrtmgp_gas_vmr* gases,      \
+    int sfc_lay, const T* cloud_tau, T* tau, T* planck_frac, T* band_lay_src, T* band_lev_src,       \
+    T* sfc_src, T* sfc_src_jac, void* stream)                                                        \
+{                                                                                                    \
+    if (!band_lay_src || !band_lev_src)                                                              \
+        return arg_error("gas_optics_lw_bands_factored: NULL band array");                           \
+    return gas_optics_lw<T>(kd, band_start, band_count, ncol, nlay, play, tlay, tlev, tsfc, col_dry, \
+                            gases, sfc_lay, cloud_tau, tau, planck_frac, nullptr, nullptr, sfc_src,  \
+                            sfc_src_jac, stream, nullptr, 0, band_lay_src, band_lev_src);            \
+}                                                                                                    \
+extern "C" int rrtmgp_hip_gas_optics_lw_adjoint_bands_##S(const rrtmgp_kdist_dev* kd,               \
+    int64_t band_start, int64_t band_count, int64_t ncol, int64_t nlay, const T* play,               \
+    const T* tlay, const T* tlev, const T* tsfc, const T* col_dry, const rrtmgp_gas_vmr* gases,      \
+    int sfc_lay, const T* g_tau, const T* g_planck_frac, const T* g_lay_src, const T* g_lev_src_lo,  \
+    const T* g_lev_src_hi, const T* g_sfc_src, T* d_col_gas, T* d_tlay, T* d_lnp_lay, T* d_tlev_lo,  \
+    T* d_tlev_hi, T* d_tsfc, void* stream)                                                           \
+{                                                                                                    \
+    GaCot<T> ct{};                                                                                   \
+    ct.a = g_tau; ct.b = g_planck_frac; ct.s = g_sfc_src;                                            \
+    ct.blay = g_lay_src; ct.blo = g_lev_src_lo; ct.bhi = g_lev_src_hi;                               \
+    return gas_optics_adjoint<T, GA_LWF>(kd, band_start, band_count, ncol, nlay, play, tlay, tlev,   \
+                                         tsfc, col_dry, gases, sfc_lay, ct,                          \
+                                         {d_col_gas, d_tlay, d_lnp_lay, d_tlev_lo, d_tlev_hi, d_tsfc}, \
+                                         stream);                                                    \
+}                                                                                                    \
+extern "C" int rrtmgp_hip_gas_optics_sw_adjoint_bands_##S(const rrtmgp_kdist_dev* kd,               \
+    int64_t band_start, int64_t band_count, int64_t ncol, int64_t nlay, const T* play,               \
+    const T* tlay, const T* col_dry, const rrtmgp_gas_vmr* gases, const T* g_tau_abs,                \
+    const T* g_tau_ray, T* d_col_gas, T* d_tlay, T* d_lnp_lay, void* stream)                         \
+{                                                                                                    \
+    GaCot<T> ct{};                                                                                   \
+    ct.a = g_tau_abs; ct.b = g_tau_ray;                                                              \
+    return gas_optics_adjoint<T, GA_SW2>(kd, band_start, band_count, ncol, nlay, play, tlay, nullptr, \
+                                         nullptr, col_dry, gases, 1, ct,                             \
+                                         {d_col_gas, d_tlay, d_lnp_lay, nullptr, nullptr, nullptr},  \
+                                         stream);                                                    \
 }                                                                                                    \
 extern "C" int rrtmgp_hip_get_col_dry_adjoint_##S(int64_t ncol, int64_t nlay, const T* vmr_h2o,     \
     int64_t h2o_dim1, int64_t h2o_dim2, const T* plev, const T* g_col_dry, T* d_vmr_h2o, T* d_plev,  \

@@ -35,6 +35,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "solver_groups.h"
 #include "solver_math.h"
 
 namespace rrtmgp_hip
@@ -288,6 +289,207 @@ int lw_adjoint(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t n
     return rc;
 }
 // ---------------------------------------------------------------------------------------------
+// The longwave adjoint on factored sources: each source is a Planck fraction (per g-point) times the band's
+// Planck function at the layer or a level (lw_solver_kernel's FACT form), one Gaussian angle.  Read and
+// written per g-point are tau, the fraction and their cotangents (24 values of traffic a layer became 8); the
+// cotangents of the band Planck functions are summed over the work-group's g-points (one band's) in LDS every
+// K layers, in a fixed order, into (ncol, nlay, groups).  Layers and recurrences as in lw_adjoint_kernel.
+template<typename Real> struct AdjFactSeg;
+template<> struct AdjFactSeg<float> { static constexpr int K = 4; };    // 48 KiB of LDS: two work-groups a CU
+template<> struct AdjFactSeg<double> { static constexpr int K = 2; };
+
+template<typename Real>
+struct LwAdjFactArgs
+{
+    int64_t ncol, nlay, ngpt, emis_nbnd;
+    int top_at_1;
+    Real D, fac;                                       // secant; 2 pi times the weight
+    const Real *tau, *pf, *blay, *blev, *emis, *sfc_src, *a_up, *a_dn;
+    Real *ckpt, *d_tau, *d_pf, *d_blay, *d_blo, *d_bhi, *d_sfc_src, *d_emis;
+};
+
+template<typename Real>
+__global__ __launch_bounds__(SB_COLS * SB_GPTS) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 8 : 4)))
+void lw_adjoint_factored_kernel(LwAdjFactArgs<Real> a, Groups grp)
+{
+    constexpr int K = AdjFactSeg<Real>::K;
+    __shared__ Real red[3][K][SB_GPTS][SB_COLS];
+    const int lane = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.y));
+    const int gi = blockIdx.y, gcount = grp.count[gi];
+    const int64_t ncol = a.ncol, n = a.nlay, col0 = int64_t(blockIdx.x) * SB_COLS, icol = col0 + lane;
+    const int64_t igpt = grp.start[gi] + w;
+    const bool active = icol < ncol && w < gcount;
+    const int64_t nseg = (n + K - 1) / K;
+    const int64_t c2 = icol + ncol * igpt, lslab = ncol * n * igpt;
+    const Real* tau_g = a.tau + lslab;
+    const Real* pf_g = a.pf + lslab;
+    Real* dtau_g = a.d_tau + lslab;
+    Real* dpf_g = a.d_pf + lslab;
+    const Real* blay_g = a.blay + ncol * n * grp.band[gi];
+    const Real* blev_g = a.blev + ncol * (n + 1) * grp.band[gi];
+    Real* ck_g = a.ckpt + ncol * nseg * 2 * igpt;
+    const uint32_t ucol = uint32_t(icol), uncol = uint32_t(ncol);
+    auto lay_of = [&](int64_t j) -> uint32_t { return uint32_t(a.top_at_1 ? j : n - 1 - j); };   // layer j from the top
+    auto lev_of = [&](int64_t j) -> uint32_t { return uint32_t(a.top_at_1 ? j : n - j); };       // level j from the top
+    auto ck = [&](int64_t s, int q) -> Real& { return st32(ck_g, ucol + uncol * uint32_t(s * 2 + q)); };
+    const Real D = a.D, fac = a.fac;
+
+    Real Id = Real(0), Lu = Real(0);
+    if (active)
+    {
+        // Down: forward I^d and the adjoint lu; checkpoints at the top of each segment.
+        Lu = fac * ld32(a.a_up, ucol + uncol * lev_of(0));
+        for (int64_t s = 0; s < nseg; ++s)
+        {
+            const int64_t j0 = s * K;
+            const int nk = int(std::min<int64_t>(K, n - j0));
+            ck(s, 0) = Id; ck(s, 1) = Lu;
+            Real tv[K], pv[K], bl[K], bd[K], au[K];
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk)
+                if (kk < nk)
+                {
+                    const uint32_t l = ucol + uncol * lay_of(j0 + kk);
+                    tv[kk] = ld32(tau_g, l); pv[kk] = ld32(pf_g, l); bl[kk] = ld32(blay_g, l);
+                    bd[kk] = ld32(blev_g, ucol + uncol * lev_of(j0 + kk + 1));
+                    au[kk] = ld32(a.a_up, ucol + uncol * lev_of(j0 + kk + 1));
+                }
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk)
+                if (kk < nk)
+                {
+                    Real T, f, df;
+                    lw_layer_d(tv[kk] * D, T, f, df);
+                    Id = T * Id + pv[kk] * ((Real(1) - T) * bd[kk] + Real(2) * f * (bl[kk] - bd[kk]));
+                    Lu = fac * au[kk] + T * Lu;
+                }
+        }
+    }
+    // Surface.
+    Real Iu = Real(0), Ld = Real(0);
+    if (active)
+    {
+        const Real e = a.emis[grp.band[gi] + a.emis_nbnd * icol], bs = a.sfc_src[c2];
+        Iu = (Real(1) - e) * Id + e * bs;
+        a.d_emis[c2] = Lu * (bs - Id);
+        a.d_sfc_src[c2] = e * Lu;
+        Ld = fac * ld32(a.a_dn, ucol + uncol * lev_of(n)) + (Real(1) - e) * Lu;
+    }
+    // Up: forward I^u and the adjoint ld, replaying I^d and lu per segment.
+    for (int64_t s = nseg - 1; s >= 0; --s)
+    {
+        const int64_t j0 = s * K;
+        const int nk = int(std::min<int64_t>(K, n - j0));
+        Real gbl[K], gbd[K], gbu[K];
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) { gbl[kk] = Real(0); gbd[kk] = Real(0); gbu[kk] = Real(0); }
+        if (active)
+        {
+            Real tv[K], pv[K], bl[K], bv[K + 1], au[K], adv[K], sId[K], sLu[K];
+            bv[0] = ld32(blev_g, ucol + uncol * lev_of(j0));
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk)
+                if (kk < nk)
+                {
+                    const uint32_t l = ucol + uncol * lay_of(j0 + kk);
+                    tv[kk] = ld32(tau_g, l); pv[kk] = ld32(pf_g, l); bl[kk] = ld32(blay_g, l);
+                    bv[kk + 1] = ld32(blev_g, ucol + uncol * lev_of(j0 + kk + 1));
+                    au[kk] = ld32(a.a_up, ucol + uncol * lev_of(j0 + kk + 1));
+                    adv[kk] = ld32(a.a_dn, ucol + uncol * lev_of(j0 + kk));
+                }
+            {
+                Real id = ck(s, 0), lu = ck(s, 1);
+#pragma unroll
+                for (int kk = 0; kk < K; ++kk)
+                    if (kk < nk)
+                    {
+                        Real T, f, df;
+                        lw_layer_d(tv[kk] * D, T, f, df);
+                        sId[kk] = id; sLu[kk] = lu;
+                        id = T * id + pv[kk] * ((Real(1) - T) * bv[kk + 1] + Real(2) * f * (bl[kk] - bv[kk + 1]));
+                        lu = fac * au[kk] + T * lu;
+                    }
+            }
+#pragma unroll
+            for (int kk = K - 1; kk >= 0; --kk)
+                if (kk < nk)
+                {
+                    Real T, f, df;
+                    lw_layer_d(tv[kk] * D, T, f, df);
+                    const Real p = pv[kk], Bl = bl[kk], Bu = bv[kk], Bd = bv[kk + 1];
+                    const Real gSu = sLu[kk], gSd = Ld;
+                    const Real gT = sLu[kk] * Iu + Ld * sId[kk] - p * (Bd * gSd + Bu * gSu);
+                    const Real gf = Real(2) * p * ((Bl - Bd) * gSd + (Bl - Bu) * gSu);
+                    const Real c = (Real(1) - T) - Real(2) * f, f2 = Real(2) * f;
+                    // dL/dp and, times p, dL/dB.
+                    const uint32_t l = ucol + uncol * lay_of(j0 + kk);
+                    st32(dtau_g, l) = D * (-T * gT + df * gf);
+                    st32(dpf_g, l) = gSd * (c * Bd + f2 * Bl) + gSu * (c * Bu + f2 * Bl);
+                    gbl[kk] = p * f2 * (gSd + gSu);
+                    gbd[kk] = p * c * gSd;
+                    gbu[kk] = p * c * gSu;
+                    Iu = T * Iu + p * ((Real(1) - T) * Bu + f2 * (Bl - Bu));
+                    Ld = fac * adv[kk] + T * Ld;
+                }
+        }
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk)
+        {
+            red[0][kk][w][lane] = gbl[kk]; red[1][kk][w][lane] = gbd[kk]; red[2][kk][w][lane] = gbu[kk];
+        }
+        __syncthreads();
+        // Row r of the 3 K rows: component r / K at layer j0 + r % K.
+        for (int r = w; r < 3 * K; r += SB_GPTS)
+        {
+            const int c = r / K, kk = r % K;
+            if (kk >= nk || icol >= ncol) continue;
+            Real v = red[c][kk][0][lane];
+            for (int q = 1; q < gcount; ++q) v += red[c][kk][q][lane];
+            // The lower source (c = 1) is at level L + 1 with the top at layer 1, else at level L.
+            Real* out = c == 0 ? a.d_blay : ((c == 1) == (a.top_at_1 != 0) ? a.d_bhi : a.d_blo);
+            out[icol + ncol * (int64_t(lay_of(j0 + kk)) + n * gi)] = v;
+        }
+        __syncthreads();
+    }
+}
+
+template<typename Real>
+int lw_adjoint_factored(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, double secant, double weight,
+                        const Real* tau, const Real* pf, const Real* blay, const Real* blev, int64_t nbnd,
+                        const int* band_lims, const Real* emis, int64_t emis_nbnd, const Real* sfc_src,
+                        const Real* a_up, const Real* a_dn, Real* d_tau, Real* d_pf, Real* d_blay, Real* d_blo,
+                        Real* d_bhi, Real* d_sfc_src, Real* d_emis, void* stream)
+{
+    if (ncol <= 0 || nlay <= 0 || ngpt <= 0 || nbnd <= 0) return arg_error("lw_adjoint_factored: empty extents");
+    if (!tau || !pf || !blay || !blev || !band_lims || !emis || emis_nbnd < nbnd || !sfc_src || !a_up || !a_dn ||
+        !d_tau || !d_pf || !d_blay || !d_blo || !d_bhi || !d_sfc_src || !d_emis)
+        return arg_error("lw_adjoint_factored: NULL array");
+    constexpr int K = AdjFactSeg<Real>::K;
+    const int64_t nseg = (nlay + K - 1) / K;
+    if (ncol * std::max<int64_t>(nlay + 1, 2 * nseg) * int64_t(sizeof(Real)) >= (int64_t(1) << 32))
+        return arg_error("lw_adjoint_factored: ncol * (nlay + 1) values of one g-point must stay below 4 GiB");
+    Groups grp;
+    RRTMGP_TRY(make_groups(ngpt, nbnd, band_lims, grp));
+    hipStream_t s = as_stream(stream);
+    Real* ck = nullptr;
+    RRTMGP_TRY(scratch_alloc(&ck, size_t(nseg * 2 * ngpt * ncol), s));
+    const Real pi = Real(3.14159265358979323846);
+    const LwAdjFactArgs<Real> args{ncol, nlay, ngpt, emis_nbnd, top_at_1, Real(secant), Real(2) * pi * Real(weight),
+                                   tau, pf, blay, blev, emis, sfc_src, a_up, a_dn, ck, d_tau, d_pf, d_blay, d_blo,
+                                   d_bhi, d_sfc_src, d_emis};
+    int rc;
+    {
+        RRTMGP_TIMED("lw_adjoint_factored_kernel", s);
+        hipLaunchKernelGGL(lw_adjoint_factored_kernel<Real>, dim3(grid1(ncol, SB_COLS), unsigned(grp.n)),
+                           dim3(SB_COLS, SB_GPTS), 0, s, args, grp);
+        rc = check_hip(hipGetLastError(), "lw_adjoint_factored_kernel");
+    }
+    scratch_free(ck, s);
+    return rc;
+}
+
+// ---------------------------------------------------------------------------------------------
 // Shortwave adjoint: one (column, g-point) per thread, 64 columns x 4 g-points per work-group.
 constexpr int SWA_GPTS = 4;
 constexpr int SWA_NS = 4;    // stored level states: R_up, D, E, dir
@@ -492,11 +694,16 @@ void sw_adjoint_down_kernel(SwAdjArgs<Real> a)
 }
 
 // Sweep up: the column below each level, the fluxes and multipliers of the level, the layer's gradients.
+// With CHAIN the cotangents of tau, ssa and g are carried on to the gases' absorption and Rayleigh optical
+// depths (d_tau and d_ssa receive those; the band cloud is held fixed): with the scattering optical depth
+// ts = ssa tau, tau = abs + ray + cloud and g a cloud quantity over ts,
+//     d_abs = d_tau - d_ssa ssa / tau,   d_ray = d_abs + d_ssa / tau - d_g g / ts,
+// and d_ray = d_abs where the combine rule sets ssa = 0 (tau <= 2 eps).
 // Bound by its FP64 arithmetic (153 VGPRs, 3 wavefronts per SIMD) next to 10 values of traffic a layer.
 // The pair of sweeps takes 3.4 + 5.4 ms for the 14 bands of 16384 columns x 128 layers in FP32; the four
 // it replaced (two forward and two reverse recursions through 12 stored states a level, the layer
 // Jacobian on forward-mode dual numbers) took 22.9 ms.
-template<typename Real>
+template<typename Real, bool CHAIN>
 __global__ __launch_bounds__(ADJ_COLS * SWA_GPTS)
 void sw_adjoint_up_kernel(SwAdjArgs<Real> a)
 {
@@ -547,7 +754,18 @@ void sw_adjoint_up_kernel(SwAdjArgs<Real> a)
         const double dn = (D + Ru * S) * den, mu = (E + Ru * F) * den;
         double gt, gw, gg;
         L.reverse(tau, m0, im0, lam * up + mu * dn, lam * dn + mu * up, mu * dir, lam * dir, ldir * dir, gt, gw, gg);
-        a.d_tau[lo] = Real(gt); a.d_ssa[lo] = Real(gw); a.d_g[lo] = Real(gg);
+        if constexpr (CHAIN)
+        {
+            const double op_eps = 3. * double(Limits<Real>::tiny), ts = w0 * tau;
+            const double it = tau > op_eps ? rcp_full(tau) : 0.;
+            const double da = gt - gw * w0 * it;
+            const double dr = tau > 2. * prop_eps ? gw * it - (ts > op_eps ? gg * g * rcp_full(ts) : 0.) : 0.;
+            a.d_tau[lo] = Real(da); a.d_ssa[lo] = Real(da + dr);
+        }
+        else
+        {
+            a.d_tau[lo] = Real(gt); a.d_ssa[lo] = Real(gw); a.d_g[lo] = Real(gg);
+        }
         ldir = cd + cr + mu * L.Rd + lam * L.Td + ldir * L.Tn;
         up = A * dn + S;
         lam = A * mu + F;
@@ -559,11 +777,11 @@ template<typename Real>
 int sw_adjoint(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real* tau, const Real* ssa,
                const Real* g, const Real* mu0, const Real* alb_dir, const Real* alb_dif, const Real* inc_dir,
                const Real* inc_dif, const Real* a_up, const Real* a_dn, const Real* a_dir, Real* d_tau,
-               Real* d_ssa, Real* d_g, Real* d_alb_dir, Real* d_alb_dif, void* stream)
+               Real* d_ssa, Real* d_g, Real* d_alb_dir, Real* d_alb_dif, void* stream, bool chain = false)
 {
     if (ncol <= 0 || nlay <= 0 || ngpt <= 0) return arg_error("sw_adjoint: empty extents");
     if (!tau || !ssa || !g || !mu0 || !alb_dir || !alb_dif || !inc_dir || !a_up || !a_dn || !a_dir || !d_tau ||
-        !d_ssa || !d_g || !d_alb_dir || !d_alb_dif)
+        !d_ssa || (!chain && !d_g) || !d_alb_dir || !d_alb_dif)
         return arg_error("sw_adjoint: NULL array");
     hipStream_t s = as_stream(stream);
     Real* st = nullptr;
@@ -581,7 +799,8 @@ int sw_adjoint(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Rea
     if (rc == RRTMGP_OK)
     {
         RRTMGP_TIMED("sw_adjoint_up_kernel", s);
-        hipLaunchKernelGGL(sw_adjoint_up_kernel<Real>, grid, block, 0, s, args);
+        auto kernel = chain ? sw_adjoint_up_kernel<Real, true> : sw_adjoint_up_kernel<Real, false>;
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, args);
         rc = check_hip(hipGetLastError(), "sw_adjoint_up_kernel");
     }
     scratch_free(st, s);
@@ -666,6 +885,34 @@ extern "C" int rrtmgp_hip_sw_solver_2stream_adjoint_##S(int64_t ncol, int64_t nl
 
 RRTMGP_DEF_ADJOINT(f32, float)
 RRTMGP_DEF_ADJOINT(f64, double)
+
+#define RRTMGP_DEF_ADJOINT_BANDS(S, T)                                                             \
+extern "C" int rrtmgp_hip_lw_adjoint_factored_##S(int64_t ncol, int64_t nlay, int64_t ngpt,        \
+    int top_at_1, double secant, double weight, const T* tau, const T* planck_frac,                 \
+    const T* band_lay_src, const T* band_lev_src, int64_t nbnd, const int* band_lims_gpt,           \
+    const T* sfc_emis, int64_t emis_nbnd, const T* sfc_src, const T* bb_up_cot,                     \
+    const T* bb_dn_cot, T* d_tau, T* d_planck_frac, T* d_lay_src, T* d_lev_src_lo, T* d_lev_src_hi, \
+    T* d_sfc_src, T* d_sfc_emis, void* stream)                                                      \
+{                                                                                                   \
+    return lw_adjoint_factored<T>(ncol, nlay, ngpt, top_at_1, secant, weight, tau, planck_frac,     \
+                                  band_lay_src, band_lev_src, nbnd, band_lims_gpt, sfc_emis,        \
+                                  emis_nbnd, sfc_src, bb_up_cot, bb_dn_cot, d_tau, d_planck_frac,   \
+                                  d_lay_src, d_lev_src_lo, d_lev_src_hi, d_sfc_src, d_sfc_emis,     \
+                                  stream);                                                          \
+}                                                                                                   \
+extern "C" int rrtmgp_hip_sw_adjoint_gases_##S(int64_t ncol, int64_t nlay, int64_t ngpt,           \
+    int top_at_1, const T* tau, const T* ssa, const T* g, const T* mu0, const T* sfc_alb_dir,       \
+    const T* sfc_alb_dif, const T* inc_flux_dir, const T* inc_flux_dif, const T* bb_up_cot,         \
+    const T* bb_dn_cot, const T* bb_dir_cot, T* d_tau_abs, T* d_tau_ray, T* d_sfc_alb_dir,           \
+    T* d_sfc_alb_dif, void* stream)                                                                 \
+{                                                                                                   \
+    return sw_adjoint<T>(ncol, nlay, ngpt, top_at_1, tau, ssa, g, mu0, sfc_alb_dir, sfc_alb_dif,    \
+                         inc_flux_dir, inc_flux_dif, bb_up_cot, bb_dn_cot, bb_dir_cot, d_tau_abs,   \
+                         d_tau_ray, nullptr, d_sfc_alb_dir, d_sfc_alb_dif, stream, true);           \
+}
+
+RRTMGP_DEF_ADJOINT_BANDS(f32, float)
+RRTMGP_DEF_ADJOINT_BANDS(f64, double)
 
 #define RRTMGP_DEF_ADJ_HELPERS(S, T)                                                               \
 extern "C" int rrtmgp_hip_adjoint_col_chain_##S(int64_t ncol, int64_t nlay,                        \

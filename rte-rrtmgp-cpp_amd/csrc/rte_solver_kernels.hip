@@ -38,15 +38,12 @@
 #include <vector>
 
 #include "common.h"
+#include "solver_groups.h"
 #include "solver_math.h"
 #include "two_stream.h"
 
 namespace rrtmgp_hip
 {
-constexpr int SB_COLS = 64;     // columns per work-group: the lanes of each wavefront
-constexpr int SB_GPTS = 16;     // g-points per work-group: one wavefront each, within one band
-constexpr int MAX_GROUPS = 256;
-
 // Segment lengths: levels per LDS reduction round (LW, SW) and the SW checkpoint spacing.  The
 // LW segment inputs are double-buffered in registers (K1 for one angle, K4 for up to four), sized
 // for 64 VGPRs in FP32 (two 1024-thread work-groups per CU) without spills; the SW segment
@@ -58,48 +55,6 @@ template<> struct LwSeg<double> { static constexpr int K1 = 4, K4 = 4; };
 // K = 3, so two 1024-thread work-groups share a CU; the others keep K = 4 at up to 128 VGPRs.
 constexpr bool sw_wide(bool fp32, bool co, bool hr) { return fp32 && co && !hr; }
 constexpr int sw_seg_k(bool fp32, bool co, bool hr) { return sw_wide(fp32, co, hr) ? 3 : 4; }
-
-// G-point groups: consecutive g-points of one band, at most SB_GPTS each.
-struct Groups
-{
-    int n;
-    int start[MAX_GROUPS];
-    int count[MAX_GROUPS];
-    int band[MAX_GROUPS];
-};
-
-// Groups from band limits (2, nbnd), 1-based inclusive; without band limits the g-points are cut
-// into consecutive chunks (enough for broadband sums).
-int make_groups(int64_t ngpt, int64_t nbnd, const int* band_lims, Groups& g)
-{
-    g.n = 0;
-    auto add = [&](int s, int e, int b) {
-        for (int x = s; x < e; x += SB_GPTS)
-        {
-            if (g.n == MAX_GROUPS) return false;
-            g.start[g.n] = x;
-            g.count[g.n] = std::min(SB_GPTS, e - x);
-            g.band[g.n] = b;
-            ++g.n;
-        }
-        return true;
-    };
-    if (band_lims)
-    {
-        int expect = 1;
-        for (int64_t b = 0; b < nbnd; ++b)
-        {
-            const int s = band_lims[2 * b], e = band_lims[2 * b + 1];
-            if (s != expect || e < s || e > ngpt) return arg_error("solver: band limits do not tile the g-points");
-            if (!add(s - 1, e, int(b))) return arg_error("solver: too many g-point groups");
-            expect = e + 1;
-        }
-        if (expect != ngpt + 1) return arg_error("solver: band limits do not cover all g-points");
-    }
-    else if (!add(0, int(ngpt), 0))
-        return arg_error("solver: too many g-point groups");
-    return RRTMGP_OK;
-}
 
 // Writes the LDS slots kk < nslots, components c < NC, summed over the group's g-points, to
 // out[c] at level lev_of(kk) (skipped when negative).

@@ -2,6 +2,7 @@
 // sequence they differentiate is src_test/Radiation_solver.cu:489-580 LW and :763-893 SW).
 #include "Radiation_adjoint.h"
 
+#include <algorithm>
 #include <stdexcept>
 #include <vector>
 
@@ -37,12 +38,40 @@ Array_gpu<Float,2> expand(const Gas_optics_rrtmgp_gpu& kd, const Array_gpu<Float
     return out;
 }
 
-// Largest number of g-points in one band.
-int max_band_gpts(const Gas_optics_rrtmgp_gpu& kd)
+// Bands processed together: consecutive bands whose per-g-point scratch (`arrays` values per column, layer
+// and g-point) stays below 2.25 GiB, at least one.  One launch per kernel then covers them: at a few
+// thousand columns and fewer a single band's work-groups leave most of the GPU idle (250 x 60 columns and
+// layers: 4 tiles x 16 g-points), at 16384 x 128 in FP32 two shortwave and four longwave bands share the
+// staging of the gas-optics inputs, with the peak scratch of one band's former 12-state store.
+struct Batch
 {
+    int b0, nb, g0, ng;              // bands, first g-point (0-based), g-points
+    std::vector<int> lims;           // (2, nb) band limits, 1-based within the batch
+};
+
+std::vector<Batch> make_batches(const Gas_optics_rrtmgp_gpu& kd, int64_t ncl, double arrays)
+{
+    const double most = 2.25 * 1024. * 1024. * 1024. / (arrays * double(sizeof(Float)) * double(ncl));
     const Array<int,2>& bl = kd.get_band_lims_gpoint();
+    std::vector<Batch> out;
+    for (int b = 0; b < kd.get_nband(); ++b)
+    {
+        const int s = bl({1, b + 1}), e = bl({2, b + 1});
+        if (out.empty() || double(out.back().ng + e - s + 1) > most) out.push_back({b, 0, s - 1, 0, {}});
+        Batch& t = out.back();
+        t.lims.push_back(s - t.g0);
+        t.lims.push_back(e - t.g0);
+        ++t.nb;
+        t.ng += e - s + 1;
+    }
+    return out;
+}
+
+template<typename F>
+int most_of(const std::vector<Batch>& v, F f)
+{
     int m = 0;
-    for (int b = 1; b <= kd.get_nband(); ++b) m = std::max(m, bl({2, b}) - bl({1, b}) + 1);
+    for (const Batch& t : v) m = std::max(m, f(t));
     return m;
 }
 
@@ -80,8 +109,9 @@ void lw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
     const rrtmgp_kdist_dev& kd = kdist.device_tables();
     rrtmgp_gas_vmr vmr;
     kdist.vmr_descriptor(gas_concs, ncol, nlay, vmr);
-    const Bool top_at_1 = p_lay({1, 1}) < p_lay({1, nlay});
-    const int sfc_lay = p_lay({1, 1}) > p_lay({1, nlay}) ? 1 : nlay;
+    const Float p_first = p_lay({1, 1}), p_last = p_lay({1, nlay});
+    const Bool top_at_1 = p_first < p_last;
+    const int sfc_lay = p_first > p_last ? 1 : nlay;
 
     ensure<2>(out.d_t_lay, {ncol, nlay}); ensure<2>(out.d_t_lev, {ncol, nlev}); ensure<1>(out.d_t_sfc, {ncol});
     ensure<2>(out.d_lnp_lay, {ncol, nlay}); ensure<2>(out.d_p_lev, {ncol, nlev});
@@ -97,39 +127,38 @@ void lw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
         cloud_optics->cloud_optics(lwp, iwp, rel, rei, *cl);
     }
 
-    // One Gaussian angle, as the forward driver (src_test/Radiation_solver.cpp:533): D = 1.66, w = 0.5.
-    Array_gpu<Float,2> emis_gpt = expand(kdist, emis_sfc, ncol);
-    Array<Float,2> sec_h({ncol, ngpt});
-    for (auto& x : sec_h.v()) x = Float(1.66);
-    Array_gpu<Float,2> secants(sec_h);
-    Array<Float,1> w_h({1});
-    w_h({1}) = Float(0.5);
-    Array_gpu<Float,1> weights(w_h);
-
     Array_gpu<Float,3> d_col({ncol, nlay, ngas + 2});
     Array_gpu<Float,2> d_lo({ncol, nlay}), d_hi({ncol, nlay}), d_col_dry({ncol, nlay}), d_emis_gpt({ncol, ngpt});
     zero(d_col); zero(d_lo); zero(d_hi); zero(out.d_t_lay); zero(out.d_t_sfc); zero(out.d_lnp_lay); zero(out.d_p_lev);
 
-    const int mb = max_band_gpts(kdist);
-    Array_gpu<Float,3> tau({ncol, nlay, mb}), lay({ncol, nlay, mb}), linc({ncol, nlay, mb}), ldec({ncol, nlay, mb});
-    Array_gpu<Float,3> dtau({ncol, nlay, mb}), dlay({ncol, nlay, mb}), dlinc({ncol, nlay, mb}), dldec({ncol, nlay, mb});
-    Array_gpu<Float,2> sfc({ncol, mb}), sfcj({ncol, mb}), dsfc({ncol, mb});
-    const Array<int,2>& bl = kdist.get_band_lims_gpoint();
-    for (int b = 0; b < nbnd; ++b)
+    // Factored sources, as the forward driver: per g-point only tau, the Planck fractions and their cotangents.
+    const std::vector<Batch> batches = make_batches(kdist, ncl, 4.5);
+    const int mg = most_of(batches, [](const Batch& t) { return t.ng; });
+    const int mb = most_of(batches, [](const Batch& t) { return t.nb; });
+    const int mq = most_of(batches, [](const Batch& t) {
+        int n = 0;
+        for (int i = 0; i < t.nb; ++i) n += (t.lims[2 * i + 1] - t.lims[2 * i] + 16) / 16;   // groups of 16 g-points
+        return n;
+    });
+    Array_gpu<Float,3> tau({ncol, nlay, mg}), pf({ncol, nlay, mg}), dtau({ncol, nlay, mg}), dpf({ncol, nlay, mg});
+    Array_gpu<Float,3> blay({ncol, nlay, mb}), blev({ncol, nlev, mb});
+    Array_gpu<Float,3> dblay({ncol, nlay, mq}), dblo({ncol, nlay, mq}), dbhi({ncol, nlay, mq});
+    Array_gpu<Float,2> sfc({ncol, mg}), sfcj({ncol, mg}), dsfc({ncol, mg});
+    const Float* ctau = cl ? cl->get_tau().ptr() : nullptr;
+    for (const Batch& t : batches)
     {
-        const int g0 = bl({1, b + 1}) - 1, ngb = bl({2, b + 1}) - g0;
-        hip_check(K<Float>::gas_optics_lw_bands(&kd, b, 1, ncol, nlay, p_lay.ptr(), t_lay.ptr(), t_lev.ptr(),
-                                                t_sfc.ptr(), col_dry.ptr(), &vmr, sfc_lay,
-                                                cl ? cl->get_tau().ptr() : nullptr, tau.ptr(), lay.ptr(),
-                                                linc.ptr(), ldec.ptr(), sfc.ptr(), sfcj.ptr(), stream()));
-        hip_check(K<Float>::lw_solver_noscat_adjoint(
-                ncol, nlay, ngb, top_at_1, 1, secants.ptr() + int64_t(ncol) * g0, weights.ptr(), tau.ptr(),
-                lay.ptr(), linc.ptr(), ldec.ptr(), emis_gpt.ptr() + int64_t(ncol) * g0, sfc.ptr(), nullptr,
-                g_flux_up.ptr(), g_flux_dn.ptr(), dtau.ptr(), dlay.ptr(), dlinc.ptr(), dldec.ptr(), dsfc.ptr(),
-                d_emis_gpt.ptr() + int64_t(ncol) * g0, stream()));
-        hip_check(K<Float>::gas_optics_lw_adjoint(
-                &kd, b, ncol, nlay, p_lay.ptr(), t_lay.ptr(), t_lev.ptr(), t_sfc.ptr(), col_dry.ptr(), &vmr,
-                sfc_lay, dtau.ptr(), dlay.ptr(), dlinc.ptr(), dldec.ptr(), dsfc.ptr(), d_col.ptr(),
+        hip_check(K<Float>::gas_optics_lw_bands_factored(
+                &kd, t.b0, t.nb, ncol, nlay, p_lay.ptr(), t_lay.ptr(), t_lev.ptr(), t_sfc.ptr(), col_dry.ptr(), &vmr,
+                sfc_lay, ctau, tau.ptr(), pf.ptr(), blay.ptr(), blev.ptr(), sfc.ptr(), sfcj.ptr(), stream()));
+        // One Gaussian angle, as the forward driver (src_test/Radiation_solver.cpp:533): D = 1.66, w = 0.5.
+        hip_check(K<Float>::lw_adjoint_factored(
+                ncol, nlay, t.ng, top_at_1, 1.66, 0.5, tau.ptr(), pf.ptr(), blay.ptr(), blev.ptr(), t.nb,
+                t.lims.data(), emis_sfc.ptr() + t.b0, nbnd, sfc.ptr(), g_flux_up.ptr(), g_flux_dn.ptr(), dtau.ptr(),
+                dpf.ptr(), dblay.ptr(), dblo.ptr(), dbhi.ptr(), dsfc.ptr(),
+                d_emis_gpt.ptr() + int64_t(ncol) * t.g0, stream()));
+        hip_check(K<Float>::gas_optics_lw_adjoint_bands(
+                &kd, t.b0, t.nb, ncol, nlay, p_lay.ptr(), t_lay.ptr(), t_lev.ptr(), t_sfc.ptr(), col_dry.ptr(), &vmr,
+                sfc_lay, dtau.ptr(), dpf.ptr(), dblay.ptr(), dblo.ptr(), dbhi.ptr(), dsfc.ptr(), d_col.ptr(),
                 out.d_t_lay.ptr(), out.d_lnp_lay.ptr(), d_lo.ptr(), d_hi.ptr(), out.d_t_sfc.ptr(), stream()));
     }
     hip_check(K<Float>::adjoint_levels(ncol, nlay, d_lo.ptr(), d_hi.ptr(), out.d_t_lev.ptr(), stream()));
@@ -188,26 +217,25 @@ void sw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
     Array_gpu<Float,2> d_col_dry({ncol, nlay}), d_ad({ncol, ngpt}), d_af({ncol, ngpt});
     zero(d_col); zero(out.d_t_lay); zero(out.d_lnp_lay); zero(out.d_p_lev);
 
-    const int mb = max_band_gpts(kdist);
-    Array_gpu<Float,3> tau({ncol, nlay, mb}), ssa({ncol, nlay, mb}), g({ncol, nlay, mb});
-    Array_gpu<Float,3> dtau({ncol, nlay, mb}), dssa({ncol, nlay, mb}), dg({ncol, nlay, mb});
+    const std::vector<Batch> batches = make_batches(kdist, ncl, 9.);     // 5 arrays and the solver's 4 level states
+    const int mg = most_of(batches, [](const Batch& t) { return t.ng; });
+    Array_gpu<Float,3> tau({ncol, nlay, mg}), ssa({ncol, nlay, mg}), g({ncol, nlay, mg});
+    Array_gpu<Float,3> dabs({ncol, nlay, mg}), dray({ncol, nlay, mg});
     const Float* ct = cl ? cl->get_tau().ptr() : nullptr;
     const Float* cs = cl ? cl->get_ssa().ptr() : nullptr;
     const Float* cg = cl ? cl->get_g().ptr() : nullptr;
-    const Array<int,2>& bl = kdist.get_band_lims_gpoint();
-    for (int b = 0; b < nbnd; ++b)
+    for (const Batch& t : batches)
     {
-        const int g0 = bl({1, b + 1}) - 1, ngb = bl({2, b + 1}) - g0;
-        const int64_t o = int64_t(ncol) * g0;
-        hip_check(K<Float>::gas_optics_sw_bands(&kd, b, 1, ncol, nlay, p_lay.ptr(), t_lay.ptr(), col_dry.ptr(), &vmr,
-                                                ct, cs, cg, tau.ptr(), ssa.ptr(), g.ptr(), stream()));
-        hip_check(K<Float>::sw_solver_2stream_adjoint(
-                ncol, nlay, ngb, top_at_1, tau.ptr(), ssa.ptr(), g.ptr(), mu0.ptr(), ad_gpt.ptr() + o,
+        const int64_t o = int64_t(ncol) * t.g0;
+        hip_check(K<Float>::gas_optics_sw_bands(&kd, t.b0, t.nb, ncol, nlay, p_lay.ptr(), t_lay.ptr(), col_dry.ptr(),
+                                                &vmr, ct, cs, cg, tau.ptr(), ssa.ptr(), g.ptr(), stream()));
+        hip_check(K<Float>::sw_adjoint_gases(
+                ncol, nlay, t.ng, top_at_1, tau.ptr(), ssa.ptr(), g.ptr(), mu0.ptr(), ad_gpt.ptr() + o,
                 af_gpt.ptr() + o, toa.ptr() + o, nullptr, g_flux_up.ptr(), g_flux_dn.ptr(), g_flux_dir.ptr(),
-                dtau.ptr(), dssa.ptr(), dg.ptr(), d_ad.ptr() + o, d_af.ptr() + o, stream()));
-        hip_check(K<Float>::gas_optics_sw_adjoint(&kd, b, ncol, nlay, p_lay.ptr(), t_lay.ptr(), col_dry.ptr(), &vmr,
-                                                  ct, cs, cg, dtau.ptr(), dssa.ptr(), dg.ptr(), d_col.ptr(),
-                                                  out.d_t_lay.ptr(), out.d_lnp_lay.ptr(), stream()));
+                dabs.ptr(), dray.ptr(), d_ad.ptr() + o, d_af.ptr() + o, stream()));
+        hip_check(K<Float>::gas_optics_sw_adjoint_bands(&kd, t.b0, t.nb, ncol, nlay, p_lay.ptr(), t_lay.ptr(),
+                                                        col_dry.ptr(), &vmr, dabs.ptr(), dray.ptr(), d_col.ptr(),
+                                                        out.d_t_lay.ptr(), out.d_lnp_lay.ptr(), stream()));
     }
     hip_check(K<Float>::adjoint_col_chain(ncol, nlay, &vmr, col_dry.ptr(), d_col.ptr(), out.d_vmr.ptr(),
                                           d_col_dry.ptr(), stream()));
