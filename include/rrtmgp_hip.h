@@ -77,6 +77,13 @@ int rrtmgp_hip_cache_free(void* ptr, void* stream);
 int rrtmgp_hip_cache_release(void);
 int rrtmgp_hip_cache_stats(size_t* live_bytes, size_t* cached_bytes);
 
+/* Pool for arrays that any stream or library may use: pool_malloc / pool_free stand in for    */
+/* rrtmgp_hip_malloc / _free.  A freed block is handed out again only after a device            */
+/* synchronisation that began after its free, so one wait covers all blocks freed before it.   */
+/* Per device the pool keeps at most a sixteenth of the memory; cache_release gives it back.   */
+int rrtmgp_hip_pool_malloc(void** ptr, size_t bytes);
+int rrtmgp_hip_pool_free(void* ptr);
+
 /* Array_gpu element operations (reference include/Array.h): fill sets n elements of          */
 /* elem_size bytes (1, 2, 4 or 8) to *value (a host pointer), as Array_gpu::fill and fill_kernel*/
 /* (:296-335, :501-511).  subset copies dst(d_1..d_n) = src(s_1..s_n), s_k = d_k + starts_k - 1 */

@@ -98,6 +98,11 @@ def _dev(x, dtype):
     return DeviceArray.from_host(np.asarray(x), dtype=dtype)
 
 
+def _out(shape, dtype):
+    """An output array: not cleared, since every call here writes all elements of its outputs."""
+    return DeviceArray(shape, dtype, zero=False)
+
+
 def _p(d):
     return None if d is None else d.ptr
 
@@ -244,9 +249,9 @@ class Cloud(_Handle):
         dt = real_dtype(self.precision)
         lwp, iwp, rel, rei = (_dev(a, dt) for a in (lwp, iwp, rel, rei))
         ncol, nlay = lwp.shape
-        tau = DeviceArray((ncol, nlay, self.nbnd), dt)
-        ssa = DeviceArray((ncol, nlay, self.nbnd), dt) if two_stream else None
-        g = DeviceArray((ncol, nlay, self.nbnd), dt) if two_stream else None
+        tau = _out((ncol, nlay, self.nbnd), dt)
+        ssa = _out((ncol, nlay, self.nbnd), dt) if two_stream else None
+        g = _out((ncol, nlay, self.nbnd), dt) if two_stream else None
         self._check(self.L.rrtmgp_api_cloud_optics(self.h, ncol, nlay, lwp.ptr, iwp.ptr, rel.ptr, rei.ptr,
                                                    2 if two_stream and coalbedo else int(two_stream),
                                                    int(delta_scale), tau.ptr, _p(ssa), _p(g)))
@@ -289,7 +294,7 @@ class Aerosol(_Handle):
         dt = real_dtype(self.precision)
         rh, plev = _dev(rh, dt), _dev(plev, dt)
         ncol, nlay = rh.shape
-        out = [DeviceArray((ncol, nlay, self.nbnd), dt) for _ in range(3)]
+        out = [_out((ncol, nlay, self.nbnd), dt) for _ in range(3)]
         self._check(self.L.rrtmgp_api_aerosol_optics(self.h, ncol, nlay, concs.h, rh.ptr, plev.ptr,
                                                      int(delta_scale), int(coalbedo), *[o.ptr for o in out]))
         return tuple(out)
@@ -299,7 +304,7 @@ def get_col_dry(vmr_h2o, plev, precision=8):
     dt = real_dtype(precision)
     h2o, plev = _dev(vmr_h2o, dt), _dev(plev, dt)
     ncol, nlev = plev.shape
-    out = DeviceArray((ncol, nlev - 1), dt)
+    out = _out((ncol, nlev - 1), dt)
     _lib.check_api(_lib.cpp(precision).rrtmgp_api_get_col_dry(ncol, nlev - 1, h2o.ptr, C.c_int64(h2o.shape[0]),
                                                               C.c_int64(h2o.shape[1]), plev.ptr, out.ptr), precision)
     return out
@@ -313,22 +318,22 @@ def gas_optics(kd: KDist, atm, gas_concs: GasConcs, col_dry, coalbedo=False):
     ng = kd.ngpt
     play, plev, tlay = (_dev(a, dt) for a in (atm.p_lay, atm.p_lev, atm.t_lay))
     cd = _dev(col_dry, dt)
-    o = {"tau": DeviceArray((ncol, nlay, ng), dt)}
+    o = {"tau": _out((ncol, nlay, ng), dt)}
     if kd.is_lw:
         tlev, tsfc = _dev(atm.t_lev, dt), _dev(atm.t_sfc, dt)
         for k in ("lay_src", "lev_src_inc", "lev_src_dec"):
-            o[k] = DeviceArray((ncol, nlay, ng), dt)
-        o["sfc_src"] = DeviceArray((ncol, ng), dt)
-        o["sfc_src_jac"] = DeviceArray((ncol, ng), dt)
+            o[k] = _out((ncol, nlay, ng), dt)
+        o["sfc_src"] = _out((ncol, ng), dt)
+        o["sfc_src_jac"] = _out((ncol, ng), dt)
         kd._check(kd.L.rrtmgp_api_gas_optics_lw(
             kd.h, ncol, nlay, play.ptr, plev.ptr, tlay.ptr, tsfc.ptr, tlev.ptr, gas_concs.h, cd.ptr,
             o["tau"].ptr, o["lay_src"].ptr, o["lev_src_inc"].ptr, o["lev_src_dec"].ptr,
             o["sfc_src"].ptr, o["sfc_src_jac"].ptr))
     else:
         key = "coalbedo" if coalbedo else "ssa"
-        o[key] = DeviceArray((ncol, nlay, ng), dt)
-        o["g"] = DeviceArray((ncol, nlay, ng), dt)
-        o["toa_src"] = DeviceArray((ncol, ng), dt)
+        o[key] = _out((ncol, nlay, ng), dt)
+        o["g"] = _out((ncol, nlay, ng), dt)
+        o["toa_src"] = _out((ncol, ng), dt)
         fn = kd.L.rrtmgp_api_gas_optics_sw_coalbedo if coalbedo else kd.L.rrtmgp_api_gas_optics_sw
         kd._check(fn(kd.h, ncol, nlay, play.ptr, plev.ptr, tlay.ptr, gas_concs.h, cd.ptr, o["tau"].ptr,
                      o[key].ptr, o["g"].ptr, o["toa_src"].ptr))
@@ -359,7 +364,7 @@ def rte_lw(kd: KDist, top_at_1, tau, lay_src, lev_src_inc, lev_src_dec, sfc_src,
     emis = _dev(sfc_emis, dt)
     inc = _dev(inc_flux, dt)
     shape = (ncol, nlay + 1) if do_broadband else (ncol, nlay + 1, ng)
-    up, dn = DeviceArray(shape, dt), DeviceArray(shape, dt)
+    up, dn = _out(shape, dt), _out(shape, dt)
     kd._check(kd.L.rrtmgp_api_rte_lw(kd.h, ncol, nlay, int(top_at_1), tau.ptr, lay_src.ptr, lev_src_inc.ptr,
                                      lev_src_dec.ptr, sfc_src.ptr, emis.ptr, _p(inc), n_gauss_angles,
                                      int(do_broadband), up.ptr, dn.ptr))
@@ -373,7 +378,7 @@ def rte_sw(kd: KDist, top_at_1, tau, ssa, g, mu0, inc_flux_dir, sfc_alb_dir, sfc
     mu0, inc, ad, af = (_dev(a, dt) for a in (mu0, inc_flux_dir, sfc_alb_dir, sfc_alb_dif))
     dif = _dev(inc_flux_dif, dt)
     shape = (ncol, nlay + 1) if do_broadband else (ncol, nlay + 1, ng)
-    up, dn, dr = DeviceArray(shape, dt), DeviceArray(shape, dt), DeviceArray(shape, dt)
+    up, dn, dr = _out(shape, dt), _out(shape, dt), _out(shape, dt)
     kd._check(kd.L.rrtmgp_api_rte_sw(kd.h, ncol, nlay, int(top_at_1), tau.ptr, ssa.ptr, g.ptr, mu0.ptr,
                                      inc.ptr, ad.ptr, af.ptr, _p(dif), int(do_broadband), up.ptr, dn.ptr, dr.ptr))
     return up, dn, dr
@@ -388,8 +393,8 @@ def rte_sw_bnd(kd: KDist, top_at_1, tau, ssa, g, mu0, inc_flux_dir, sfc_alb_dir,
     dt = real_dtype(kd.precision)
     ncol, nlay, ng = tau.shape
     mu0, inc, ad, af, pl = (_dev(a, dt) for a in (mu0, inc_flux_dir, sfc_alb_dir, sfc_alb_dif, p_lev))
-    o = {k: DeviceArray((ncol, nlay + 1), dt) for k in ("flux_up", "flux_dn", "flux_dn_dir")}
-    o["heating_rate"] = DeviceArray((ncol, nlay), dt) if pl is not None else None
+    o = {k: _out((ncol, nlay + 1), dt) for k in ("flux_up", "flux_dn", "flux_dn_dir")}
+    o["heating_rate"] = _out((ncol, nlay), dt) if pl is not None else None
     fn = getattr(_lib.hip(), "rrtmgp_hip_sw_solver_2stream_bnd_" + ("coalbedo_" if coalbedo else "")
                  + ("f64" if kd.precision == 8 else "f32"))
     bl = kd.band_lims
@@ -404,10 +409,10 @@ def rte_sw_bnd(kd: KDist, top_at_1, tau, ssa, g, mu0, inc_flux_dir, sfc_alb_dir,
 def fluxes_reduce(kd: KDist, gpt_up, gpt_dn, gpt_dir=None, byband=False):
     dt = real_dtype(kd.precision)
     ncol, nlev, _ = gpt_up.shape
-    o = {k: DeviceArray((ncol, nlev), dt) for k in ("flux_up", "flux_dn", "flux_net")}
-    o["flux_dn_dir"] = DeviceArray((ncol, nlev), dt) if gpt_dir is not None else None
+    o = {k: _out((ncol, nlev), dt) for k in ("flux_up", "flux_dn", "flux_net")}
+    o["flux_dn_dir"] = _out((ncol, nlev), dt) if gpt_dir is not None else None
     for k in ("bnd_flux_up", "bnd_flux_dn", "bnd_flux_net", "bnd_flux_dn_dir"):
-        o[k] = DeviceArray((ncol, nlev, kd.nbnd), dt) if byband else None
+        o[k] = _out((ncol, nlev, kd.nbnd), dt) if byband else None
     if gpt_dir is None:
         o["bnd_flux_dn_dir"] = None
     kd._check(kd.L.rrtmgp_api_fluxes_reduce(
@@ -421,7 +426,7 @@ def heating_rate(flux_up, flux_dn, plev, precision=8):
     dt = real_dtype(precision)
     up, dn, p = (_dev(a, dt) for a in (flux_up, flux_dn, plev))
     ncol, nlev = up.shape
-    out = DeviceArray((ncol, nlev - 1), dt)
+    out = _out((ncol, nlev - 1), dt)
     _lib.check_api(_lib.cpp(precision).rrtmgp_api_heating_rate(ncol, nlev - 1, up.ptr, dn.ptr, p.ptr, out.ptr),
                    precision)
     return out
@@ -479,11 +484,11 @@ class SolverLW(_Solver):
         nlev = nlay + 1
         o = outputs
         if o is None:
-            o = {k: DeviceArray((ncol, nlev), dt) for k in ("flux_up", "flux_dn", "flux_net")}
+            o = {k: _out((ncol, nlev), dt) for k in ("flux_up", "flux_dn", "flux_net")}
             for k in ("bnd_flux_up", "bnd_flux_dn", "bnd_flux_net"):
-                o[k] = DeviceArray((ncol, nlev, self.kd.nbnd), dt) if bnd else None
+                o[k] = _out((ncol, nlev, self.kd.nbnd), dt) if bnd else None
         if heating_rate and o.get("heating_rate") is None:
-            o["heating_rate"] = DeviceArray((ncol, nlay), dt)
+            o["heating_rate"] = _out((ncol, nlay), dt)
         cloudy = da.cloudy and self.cloud is not None
         col_dry = _dev(col_dry, dt)
         self._check(self.L.rrtmgp_api_solve_lw(
@@ -505,10 +510,10 @@ class SolverLW(_Solver):
         ncol, nlay = da.ncol, da.nlay
         nlev = nlay + 1
         gu, gd = _dev(g_flux_up, dt), _dev(g_flux_dn, dt)
-        o = {"t_lay": DeviceArray((ncol, nlay), dt), "t_lev": DeviceArray((ncol, nlev), dt),
-             "t_sfc": DeviceArray((ncol,), dt), "lnp_lay": DeviceArray((ncol, nlay), dt),
-             "p_lev": DeviceArray((ncol, nlev), dt), "vmr": DeviceArray((ncol, nlay, self.kd.ngas), dt),
-             "emis_sfc": DeviceArray((self.kd.nbnd, ncol), dt)}
+        o = {"t_lay": _out((ncol, nlay), dt), "t_lev": _out((ncol, nlev), dt),
+             "t_sfc": _out((ncol,), dt), "lnp_lay": _out((ncol, nlay), dt),
+             "p_lev": _out((ncol, nlev), dt), "vmr": _out((ncol, nlay, self.kd.ngas), dt),
+             "emis_sfc": _out((self.kd.nbnd, ncol), dt)}
         cloudy = da.cloudy and self.cloud is not None
         self._check(self.L.rrtmgp_api_adjoint_lw(
             self.h, ncol, nlay, int(cloudy), da.p_lay.ptr, da.p_lev.ptr, da.t_lay.ptr, da.t_lev.ptr, da.t_sfc.ptr,
@@ -542,11 +547,11 @@ class SolverSW(_Solver):
         tsi = _dev(tsi_scaling, dt)
         o = outputs
         if o is None:
-            o = {k: DeviceArray((ncol, nlev), dt) for k in ("flux_up", "flux_dn", "flux_dn_dir", "flux_net")}
+            o = {k: _out((ncol, nlev), dt) for k in ("flux_up", "flux_dn", "flux_dn_dir", "flux_net")}
             for k in ("bnd_flux_up", "bnd_flux_dn", "bnd_flux_dn_dir", "bnd_flux_net"):
-                o[k] = DeviceArray((ncol, nlev, self.kd.nbnd), dt) if bnd else None
+                o[k] = _out((ncol, nlev, self.kd.nbnd), dt) if bnd else None
         if heating_rate and o.get("heating_rate") is None:
-            o["heating_rate"] = DeviceArray((ncol, nlay), dt)
+            o["heating_rate"] = _out((ncol, nlay), dt)
         cloudy = da.cloudy and self.cloud is not None
         rh, aconcs = (None, None) if aerosol is None else aerosol
         rh = _dev(rh, dt) if aerosol is not None else None
@@ -576,10 +581,10 @@ class SolverSW(_Solver):
         tsi = _dev(tsi_scaling, dt)
         af = da.sfc_alb if sfc_alb_dif is None else _dev(sfc_alb_dif, dt)
         gu, gd, gr = _dev(g_flux_up, dt), _dev(g_flux_dn, dt), _dev(g_flux_dir, dt)
-        o = {"t_lay": DeviceArray((ncol, nlay), dt), "lnp_lay": DeviceArray((ncol, nlay), dt),
-             "p_lev": DeviceArray((ncol, nlev), dt), "vmr": DeviceArray((ncol, nlay, self.kd.ngas), dt),
-             "sfc_alb_dir": DeviceArray((self.kd.nbnd, ncol), dt),
-             "sfc_alb_dif": DeviceArray((self.kd.nbnd, ncol), dt)}
+        o = {"t_lay": _out((ncol, nlay), dt), "lnp_lay": _out((ncol, nlay), dt),
+             "p_lev": _out((ncol, nlev), dt), "vmr": _out((ncol, nlay, self.kd.ngas), dt),
+             "sfc_alb_dir": _out((self.kd.nbnd, ncol), dt),
+             "sfc_alb_dif": _out((self.kd.nbnd, ncol), dt)}
         cloudy = da.cloudy and self.cloud is not None
         self._check(self.L.rrtmgp_api_adjoint_sw(
             self.h, ncol, nlay, int(cloudy), int(delta_cloud), da.p_lay.ptr, da.p_lev.ptr, da.t_lay.ptr,

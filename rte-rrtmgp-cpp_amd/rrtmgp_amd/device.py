@@ -1,4 +1,4 @@
-"""Device arrays owned through the C ABI (rrtmgp_hip_malloc / memcpy), Fortran layout."""
+"""Device arrays owned through the C ABI (rrtmgp_hip_pool_malloc / memcpy), Fortran layout."""
 from __future__ import annotations
 
 import ctypes as C
@@ -17,7 +17,7 @@ class DeviceArray:
         self.size = int(np.prod(self.shape)) if self.shape else 1
         self.nbytes = self.size * self.dtype.itemsize
         p = C.c_void_p()
-        _lib.check_hip(_lib.hip().rrtmgp_hip_malloc(C.byref(p), C.c_size_t(max(self.nbytes, 1))))
+        _lib.check_hip(_lib.hip().rrtmgp_hip_pool_malloc(C.byref(p), C.c_size_t(max(self.nbytes, 1))))
         self._p = p
         if zero:
             _lib.check_hip(_lib.hip().rrtmgp_hip_memset(p, 0, C.c_size_t(max(self.nbytes, 1)), None))
@@ -44,7 +44,7 @@ class DeviceArray:
 
     def free(self):
         if getattr(self, "_p", None) is not None and self._p.value:
-            _lib.hip().rrtmgp_hip_free(self._p)
+            _lib.hip().rrtmgp_hip_pool_free(self._p)
         self._p = None
 
     def __del__(self):

@@ -1,0 +1,95 @@
+// Host-side checks of the device-array pool's reuse rules (rte-rrtmgp-cpp_amd/csrc/device_pool.h).
+// Pointers are opaque here; the checks print "ok" and return 0 when all hold.
+#include <cstdio>
+
+#include "device_pool.h"
+
+using rrtmgp_hip::PoolBlock;
+using rrtmgp_hip::PoolPolicy;
+
+#define CHECK(c)                                                                  \
+    do { if (!(c)) { std::printf("FAILED line %d: %s\n", __LINE__, #c); return 1; } } while (0)
+
+int main()
+{
+    char mem[8][8];
+    const size_t MiB = size_t(1) << 20;
+    std::vector<PoolBlock> out;
+    PoolBlock b;
+    bool wait = false;
+
+    CHECK(PoolPolicy::round_block(1) == 512);
+    CHECK(PoolPolicy::round_block(512) == 512);
+    CHECK(PoolPolicy::round_block(MiB) == MiB);
+    CHECK(PoolPolicy::round_block(MiB + 1) == 2 * MiB);
+
+    // One wait covers every block freed before it began, none freed after.
+    {
+        PoolPolicy p;
+        for (int i = 0; i < 3; ++i) p.add_live(mem[i], 4096, 0);
+        CHECK(p.give(mem[0], MiB, out) && p.give(mem[1], MiB, out) && out.empty());
+        CHECK(p.held(0) == 8192 && p.n_live() == 1);
+        CHECK(p.take(0, 4096, b, wait) && wait);
+        const uint64_t n = p.start_wait();
+        CHECK(p.give(mem[2], MiB, out));               // freed while the wait runs
+        p.waited(0, n);
+        CHECK(p.take(0, 4096, b, wait) && !wait && b.ptr == mem[1]);
+        CHECK(p.take(0, 4096, b, wait) && wait && b.ptr == mem[2]);
+        CHECK(!p.take(0, 4096, b, wait));
+        CHECK(p.held(0) == 0 && p.n_live() == 3);
+    }
+
+    // A block that needs no wait is preferred to a smaller one that needs one.
+    {
+        PoolPolicy p;
+        p.add_live(mem[0], 4608, 0);
+        CHECK(p.give(mem[0], MiB, out));
+        p.waited(0, p.start_wait());
+        p.add_live(mem[1], 4096, 0);
+        CHECK(p.give(mem[1], MiB, out));
+        CHECK(p.take(0, 4096, b, wait) && !wait && b.ptr == mem[0]);
+    }
+
+    // A wait on one device says nothing of another, and blocks stay on theirs.
+    {
+        PoolPolicy p;
+        p.add_live(mem[0], 4096, 1);
+        CHECK(p.give(mem[0], MiB, out));
+        p.waited(0, p.start_wait());
+        CHECK(!p.take(0, 4096, b, wait));
+        CHECK(p.take(1, 4096, b, wait) && wait);
+    }
+
+    // Too small, or more than an eighth too large: not taken.  The smallest that fits is.
+    {
+        PoolPolicy p;
+        p.add_live(mem[0], 4096, 0);
+        p.add_live(mem[1], 8192, 0);
+        p.add_live(mem[2], 8704, 0);
+        for (int i = 2; i >= 0; --i) CHECK(p.give(mem[i], MiB, out));
+        CHECK(p.take(0, 8192, b, wait) && b.ptr == mem[1]);
+        CHECK(p.take(0, 8192, b, wait) && b.ptr == mem[2]);
+        CHECK(!p.take(0, 8192, b, wait));
+        CHECK(!p.take(0, 2048, b, wait));
+    }
+
+    // The bound: oldest blocks leave first; a block beyond the bound is never kept.
+    {
+        PoolPolicy p;
+        for (int i = 0; i < 3; ++i) p.add_live(mem[i], 4096, 0);
+        p.add_live(mem[3], 16384, 0);
+        p.add_live(mem[4], 4096, 1);
+        CHECK(p.give(mem[4], 8192, out) && p.give(mem[0], 8192, out) && p.give(mem[1], 8192, out) && out.empty());
+        CHECK(p.give(mem[2], 8192, out) && out.size() == 1 && out[0].ptr == mem[0]);
+        out.clear();
+        CHECK(p.give(mem[3], 8192, out) && out.size() == 1 && out[0].ptr == mem[3]);
+        out.clear();
+        CHECK(p.held(0) == 8192 && p.held(1) == 4096 && p.n_live() == 0);
+        CHECK(!p.give(mem[3], 8192, out));             // not live any more
+        CHECK(p.drain().size() == 3 && p.held(0) == 0 && p.held(1) == 0);
+        CHECK(!p.take(0, 4096, b, wait));
+    }
+
+    std::printf("ok\n");
+    return 0;
+}
