@@ -664,6 +664,9 @@ RRTMGP_DECLARE_BOTH(RRTMGP_DECL_ADJ_HELPERS)
 /* Fortran rte_sum_broadband / rte_net_broadband_precalc / sum_byband / net_byband_precalc,   */
 /* rrtmgp_kernels.h:34-52).  By-band sums use the CPU semantics (1-based inclusive band_lims, */
 /* mo_fluxes_byband_kernels.F90:22-79).                                                       */
+/* reduce_fluxes makes all of them in one pass over the fluxes: gpt_dir and any output may be  */
+/* NULL; band_lims (device) is NULL for broadband only, else the nbnd bands must follow each   */
+/* other from g-point 1 to ngpt.                                                               */
 /* ------------------------------------------------------------------------------------------ */
 #define RRTMGP_DECL_FLUXES(S, T)                                                               \
     int rrtmgp_hip_sum_broadband_##S(int64_t ncol, int64_t nlev, int64_t ngpt,                \
@@ -674,7 +677,11 @@ RRTMGP_DECLARE_BOTH(RRTMGP_DECL_ADJ_HELPERS)
         const int* band_lims, const T* gpt_flux, T* bnd_flux, void* stream);                   \
     int rrtmgp_hip_net_byband_full_##S(int64_t ncol, int64_t nlev, int64_t ngpt,              \
         int64_t nbnd, const int* band_lims, const T* gpt_flux_dn, const T* gpt_flux_up,        \
-        T* bnd_flux_net, void* stream);
+        T* bnd_flux_net, void* stream);                                                        \
+    int rrtmgp_hip_reduce_fluxes_##S(int64_t ncol, int64_t nlev, int64_t ngpt, int64_t nbnd,  \
+        const int* band_lims, const T* gpt_up, const T* gpt_dn, const T* gpt_dir, T* flux_up,  \
+        T* flux_dn, T* flux_net, T* flux_dir, T* bnd_up, T* bnd_dn, T* bnd_net, T* bnd_dir,    \
+        void* stream);
 RRTMGP_DECLARE_BOTH(RRTMGP_DECL_FLUXES)
 
 /* Heating rate, no reference counterpart: hr(ncol, nlay) [K/day] =                          */

@@ -225,46 +225,93 @@ __global__ void increment_kernel(int64_t n, Real* __restrict__ tau1, Real* __res
     tau1[i] = tau12;
 }
 
-// inc_*_bybnd: thread per (col, lay, gpt); the band of a g-point is found by scanning the
-// (few) band limits, as the reference kernel does (optical_props_kernels.cu:86-95).
-template<typename Real>
-__global__ void inc_bybnd_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, Real* __restrict__ tau1,
-                                 Real* __restrict__ ssa1, Real* __restrict__ g1,
-                                 const Real* __restrict__ tau2, const Real* __restrict__ ssa2,
-                                 const Real* __restrict__ g2, int64_t nbnd, const int* __restrict__ band_lims,
-                                 int coalb = 0)
+template<typename Real, int N>
+struct alignas(sizeof(Real) * N) Vec { Real v[N]; };
+
+enum IncMode { INC_1SCL = 0, INC_2STR = 1, INC_COALB = 2 };
+
+// inc_*_bybnd (optical_props_kernels.cu:86-95): bound by HBM (three arrays read and written per element, the
+// band-resolved ones come from the L2).  A work-group covers 256 * NV elements (col, lay) of one g-point, so
+// the band of the g-point is found by scalar code and every lane moves 16 bytes an access.  A flat thread per
+// element, with a 64-bit division and a per-lane scan of the limits, ran at half the copy rate: at 4096 x 72
+// FP32 the LW and the 2-stream SW increment (256 and 224 g-points) took 938 us together and take 413 us
+// (5.3 TB/s); the FP64 co-albedo increment at 1000 x 72 x 224 took 157 us and takes 148 us (5.2 TB/s).
+template<typename Real, int MODE, int NV>
+__global__ void inc_bybnd_kernel(int64_t ncl, int64_t ngpt, Real* __restrict__ tau1, Real* __restrict__ ssa1,
+                                 Real* __restrict__ g1, const Real* __restrict__ tau2,
+                                 const Real* __restrict__ ssa2, const Real* __restrict__ g2, int64_t nbnd,
+                                 const int* __restrict__ band_lims)
 {
-    const int64_t ncl = ncol * nlay;
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= ncl * ngpt) return;
-    const int64_t cl = i % ncl;
-    const int gpt1 = int(i / ncl) + 1;
+    using V = Vec<Real, NV>;
+    const int64_t cl = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) * NV;
+    if (cl >= ncl) return;
     const Real eps = Real(3) * Limits<Real>::tiny;
-    for (int64_t b = 0; b < nbnd; ++b)
+    for (int64_t gpt = blockIdx.y; gpt < ngpt; gpt += gridDim.y)
     {
-        if (gpt1 >= band_lims[2 * b] && gpt1 <= band_lims[2 * b + 1])
+        const int64_t i = cl + ncl * gpt;
+        for (int64_t b = 0; b < nbnd; ++b)
         {
+            if (gpt + 1 < band_lims[2 * b] || gpt + 1 > band_lims[2 * b + 1]) continue;
             const int64_t ib = cl + ncl * b;
-            if (!ssa1) { tau1[i] = tau1[i] + tau2[ib]; continue; }
-            if (coalb)
+            V t1 = *reinterpret_cast<const V*>(tau1 + i);
+            const V t2 = *reinterpret_cast<const V*>(tau2 + ib);
+            if constexpr (MODE == INC_1SCL)
             {
-                // ssa1, ssa2 hold co-albedos 1 - ssa: the same increment in those terms.
-                const Real t1 = tau1[i], t2 = tau2[ib], c1 = ssa1[i], c2 = ssa2[ib];
-                const Real tau12 = t1 + t2;
-                const Real tauscat12 = (t1 * (Real(1) - c1)) + (t2 * (Real(1) - c2));
-                g1[i] = ((t1 * (Real(1) - c1) * g1[i]) + (t2 * (Real(1) - c2) * g2[ib])) / max(tauscat12, eps);
-                ssa1[i] = (tau12 > eps) ? ((t1 * c1) + (t2 * c2)) / tau12 : Real(1) - tauscat12 / eps;
-                tau1[i] = tau12;
-                continue;
+#pragma unroll
+                for (int k = 0; k < NV; ++k) t1.v[k] = t1.v[k] + t2.v[k];
             }
-            const Real t1 = tau1[i], t2 = tau2[ib], s1 = ssa1[i], s2 = ssa2[ib];
-            const Real tau12 = t1 + t2;
-            const Real tauscat12 = (t1 * s1) + (t2 * s2);
-            g1[i] = ((t1 * s1 * g1[i]) + (t2 * s2 * g2[ib])) / max(tauscat12, eps);
-            ssa1[i] = tauscat12 / max(eps, tau12);
-            tau1[i] = tau12;
+            else
+            {
+                V s1 = *reinterpret_cast<const V*>(ssa1 + i), a1 = *reinterpret_cast<const V*>(g1 + i);
+                const V s2 = *reinterpret_cast<const V*>(ssa2 + ib), a2 = *reinterpret_cast<const V*>(g2 + ib);
+#pragma unroll
+                for (int k = 0; k < NV; ++k)
+                {
+                    const Real x1 = t1.v[k], x2 = t2.v[k], w1 = s1.v[k], w2 = s2.v[k];
+                    const Real tau12 = x1 + x2;
+                    if constexpr (MODE == INC_COALB)
+                    {
+                        // ssa1, ssa2 hold co-albedos 1 - ssa: the same increment in those terms.
+                        const Real tauscat12 = (x1 * (Real(1) - w1)) + (x2 * (Real(1) - w2));
+                        a1.v[k] = ((x1 * (Real(1) - w1) * a1.v[k]) + (x2 * (Real(1) - w2) * a2.v[k]))
+                                  / max(tauscat12, eps);
+                        s1.v[k] = (tau12 > eps) ? ((x1 * w1) + (x2 * w2)) / tau12 : Real(1) - tauscat12 / eps;
+                    }
+                    else
+                    {
+                        const Real tauscat12 = (x1 * w1) + (x2 * w2);
+                        a1.v[k] = ((x1 * w1 * a1.v[k]) + (x2 * w2 * a2.v[k])) / max(tauscat12, eps);
+                        s1.v[k] = tauscat12 / max(eps, tau12);
+                    }
+                    t1.v[k] = tau12;
+                }
+                *reinterpret_cast<V*>(ssa1 + i) = s1;
+                *reinterpret_cast<V*>(g1 + i) = a1;
+            }
+            *reinterpret_cast<V*>(tau1 + i) = t1;
         }
     }
+}
+
+// 16-byte accesses need every g-point's slice to start on 16 bytes: whole vectors per slice and aligned
+// arrays.  Other shapes (odd column counts times odd layer counts, arrays inside others) go element by element.
+template<typename Real, int MODE>
+void launch_inc_bybnd(int64_t ncl, int64_t ngpt, Real* tau1, Real* ssa1, Real* g1, const Real* tau2,
+                      const Real* ssa2, const Real* g2, int64_t nbnd, const int* band_lims, hipStream_t stream)
+{
+    if (ncl <= 0 || ngpt <= 0) return;
+    constexpr int NV = 16 / int(sizeof(Real));
+    uintptr_t bits = 0;
+    for (const void* p : {(const void*)tau1, (const void*)ssa1, (const void*)g1, (const void*)tau2,
+                          (const void*)ssa2, (const void*)g2})
+        bits |= reinterpret_cast<uintptr_t>(p);
+    const unsigned gy = unsigned(std::min<int64_t>(ngpt, 65535));
+    if (ncl % NV == 0 && bits % 16 == 0)
+        hipLaunchKernelGGL((inc_bybnd_kernel<Real, MODE, NV>), dim3(grid1(ncl / NV, 256), gy), dim3(256), 0, stream,
+                           ncl, ngpt, tau1, ssa1, g1, tau2, ssa2, g2, nbnd, band_lims);
+    else
+        hipLaunchKernelGGL((inc_bybnd_kernel<Real, MODE, 1>), dim3(grid1(ncl, 256), gy), dim3(256), 0, stream,
+                           ncl, ngpt, tau1, ssa1, g1, tau2, ssa2, g2, nbnd, band_lims);
 }
 
 template<typename Real>
@@ -280,15 +327,98 @@ __global__ void delta_scale_kernel(int64_t n, Real* __restrict__ tau, Real* __re
     g[i] = (gv - f) / max(eps, Real(1) - f);
 }
 
+// Adds f[0 .. n), strided, to s in order, with 16 loads in flight.
+template<typename Real>
+__device__ __forceinline__ Real add_in_order(Real s, const Real* __restrict__ f, int64_t stride, int64_t n)
+{
+    int64_t g = 0;
+    for (; g + 16 <= n; g += 16)
+    {
+        Real x[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = f[(g + k) * stride];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) s += x[k];
+    }
+    for (; g < n; ++g) s += f[g * stride];
+    return s;
+}
+
 // Broadband sum over g-points in order (fluxes_kernels.cu:26-43).
 template<typename Real>
 __global__ void sum_broadband_kernel(int64_t ncv, int64_t ngpt, const Real* __restrict__ f, Real* __restrict__ out)
 {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= ncv) return;
-    Real s = Real(0);
-    for (int64_t g = 0; g < ngpt; ++g) s += f[i + ncv * g];
-    out[i] = s;
+    out[i] = add_in_order(Real(0), f + i, ncv, ngpt);
+}
+
+// All reductions of one set of g-point fluxes in one pass: broadband up, down, net and (DIR) direct, and with
+// BANDS the same per band, for bands that follow each other from the first g-point to the last; outputs that are
+// NULL are left out.  Sums run in g-point order, as in the separate kernels.  Bound by HBM: each flux is read once, where the separate sums
+// read it twice and the nets re-read the sums.  There are only ncol * nlev threads, so each keeps 8 loads of
+// every flux in flight (the plain loop kept too few: 1.4 TB/s).  At 2048 x 73 x 256 FP32 with bands six launches
+// took 330 us, this one takes 74 us (4.1 TB/s); three broadband sums at 3000 x 61 x 224 342 us, now 165 us.
+template<typename Real, bool DIR, bool BANDS>
+__global__ __launch_bounds__(256) void reduce_fluxes_kernel(int64_t ncv, int64_t ngpt, int64_t nbnd,
+                                     const int* __restrict__ bl, const Real* __restrict__ up,
+                                     const Real* __restrict__ dn, const Real* __restrict__ dir,
+                                     Real* __restrict__ b_up, Real* __restrict__ b_dn, Real* __restrict__ b_net,
+                                     Real* __restrict__ b_dir, Real* __restrict__ bnd_up, Real* __restrict__ bnd_dn,
+                                     Real* __restrict__ bnd_net, Real* __restrict__ bnd_dir)
+{
+    constexpr int U = 8;
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= ncv) return;
+    Real su = Real(0), sd = Real(0), sr = Real(0);
+    int64_t g = 0;
+    for (int64_t b = 0; b < (BANDS ? nbnd : 1); ++b)
+    {
+        const int64_t ge = BANDS ? int64_t(bl[2 * b + 1]) : ngpt;
+        Real bu = Real(0), bd = Real(0), br = Real(0);
+        for (; g + U <= ge; g += U)
+        {
+            Real xu[U], xd[U], xr[U];
+#pragma unroll
+            for (int k = 0; k < U; ++k)
+            {
+                xu[k] = up[i + (g + k) * ncv];
+                xd[k] = dn[i + (g + k) * ncv];
+                if constexpr (DIR) xr[k] = dir[i + (g + k) * ncv];
+            }
+#pragma unroll
+            for (int k = 0; k < U; ++k)
+            {
+                su += xu[k]; sd += xd[k];
+                if constexpr (BANDS) { bu += xu[k]; bd += xd[k]; }
+                if constexpr (DIR) { sr += xr[k]; if constexpr (BANDS) br += xr[k]; }
+            }
+        }
+        for (; g < ge; ++g)
+        {
+            const Real xu = up[i + g * ncv], xd = dn[i + g * ncv];
+            su += xu; sd += xd;
+            if constexpr (BANDS) { bu += xu; bd += xd; }
+            if constexpr (DIR)
+            {
+                const Real xr = dir[i + g * ncv];
+                sr += xr;
+                if constexpr (BANDS) br += xr;
+            }
+        }
+        if constexpr (BANDS)
+        {
+            const int64_t o = i + ncv * b;
+            if (bnd_up) bnd_up[o] = bu;
+            if (bnd_dn) bnd_dn[o] = bd;
+            if (bnd_net) bnd_net[o] = bd - bu;
+            if constexpr (DIR) { if (bnd_dir) bnd_dir[o] = br; }
+        }
+    }
+    if (b_up) b_up[i] = su;
+    if (b_dn) b_dn[i] = sd;
+    if (b_net) b_net[i] = sd - su;
+    if constexpr (DIR) { if (b_dir) b_dir[i] = sr; }
 }
 
 template<typename Real>
@@ -308,9 +438,7 @@ __global__ void sum_byband_kernel(int64_t ncv, int64_t nbnd, const int* __restri
     if (i >= ncv * nbnd) return;
     const int64_t cv = i % ncv, b = i / ncv;
     const int gs = bl[2 * b], ge = bl[2 * b + 1];
-    Real s = f[cv + ncv * (gs - 1)];
-    for (int g = gs; g < ge; ++g) s += f[cv + ncv * g];
-    out[i] = s;
+    out[i] = add_in_order(f[cv + ncv * (gs - 1)], f + cv + ncv * gs, ncv, ge - gs);
 }
 
 // net_byband_full (mo_fluxes_byband_kernels.F90:46-69): (net + dn) - up in g-point order.
@@ -494,28 +622,28 @@ extern "C" int rrtmgp_hip_inc_bybnd_##S(int64_t ncol, int64_t nlay, int64_t ngpt
     T* ssa_inout, T* g_inout, const T* tau_in, const T* ssa_in, const T* g_in, int64_t nbnd,        \
     const int* band_lims_gpt, void* stream)                                                          \
 {                                                                                                    \
-    const int64_t n = ncol * nlay * ngpt;                                                            \
-    RRTMGP_TIMED("inc_bybnd_kernel", as_stream(stream));                                             \
-    hipLaunchKernelGGL(inc_bybnd_kernel<T>, dim3(grid1(n, 256)), dim3(256), 0, as_stream(stream),   \
-                       ncol, nlay, ngpt, tau_inout, ssa_inout, g_inout, tau_in, ssa_in, g_in, nbnd, \
-                       band_lims_gpt);                                                               \
+    RRTMGP_TIMED("inc_bybnd_kernel", as_stream(stream));                                            \
+    if (ssa_inout)                                                                                  \
+        launch_inc_bybnd<T, INC_2STR>(ncol * nlay, ngpt, tau_inout, ssa_inout, g_inout, tau_in, ssa_in, \
+                                      g_in, nbnd, band_lims_gpt, as_stream(stream));                \
+    else                                                                                            \
+        launch_inc_bybnd<T, INC_1SCL>(ncol * nlay, ngpt, tau_inout, nullptr, nullptr, tau_in, nullptr, \
+                                      nullptr, nbnd, band_lims_gpt, as_stream(stream));             \
     RRTMGP_LAUNCHED("inc_bybnd_kernel");                                                            \
-    return RRTMGP_OK;                                                                                \
-}                                                                                                    \
+    return RRTMGP_OK;                                                                               \
+}                                                                                                   \
 extern "C" int rrtmgp_hip_inc_bybnd_coalbedo_##S(int64_t ncol, int64_t nlay, int64_t ngpt,       \
     T* tau_inout, T* coalbedo_inout, T* g_inout, const T* tau_in, const T* coalbedo_in,             \
     const T* g_in, int64_t nbnd, const int* band_lims_gpt, void* stream)                             \
 {                                                                                                    \
     if (!coalbedo_inout || !coalbedo_in || !g_inout || !g_in)                                        \
         return arg_error("inc_bybnd_coalbedo: two-stream arrays required");                         \
-    const int64_t n = ncol * nlay * ngpt;                                                            \
-    RRTMGP_TIMED("inc_bybnd_kernel", as_stream(stream));                                             \
-    hipLaunchKernelGGL(inc_bybnd_kernel<T>, dim3(grid1(n, 256)), dim3(256), 0, as_stream(stream),   \
-                       ncol, nlay, ngpt, tau_inout, coalbedo_inout, g_inout, tau_in, coalbedo_in,   \
-                       g_in, nbnd, band_lims_gpt, 1);                                                \
+    RRTMGP_TIMED("inc_bybnd_kernel", as_stream(stream));                                            \
+    launch_inc_bybnd<T, INC_COALB>(ncol * nlay, ngpt, tau_inout, coalbedo_inout, g_inout, tau_in,   \
+                                   coalbedo_in, g_in, nbnd, band_lims_gpt, as_stream(stream));      \
     RRTMGP_LAUNCHED("inc_bybnd_kernel");                                                            \
-    return RRTMGP_OK;                                                                                \
-}                                                                                                    \
+    return RRTMGP_OK;                                                                               \
+}                                                                                                   \
 extern "C" int rrtmgp_hip_delta_scale_2str_##S(int64_t ncol, int64_t nlay, int64_t ngpt, T* tau,  \
     T* ssa, T* g, void* stream)                                                                      \
 {                                                                                                    \
@@ -557,6 +685,25 @@ extern "C" int rrtmgp_hip_sum_byband_##S(int64_t ncol, int64_t nlev, int64_t ngp
     (void)ngpt;                                                                                      \
     return RRTMGP_OK;                                                                                \
 }                                                                                                    \
+extern "C" int rrtmgp_hip_reduce_fluxes_##S(int64_t ncol, int64_t nlev, int64_t ngpt, int64_t nbnd, \
+    const int* band_lims, const T* gpt_up, const T* gpt_dn, const T* gpt_dir, T* flux_up, T* flux_dn, \
+    T* flux_net, T* flux_dir, T* bnd_up, T* bnd_dn, T* bnd_net, T* bnd_dir, void* stream)           \
+{                                                                                                   \
+    const int64_t n = ncol * nlev;                                                                  \
+    const bool bands = band_lims != nullptr;                                                        \
+    if (n <= 0 || ngpt < 0 || !gpt_up || !gpt_dn || (bands && nbnd <= 0))                           \
+        return arg_error("reduce_fluxes: bad arguments");                                           \
+    RRTMGP_TIMED("reduce_fluxes_kernel", as_stream(stream));                                        \
+    const auto go = [&](auto kernel) {                                                              \
+        hipLaunchKernelGGL(kernel, dim3(grid1(n, 256)), dim3(256), 0, as_stream(stream), n, ngpt, nbnd, \
+                           band_lims, gpt_up, gpt_dn, gpt_dir, flux_up, flux_dn, flux_net, flux_dir, bnd_up, \
+                           bnd_dn, bnd_net, bnd_dir);                                               \
+    };                                                                                              \
+    if (bands) gpt_dir ? go(reduce_fluxes_kernel<T, true, true>) : go(reduce_fluxes_kernel<T, false, true>); \
+    else gpt_dir ? go(reduce_fluxes_kernel<T, true, false>) : go(reduce_fluxes_kernel<T, false, false>); \
+    RRTMGP_LAUNCHED("reduce_fluxes_kernel");                                                        \
+    return RRTMGP_OK;                                                                               \
+}                                                                                                   \
 extern "C" int rrtmgp_hip_net_byband_full_##S(int64_t ncol, int64_t nlev, int64_t ngpt,           \
     int64_t nbnd, const int* band_lims, const T* gpt_flux_dn, const T* gpt_flux_up,                 \
     T* bnd_flux_net, void* stream)                                                                   \

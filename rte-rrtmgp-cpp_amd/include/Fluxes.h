@@ -10,7 +10,19 @@
 #include "Array.h"
 #include "types.h"
 
+class Optical_props_gpu;
 class Optical_props_arry_gpu;
+
+// Where reduce_fluxes() leaves its results; nullptr for what is not wanted.
+struct Flux_outputs
+{
+    Float* up = nullptr;     Float* dn = nullptr;     Float* net = nullptr;     Float* dir = nullptr;
+    Float* bnd_up = nullptr; Float* bnd_dn = nullptr; Float* bnd_net = nullptr; Float* bnd_dir = nullptr;
+};
+
+// Broadband and, given the bands, by-band sums of g-point fluxes (ncol, nlev, ngpt); dir may be nullptr.
+void reduce_fluxes(int ncol, int nlev, int ngpt, const Float* up, const Float* dn, const Float* dir,
+                   const Optical_props_gpu* bands, const Flux_outputs& out);
 
 class Fluxes_gpu
 {

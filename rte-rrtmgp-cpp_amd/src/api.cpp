@@ -585,27 +585,10 @@ int rrtmgp_api_fluxes_reduce(void* h, int ncol, int nlev, const rrtmgp_real* gpt
 {
     return guarded([&] {
         auto& k = *K_(h).k;
-        const int ngpt = k.get_ngpt(), nbnd = k.get_nband();
-        std::unique_ptr<Optical_props_arry_gpu> p(new ViewProps(k, gpt_up, nullptr, nullptr, ncol, nlev, ngpt));
-        auto up = view<3>(gpt_up, {ncol, nlev, ngpt}), dn = view<3>(gpt_dn, {ncol, nlev, ngpt});
-        std::unique_ptr<Fluxes_broadband_gpu> f;
-        if (bnd_up) f.reset(new Fluxes_byband_gpu(ncol, nlev, nbnd));
-        else f.reset(new Fluxes_broadband_gpu(ncol, nlev));
-        if (gpt_dir) f->reduce(up, dn, view<3>(gpt_dir, {ncol, nlev, ngpt}), p, true);
-        else f->reduce(up, dn, p, true);
-        auto out2 = [&](rrtmgp_real* dst, const Array_gpu<Float,2>& a) {
-            if (dst) rrtmgp_cpp::hip_check(rrtmgp_hip_memcpy_d2d(dst, a.ptr(), a.bytes(), rrtmgp_cpp::stream()));
-        };
-        auto out3 = [&](rrtmgp_real* dst, const Array_gpu<Float,3>& a) {
-            if (dst) rrtmgp_cpp::hip_check(rrtmgp_hip_memcpy_d2d(dst, a.ptr(), a.bytes(), rrtmgp_cpp::stream()));
-        };
-        out2(flux_up, f->get_flux_up()); out2(flux_dn, f->get_flux_dn()); out2(flux_net, f->get_flux_net());
-        if (gpt_dir) out2(flux_dir, f->get_flux_dn_dir());
-        if (bnd_up)
-        {
-            out3(bnd_up, f->get_bnd_flux_up()); out3(bnd_dn, f->get_bnd_flux_dn()); out3(bnd_net, f->get_bnd_flux_net());
-            if (gpt_dir) out3(bnd_dir, f->get_bnd_flux_dn_dir());
-        }
+        Flux_outputs o;
+        o.up = flux_up; o.dn = flux_dn; o.net = flux_net; o.dir = flux_dir;
+        o.bnd_up = bnd_up; o.bnd_dn = bnd_dn; o.bnd_net = bnd_net; o.bnd_dir = bnd_dir;
+        reduce_fluxes(ncol, nlev, k.get_ngpt(), gpt_up, gpt_dn, gpt_dir, bnd_up ? &k : nullptr, o);
         rrtmgp_cpp::hip_check(rrtmgp_hip_stream_synchronize(rrtmgp_cpp::stream()));
     });
 }

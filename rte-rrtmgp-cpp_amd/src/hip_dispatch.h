@@ -50,6 +50,7 @@ template<typename T> struct K;
     static constexpr auto net_broadband = rrtmgp_hip_net_broadband_##S;  \
     static constexpr auto sum_byband = rrtmgp_hip_sum_byband_##S;        \
     static constexpr auto net_byband_full = rrtmgp_hip_net_byband_full_##S; \
+    static constexpr auto reduce_fluxes = rrtmgp_hip_reduce_fluxes_##S; \
     static constexpr auto heating_rate = rrtmgp_hip_heating_rate_##S;    \
     static constexpr auto count_outside = rrtmgp_hip_count_outside_##S;  \
     static constexpr auto check_ranges = rrtmgp_hip_check_ranges_##S;    \
