@@ -777,6 +777,17 @@ int rrtmgp_hip_mlp_bias_grad(int64_t rows, int n, const float* dZ, float* db, vo
 /* p_bf16 when it is not NULL.                                                                   */
 int rrtmgp_hip_mlp_adam(int64_t n, float* p, const float* g, float* m, float* v, void* p_bf16, float lr,
                         float beta1, float beta2, float eps, int64_t step, void* stream);
+/* The same step on up to 16 arrays in one launch.                                               */
+typedef struct { float* p; const float* g; float* m; float* v; void* p_bf16; int64_t n; } rrtmgp_mlp_param;
+int rrtmgp_hip_mlp_adam_arrays(int count, const rrtmgp_mlp_param* params, float lr, float beta1, float beta2,
+                               float eps, int64_t step, void* stream);
+/* Gradients of the mean squared normalised error over the rows idx (device) of a training set   */
+/* (X (rows, 16) raw inputs, Y (rows, n_out) raw targets), with respect to net's weights and      */
+/* biases.  loss_parts (n_loss >= 2 ceil(batch / 32)) receives sums of squared errors of groups  */
+/* of 16 rows, then zeros.                                                                       */
+int rrtmgp_hip_mlp_train_grads(const rrtmgp_mlp_net* net, const float* X, const float* Y, const int64_t* idx,
+                               int64_t batch, float* gW1, float* gb1, float* gW2, float* gb2, float* gW3,
+                               float* gb3, float* loss_parts, int64_t n_loss, void* stream);
 int rrtmgp_hip_mlp_to_bf16(int64_t n, const float* x, void* y, void* stream);
 /* Training data from the plain gas optics: raw inputs X (ncol nlay, 16) with row = icol +      */
 /* ncol ilay; targets Y (ncol nlay, 2 ngpt) from LW (a = tau, b = lay_src) or SW (a = tau,       */

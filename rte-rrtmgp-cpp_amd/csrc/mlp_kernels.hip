@@ -190,12 +190,10 @@ void bias_partial_kernel(int64_t rows, int n, int64_t chunk, const float* __rest
 }
 
 // Adam on FP32 master weights; writes the BF16 copy (Kingma & Ba 2015, bias-corrected).
-__global__ void adam_kernel(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                            float* __restrict__ v, __bf16* __restrict__ p16, float lr, float b1, float b2, float eps,
-                            float c1, float c2)
+__device__ __forceinline__ void adam_element(int64_t i, float* __restrict__ p, const float* __restrict__ g,
+                                             float* __restrict__ m, float* __restrict__ v, __bf16* __restrict__ p16,
+                                             float lr, float b1, float b2, float eps, float c1, float c2)
 {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
     const float gi = g[i];
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
@@ -204,6 +202,14 @@ __global__ void adam_kernel(int64_t n, float* __restrict__ p, const float* __res
     const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     p[i] = pi;
     if (p16) p16[i] = __bf16(pi);
+}
+
+__global__ void adam_kernel(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
+                            float* __restrict__ v, __bf16* __restrict__ p16, float lr, float b1, float b2, float eps,
+                            float c1, float c2)
+{
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) adam_element(i, p, g, m, v, p16, lr, b1, b2, eps, c1, c2);
 }
 
 // FP32 -> BF16.
@@ -679,6 +685,396 @@ __global__ void normalize_rows_kernel(int64_t rows, int n, int n_norm, const flo
 }
 
 // ---------------------------------------------------------------------------------------------
+// One training step's gradients.  Everything from the gathered inputs to dZ1 is local to a row, so one kernel
+// carries 16 rows of the batch through the forward and the backward pass in LDS and registers, and only what
+// the weight gradients sum over the rows leaves it: bf16 activations and errors, stored with the rows fastest
+// so that both operands of the weight-gradient products are read as 16-byte pieces along their summed index,
+// and FP32 row sums of the errors for the biases.  Three launches instead of 21; each of those was far from any
+// bandwidth or matrix-core bound (8 products of 24 us at a batch of 4096, with scalar bf16 loads).
+// 16 rows a work-group: 256 work-groups at a batch of 4096, one per compute unit; the weights (164 KB at 512
+// outputs) come from the L2.  Batch 4096, 512 outputs: 26 us here, 13 us weight gradients, 6 us sums and 6 us
+// Adam; a training step took 332 us with the separate kernels and takes 69 us.
+//
+// v_mfma_f32_16x16x32_bf16: for D(16x16) += A(16x32) B(32x16), lane l holds A[l%16][8(l/16) .. +7],
+// B[8(l/16) .. +7][l%16] and D rows 4(l/16) + r (register r = 0..3) of column l%16.
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int TR_ROWS = 16;          // rows per work-group
+constexpr int TR_WAVES = 8;          // one 16-column tile of the 128-wide layers each
+constexpr int TR_LD = MLP_H + 8;     // activations in LDS: 16-byte rows
+// Weights in LDS, read along k (forward: two 8-byte pieces) and along the rows (backward: eight 2-byte reads a
+// lane, rows 8(l/16) + e): with 264-byte rows the four row groups fall into different banks.
+constexpr int TR_LDW = MLP_H + 4;
+
+struct MlpTrain
+{
+    const float* X;          // (set rows, 16) raw inputs, (set rows, no) targets
+    const float* Y;
+    const int64_t* idx;      // rows of the batch
+    int64_t rows, ldr;       // batch, and rounded up to 32: rows of the transposed arrays
+    __bf16* xT;              // (16, ldr), (128, ldr) x 4, (no, ldr)
+    __bf16* h1T;
+    __bf16* h2T;
+    __bf16* dz1T;
+    __bf16* dz2T;
+    __bf16* dyT;
+    float* bias_part;        // (ldr / 16, 128 + 128 + no): row sums of dZ1, dZ2, dY per work-group
+    float* loss;             // (nloss): squared error per work-group, then zeros
+    int64_t nloss;
+};
+
+__device__ __forceinline__ bf16x8 lds_bf16x8(const __bf16* p)      // 8-byte aligned
+{
+    const bf16x4 a = *reinterpret_cast<const bf16x4*>(p), b = *reinterpret_cast<const bf16x4*>(p + 4);
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// D = A W^T for A (16 x 128) as fragments and a wavefront's 16 rows (n) of W in LDS.
+__device__ __forceinline__ f32x4 train_forward(const bf16x8* a, const __bf16* W, int lane)
+{
+    f32x4 acc = {};
+    const __bf16* p = W + (lane % 16) * TR_LDW + 8 * (lane / 16);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc = mfma16(a[s], lds_bf16x8(p + 32 * s), acc);
+    return acc;
+}
+
+// D += E W for E (16 x 128) in LDS and a wavefront's 16 columns (h0 ..) of W in LDS.
+__device__ __forceinline__ f32x4 train_backward(f32x4 acc, const __bf16 (*E)[TR_LD], const __bf16* W, int h0, int lane)
+{
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+    {
+        const int k = 32 * s + 8 * (lane / 16);
+        bf16x8 b;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b[e] = W[(k + e) * TR_LDW + h0 + lane % 16];
+        acc = mfma16(load_bf16x8(&E[lane % 16][k]), b, acc);
+    }
+    return acc;
+}
+
+// A wavefront's 16 x 16 tile (rows 4(l/16) + r, column l%16): to LDS and to the transposed array.
+__device__ __forceinline__ void train_put(const float* v, __bf16 (*S)[TR_LD], int col, __bf16* T, int64_t ldr,
+                                          int64_t row0, int lane)
+{
+    bf16x4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+    {
+        o[r] = __bf16(v[r]);
+        if (S) S[4 * (lane / 16) + r][col] = o[r];
+    }
+    *reinterpret_cast<bf16x4*>(T + int64_t(col) * ldr + row0 + 4 * (lane / 16)) = o;
+}
+
+__device__ __forceinline__ void train_bias(const float* v, float* part, int lane)
+{
+    float s = (v[0] + v[1]) + (v[2] + v[3]);
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (lane < 16) part[lane] = s;
+}
+
+__global__ __launch_bounds__(64 * TR_WAVES)
+void mlp_train_kernel(MlpNet net, MlpTrain t)
+{
+    __shared__ __align__(16) __bf16 sW2[MLP_H * TR_LDW];
+    __shared__ __align__(16) __bf16 sW3[MLP_H * TR_LDW];      // 128 outputs at a time
+    __shared__ __align__(16) __bf16 sX[TR_ROWS][32 + 8];
+    __shared__ __align__(16) __bf16 sH1[TR_ROWS][TR_LD];
+    __shared__ __align__(16) __bf16 sH2[TR_ROWS][TR_LD];
+    __shared__ __align__(16) __bf16 sE[TR_ROWS][TR_LD];
+    __shared__ float s_loss[TR_WAVES];
+    const int tid = threadIdx.x, lane = tid % 64;
+    const int w = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int col = 16 * w + lane % 16;                       // of the 128-wide layers
+    const int64_t row0 = int64_t(blockIdx.x) * TR_ROWS;
+    const int no = net.no, nb = 2 * MLP_H + no;
+    float* bias_part = t.bias_part + int64_t(blockIdx.x) * nb;
+
+    // 128 x 128 weights through registers: four 16-byte pieces a thread.
+    bf16x8 wreg[4];
+    const auto fetch = [&](const __bf16* W, int n) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+        {
+            const int v = tid + 64 * TR_WAVES * i;
+            wreg[i] = v / 16 < n ? load_bf16x8(W + (v / 16) * MLP_H + v % 16 * 8) : bf16x8{};
+        }
+    };
+    const auto put = [&](__bf16* S) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+        {
+            const int v = tid + 64 * TR_WAVES * i;
+            __bf16* p = S + (v / 16) * TR_LDW + v % 16 * 8;
+            *reinterpret_cast<bf16x4*>(p) = __builtin_shufflevector(wreg[i], wreg[i], 0, 1, 2, 3);
+            *reinterpret_cast<bf16x4*>(p + 4) = __builtin_shufflevector(wreg[i], wreg[i], 4, 5, 6, 7);
+        }
+    };
+    fetch(net.W2, MLP_H);
+
+    // Set rows of this lane's four rows of a tile (-1: past the batch).
+    int64_t src[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+    {
+        const int64_t row = row0 + 4 * (lane / 16) + r;
+        src[r] = row < t.rows ? t.idx[row] : -1;
+    }
+    if (tid < TR_ROWS * 32)
+    {
+        const int r = tid / 32, c = tid % 32;
+        float v = 0.f;
+        if (c < MLP_IN && row0 + r < t.rows)
+            v = (t.X[t.idx[row0 + r] * MLP_INP + c] - net.x_mean[c]) / net.x_std[c];
+        const __bf16 x = __bf16(v);
+        sX[r][c] = x;
+        if (c < MLP_INP) t.xT[int64_t(c) * t.ldr + row0 + r] = x;
+    }
+    put(sW2);
+    fetch(net.W3, no);
+    __syncthreads();
+
+    float z1[4], z2[4], v[4];
+    {
+        // K = 16, padded with zeros to 32.
+        const int k = 8 * (lane / 16);
+        const bf16x8 b = k < MLP_INP ? load_bf16x8(net.W1 + col * MLP_INP + k) : bf16x8{};
+        const f32x4 acc = mfma16(load_bf16x8(&sX[lane % 16][k]), b, f32x4{});
+        const float bias = net.b1[col];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            z1[r] = acc[r] + bias;
+            v[r] = softplus(z1[r]);
+        }
+        train_put(v, sH1, col, t.h1T, t.ldr, row0, lane);
+    }
+    put(sW3);
+    __syncthreads();
+    bf16x8 a[4];
+    {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[s] = load_bf16x8(&sH1[lane % 16][32 * s + 8 * (lane / 16)]);
+        const f32x4 acc = train_forward(a, sW2 + 16 * w * TR_LDW, lane);
+        const float bias = net.b2[col];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            z2[r] = acc[r] + bias;
+            v[r] = softplus(z2[r]);
+        }
+        train_put(v, sH2, col, t.h2T, t.ldr, row0, lane);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) a[s] = load_bf16x8(&sH2[lane % 16][32 * s + 8 * (lane / 16)]);
+
+    // Output layer, its error and dH2, 128 outputs at a time.
+    f32x4 dh = {};
+    float loss = 0.f;
+    const float count = float(t.rows * no);
+    for (int n0 = 0; n0 < no; n0 += MLP_H)
+    {
+        const int n = n0 + col;
+        float y[4] = {}, mean = 0.f, std_ = 1.f, bias = 0.f;
+        if (n < no)
+        {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = src[r] >= 0 ? t.Y[src[r] * no + n] : 0.f;
+            mean = net.y_mean[n];
+            std_ = net.y_std[n];
+            bias = net.b3[n];
+        }
+        if (n0 + MLP_H < no) fetch(net.W3 + int64_t(n0 + MLP_H) * MLP_H, no - (n0 + MLP_H));
+        const f32x4 acc = train_forward(a, sW3 + 16 * w * TR_LDW, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const float d = (acc[r] + bias) - (y[r] - mean) / std_;
+            const bool in = n < no && src[r] >= 0;
+            v[r] = in ? 2.f * d / count : 0.f;
+            loss += in ? d * d : 0.f;
+        }
+        // Outputs come in whole tiles of 32, so a wavefront's 16 columns are all in or all out.
+        if (n < no)
+        {
+            train_put(v, nullptr, n, t.dyT, t.ldr, row0, lane);
+            train_bias(v, bias_part + 2 * MLP_H + n0 + 16 * w, lane);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sE[4 * (lane / 16) + r][col] = __bf16(v[r]);
+        __syncthreads();
+        dh = train_backward(dh, sE, sW3, 16 * w, lane);
+        __syncthreads();
+        if (n0 + MLP_H < no)
+        {
+            put(sW3);
+            __syncthreads();
+        }
+    }
+
+    // dZ = dH softplus'(Z) of the two hidden layers.
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = dh[r] * sigmoid(z2[r]);
+    train_put(v, sE, col, t.dz2T, t.ldr, row0, lane);
+    train_bias(v, bias_part + MLP_H + 16 * w, lane);
+    __syncthreads();
+    dh = train_backward(f32x4{}, sE, sW2, 16 * w, lane);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = dh[r] * sigmoid(z1[r]);
+    train_put(v, nullptr, col, t.dz1T, t.ldr, row0, lane);
+    train_bias(v, bias_part + 16 * w, lane);
+
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) loss += __shfl_xor(loss, m);
+    if (lane == 0) s_loss[w] = loss;
+    __syncthreads();
+    if (tid == 0)
+    {
+        float s = 0.f;
+        for (int i = 0; i < TR_WAVES; ++i) s += s_loss[i];
+        for (int64_t i = blockIdx.x; i < t.nloss; i += gridDim.x) t.loss[i] = i == blockIdx.x ? s : 0.f;
+    }
+}
+
+// Weight gradients dW(m, n) = sum over rows of E(row, m) H(row, n), from the transposed arrays: a wavefront
+// takes a 32 x 32 tile (32 x 16 for W1) over a range of rows, operands straight from the L2 (each piece is read
+// by four wavefronts at most); the four wavefronts of a work-group share the tile and add their parts in LDS.
+// Work-group (tile, z) leaves its part in part[z]: W1, W2, W3 after each other, row-major.
+constexpr int WG_WAVES = 4;
+
+struct MlpGradTiles { int no; int64_t ldr, chunk; };
+
+__global__ __launch_bounds__(64 * WG_WAVES)
+void mlp_weight_grad_kernel(MlpGradTiles q, MlpTrain t, float* __restrict__ part)
+{
+    __shared__ float red[WG_WAVES - 1][64][16 + 1];
+    const int lane = threadIdx.x % 64;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int n3 = q.no / 32 * 4;
+    int b = blockIdx.x;
+    const __bf16 *E, *H;
+    int m0, h0, N, nt = 2;
+    float* out = part + int64_t(blockIdx.y) * (MLP_H * MLP_INP + MLP_H * MLP_H + q.no * MLP_H);
+    if (b < n3)
+    {
+        E = t.dyT; H = t.h2T; N = MLP_H;
+        m0 = b / 4 * 32; h0 = b % 4 * 32;
+        out += MLP_H * MLP_INP + MLP_H * MLP_H;
+    }
+    else if ((b -= n3) < 16)
+    {
+        E = t.dz2T; H = t.h1T; N = MLP_H;
+        m0 = b / 4 * 32; h0 = b % 4 * 32;
+        out += MLP_H * MLP_INP;
+    }
+    else
+    {
+        b -= 16;
+        E = t.dz1T; H = t.xT; N = MLP_INP;
+        m0 = b * 32; h0 = 0; nt = 1;
+    }
+    const int64_t k0 = (int64_t(blockIdx.y) * WG_WAVES + w) * q.chunk, k1 = min(q.ldr, k0 + q.chunk);
+    const __bf16* pe = E + (m0 + lane % 16) * q.ldr + 8 * (lane / 16);
+    const __bf16* ph = H + (h0 + lane % 16) * q.ldr + 8 * (lane / 16);
+    const int64_t up = 16 * q.ldr, uh = nt == 2 ? up : 0;
+    f32x4 acc[4] = {};
+#pragma unroll 4
+    for (int64_t k = k0; k < k1; k += 32)
+    {
+        const bf16x8 e0 = load_bf16x8(pe + k), e1 = load_bf16x8(pe + up + k);
+        const bf16x8 x0 = load_bf16x8(ph + k), x1 = load_bf16x8(ph + uh + k);
+        acc[0] = mfma16(e0, x0, acc[0]);
+        acc[1] = mfma16(e1, x0, acc[1]);
+        acc[2] = mfma16(e0, x1, acc[2]);
+        acc[3] = mfma16(e1, x1, acc[3]);
+    }
+    if (w > 0)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) red[w - 1][lane][i] = acc[i / 4][i % 4];
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+    {
+        float s = acc[i / 4][i % 4];
+#pragma unroll
+        for (int v = 0; v < WG_WAVES - 1; ++v) s += red[v][lane][i];
+        const int m = m0 + 16 * (i / 4 % 2) + 4 * (lane / 16) + i % 4, h = h0 + 16 * (i / 8) + lane % 16;
+        if (i < 8 || nt == 2) out[int64_t(m) * N + h] = s;
+    }
+}
+
+// The gradients: parts of the weights added in order, 16 slices of the biases' row sums each in order and then
+// the slices, so the result does not depend on scheduling.
+struct MlpGrads { float *W1, *W2, *W3, *b1, *b2, *b3; };
+
+__global__ __launch_bounds__(256)
+void mlp_grad_sum_kernel(int no, int nz, const float* __restrict__ part, int nwg, const float* __restrict__ bias_part,
+                         unsigned weight_blocks, MlpGrads g)
+{
+    __shared__ float red[16][16];
+    constexpr int n1 = MLP_H * MLP_INP, n2 = MLP_H * MLP_H;
+    const int total = n1 + n2 + no * MLP_H, nb = 2 * MLP_H + no;
+    if (blockIdx.x < weight_blocks)
+    {
+        const int i = blockIdx.x * 256 + threadIdx.x;
+        if (i >= total) return;
+        float s = 0.f;
+        for (int z = 0; z < nz; ++z) s += part[int64_t(z) * total + i];
+        if (i < n1) g.W1[i] = s;
+        else if (i < n1 + n2) g.W2[i - n1] = s;
+        else g.W3[i - n1 - n2] = s;
+        return;
+    }
+    const int c = threadIdx.x % 16, q = threadIdx.x / 16;
+    const int j = (blockIdx.x - weight_blocks) * 16 + c;       // nb is a multiple of 16
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = q; k < nwg; k += 16) s += bias_part[int64_t(k) * nb + j];
+    red[q][c] = s;
+    __syncthreads();
+    if (q > 0) return;
+    s = 0.f;
+    for (int k = 0; k < 16; ++k) s += red[k][c];
+    if (j < MLP_H) g.b1[j] = s;
+    else if (j < 2 * MLP_H) g.b2[j - MLP_H] = s;
+    else g.b3[j - 2 * MLP_H] = s;
+}
+
+// Adam over several parameter arrays in one launch; work-groups first[i] .. first[i + 1) belong to array i.
+constexpr int ADAM_MAX = 16;
+struct AdamArrays
+{
+    float* p[ADAM_MAX];
+    const float* g[ADAM_MAX];
+    float* m[ADAM_MAX];
+    float* v[ADAM_MAX];
+    __bf16* p16[ADAM_MAX];
+    int64_t n[ADAM_MAX];
+    unsigned first[ADAM_MAX + 1];
+    int count;
+};
+
+__global__ void adam_arrays_kernel(AdamArrays a, float lr, float b1, float b2, float eps, float c1, float c2)
+{
+    int k = 0;
+    while (k + 1 < a.count && blockIdx.x >= a.first[k + 1]) ++k;
+    const int64_t i = int64_t(blockIdx.x - a.first[k]) * blockDim.x + threadIdx.x;
+    if (i >= a.n[k]) return;
+    adam_element(i, a.p[k], a.g[k], a.m[k], a.v[k], a.p16[k], lr, b1, b2, eps, c1, c2);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Launchers.
 int gemm_bf16(int64_t M, int64_t N, int64_t K, const void* A, int64_t sAm, int64_t sAk, const void* B, int64_t sBk,
               int64_t sBn, float* C, int64_t sCm, int64_t sCn, int accumulate, void* stream)
@@ -841,6 +1237,103 @@ static int make_mlp_gases(const rrtmgp_gas_vmr* g, int64_t ncol, int64_t nlay, M
         out.scol[i] = d1 == 1 ? 0 : 1;
         out.slay[i] = d2 == 1 ? 0 : d1;
     }
+    return RRTMGP_OK;
+}
+
+extern "C++" {
+namespace
+{
+template<typename T>
+T* carve(char*& p, size_t n)
+{
+    T* r = reinterpret_cast<T*>(p);
+    p += (n * sizeof(T) + 255) / 256 * 256;
+    return r;
+}
+}
+}
+
+int rrtmgp_hip_mlp_train_grads(const rrtmgp_mlp_net* n, const float* X, const float* Y, const int64_t* idx,
+                               int64_t batch, float* gW1, float* gb1, float* gW2, float* gb2, float* gW3, float* gb3,
+                               float* loss_parts, int64_t n_loss, void* stream)
+{
+    MlpNet net;
+    RRTMGP_TRY(make_mlp_net(n, net));
+    if (batch <= 0 || !X || !Y || !idx || !gW1 || !gb1 || !gW2 || !gb2 || !gW3 || !gb3 || !loss_parts)
+        return arg_error("mlp_train_grads: bad arguments");
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(net.W1) | reinterpret_cast<uintptr_t>(net.W2) |
+                           reinterpret_cast<uintptr_t>(net.W3);
+    if (bits & 15) return arg_error("mlp_train_grads: weights must be 16-byte aligned");
+    const int64_t ldr = (batch + 31) / 32 * 32, nwg = ldr / TR_ROWS;
+    if (n_loss < nwg) return arg_error("mlp_train_grads: one loss part per 16 rows, rounded up to 32 rows");
+    const int no = net.no, nb = 2 * MLP_H + no;
+    const int64_t total = MLP_H * MLP_INP + MLP_H * MLP_H + int64_t(no) * MLP_H;
+    // Rows per wavefront of the weight gradients: 256 where the batch is long enough to keep the chip busy so
+    // (84 tiles at 512 outputs; 336 work-groups of four wavefronts at a batch of 4096), and 16 parts at most.
+    const int64_t nz = std::max<int64_t>(1, std::min<int64_t>(16, ldr / (256 * WG_WAVES)));
+    const int64_t chunk = ((ldr + nz * WG_WAVES - 1) / (nz * WG_WAVES) + 31) / 32 * 32;
+    const hipStream_t s = as_stream(stream);
+    char* base = nullptr;
+    const size_t bytes = size_t(ldr) * size_t(MLP_INP + 4 * MLP_H + no) * 2 + size_t(nwg * nb) * 4 +
+                         size_t(nz * total) * 4 + 16 * 256;
+    RRTMGP_TRY(scratch_alloc(&base, bytes, s));
+    char* p = base;
+    MlpTrain t;
+    t.X = X; t.Y = Y; t.idx = idx; t.rows = batch; t.ldr = ldr;
+    t.xT = carve<__bf16>(p, size_t(ldr) * MLP_INP);
+    t.h1T = carve<__bf16>(p, size_t(ldr) * MLP_H);
+    t.h2T = carve<__bf16>(p, size_t(ldr) * MLP_H);
+    t.dz1T = carve<__bf16>(p, size_t(ldr) * MLP_H);
+    t.dz2T = carve<__bf16>(p, size_t(ldr) * MLP_H);
+    t.dyT = carve<__bf16>(p, size_t(ldr) * no);
+    t.bias_part = carve<float>(p, size_t(nwg * nb));
+    float* part = carve<float>(p, size_t(nz * total));
+    t.loss = loss_parts; t.nloss = n_loss;
+    const auto run = [&]() -> int {
+        {
+            RRTMGP_TIMED("mlp_train_kernel", s);
+            hipLaunchKernelGGL(mlp_train_kernel, dim3(unsigned(nwg)), dim3(64 * TR_WAVES), 0, s, net, t);
+            RRTMGP_LAUNCHED("mlp_train_kernel");
+        }
+        {
+            RRTMGP_TIMED("mlp_weight_grad_kernel", s);
+            hipLaunchKernelGGL(mlp_weight_grad_kernel, dim3(no / 32 * 4 + 16 + 4, unsigned(nz)), dim3(64 * WG_WAVES), 0,
+                               s, MlpGradTiles{no, ldr, chunk}, t, part);
+            RRTMGP_LAUNCHED("mlp_weight_grad_kernel");
+        }
+        RRTMGP_TIMED("mlp_grad_sum_kernel", s);
+        const unsigned wb = grid1(total, 256);
+        hipLaunchKernelGGL(mlp_grad_sum_kernel, dim3(wb + nb / 16), dim3(256), 0, s, no, int(nz), part, int(nwg),
+                           t.bias_part, wb, MlpGrads{gW1, gW2, gW3, gb1, gb2, gb3});
+        RRTMGP_LAUNCHED("mlp_grad_sum_kernel");
+        return RRTMGP_OK;
+    };
+    const int rc = run();
+    scratch_free(base, s);
+    return rc;
+}
+
+int rrtmgp_hip_mlp_adam_arrays(int count, const rrtmgp_mlp_param* params, float lr, float beta1, float beta2, float eps,
+                               int64_t step, void* stream)
+{
+    if (count <= 0 || count > ADAM_MAX || !params || step < 1) return arg_error("mlp_adam_arrays: bad arguments");
+    AdamArrays a;
+    a.count = count;
+    a.first[0] = 0;
+    for (int i = 0; i < count; ++i)
+    {
+        const rrtmgp_mlp_param& q = params[i];
+        if (q.n <= 0 || !q.p || !q.g || !q.m || !q.v) return arg_error("mlp_adam_arrays: bad arguments");
+        a.p[i] = q.p; a.g[i] = q.g; a.m[i] = q.m; a.v[i] = q.v;
+        a.p16[i] = static_cast<__bf16*>(q.p_bf16);
+        a.n[i] = q.n;
+        a.first[i + 1] = a.first[i] + grid1(q.n, 256);
+    }
+    const float c1 = 1.f - std::pow(beta1, float(step)), c2 = 1.f - std::pow(beta2, float(step));
+    RRTMGP_TIMED("adam_arrays_kernel", as_stream(stream));
+    hipLaunchKernelGGL(adam_arrays_kernel, dim3(a.first[count]), dim3(256), 0, as_stream(stream), a, lr, beta1, beta2,
+                       eps, c1, c2);
+    RRTMGP_LAUNCHED("adam_arrays_kernel");
     return RRTMGP_OK;
 }
 

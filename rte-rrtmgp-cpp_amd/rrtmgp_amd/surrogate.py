@@ -43,6 +43,10 @@ class MlpNetC(C.Structure):
                                           "x_hi", "y_mean", "y_std")] + [("n_out", C.c_int64), ("p_trop", C.c_double)]
 
 
+class MlpParamC(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("p", "g", "m", "v", "p_bf16")] + [("n", C.c_int64)]
+
+
 def _L():
     return _lib.hip()
 
@@ -262,66 +266,32 @@ class MlpGasOptics:
 
     # -- training ------------------------------------------------------------------------------
     def _workspace(self, B):
-        if self._ws is not None and self._ws["B"] == B:
-            return self._ws
-        H, no = HIDDEN, self.n_out
-        f32 = lambda *s: DeviceArray(s, np.float32)                         # noqa: E731
-        b16 = lambda *s: DeviceArray(s, np.uint16)                          # noqa: E731
-        ws = dict(B=B, idx=DeviceArray((B,), np.int64), xr=f32(B * N_INP), yr=f32(B * no), X16=b16(B * N_INP),
-                  Yn=f32(B * no), Z1=f32(B * H), H1=b16(B * H), Z2=f32(B * H), H2=b16(B * H), Yp=f32(B * no),
-                  dY16=b16(B * no), dYf=f32(B * no), loss=f32((B * no + 255) // 256), dH=f32(B * H),
-                  dZ16=b16(B * H), dZf=f32(B * H))
-        self._ws = ws
-        return ws
-
-    def _gemm(self, M, N, K, A, sAm, sAk, B, sBk, sBn, Cm, sCm, sCn, acc=0):
-        _chk(_L().rrtmgp_hip_mlp_gemm_bf16(_i(M), _i(N), _i(K), A.ptr, _i(sAm), _i(sAk), B.ptr, _i(sBk), _i(sBn),
-                                           Cm.ptr, _i(sCm), _i(sCn), C.c_int(acc), None))
+        if self._ws is None or self._ws["B"] != B:
+            parts = max((B * self.n_out + 255) // 256, 2 * ((B + 31) // 32))
+            self._ws = dict(B=B, idx=DeviceArray((B,), np.int64, zero=False),
+                            loss=DeviceArray((parts,), np.float32, zero=False))
+        return self._ws
 
     def forward_backward(self, ts: TrainingSet, idx: np.ndarray) -> DeviceArray:
         """One forward/backward pass over rows idx; leaves gradients in the parameters' g buffers and
-        returns the per-block loss partial sums (sum of squared normalised errors)."""
-        L = _L()
-        B, H, no = len(idx), HIDDEN, self.n_out
+        returns the loss as partial sums (of squared normalised errors)."""
+        B = len(idx)
         ws = self._workspace(B)
-        st = self.stats
-        _chk(L.rrtmgp_hip_memcpy_h2d(ws["idx"].ptr, np.ascontiguousarray(idx, np.int64).ctypes.data_as(C.c_void_p),
-                                     C.c_size_t(8 * B), None))
-        _chk(L.rrtmgp_hip_mlp_gather_rows(_i(B), C.c_int(N_INP), ws["idx"].ptr, ts.X.ptr, ws["xr"].ptr, None))
-        _chk(L.rrtmgp_hip_mlp_normalize_rows(_i(B), C.c_int(N_INP), C.c_int(N_IN), ws["xr"].ptr, st["x_mean"].ptr,
-                                             st["x_std"].ptr, ws["X16"].ptr, None, None))
-        _chk(L.rrtmgp_hip_mlp_gather_rows(_i(B), C.c_int(no), ws["idx"].ptr, ts.Y.ptr, ws["yr"].ptr, None))
-        _chk(L.rrtmgp_hip_mlp_normalize_rows(_i(B), C.c_int(no), C.c_int(no), ws["yr"].ptr, st["y_mean"].ptr,
-                                             st["y_std"].ptr, None, ws["Yn"].ptr, None))
-        # Forward: Z1 = X W1^T, H1 = softplus(Z1 + b1), ..., Y = H2 W3^T + b3.
-        self._gemm(B, H, N_INP, ws["X16"], N_INP, 1, self.W1.b16, 1, N_INP, ws["Z1"], H, 1)
-        _chk(L.rrtmgp_hip_mlp_bias_softplus(_i(B), C.c_int(H), ws["Z1"].ptr, self.b1.p.ptr, ws["H1"].ptr, None))
-        self._gemm(B, H, H, ws["H1"], H, 1, self.W2.b16, 1, H, ws["Z2"], H, 1)
-        _chk(L.rrtmgp_hip_mlp_bias_softplus(_i(B), C.c_int(H), ws["Z2"].ptr, self.b2.p.ptr, ws["H2"].ptr, None))
-        self._gemm(B, no, H, ws["H2"], H, 1, self.W3.b16, 1, H, ws["Yp"], no, 1)
-        _chk(L.rrtmgp_hip_mlp_mse_grad(_i(B), C.c_int(no), ws["Yp"].ptr, self.b3.p.ptr, ws["Yn"].ptr,
-                                       ws["dY16"].ptr, ws["dYf"].ptr, ws["loss"].ptr, None))
-        # Backward.
-        self._gemm(no, H, B, ws["dY16"], 1, no, ws["H2"], H, 1, self.W3.g, H, 1)          # dW3 = dY^T H2
-        _chk(L.rrtmgp_hip_mlp_bias_grad(_i(B), C.c_int(no), ws["dYf"].ptr, self.b3.g.ptr, None))
-        self._gemm(B, H, no, ws["dY16"], no, 1, self.W3.b16, H, 1, ws["dH"], H, 1)        # dH2 = dY W3
-        _chk(L.rrtmgp_hip_mlp_softplus_back(_i(B * H), ws["dH"].ptr, ws["Z2"].ptr, ws["dZ16"].ptr, ws["dZf"].ptr,
-                                            None))
-        self._gemm(H, H, B, ws["dZ16"], 1, H, ws["H1"], H, 1, self.W2.g, H, 1)            # dW2 = dZ2^T H1
-        _chk(L.rrtmgp_hip_mlp_bias_grad(_i(B), C.c_int(H), ws["dZf"].ptr, self.b2.g.ptr, None))
-        self._gemm(B, H, H, ws["dZ16"], H, 1, self.W2.b16, H, 1, ws["dH"], H, 1)          # dH1 = dZ2 W2
-        _chk(L.rrtmgp_hip_mlp_softplus_back(_i(B * H), ws["dH"].ptr, ws["Z1"].ptr, ws["dZ16"].ptr, ws["dZf"].ptr,
-                                            None))
-        self._gemm(H, N_INP, B, ws["dZ16"], 1, H, ws["X16"], N_INP, 1, self.W1.g, N_INP, 1)  # dW1 = dZ1^T X
-        _chk(L.rrtmgp_hip_mlp_bias_grad(_i(B), C.c_int(H), ws["dZf"].ptr, self.b1.g.ptr, None))
+        _chk(_L().rrtmgp_hip_memcpy_h2d(ws["idx"].ptr, np.ascontiguousarray(idx, np.int64).ctypes.data_as(C.c_void_p),
+                                        C.c_size_t(8 * B), None))
+        net = self._net_struct()
+        _chk(_L().rrtmgp_hip_mlp_train_grads(
+            C.byref(net), ts.X.ptr, ts.Y.ptr, ws["idx"].ptr, _i(B), self.W1.g.ptr, self.b1.g.ptr, self.W2.g.ptr,
+            self.b2.g.ptr, self.W3.g.ptr, self.b3.g.ptr, ws["loss"].ptr, _i(ws["loss"].size), None))
         return ws["loss"]
 
     def adam_step(self, lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8):
         self.step += 1
-        for p in self.params:
-            _chk(_L().rrtmgp_hip_mlp_adam(_i(p.n), p.p.ptr, p.g.ptr, p.m.ptr, p.v.ptr,
-                                          p.b16.ptr if p.b16 is not None else None, _f(lr), _f(beta1), _f(beta2),
-                                          _f(eps), _i(self.step), None))
+        q = (MlpParamC * len(self.params))(*[
+            MlpParamC(p.p.ptr, p.g.ptr, p.m.ptr, p.v.ptr, p.b16.ptr if p.b16 is not None else None, p.n)
+            for p in self.params])
+        _chk(_L().rrtmgp_hip_mlp_adam_arrays(C.c_int(len(q)), q, _f(lr), _f(beta1), _f(beta2), _f(eps),
+                                             _i(self.step), None))
         self._cnet = None
 
     def train(self, ts: TrainingSet, steps=60000, batch=4096, lr=1e-3, lr_final=1e-5, decay_from=0.5, seed=2,
@@ -350,16 +320,19 @@ class MlpGasOptics:
         return float(l.to_host().sum()) / (len(idx) * self.n_out)
 
     # -- inference -----------------------------------------------------------------------------
+    def _net_struct(self) -> MlpNetC:
+        st = self.stats
+        return MlpNetC(self.W1.b16.ptr.value, self.W2.b16.ptr.value, self.W3.b16.ptr.value,
+                       self.b1.p.ptr.value, self.b2.p.ptr.value, self.b3.p.ptr.value,
+                       st["x_mean"].ptr.value, st["x_std"].ptr.value, st["x_lo"].ptr.value,
+                       st["x_hi"].ptr.value, st["y_mean"].ptr.value, st["y_std"].ptr.value, self.n_out,
+                       self.p_trop)
+
     def c_net(self) -> MlpNetC:
         if self.stats is None:
             raise RuntimeError("the surrogate has no normalisation (train it or load weights first)")
         if getattr(self, "_cnet", None) is None:
-            st = self.stats
-            self._cnet = MlpNetC(self.W1.b16.ptr.value, self.W2.b16.ptr.value, self.W3.b16.ptr.value,
-                                 self.b1.p.ptr.value, self.b2.p.ptr.value, self.b3.p.ptr.value,
-                                 st["x_mean"].ptr.value, st["x_std"].ptr.value, st["x_lo"].ptr.value,
-                                 st["x_hi"].ptr.value, st["y_mean"].ptr.value, st["y_std"].ptr.value, self.n_out,
-                                 self.p_trop)
+            self._cnet = self._net_struct()
         return self._cnet
 
     def host_weights(self) -> dict:
