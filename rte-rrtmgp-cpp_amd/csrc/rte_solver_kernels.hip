@@ -6,7 +6,7 @@
 // src_kernels_cuda/rte_solver_kernels.cu:581-583.
 //
 // Layout of the work.  A work-group is 64 columns (the lanes of each wavefront) x up to 16
-// g-points of one band (one wavefront each).  Each thread runs the layer recurrences of one
+// g-points of one band (one wavefront each; up to 8 or 4 where there are few columns).  Each thread runs the layer recurrences of one
 // (column, g-point); every layer step of a wavefront reads one contiguous 256-byte row of the
 // (ncol, nlay, ngpt) inputs.  Fluxes are summed over the g-points of the work-group in LDS
 // every K levels (a fixed order, so results are reproducible), giving per-band partial fluxes
@@ -48,25 +48,34 @@ namespace rrtmgp_hip
 // LW segment inputs are double-buffered in registers (K1 for one angle, K4 for up to four), sized
 // for 64 VGPRs in FP32 (two 1024-thread work-groups per CU) without spills; the SW segment
 // registers fit the 128 VGPRs of a 1024-thread work-group.
+// Work-groups cut for few columns (GP = 8 g-points at most, solver_groups.h) run one or two wavefronts
+// per SIMD and wait for memory at every segment: they have registers for longer segments (SEG8).
 template<typename Real> struct LwSeg;
 template<> struct LwSeg<float> { static constexpr int K1 = 6, K4 = 4; };
 template<> struct LwSeg<double> { static constexpr int K1 = 4, K4 = 4; };
+constexpr int SEG8 = 8;
+constexpr int SMALL_GPTS = 8;
+template<typename Real, int NMU, int GP>
+constexpr int lw_seg_k() { return GP < SB_GPTS ? SEG8 : NMU == 1 ? LwSeg<Real>::K1 : LwSeg<Real>::K4; }
 // The SW kernel's wide variant (FP32, co-albedo input, no heating rates) fits 64 VGPRs with
 // K = 3, so two 1024-thread work-groups share a CU; the others keep K = 4 at up to 128 VGPRs.
 constexpr bool sw_wide(bool fp32, bool co, bool hr) { return fp32 && co && !hr; }
-constexpr int sw_seg_k(bool fp32, bool co, bool hr) { return sw_wide(fp32, co, hr) ? 3 : 4; }
+constexpr int sw_seg_k(bool fp32, bool co, bool hr, int gp)
+{
+    return gp < SB_GPTS ? SEG8 : sw_wide(fp32, co, hr) ? 3 : 4;
+}
 
 // Writes the LDS slots kk < nslots, components c < NC, summed over the group's g-points, to
 // out[c] at level lev_of(kk) (skipped when negative).
-// red layout: ((kk * NC + c) * SB_GPTS + w) * SB_COLS + lane.
-template<typename Real, int NC, int STRIDE = NC, typename LevOf>
+// red layout: ((kk * NC + c) * GP + w) * SB_COLS + lane.
+template<int GP, typename Real, int NC, int STRIDE = NC, typename LevOf>
 __device__ __forceinline__ void write_group_sums(const Real* red, int nslots, int gcount, int64_t col0,
                                                  int64_t ncol, int64_t nlev, int gi, Real* const (&out)[NC],
                                                  LevOf lev_of)
 {
     const int tid = threadIdx.y * SB_COLS + threadIdx.x;
     const int items = nslots * NC * SB_COLS;
-    for (int it = tid; it < items; it += SB_COLS * SB_GPTS)
+    for (int it = tid; it < items; it += SB_COLS * int(blockDim.y))
     {
         const int lane = it % SB_COLS;
         const int rest = it / SB_COLS;
@@ -74,7 +83,7 @@ __device__ __forceinline__ void write_group_sums(const Real* red, int nslots, in
         const int64_t icol = col0 + lane;
         const int64_t lev = lev_of(kk);
         if (icol >= ncol || lev < 0) continue;
-        const Real* r = red + (int64_t(kk) * STRIDE + c) * SB_GPTS * SB_COLS + lane;
+        const Real* r = red + (int64_t(kk) * STRIDE + c) * GP * SB_COLS + lane;
         Real s = r[0];
         for (int w = 1; w < gcount; ++w) s += r[w * SB_COLS];
         out[c][icol + ncol * (lev + nlev * gi)] = s;
@@ -82,21 +91,21 @@ __device__ __forceinline__ void write_group_sums(const Real* red, int nslots, in
 }
 
 // write_group_sums for component 0 only of an LDS layout with NC components per slot.
-template<typename Real, int NC, typename LevOf>
+template<int GP, typename Real, int NC, typename LevOf>
 __device__ __forceinline__ void write_group_sums_stride(const Real* red, int nslots, int gcount, int64_t col0,
                                                         int64_t ncol, int64_t nlev, int gi,
                                                         Real* const (&out)[1], LevOf lev_of)
 {
     const int tid = threadIdx.y * SB_COLS + threadIdx.x;
     const int items = nslots * SB_COLS;
-    for (int it = tid; it < items; it += SB_COLS * SB_GPTS)
+    for (int it = tid; it < items; it += SB_COLS * int(blockDim.y))
     {
         const int lane = it % SB_COLS;
         const int kk = it / SB_COLS;
         const int64_t icol = col0 + lane;
         const int64_t lev = lev_of(kk);
         if (icol >= ncol || lev < 0) continue;
-        const Real* r = red + int64_t(kk) * NC * SB_GPTS * SB_COLS + lane;
+        const Real* r = red + int64_t(kk) * NC * GP * SB_COLS + lane;
         Real s = r[0];
         for (int w = 1; w < gcount; ++w) s += r[w * SB_COLS];
         out[0][icol + ncol * (lev + nlev * gi)] = s;
@@ -106,21 +115,21 @@ __device__ __forceinline__ void write_group_sums_stride(const Real* red, int nsl
 // Heating-rate island: each layer's absorbed flux (net-flux convergence) summed over the group's
 // g-points in FP64, for the LDS slots kk < nslots of component comp (NCH components per slot),
 // written to out[icol + ncol (layer + nlay gi)] for layer lay_of(kk) (skipped when negative).
-template<typename Real, int NCH, typename LayOf>
+template<int GP, typename Real, int NCH, typename LayOf>
 __device__ __forceinline__ void write_group_layer_sums(const Real* red, int comp, int nslots, int gcount,
                                                        int64_t col0, int64_t ncol, int64_t nlay, int gi,
                                                        double* out, LayOf lay_of)
 {
     const int tid = threadIdx.y * SB_COLS + threadIdx.x;
     const int items = nslots * SB_COLS;
-    for (int it = tid; it < items; it += SB_COLS * SB_GPTS)
+    for (int it = tid; it < items; it += SB_COLS * int(blockDim.y))
     {
         const int lane = it % SB_COLS;
         const int kk = it / SB_COLS;
         const int64_t icol = col0 + lane;
         const int64_t lay = lay_of(kk);
         if (icol >= ncol || lay < 0) continue;
-        const Real* r = red + (int64_t(kk) * NCH + comp) * SB_GPTS * SB_COLS + lane;
+        const Real* r = red + (int64_t(kk) * NCH + comp) * GP * SB_COLS + lane;
         double s = double(r[0]);
         for (int w = 1; w < gcount; ++w) s += double(r[w * SB_COLS]);
         out[icol + ncol * (lay + nlay * gi)] = s;
@@ -139,9 +148,21 @@ __global__ void absorbed_heating_rate_kernel(int64_t ncol, int64_t nlay, int ngr
     if (i >= ncol * nlay) return;
     const int64_t ncl = ncol * nlay;
     double s = 0.;
-    for (int g = 0; g < ngroups; ++g)
-        for (int p = 0; p < nparts; ++p)
-            s += parts[i + ncl * (g + int64_t(ngroups) * p)];
+    // Eight groups' loads in flight; added in order.
+    for (int g0 = 0; g0 < ngroups; g0 += 8)
+    {
+        double v[8][2];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                v[k][p] = (g0 + k < ngroups && p < nparts) ? parts[i + ncl * (g0 + k + int64_t(ngroups) * p)] : 0.;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                if (g0 + k < ngroups && p < nparts) s += v[k][p];
+    }
     const double dp = fabs(double(plev[i + ncol]) - double(plev[i]));
     const double g0 = 9.80665, cp = 1004.64, sec_per_day = 86400.0;
     hr[i] = Real(g0 / cp * s / dp * sec_per_day);
@@ -150,8 +171,9 @@ __global__ void absorbed_heating_rate_kernel(int64_t ncol, int64_t nlay, int ngr
 // ---------------------------------------------------------------------------------------------
 // Longwave: no scattering, linear-in-tau source, nmus <= NMU Gaussian angles.  The layer inputs
 // of the next K-level segment are read while the current segment is computed.
-template<typename Real, bool JAC, int NMU, bool FACT, bool HR = false>
-__global__ __launch_bounds__(SB_COLS * SB_GPTS) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 8 : 4)))
+template<int GP, typename Real, bool JAC, int NMU, bool FACT, bool HR = false>
+__global__ __launch_bounds__(SB_COLS * GP)
+__attribute__((amdgpu_waves_per_eu(GP < SB_GPTS ? 2 : sizeof(Real) == 4 ? 8 : 4)))
 void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int nmus,
                       const Real* __restrict__ secants, const Real* __restrict__ weights,
                       const Real* __restrict__ tau, const Real* __restrict__ lay_src,
@@ -164,12 +186,12 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
                       const Real* __restrict__ bnd_lev, int64_t emis_nbnd, int secants_per_angle,
                       double* __restrict__ absorbed)
 {
-    constexpr int K = NMU == 1 ? LwSeg<Real>::K1 : LwSeg<Real>::K4;
+    constexpr int K = lw_seg_k<Real, NMU, GP>();
     constexpr int NC = JAC ? 2 : 1;
     // With HR, one more LDS component per slot: the layer's absorbed flux of this g-point,
     // -sum_mu fac (S - (1 - T) I_in), from the sweep's own terms (no difference of level fluxes).
     constexpr int NCH = NC + (HR ? 1 : 0);
-    __shared__ Real red[K * NCH * SB_GPTS * SB_COLS];
+    __shared__ Real red[K * NCH * GP * SB_COLS];
 
     const int lane = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.y));   // wavefront = g-point
@@ -218,29 +240,37 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
     // The up sweep (nt) reads tau and the Planck fractions for the last time and streams them; the
     // down sweep's reads stay cacheable, so the bottom layers it read last are partly still in the
     // last-level cache when the up sweep starts there.
-    Real bt[K], bl[K], bx[K];
+    // Levels outside 1 .. nlay read the nearest layer instead (their values are not used): a test per level
+    // would put each level's loads, and with FACT the wait for them, behind a branch of its own.  The small
+    // work-groups keep the factors and multiply at the use, so that the next segment's loads stay in flight;
+    // the large ones have no registers for that, and other wavefronts to run meanwhile.
+    constexpr bool LATE = FACT && GP < SB_GPTS;
+    constexpr bool AHEAD = NMU == 1 && GP < SB_GPTS && (sizeof(Real) == 4 || !HR);   // FP64 with HR would spill
+    Real bt[K] = {}, bl[K] = {}, bx[K] = {}, bp[LATE ? K : 1] = {};
     auto fetch = [&](int64_t s0, const Real* lev_g, int lsh, auto layer_of, bool nt) {
+        if (!active) return;
 #pragma unroll
         for (int kk = 0; kk < K; ++kk)
         {
-            const int64_t j = s0 + kk;
-            bt[kk] = Real(0); bl[kk] = Real(0); bx[kk] = Real(0);
-            if (active && j >= 1 && j <= nlay)
+            const int64_t j = min(max(s0 + kk, int64_t(1)), nlay);
+            const uint32_t L = uint32_t(layer_of(j));
+            const uint32_t l = ucol + uncol * L;
+            bt[kk] = nt ? ld_nt(tau_g, l) : at32(tau_g, l);
+            if constexpr (FACT)
             {
-                const uint32_t L = uint32_t(layer_of(j));
-                const uint32_t l = ucol + uncol * L;
-                bt[kk] = nt ? ld_nt(tau_g, l) : at32(tau_g, l);
-                if constexpr (FACT)
+                bp[LATE ? kk : 0] = nt ? ld_nt(lay_g, l) : at32(lay_g, l);
+                bl[kk] = at32(blay_g, l);
+                bx[kk] = at32(blev_g, ucol + uncol * (L + uint32_t(lsh)));
+                if constexpr (!LATE)
                 {
 #pragma clang fp contract(off)
-                    const Real pf = nt ? ld_nt(lay_g, l) : at32(lay_g, l);
-                    bl[kk] = pf * at32(blay_g, l);
-                    bx[kk] = pf * at32(blev_g, ucol + uncol * (L + uint32_t(lsh)));
+                    bl[kk] = bp[0] * bl[kk];
+                    bx[kk] = bp[0] * bx[kk];
                 }
-                else
-                {
-                    bl[kk] = at32(lay_g, l); bx[kk] = at32(lev_g, l);
-                }
+            }
+            else
+            {
+                bl[kk] = at32(lay_g, l); bx[kk] = at32(lev_g, l);
             }
         }
     };
@@ -251,8 +281,33 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
         {
             Real ct[K], cl[K], cx[K];
 #pragma unroll
-            for (int kk = 0; kk < K; ++kk) { ct[kk] = bt[kk]; cl[kk] = bl[kk]; cx[kk] = bx[kk]; }
+            for (int kk = 0; kk < K; ++kk)
+            {
+#pragma clang fp contract(off)
+                ct[kk] = bt[kk];
+                cl[kk] = LATE ? bp[LATE ? kk : 0] * bl[kk] : bl[kk];
+                cx[kk] = LATE ? bp[LATE ? kk : 0] * bx[kk] : bx[kk];
+            }
             if (s0 + K <= nlay) fetch(s0 + K, lev_g, lsh, layer_of, up);
+            // Small work-groups have one or two wavefronts per SIMD: the levels' transmittances and sources,
+            // which do not depend on each other, are evaluated side by side before the recurrence.
+            Real pT[AHEAD ? K : 1], pS[AHEAD ? K : 1], pA[AHEAD && HR ? K : 1], pB[AHEAD && HR ? K : 1];
+            if constexpr (AHEAD)
+            {
+#pragma unroll
+                for (int kk = 0; kk < K; ++kk)
+                {
+                    Real fact;
+                    const Real t = ct[kk] * D[0];
+                    lw_layer(t, pT[kk], fact);
+                    pS[kk] = (Real(1) - pT[kk]) * cx[kk] + Real(2) * fact * (cl[kk] - cx[kk]);
+                    if constexpr (HR)
+                    {
+                        pA[kk] = one_minus_T(t, pT[kk]);
+                        pB[kk] = Real(2) * fact * (cl[kk] - cx[kk]);
+                    }
+                }
+            }
 #pragma unroll
             for (int kk = 0; kk < K; ++kk)
             {
@@ -260,7 +315,16 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
                 Real f = Real(0), fj = Real(0), ab = Real(0);
                 if (active && j <= nlay)
                 {
-                    if (j > 0)
+                    if constexpr (AHEAD)
+                    {
+                        if (j > 0)
+                        {
+                            if constexpr (HR) ab -= fac[0] * (pA[kk] * (cx[kk] - I[0]) + pB[kk]);
+                            I[0] = pT[kk] * I[0] + pS[kk];
+                            if (JAC && up) Ij[0] = pT[kk] * Ij[0];
+                        }
+                    }
+                    else if (j > 0)
                     {
 #pragma unroll
                         for (int mu = 0; mu < NMU; ++mu)
@@ -287,9 +351,9 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
                 }
                 if (reduce)
                 {
-                    red[(kk * NCH) * SB_GPTS * SB_COLS + w * SB_COLS + lane] = f;
-                    if (JAC && up) red[(kk * NCH + 1) * SB_GPTS * SB_COLS + w * SB_COLS + lane] = fj;
-                    if constexpr (HR) red[(kk * NCH + NC) * SB_GPTS * SB_COLS + w * SB_COLS + lane] = ab;
+                    red[(kk * NCH) * GP * SB_COLS + w * SB_COLS + lane] = f;
+                    if (JAC && up) red[(kk * NCH + 1) * GP * SB_COLS + w * SB_COLS + lane] = fj;
+                    if constexpr (HR) red[(kk * NCH + NC) * GP * SB_COLS + w * SB_COLS + lane] = ab;
                 }
             }
             if (reduce)
@@ -300,20 +364,20 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
                 if (JAC && up)
                 {
                     Real* const outs[2] = {grp_out, grp_jac};
-                    write_group_sums<Real, 2, NCH>(red, nsl, gcount, col0, ncol, nlev, gi, outs, lev_of);
+                    write_group_sums<GP, Real, 2, NCH>(red, nsl, gcount, col0, ncol, nlev, gi, outs, lev_of);
                 }
                 else
                 {
                     // NCH keeps the component stride of the Jacobian / heating-rate layouts.
                     Real* const outs[1] = {grp_out};
-                    write_group_sums_stride<Real, NCH>(red, nsl, gcount, col0, ncol, nlev, gi, outs, lev_of);
+                    write_group_sums_stride<GP, Real, NCH>(red, nsl, gcount, col0, ncol, nlev, gi, outs, lev_of);
                 }
                 if constexpr (HR)
                 {
                     // Sweep level j > 0 closes layer layer_of(j); the down sweep's parts go to
                     // absorbed[.., 0], the up sweep's to absorbed[.., 1].
                     double* part = absorbed + (up ? ncol * nlay * int64_t(grp.n) : int64_t(0));
-                    write_group_layer_sums<Real, NCH>(red, NC, nsl, gcount, col0, ncol, nlay, gi, part,
+                    write_group_layer_sums<GP, Real, NCH>(red, NC, nsl, gcount, col0, ncol, nlay, gi, part,
                                                       [&](int kk) -> int64_t {
                                                           const int64_t jj = s0 + kk;
                                                           return jj >= 1 ? int64_t(layer_of(jj)) : int64_t(-1);
@@ -505,9 +569,9 @@ template<typename St> struct Beam<float, St>
 // CO: the ssa argument holds the co-albedo 1 - ssa (see sw_layer).  The adding states and
 // denominators are carried in the build's precision (with FP32 states the FP32 build stays within
 // 2e-3 W m-2 of the FP64 build, near-conservative cloud layers included).
-template<typename Real, bool HR = false, bool CO = false>
-__global__ __launch_bounds__(SB_COLS * SB_GPTS)
-__attribute__((amdgpu_waves_per_eu(sw_wide(sizeof(Real) == 4, CO, HR) ? 8 : 4)))
+template<int GP, typename Real, bool HR, bool CO>
+__global__ __launch_bounds__(SB_COLS * GP)
+__attribute__((amdgpu_waves_per_eu(GP < SB_GPTS ? 2 : sw_wide(sizeof(Real) == 4, CO, HR) ? 8 : 4)))
 void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
                       const Real* __restrict__ tau, const Real* __restrict__ ssa,
                       const Real* __restrict__ gasy, const Real* __restrict__ mu0,
@@ -519,14 +583,14 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
                       double* __restrict__ absorbed)
 {
     using St = Real;
-    constexpr int K = sw_seg_k(sizeof(Real) == 4, CO, HR);
+    constexpr int K = sw_seg_k(sizeof(Real) == 4, CO, HR, GP);
     constexpr int NC = 3;
     // With HR a fourth component per slot: the absorbed flux of the layer below the slot's level,
     // (dn_dif(top) + up(bottom)) (1 - R - T) + dir(top) (1 - Tn) - SU - SD for this g-point, from the
     // layer's own terms instead of a difference of level fluxes.
     constexpr int NCH = NC + (HR ? 1 : 0);
     // Slots 0..K-1: the levels of a segment; slot K: the surface level.
-    __shared__ Real red[(K + 1) * NCH * SB_GPTS * SB_COLS];
+    __shared__ Real red[(K + 1) * NCH * GP * SB_COLS];
 
     const int lane = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.y));   // wavefront = g-point
@@ -572,7 +636,7 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
             const int nk = int(std::min<int64_t>(K, nlay - j0));
             beam.refresh();
             ck(s, 0) = Real(R_up); ck(s, 1) = Real(D); ck(s, 2) = Real(beam.saved());
-            Real tv[K], wv[K], gv[K];
+            Real tv[K] = {}, wv[K] = {}, gv[K] = {};
 #pragma unroll
             for (int kk = 0; kk < K; ++kk)
                 if (kk < nk)
@@ -608,9 +672,9 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
         }
         if (reduce)
         {
-            red[((K * NCH + 0) * SB_GPTS + w) * SB_COLS + lane] = Real(up);
-            red[((K * NCH + 1) * SB_GPTS + w) * SB_COLS + lane] = Real(dn + dir);
-            red[((K * NCH + 2) * SB_GPTS + w) * SB_COLS + lane] = Real(dir);
+            red[((K * NCH + 0) * GP + w) * SB_COLS + lane] = Real(up);
+            red[((K * NCH + 1) * GP + w) * SB_COLS + lane] = Real(dn + dir);
+            red[((K * NCH + 2) * GP + w) * SB_COLS + lane] = Real(dir);
         }
         up_below = up;
     }
@@ -627,7 +691,7 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
             St r_up = St(ck(s, 0)), d = St(ck(s, 1));
             Beam<Real, St> bm = beam;
             bm.restore(ck(s, 2));
-            Real tv[K], wv[K], gv[K];
+            Real tv[K] = {}, wv[K] = {}, gv[K] = {};
 #pragma unroll
             for (int kk = 0; kk < K; ++kk)
                 if (kk < nk)
@@ -665,15 +729,15 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
                     }
                     if (reduce)
                     {
-                        red[((kk * NCH + 0) * SB_GPTS + w) * SB_COLS + lane] = Real(up);
-                        red[((kk * NCH + 1) * SB_GPTS + w) * SB_COLS + lane] = Real(dn + dd);
-                        red[((kk * NCH + 2) * SB_GPTS + w) * SB_COLS + lane] = Real(dd);
+                        red[((kk * NCH + 0) * GP + w) * SB_COLS + lane] = Real(up);
+                        red[((kk * NCH + 1) * GP + w) * SB_COLS + lane] = Real(dn + dd);
+                        red[((kk * NCH + 2) * GP + w) * SB_COLS + lane] = Real(dd);
                     }
                     if constexpr (HR)
                     {
                         const St ab = (dn + up_below) * St(sAb[kk]) + dd * St(sOmTn[kk]) - St(sSU[kk]) -
                                       St(sSD[kk]);
-                        red[((kk * NCH + NC) * SB_GPTS + w) * SB_COLS + lane] = Real(ab);
+                        red[((kk * NCH + NC) * GP + w) * SB_COLS + lane] = Real(ab);
                         up_below = up;
                     }
                 }
@@ -684,13 +748,13 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
             Real* const outs[3] = {grp_up, grp_dn, grp_dir};
             // The surface slot K goes out with the first (bottom) segment.
             const int nsl = (s == nseg - 1) ? K + 1 : nk;
-            write_group_sums<Real, 3, NCH>(red, nsl, gcount, col0, ncol, nlev, gi, outs,
+            write_group_sums<GP, Real, 3, NCH>(red, nsl, gcount, col0, ncol, nlev, gi, outs,
                                                               [&](int kk) -> int64_t {
                 if (kk == K) return lev_of(nlay);
                 return kk < nk ? int64_t(lev_of(j0 + kk)) : int64_t(-1);
             });
             if constexpr (HR)
-                write_group_layer_sums<Real, NCH>(red, NC, nk, gcount, col0, ncol, nlay, gi, absorbed,
+                write_group_layer_sums<GP, Real, NCH>(red, NC, nk, gcount, col0, ncol, nlay, gi, absorbed,
                                                   [&](int kk) -> int64_t { return int64_t(lay_of(j0 + kk)); });
             __syncthreads();
         }
@@ -698,34 +762,75 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
 }
 
 // Band sums (when a band spans several groups) and broadband sums of group fluxes
-// (ncol, nlev, ngroups): per (column, level), groups in order, then bands in order.
+// (ncol, nlev, ngroups): per (column, level), groups in order, then bands in order.  blockIdx.y selects the
+// flux component.  Loads of 16 groups are in flight at a time, and where bands begin comes as a bit mask that
+// stays in scalar registers (indexing the groups' band numbers cost a scalar load per group, one after the
+// other: 64 groups took 15 us).
+constexpr int MAX_SUMS = 3;
 template<typename Real>
-__global__ void group_sums_kernel(int64_t ncv, Groups grp, const Real* __restrict__ gf,
-                                  Real* __restrict__ bnd, Real* __restrict__ bb)
+struct GroupSums
+{
+    int n, ngroups;
+    uint64_t begins[MAX_GROUPS / 64];      // bit g: group g begins a band (bands are numbered in this order)
+    const Real* gf[MAX_SUMS];
+    Real* bnd[MAX_SUMS];
+    Real* bb[MAX_SUMS];
+};
+
+template<typename Real>
+__global__ void group_sums_kernel(int64_t ncv, GroupSums<Real> q)
 {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= ncv) return;
+    const Real* gf = q.gf[blockIdx.y];
+    Real* bnd = q.bnd[blockIdx.y];
+    Real* bb = q.bb[blockIdx.y];
     Real total = Real(0), band = Real(0);
-    for (int g = 0; g < grp.n; ++g)
+    int64_t o = i;
+    bool first = true;
+    for (int g0 = 0; g0 < q.ngroups; g0 += 16)
     {
-        const Real v = gf[i + ncv * g];
-        band = (g > 0 && grp.band[g] == grp.band[g - 1]) ? band + v : v;
-        const bool last = (g + 1 == grp.n) || grp.band[g + 1] != grp.band[g];
-        if (last)
+        const uint32_t bits = uint32_t(q.begins[g0 / 64] >> (g0 % 64)) & 0xffffu;
+        Real v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = gf[i + ncv * min(g0 + k, q.ngroups - 1)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
         {
-            if (bnd) bnd[i + ncv * grp.band[g]] = band;
-            total = (grp.band[g] == grp.band[0]) ? band : total + band;
+            if (g0 + k >= q.ngroups) break;
+            if (!(bits >> k & 1)) { band = band + v[k]; continue; }
+            if (g0 + k > 0)
+            {
+                if (bnd) bnd[o] = band;
+                o += ncv;
+                total = first ? band : total + band;
+                first = false;
+            }
+            band = v[k];
         }
     }
-    if (bb) bb[i] = total;
+    if (bnd) bnd[o] = band;
+    if (bb) bb[i] = first ? band : total + band;
 }
 
+// The sums that some output wants, in one launch.
 template<typename Real>
-int group_sums(int64_t ncv, const Groups& grp, const Real* gf, Real* bnd, Real* bb, hipStream_t s)
+int group_sums(int64_t ncv, const Groups& grp, int n, const Real* const* gf, Real* const* bnd, Real* const* bb,
+               hipStream_t s)
 {
-    if (!bnd && !bb) return RRTMGP_OK;
+    GroupSums<Real> q{};
+    for (int c = 0; c < n; ++c)
+    {
+        if (!bnd[c] && !bb[c]) continue;
+        q.gf[q.n] = gf[c]; q.bnd[q.n] = bnd[c]; q.bb[q.n] = bb[c];
+        ++q.n;
+    }
+    if (q.n == 0) return RRTMGP_OK;
+    q.ngroups = grp.n;
+    for (int g = 0; g < grp.n; ++g)
+        if (g == 0 || grp.band[g] != grp.band[g - 1]) q.begins[g / 64] |= uint64_t(1) << (g % 64);
     RRTMGP_TIMED("group_sums_kernel", s);
-    hipLaunchKernelGGL(group_sums_kernel<Real>, dim3(grid1(ncv, 256)), dim3(256), 0, s, ncv, grp, gf, bnd, bb);
+    hipLaunchKernelGGL(group_sums_kernel<Real>, dim3(grid1(ncv, 256), unsigned(q.n)), dim3(256), 0, s, ncv, q);
     RRTMGP_LAUNCHED("group_sums_kernel");
     return RRTMGP_OK;
 }
@@ -798,11 +903,12 @@ int lw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t nm
     if (by_band && (!band_lims || nbnd < 1)) return arg_error("lw_solver: band surface inputs need band limits");
     hipStream_t s = as_stream(stream);
     Groups grp;
-    RRTMGP_TRY(make_groups(ngpt, band_lims ? nbnd : 1, band_lims, grp));
+    int gpts = SB_GPTS;
+    RRTMGP_TRY(make_groups_for(grid1(ncol, SB_COLS), ngpt, band_lims ? nbnd : 1, band_lims, grp, gpts));
     const int64_t ncv = ncol * (nlay + 1);
     const bool direct = bnd_up != nullptr && grp.n == int(nbnd);
     const dim3 grid(grid1(ncol, SB_COLS), unsigned(grp.n));
-    const dim3 block(SB_COLS, SB_GPTS);
+    const dim3 block(SB_COLS, unsigned(gpts));
 
     Real *g_up = nullptr, *g_dn = nullptr, *g_jac = nullptr, *scratch = nullptr;
     double* absorbed = nullptr;
@@ -829,28 +935,34 @@ int lw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t nm
                                jac_src, grp, g_up, g_dn, jac_out, bnd_lay, bnd_lev, by_band ? nbnd : int64_t(0),
                                by_band ? 1 : 0, absorbed);
         };
-        if (do_jac)
-            launch(nmus == 1 ? lw_solver_kernel<Real, true, 1, false> : lw_solver_kernel<Real, true, 4, false>,
-                   sfc_src_jac, g_jac);
-        else if (heating_rate && factored)
-            launch(nmus == 1 ? lw_solver_kernel<Real, false, 1, true, true> : lw_solver_kernel<Real, false, 4, true, true>,
-                   nullptr, nullptr);
-        else if (heating_rate)
-            launch(nmus == 1 ? lw_solver_kernel<Real, false, 1, false, true> : lw_solver_kernel<Real, false, 4, false, true>,
-                   nullptr, nullptr);
-        else if (factored)
-            launch(nmus == 1 ? lw_solver_kernel<Real, false, 1, true> : lw_solver_kernel<Real, false, 4, true>,
-                   nullptr, nullptr);
-        else
-            launch(nmus == 1 ? lw_solver_kernel<Real, false, 1, false> : lw_solver_kernel<Real, false, 4, false>,
-                   nullptr, nullptr);
+        auto choose = [&](auto gp) {
+            constexpr int GP = decltype(gp)::value;
+            if (do_jac)
+                launch(nmus == 1 ? lw_solver_kernel<GP, Real, true, 1, false> : lw_solver_kernel<GP, Real, true, 4, false>,
+                       sfc_src_jac, g_jac);
+            else if (heating_rate && factored)
+                launch(nmus == 1 ? lw_solver_kernel<GP, Real, false, 1, true, true>
+                                 : lw_solver_kernel<GP, Real, false, 4, true, true>, nullptr, nullptr);
+            else if (heating_rate)
+                launch(nmus == 1 ? lw_solver_kernel<GP, Real, false, 1, false, true>
+                                 : lw_solver_kernel<GP, Real, false, 4, false, true>, nullptr, nullptr);
+            else if (factored)
+                launch(nmus == 1 ? lw_solver_kernel<GP, Real, false, 1, true> : lw_solver_kernel<GP, Real, false, 4, true>,
+                       nullptr, nullptr);
+            else
+                launch(nmus == 1 ? lw_solver_kernel<GP, Real, false, 1, false> : lw_solver_kernel<GP, Real, false, 4, false>,
+                       nullptr, nullptr);
+        };
+        if (gpts <= SMALL_GPTS) choose(std::integral_constant<int, SMALL_GPTS>());
+        else choose(std::integral_constant<int, SB_GPTS>());
         rc = check_hip(hipGetLastError(), "lw_solver_kernel");
     }
     if (rc == RRTMGP_OK && !spectral)
     {
-        rc = group_sums<Real>(ncv, grp, g_up, direct ? nullptr : bnd_up, bb_up, s);
-        if (rc == RRTMGP_OK) rc = group_sums<Real>(ncv, grp, g_dn, direct ? nullptr : bnd_dn, bb_dn, s);
-        if (rc == RRTMGP_OK && do_jac) rc = group_sums<Real>(ncv, grp, g_jac, nullptr, flux_up_jac, s);
+        const Real* const gf[3] = {g_up, g_dn, g_jac};
+        Real* const bo[3] = {direct ? nullptr : bnd_up, direct ? nullptr : bnd_dn, nullptr};
+        Real* const bbo[3] = {bb_up, bb_dn, do_jac ? flux_up_jac : nullptr};
+        rc = group_sums<Real>(ncv, grp, 3, gf, bo, bbo, s);
     }
     if (rc == RRTMGP_OK && heating_rate)
         rc = absorbed_heating_rate<Real>(ncol, nlay, grp.n, 2, absorbed, plev, heating_rate, s);
@@ -902,7 +1014,7 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
         return arg_error("sw_solver: heating rates need plev and summed (not g-point) flux outputs");
     if (by_band && (!band_lims || nbnd < 1)) return arg_error("sw_solver: band surface inputs need band limits");
     // 32-bit lane offsets within one g-point's slab of levels or of checkpoints.
-    const int K = sw_seg_k(sizeof(Real) == 4, coalbedo, heating_rate != nullptr);
+    int K = sw_seg_k(sizeof(Real) == 4, coalbedo, heating_rate != nullptr, SB_GPTS);
     if (ncol * std::max<int64_t>(nlay + 1, 3 * ((nlay + K - 1) / K)) * int64_t(sizeof(Real)) >= (int64_t(1) << 32))
         return arg_error("sw_solver: ncol * (nlay + 1) values of one g-point must stay below 4 GiB");
     if (!tau || !ssa || !g || !mu0 || !alb_dir || !alb_dif || !inc_dir) return arg_error("sw_solver: NULL input");
@@ -916,23 +1028,38 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
     if (has_dif_bc && !inc_dif) return arg_error("sw_solver: has_dif_bc without inc_flux_dif");
     hipStream_t s = as_stream(stream);
     Groups grp;
-    RRTMGP_TRY(make_groups(ngpt, band_lims ? nbnd : 1, band_lims, grp));
-    const int64_t ncv = ncol * (nlay + 1), nseg = (nlay + K - 1) / K;
-    const bool direct = want_bnd && grp.n == int(nbnd);
-    const dim3 grid(grid1(ncol, SB_COLS), unsigned(grp.n));
-    const dim3 block(SB_COLS, SB_GPTS);
+    int gpts = SB_GPTS;
+    RRTMGP_TRY(make_groups_for(grid1(ncol, SB_COLS), ngpt, band_lims ? nbnd : 1, band_lims, grp, gpts));
+    if (gpts <= SMALL_GPTS) K = SEG8;
+    const int64_t ncv = ncol * (nlay + 1);
 
     // Every element of the checkpoints, group partials and heating-rate parts is written by the
     // kernel before it is read, so none of them needs clearing.
     Real *ckpt = nullptr, *scratch = nullptr;
     double* absorbed = nullptr;
-    const size_t n_ck = size_t(nseg * 3 * ngpt * ncol);
-    const size_t n_part = (!spectral && !direct) ? size_t(ncv * grp.n * 3) : 0;
-    const size_t n_abs = heating_rate ? size_t(ncol * nlay * grp.n) : 0;
+    const auto checkpoints = [&] { return size_t((nlay + K - 1) / K * 3 * ngpt * ncol); };
+    const auto is_direct = [&] { return want_bnd && grp.n == int(nbnd); };
+    const auto parts = [&] { return (!spectral && !is_direct()) ? size_t(ncv * grp.n * 3) : size_t(0); };
+    const auto abs_parts = [&] { return heating_rate ? size_t(ncol * nlay * grp.n) : size_t(0); };
+    auto round256 = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const auto needed = [&] {
+        return round256(checkpoints() * sizeof(Real)) + round256(parts() * sizeof(Real)) +
+               round256(abs_parts() * sizeof(double));
+    };
+    // Smaller groups have more partial sums: where a fixed workspace does not hold them, whole ones.
+    if (workspace && gpts < SB_GPTS && needed() > workspace_bytes)
+    {
+        gpts = SB_GPTS;
+        K = sw_seg_k(sizeof(Real) == 4, coalbedo, heating_rate != nullptr, SB_GPTS);
+        RRTMGP_TRY(make_groups(ngpt, band_lims ? nbnd : 1, band_lims, grp));
+    }
+    const bool direct = is_direct();
+    const size_t n_ck = checkpoints(), n_part = parts(), n_abs = abs_parts();
+    const dim3 grid(grid1(ncol, SB_COLS), unsigned(grp.n));
+    const dim3 block(SB_COLS, unsigned(gpts));
     if (workspace)
     {
-        auto round256 = [](size_t b) { return (b + 255) & ~size_t(255); };
-        const size_t need = round256(n_ck * sizeof(Real)) + round256(n_part * sizeof(Real)) + round256(n_abs * sizeof(double));
+        const size_t need = needed();
         if (need > workspace_bytes)
             return arg_error("sw_solver (no allocation): this call needs " + std::to_string(need) +
                              " bytes of scratch; the entry point without allocation holds " +
@@ -965,15 +1092,24 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
     int rc = RRTMGP_OK;
     {
         RRTMGP_TIMED("sw_solver_kernel", s);
-        auto kernel = heating_rate ? (coalbedo ? sw_solver_kernel<Real, true, true> : sw_solver_kernel<Real, true>)
-                                   : (coalbedo ? sw_solver_kernel<Real, false, true> : sw_solver_kernel<Real, false>);
-        hipLaunchKernelGGL(kernel, grid, block, 0, s, ncol, nlay, ngpt, top_at_1, tau, ssa, g, mu0, alb_dir, alb_dif, inc_dir,
-                           has_dif_bc ? inc_dif : nullptr, flux_up, flux_dn, flux_dir, ckpt, grp, gf[0], gf[1], gf[2],
-                           by_band ? nbnd : int64_t(0), absorbed);
+        auto choose = [&](auto gp) {
+            constexpr int GP = decltype(gp)::value;
+            auto kernel = heating_rate
+                ? (coalbedo ? sw_solver_kernel<GP, Real, true, true> : sw_solver_kernel<GP, Real, true, false>)
+                : (coalbedo ? sw_solver_kernel<GP, Real, false, true> : sw_solver_kernel<GP, Real, false, false>);
+            hipLaunchKernelGGL(kernel, grid, block, 0, s, ncol, nlay, ngpt, top_at_1, tau, ssa, g, mu0, alb_dir,
+                               alb_dif, inc_dir, has_dif_bc ? inc_dif : nullptr, flux_up, flux_dn, flux_dir, ckpt, grp,
+                               gf[0], gf[1], gf[2], by_band ? nbnd : int64_t(0), absorbed);
+        };
+        if (gpts <= SMALL_GPTS) choose(std::integral_constant<int, SMALL_GPTS>());
+        else choose(std::integral_constant<int, SB_GPTS>());
         rc = check_hip(hipGetLastError(), "sw_solver_kernel");
     }
-    for (int c = 0; c < 3 && rc == RRTMGP_OK && !spectral; ++c)
-        rc = group_sums<Real>(ncv, grp, gf[c], direct ? nullptr : bo[c], bbo[c], s);
+    if (rc == RRTMGP_OK && !spectral)
+    {
+        Real* const none[3] = {nullptr, nullptr, nullptr};
+        rc = group_sums<Real>(ncv, grp, 3, gf, direct ? none : bo, bbo, s);
+    }
     if (rc == RRTMGP_OK && heating_rate)
         rc = absorbed_heating_rate<Real>(ncol, nlay, grp.n, 1, absorbed, plev, heating_rate, s);
     if (!workspace)

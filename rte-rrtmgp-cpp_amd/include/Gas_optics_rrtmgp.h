@@ -136,18 +136,20 @@ class Gas_optics_rrtmgp_gpu : public Gas_optics_gpu
         // the gas-optics write).  cloud may be nullptr.  The shortwave one with coalbedo writes
         // the co-albedo 1 - ssa in place of ssa, and reads the cloud's as co-albedo too
         // (rrtmgp_hip_gas_optics_sw_coalbedo_*; plain gas optics only, not with a surrogate).
+        // top_at_1, when given, receives play(1, 1) < play(1, nlay), read with the range checks.
         void gas_optics_with_clouds(
                 const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev,
                 const Array_gpu<Float,2>& tlay, const Array_gpu<Float,1>& tsfc,
                 const Gas_concs_gpu& gas_desc, Optical_props_arry_gpu& optical_props,
                 Source_func_lw_gpu& sources, const Array_gpu<Float,2>& col_dry,
-                const Array_gpu<Float,2>& tlev, const Optical_props_arry_gpu* cloud);
+                const Array_gpu<Float,2>& tlev, const Optical_props_arry_gpu* cloud,
+                Bool* top_at_1 = nullptr);
         void gas_optics_with_clouds(
                 const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev,
                 const Array_gpu<Float,2>& tlay, const Gas_concs_gpu& gas_desc,
                 Optical_props_arry_gpu& optical_props, Array_gpu<Float,2>& toa_src,
                 const Array_gpu<Float,2>& col_dry, const Optical_props_arry_gpu* cloud,
-                bool coalbedo = false);
+                bool coalbedo = false, Bool* top_at_1 = nullptr);
 
         // gas concentrations as the rrtmgp_gas_vmr descriptor of the kernels, in this
         // k-distribution's gas order
@@ -272,7 +274,8 @@ class Gas_optics_rrtmgp_gpu : public Gas_optics_gpu
         // layer of :1333, from one device pass and one read-back; returns sfc_lay.
         int check_inputs(const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev,
                          const Array_gpu<Float,2>& tlay, const Array_gpu<Float,2>& col_dry,
-                         const Array_gpu<Float,2>* tlev, const Array_gpu<Float,1>* tsfc) const;
+                         const Array_gpu<Float,2>* tlev, const Array_gpu<Float,1>* tsfc,
+                         Bool* top_at_1) const;
 };
 
 #endif

@@ -498,7 +498,8 @@ void Gas_optics_rrtmgp_gpu::make_vmr_desc(const Gas_concs_gpu& gas_desc, int nco
 
 int Gas_optics_rrtmgp_gpu::check_inputs(const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev,
                                         const Array_gpu<Float,2>& tlay, const Array_gpu<Float,2>& col_dry,
-                                        const Array_gpu<Float,2>* tlev, const Array_gpu<Float,1>* tsfc) const
+                                        const Array_gpu<Float,2>* tlev, const Array_gpu<Float,1>* tsfc,
+                                        Bool* top_at_1) const
 {
     const Float nan = std::nan("");
     // In the reference's order of the checks (and of its messages).
@@ -517,6 +518,7 @@ int Gas_optics_rrtmgp_gpu::check_inputs(const Array_gpu<Float,2>& play, const Ar
     hip_check(K<Float>::check_ranges(6, arrays, sizes, lo, hi, counts, play.ptr(), ncol, nlay, ends, stream()));
     for (int k = 0; k < 6; ++k)
         if (counts[k] > 0) throw std::range_error(std::string(what[k]) + " is out of range");
+    if (top_at_1) *top_at_1 = ends[0] < ends[1];
     // Surface layer from the first column (src/Gas_optics_rrtmgp.cpp:1333).
     return ends[0] > ends[1] ? 1 : nlay;
 }
@@ -545,11 +547,11 @@ void Gas_optics_rrtmgp_gpu::gas_optics_with_clouds(
         const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev, const Array_gpu<Float,2>& tlay,
         const Array_gpu<Float,1>& tsfc, const Gas_concs_gpu& gas_desc, Optical_props_arry_gpu& props,
         Source_func_lw_gpu& sources, const Array_gpu<Float,2>& col_dry, const Array_gpu<Float,2>& tlev,
-        const Optical_props_arry_gpu* cloud)
+        const Optical_props_arry_gpu* cloud, Bool* top_at_1)
 {
     if (!source_is_internal()) throw std::runtime_error("longwave gas_optics called on a shortwave k-distribution");
     const int ncol = play.dim(1), nlay = play.dim(2);
-    const int sfc_lay = check_inputs(play, plev, tlay, col_dry, &tlev, &tsfc);
+    const int sfc_lay = check_inputs(play, plev, tlay, col_dry, &tlev, &tsfc, top_at_1);
     rrtmgp_gas_vmr v;
     make_vmr_desc(gas_desc, ncol, nlay, v);
     if (cloud && cloud->get_ngpt() != get_nband())
@@ -615,12 +617,12 @@ void Gas_optics_rrtmgp_gpu::gas_optics_with_clouds(
 void Gas_optics_rrtmgp_gpu::gas_optics_with_clouds(
         const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev, const Array_gpu<Float,2>& tlay,
         const Gas_concs_gpu& gas_desc, Optical_props_arry_gpu& props, Array_gpu<Float,2>& toa_src,
-        const Array_gpu<Float,2>& col_dry, const Optical_props_arry_gpu* cloud, bool coalbedo)
+        const Array_gpu<Float,2>& col_dry, const Optical_props_arry_gpu* cloud, bool coalbedo, Bool* top_at_1)
 {
     if (krayl.size() == 0) throw std::runtime_error("shortwave gas_optics called on a longwave k-distribution");
     if (coalbedo && use_mlp) throw std::invalid_argument("co-albedo gas optics with a surrogate set");
     const int ncol = play.dim(1), nlay = play.dim(2);
-    (void)check_inputs(play, plev, tlay, col_dry, nullptr, nullptr);
+    (void)check_inputs(play, plev, tlay, col_dry, nullptr, nullptr, top_at_1);
     rrtmgp_gas_vmr v;
     make_vmr_desc(gas_desc, ncol, nlay, v);
     if (cloud && cloud->get_ngpt() != get_nband())

@@ -65,8 +65,9 @@ void Radiation_solver_longwave_gpu::solve_gpu(
     const int ncol = p_lay.dim(1), nlay = p_lay.dim(2), nlev = nlay + 1;
     const int ngpt = kdist->get_ngpt(), nbnd = kdist->get_nband();
     if (switch_cloud_optics && !cloud_optics) throw std::runtime_error("cloud optics requested but not configured");
-    // Orientation from the first column (src_test/Radiation_solver.cpp:407).
-    const Bool top_at_1 = p_lay({1, 1}) < p_lay({1, nlay});
+    // Orientation from the first column (src_test/Radiation_solver.cpp:407), read back with the first block's
+    // range checks.
+    Bool top_at_1 = false;
     const int nblk = std::max(1, std::min(n_col_block, ncol));
     if (ws_ncol != nblk || ws_nlay != nlay || ws_bnd != int(switch_output_bnd_fluxes))
     {
@@ -149,7 +150,8 @@ void Radiation_solver_longwave_gpu::solve_gpu(
                                        block_of(rel, c0, n, ws.rel), block_of(rei, c0, n, ws.rei), *cloud_props);
             cloud = cloud_props.get();
         }
-        kdist->gas_optics_with_clouds(pl, pv, tl, ts, gc, *optical_props, *sources, cd, tv, cloud);
+        kdist->gas_optics_with_clouds(pl, pv, tl, ts, gc, *optical_props, *sources, cd, tv, cloud,
+                                      c0 == 0 ? &top_at_1 : nullptr);
 
         // Band and broadband fluxes summed inside the solver, straight into the outputs when the
         // block spans all columns.
@@ -239,7 +241,7 @@ void Radiation_solver_shortwave_gpu::solve_gpu(
         throw std::runtime_error("aerosol optics requested but not configured");
     if (switch_aerosol_optics && (rh.dim(1) != ncol || rh.dim(2) != nlay))
         throw std::runtime_error("aerosol optics: rh must be (ncol, nlay)");
-    const Bool top_at_1 = p_lay({1, 1}) < p_lay({1, nlay});
+    Bool top_at_1 = false;      // as in the longwave
     const int nblk = std::max(1, std::min(n_col_block, ncol));
 
     if (ws_ncol != nblk || ws_nlay != nlay || ws_bnd != int(switch_output_bnd_fluxes))
@@ -342,7 +344,8 @@ void Radiation_solver_shortwave_gpu::solve_gpu(
             else cloud_optics->cloud_optics(a, b, c, d, *cloud_props);
             cloud = cloud_props.get();
         }
-        kdist->gas_optics_with_clouds(pl, pv, tl, gc, *optical_props, toa_src, cd, cloud, co);
+        kdist->gas_optics_with_clouds(pl, pv, tl, gc, *optical_props, toa_src, cd, cloud, co,
+                                      c0 == 0 ? &top_at_1 : nullptr);
         if (switch_aerosol_optics)
         {
             std::unique_ptr<Aerosol_concs_gpu> asub;
