@@ -95,6 +95,17 @@ int rrtmgp_hip_subset(int elem_size, int ndim, const void* src, const int64_t* s
                       const int64_t* src_offsets, const int64_t* starts, void* dst,
                       const int64_t* dst_dims, void* stream);
 
+/* Strided copies: item k writes dst (n0, n1), first index fastest, from src[i s0 + j s1] (strides  */
+/* in elements), both of float (size 4) or double (size 8), converting between them.               */
+typedef struct
+{
+    const void* src;
+    void* dst;
+    int64_t n0, n1, s0, s1;
+    int32_t src_size, dst_size;
+} rrtmgp_copy_item;
+int rrtmgp_hip_copy_arrays(int n, const rrtmgp_copy_item* items, void* stream);
+
 /* Per-kernel timing.  No counterpart in the reference (its timing is external profiling):   */
 /* with timing on, every kernel launch of this library is bracketed by two HIP events on its */
 /* launch stream.  enable(1) clears earlier records; collect() waits for the recorded events  */

@@ -1,7 +1,8 @@
 // Device kernels behind Array_gpu::fill and Array_gpu::subset (rte-rrtmgp-cpp_amd/include/Array.h),
 // the counterparts of the reference's fill_kernel and subset_kernel (include/Array.h:296-335,
 // launched at :501-511 and :583-606).  Extents and offsets are 64-bit; the element type only
-// matters through its size, so one kernel per size serves every Array_gpu<T,N>.
+// matters through its size, so one kernel per size serves every Array_gpu<T,N>.  And the strided copies
+// between other libraries' tensors and Fortran-order arrays (rrtmgp_hip_copy_arrays).
 #include <algorithm>
 #include <cstring>
 
@@ -80,9 +81,93 @@ int subset_t(int64_t n, const SubsetGeom& g, const void* src, void* dst, hipStre
     RRTMGP_LAUNCHED("subset_kernel");
     return RRTMGP_OK;
 }
+
+// Copies of several strided 2-D arrays of float or double into arrays with the first index fastest, in one
+// launch (blockIdx.y selects the array).  Latency bound at the sizes a gradient step has: one launch per array,
+// with a layout pass of its own and waits on both sides, took 33 us for each of the 58 arrays of a step at
+// 250 x 60 FP64; a launch of up to 16 arrays takes 8 us, and the step went from 4.0 to 3.1 ms.  Where the source
+// runs along its second index, 32 x 32 tiles go through LDS, so that both sides move along their rows.
+constexpr int COPY_MAX = 16;
+constexpr int COPY_TILE = 32;
+struct CopyItem
+{
+    const void* src;
+    void* dst;
+    int64_t n0, n1, s0, s1;          // extents, source strides in elements; dst is (n0, n1), n0 fastest
+    int src_size, dst_size;          // 4 (float) or 8 (double)
+};
+struct CopySet { CopyItem a[COPY_MAX]; };
+
+template<typename S, typename D>
+__device__ __forceinline__ void copy_item(const CopyItem& c, D (*tile)[COPY_TILE + 1])
+{
+    const S* __restrict__ src = static_cast<const S*>(c.src);
+    D* __restrict__ dst = static_cast<D*>(c.dst);
+    const int64_t n = c.n0 * c.n1;
+    if (c.s1 == 1 && c.s0 != 1 && c.n0 > 1 && c.n1 > 1)
+    {
+        const int64_t t0 = (c.n0 + COPY_TILE - 1) / COPY_TILE, t1 = (c.n1 + COPY_TILE - 1) / COPY_TILE;
+        const int x = threadIdx.x % COPY_TILE, y = threadIdx.x / COPY_TILE;
+        for (int64_t t = blockIdx.x; t < t0 * t1; t += gridDim.x)       // uniform over the work-group
+        {
+            const int64_t b0 = t % t0 * COPY_TILE, b1 = t / t0 * COPY_TILE;
+            for (int r = y; r < COPY_TILE; r += 256 / COPY_TILE)
+                if (b0 + r < c.n0 && b1 + x < c.n1) tile[r][x] = D(src[(b0 + r) * c.s0 + b1 + x]);
+            __syncthreads();
+            for (int r = y; r < COPY_TILE; r += 256 / COPY_TILE)
+                if (b0 + x < c.n0 && b1 + r < c.n1) dst[b0 + x + c.n0 * (b1 + r)] = tile[x][r];
+            __syncthreads();
+        }
+        return;
+    }
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256)
+        dst[i] = D(src[i % c.n0 * c.s0 + i / c.n0 * c.s1]);
+}
+
+__global__ __launch_bounds__(256)
+void copy_arrays_kernel(CopySet q)
+{
+    __shared__ double tile[COPY_TILE][COPY_TILE + 1];
+    const CopyItem& c = q.a[blockIdx.y];
+    auto* td = tile;
+    auto* tf = reinterpret_cast<float (*)[COPY_TILE + 1]>(&tile[0][0]);
+    if (c.src_size == 4 && c.dst_size == 4) copy_item<float, float>(c, tf);
+    else if (c.src_size == 4) copy_item<float, double>(c, td);
+    else if (c.dst_size == 4) copy_item<double, float>(c, tf);
+    else copy_item<double, double>(c, td);
+}
 }  // namespace rrtmgp_hip
 
 using namespace rrtmgp_hip;
+
+extern "C" int rrtmgp_hip_copy_arrays(int n, const rrtmgp_copy_item* items, void* stream)
+{
+    if (n < 0 || (n > 0 && !items)) return arg_error("copy_arrays: bad arguments");
+    hipStream_t s = as_stream(stream);
+    for (int k = 0; k < n;)
+    {
+        CopySet q{};
+        int m = 0;
+        int64_t most = 0;
+        for (; k < n && m < COPY_MAX; ++k)
+        {
+            const rrtmgp_copy_item& c = items[k];
+            if (c.n0 < 0 || c.n1 < 0) return arg_error("copy_arrays: negative extent");
+            if ((c.src_size != 4 && c.src_size != 8) || (c.dst_size != 4 && c.dst_size != 8))
+                return arg_error("copy_arrays: element sizes must be 4 or 8 bytes");
+            if (c.n0 * c.n1 == 0) continue;
+            if (!c.src || !c.dst) return arg_error("copy_arrays: NULL array");
+            q.a[m++] = CopyItem{c.src, c.dst, c.n0, c.n1, c.s0, c.s1, c.src_size, c.dst_size};
+            most = std::max(most, c.n0 * c.n1);
+        }
+        if (m == 0) continue;
+        const unsigned bx = unsigned(std::min<int64_t>((most + 1023) / 1024, int64_t(device_cu_count()) * 8));
+        RRTMGP_TIMED("copy_arrays_kernel", s);
+        hipLaunchKernelGGL(copy_arrays_kernel, dim3(bx, unsigned(m)), dim3(256), 0, s, q);
+        RRTMGP_LAUNCHED("copy_arrays_kernel");
+    }
+    return RRTMGP_OK;
+}
 
 extern "C" int rrtmgp_hip_fill(void* dst, int64_t n, int elem_size, const void* value, void* stream)
 {

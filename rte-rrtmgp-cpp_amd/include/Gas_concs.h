@@ -5,6 +5,7 @@
 
 #include <map>
 #include <string>
+#include <vector>
 
 #include "Array.h"
 #include "types.h"
@@ -19,6 +20,8 @@ class Gas_concs_gpu
         void set_vmr(const std::string& name, const Array<Float,1>& data);
         void set_vmr(const std::string& name, const Array<Float,2>& data);
         void set_vmr(const std::string& name, const Array_gpu<Float,2>& data);
+        // Several gases, range-checked together (one wait for the device per eight of them).
+        void set_vmr(const std::vector<std::string>& names, const std::vector<Array_gpu<Float,2>>& data);
 
         const Array_gpu<Float,2>& get_vmr(const std::string& name) const;
         Bool exists(const std::string& name) const;

@@ -2,6 +2,7 @@
 // src/Gas_concs.cpp:54-97).
 #include "Gas_concs.h"
 
+#include <algorithm>
 #include <stdexcept>
 
 #include "hip_dispatch.h"
@@ -50,6 +51,33 @@ void Gas_concs_gpu::set_vmr(const std::string& name, const Array_gpu<Float,2>& d
     if (bad) throw std::range_error("Gas concentration " + name + " is out of range");
     gas_concs_map.erase(name);
     gas_concs_map.emplace(name, Array_gpu<Float,2>(data));
+}
+
+void Gas_concs_gpu::set_vmr(const std::vector<std::string>& names, const std::vector<Array_gpu<Float,2>>& data)
+{
+    constexpr size_t at_once = 8;
+    for (size_t k0 = 0; k0 < names.size(); k0 += at_once)
+    {
+        const int n = int(std::min(at_once, names.size() - k0));
+        const Float* arrays[at_once];
+        int64_t sizes[at_once], bad[at_once] = {};
+        Float lo[at_once], hi[at_once];
+        for (int k = 0; k < n; ++k)
+        {
+            arrays[k] = data[k0 + k].ptr();
+            sizes[k] = data[k0 + k].size();
+            lo[k] = Float(0.);
+            hi[k] = Float(1.);
+        }
+        rrtmgp_cpp::hip_check(K<Float>::check_ranges(n, arrays, sizes, lo, hi, bad, nullptr, 0, 0, nullptr,
+                                                     rrtmgp_cpp::stream()));
+        for (int k = 0; k < n; ++k)
+        {
+            if (bad[k]) throw std::range_error("Gas concentration " + names[k0 + k] + " is out of range");
+            gas_concs_map.erase(names[k0 + k]);
+            gas_concs_map.emplace(names[k0 + k], Array_gpu<Float,2>(data[k0 + k]));
+        }
+    }
 }
 
 // Column subset (src/Gas_concs.cpp:29-42): profiles and scalars are shared.

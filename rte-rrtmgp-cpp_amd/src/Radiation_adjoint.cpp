@@ -85,6 +85,19 @@ void refuse_surrogate(const Gas_optics_rrtmgp_gpu& kdist)
                                     "before computing gradients");
 }
 
+// play(1, 1) and play(1, nlay), which decide the orientation, in one wait for the device.
+std::pair<Float, Float> column_ends(const Array_gpu<Float,2>& p_lay)
+{
+    const Float* none = nullptr;
+    const int64_t size = 0;
+    const Float lo = Float(0.), hi = Float(0.);
+    int64_t bad = 0;
+    Float ends[2] = {Float(0.), Float(0.)};
+    hip_check(K<Float>::check_ranges(1, &none, &size, &lo, &hi, &bad, p_lay.ptr(), p_lay.dim(1), p_lay.dim(2), ends,
+                                     stream()));
+    return {ends[0], ends[1]};
+}
+
 bool cloudy(const Cloud_optics_gpu* c, const Array_gpu<Float,2>& lwp)
 {
     return c != nullptr && lwp.size() > 0;
@@ -109,7 +122,7 @@ void lw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
     const rrtmgp_kdist_dev& kd = kdist.device_tables();
     rrtmgp_gas_vmr vmr;
     kdist.vmr_descriptor(gas_concs, ncol, nlay, vmr);
-    const Float p_first = p_lay({1, 1}), p_last = p_lay({1, nlay});
+    const auto [p_first, p_last] = column_ends(p_lay);
     const Bool top_at_1 = p_first < p_last;
     const int sfc_lay = p_first > p_last ? 1 : nlay;
 
@@ -190,7 +203,8 @@ void sw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
     const rrtmgp_kdist_dev& kd = kdist.device_tables();
     rrtmgp_gas_vmr vmr;
     kdist.vmr_descriptor(gas_concs, ncol, nlay, vmr);
-    const Bool top_at_1 = p_lay({1, 1}) < p_lay({1, nlay});
+    const auto [p_first, p_last] = column_ends(p_lay);
+    const Bool top_at_1 = p_first < p_last;
 
     ensure<2>(out.d_t_lay, {ncol, nlay}); ensure<2>(out.d_lnp_lay, {ncol, nlay}); ensure<2>(out.d_p_lev, {ncol, nlev});
     ensure<3>(out.d_vmr, {ncol, nlay, ngas});

@@ -238,11 +238,17 @@ int rrtmgp_api_gas_concs_create(const rrtmgp_api_gases* g, void** out)
     return guarded([&] {
         std::unique_ptr<Gas_concs_gpu> gc(new Gas_concs_gpu);
         auto nm = names(g->names, g->n);
+        std::vector<std::string> all;
+        std::vector<Array_gpu<Float,2>> data;
+        all.reserve(g->n);
+        data.reserve(g->n);
         for (int i = 0; i < g->n; ++i)
         {
             const int d1 = int(g->dims[2 * i]), d2 = int(g->dims[2 * i + 1]);
-            gc->set_vmr(nm({i + 1}), view<2>(static_cast<const rrtmgp_real*>(g->data[i]), {d1, d2}));
+            all.push_back(nm({i + 1}));
+            data.push_back(view<2>(static_cast<const rrtmgp_real*>(g->data[i]), {d1, d2}));
         }
+        gc->set_vmr(all, data);
         *out = gc.release();
     });
 }
