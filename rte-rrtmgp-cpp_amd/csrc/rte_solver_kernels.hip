@@ -55,15 +55,19 @@ template<> struct LwSeg<float> { static constexpr int K1 = 6, K4 = 4; };
 template<> struct LwSeg<double> { static constexpr int K1 = 4, K4 = 4; };
 constexpr int SEG8 = 8;
 constexpr int SMALL_GPTS = 8;
-template<typename Real, int NMU, int GP>
-constexpr int lw_seg_k() { return GP < SB_GPTS ? SEG8 : NMU == 1 ? LwSeg<Real>::K1 : LwSeg<Real>::K4; }
-// The SW kernel's wide variant (FP32, co-albedo input, no heating rates) fits 64 VGPRs with
-// K = 3, so two 1024-thread work-groups share a CU; the others keep K = 4 at up to 128 VGPRs.
-constexpr bool sw_wide(bool fp32, bool co, bool hr) { return fp32 && co && !hr; }
-constexpr int sw_seg_k(bool fp32, bool co, bool hr, int gp)
+// On factored sources the buffers hold a fourth value per level (see LATE), so one-angle segments are shorter.
+template<typename Real, int NMU, int GP, bool FACT, bool HR>
+constexpr int lw_seg_k()
 {
-    return gp < SB_GPTS ? SEG8 : sw_wide(fp32, co, hr) ? 3 : 4;
+    if (GP < SB_GPTS) return SEG8;
+    if (FACT && NMU == 1) return sizeof(Real) == 8 ? 3 : HR ? 4 : 5;
+    return NMU == 1 ? LwSeg<Real>::K1 : LwSeg<Real>::K4;
 }
+// The SW kernel's wide variant (FP32, co-albedo input, no heating rates) fits 64 VGPRs, so two 1024-thread
+// work-groups share a CU; the others take up to 128 VGPRs.  FP32 re-forms the direct beam at every segment, so
+// its segments are as long in small work-groups as in large ones, for the same bits.
+constexpr bool sw_wide(bool fp32, bool co, bool hr) { return fp32 && co && !hr; }
+constexpr int sw_seg_k(bool fp32, int gp) { return gp < SB_GPTS && !fp32 ? SEG8 : 4; }
 
 // Writes the LDS slots kk < nslots, components c < NC, summed over the group's g-points, to
 // out[c] at level lev_of(kk) (skipped when negative).
@@ -140,6 +144,14 @@ __device__ __forceinline__ void write_group_layer_sums(const Real* red, int comp
 // hr = g0 / cp * (sum over parts and groups, in order) / |p(lev+1) - p(lev)|, in FP64.  Equal to
 // g0 / cp (net_i - net_i+1) / (p_i+1 - p_i) with net = dn - up, in either orientation.
 template<typename Real>
+__device__ __forceinline__ Real absorbed_rate(double s, Real p_a, Real p_b)
+{
+    const double dp = fabs(double(p_b) - double(p_a));
+    const double g0 = 9.80665, cp = 1004.64, sec_per_day = 86400.0;
+    return Real(g0 / cp * s / dp * sec_per_day);
+}
+
+template<typename Real>
 __global__ void absorbed_heating_rate_kernel(int64_t ncol, int64_t nlay, int ngroups, int nparts,
                                              const double* __restrict__ parts, const Real* __restrict__ plev,
                                              Real* __restrict__ hr)
@@ -163,9 +175,7 @@ __global__ void absorbed_heating_rate_kernel(int64_t ncol, int64_t nlay, int ngr
             for (int p = 0; p < 2; ++p)
                 if (g0 + k < ngroups && p < nparts) s += v[k][p];
     }
-    const double dp = fabs(double(plev[i + ncol]) - double(plev[i]));
-    const double g0 = 9.80665, cp = 1004.64, sec_per_day = 86400.0;
-    hr[i] = Real(g0 / cp * s / dp * sec_per_day);
+    hr[i] = absorbed_rate(s, plev[i], plev[i + ncol]);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -186,12 +196,15 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
                       const Real* __restrict__ bnd_lev, int64_t emis_nbnd, int secants_per_angle,
                       double* __restrict__ absorbed)
 {
-    constexpr int K = lw_seg_k<Real, NMU, GP>();
+    constexpr int K = lw_seg_k<Real, NMU, GP, FACT, HR>();
     constexpr int NC = JAC ? 2 : 1;
     // With HR, one more LDS component per slot: the layer's absorbed flux of this g-point,
     // -sum_mu fac (S - (1 - T) I_in), from the sweep's own terms (no difference of level fluxes).
     constexpr int NCH = NC + (HR ? 1 : 0);
-    __shared__ Real red[K * NCH * GP * SB_COLS];
+    // Small work-groups leave the fluxes (and with HR the absorbed ones, in absorbed's memory) of every g-point;
+    // g_point_sums_kernel adds them in the order in which whole groups are added here.
+    constexpr bool SUMS = GP == SB_GPTS;
+    __shared__ Real red[SUMS ? K * NCH * GP * SB_COLS : 1];
 
     const int lane = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.y));   // wavefront = g-point
@@ -201,7 +214,7 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
     const int64_t icol = col0 + lane;
     const int64_t igpt = grp.start[gi] + w;
     const bool active = icol < ncol && w < gcount;
-    const bool reduce = grp_dn != nullptr;
+    const bool reduce = SUMS && grp_dn != nullptr;
     const int64_t nlev = nlay + 1;
     const int64_t c2 = icol + ncol * igpt;
     // Per-g-point slabs at wavefront-uniform bases; lane offsets icol + ncol * level (32-bit).
@@ -241,10 +254,11 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
     // down sweep's reads stay cacheable, so the bottom layers it read last are partly still in the
     // last-level cache when the up sweep starts there.
     // Levels outside 1 .. nlay read the nearest layer instead (their values are not used): a test per level
-    // would put each level's loads, and with FACT the wait for them, behind a branch of its own.  The small
-    // work-groups keep the factors and multiply at the use, so that the next segment's loads stay in flight;
-    // the large ones have no registers for that, and other wavefronts to run meanwhile.
-    constexpr bool LATE = FACT && GP < SB_GPTS;
+    // would put each level's loads, and with FACT the wait for them, behind a branch of its own.  With one angle
+    // the factors of FACT are kept and multiplied at the use, so that the next segment's loads stay in flight
+    // while this one is computed: 65536 x 128 x 256 FP32 7.6 -> 7.1 ms, 16384 x 128 1.91 -> 1.70, 8192 x 128 FP64
+    // 2.60 -> 2.40, all above the copy rate (part of the up sweep's reads come from the last-level cache).
+    constexpr bool LATE = FACT && (NMU == 1 || GP < SB_GPTS);
     constexpr bool AHEAD = NMU == 1 && GP < SB_GPTS && (sizeof(Real) == 4 || !HR);   // FP64 with HR would spill
     Real bt[K] = {}, bl[K] = {}, bx[K] = {}, bp[LATE ? K : 1] = {};
     auto fetch = [&](int64_t s0, const Real* lev_g, int lsh, auto layer_of, bool nt) {
@@ -348,6 +362,10 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
                             if (JAC && up) fj = (mu == 0) ? fac[0] * Ij[0] : fj + fac[mu] * Ij[mu];
                         }
                     if (flux_g) at32(flux_g, ucol + uncol * uint32_t(lev_out(j))) = f;
+                    if constexpr (HR && !SUMS)
+                        if (j > 0)
+                            at32(reinterpret_cast<Real*>(absorbed) + lslab + (up ? ncol * nlay * ngpt : int64_t(0)),
+                                 ucol + uncol * uint32_t(layer_of(j))) = ab;
                 }
                 if (reduce)
                 {
@@ -439,11 +457,12 @@ __device__ __forceinline__ bool sw_layer_fp32(float tau, float w0, float one_m_w
                                               St dir, LayerSW<St>& L)
 {
     if (ISLAND && one_m_w0 < 1e-6f) return false;
-    const float gamma1 = (8.f - w0 * (5.f + 3.f * g)) * .25f;
-    const float gamma2 = 3.f * (w0 * (1.f - g)) * .25f;
-    const float k = __builtin_amdgcn_sqrtf(fmaxf(2.f * one_m_w0 * (gamma1 + gamma2), 1e-12f));
+    const float gamma1 = 2.f - w0 * (1.25f + .75f * g);
+    const float gamma2 = w0 * (.75f - .75f * g);
+    const float om2 = 2.f * one_m_w0;
+    const float k = __builtin_amdgcn_sqrtf(fmaxf(om2 * (gamma1 + gamma2), 1e-12f));
     const float k_mu = k * mu0;
-    const float gamma3 = (2.f - 3.f * mu0 * g) * .25f;
+    const float gamma3 = .5f - (.75f * mu0) * g;
     const float gamma4 = 1.f - gamma3;
     const float alpha1 = gamma1 * gamma4 + gamma2 * gamma3;
     const float alpha2 = gamma1 * gamma3 + gamma2 * gamma4;
@@ -481,7 +500,7 @@ __device__ __forceinline__ bool sw_layer_fp32(float tau, float w0, float one_m_w
     const float td = fmaxf(eps, fminf(tdf, b - rd));
     // 1 - R - T = RT [k (2 - c2) + gamma1 c2 - gamma2 c2 - 2 k e1] = RT [k a^2 + (gamma1 - gamma2) c2] with
     // gamma1 - gamma2 = 2 (1 - w0): a sum of non-negative terms, free of the cancellation of 1 - R - T.
-    const float ab = RT * (k * a * a + 2.f * one_m_w0 * c2);
+    const float ab = RT * (k * a * a + om2 * c2);
     L = {St(RT * gamma2 * c2), St(RT * 2.f * k * e1), St(rd) * dir, St(td) * dir, St(Tn), St(ab), St(b)};
     return true;
 }
@@ -519,13 +538,25 @@ __device__ __forceinline__ LayerSW<St> sw_layer(Real tau, Real w_in, Real g, Rea
 __device__ __forceinline__ double rcp_den(double x) { return rcp_f64(x); }
 __device__ __forceinline__ float rcp_den(float x) { return rcp_f32(x); }
 
+// a + b as its own rounding, and a b + c in one.  Whether the compiler contracts an addition with the product
+// before it depends on the code around it, and the same columns have to give the same bits in every variant of
+// the kernel: the adding recurrences are written with these.
+__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template<typename St>
+__device__ __forceinline__ St add_alone(St a, St b)
+{
+#pragma clang fp contract(off)
+    return a + b;
+}
+
 // Column above the next level from the column above this one and the layer between.
 template<typename St>
 __device__ __forceinline__ void above_update(const LayerSW<St>& L, St& R_up, St& D)
 {
-    const St den = rcp_den(St(1) - L.R * R_up);
-    D = L.SD + L.T * (D + R_up * L.SU) * den;
-    R_up = L.R + L.T * L.T * R_up * den;
+    const St den = rcp_den(fma_of(-L.R, R_up, St(1)));
+    D = fma_of(L.T * fma_of(R_up, L.SU, D), den, L.SD);
+    R_up = fma_of(L.T * L.T * R_up, den, L.R);
 }
 
 // The direct beam below each layer of the top-down sweeps.  FP64 builds multiply the layer
@@ -583,14 +614,15 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
                       double* __restrict__ absorbed)
 {
     using St = Real;
-    constexpr int K = sw_seg_k(sizeof(Real) == 4, CO, HR, GP);
+    constexpr int K = sw_seg_k(sizeof(Real) == 4, GP);
     constexpr int NC = 3;
     // With HR a fourth component per slot: the absorbed flux of the layer below the slot's level,
     // (dn_dif(top) + up(bottom)) (1 - R - T) + dir(top) (1 - Tn) - SU - SD for this g-point, from the
     // layer's own terms instead of a difference of level fluxes.
     constexpr int NCH = NC + (HR ? 1 : 0);
     // Slots 0..K-1: the levels of a segment; slot K: the surface level.
-    __shared__ Real red[(K + 1) * NCH * GP * SB_COLS];
+    constexpr bool SUMS = GP == SB_GPTS;                   // see lw_solver_kernel
+    __shared__ Real red[SUMS ? (K + 1) * NCH * GP * SB_COLS : 1];
 
     const int lane = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.y));   // wavefront = g-point
@@ -600,7 +632,7 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
     const int64_t icol = col0 + lane;
     const int64_t igpt = grp.start[gi] + w;
     const bool active = icol < ncol && w < gcount;
-    const bool reduce = grp_dn != nullptr;
+    const bool reduce = SUMS && grp_dn != nullptr;
     const int64_t nlev = nlay + 1;
     const int64_t nseg = (nlay + K - 1) / K;
     const int64_t c2 = icol + ncol * igpt;
@@ -634,6 +666,8 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
         {
             const int64_t j0 = s * K;
             const int nk = int(std::min<int64_t>(K, nlay - j0));
+            // The last eighth of the layers is read with the cache: the sweep up starts with them.
+            const bool keep = j0 >= nlay - nlay / 8;
             beam.refresh();
             ck(s, 0) = Real(R_up); ck(s, 1) = Real(D); ck(s, 2) = Real(beam.saved());
             Real tv[K] = {}, wv[K] = {}, gv[K] = {};
@@ -642,7 +676,14 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
                 if (kk < nk)
                 {
                     const uint32_t l = ucol + uncol * lay_of(j0 + kk);
-                    tv[kk] = ld_nt(tau_g, l); wv[kk] = ld_nt(ssa_g, l); gv[kk] = ld_nt(gasy_g, l);
+                    if (keep)
+                    {
+                        tv[kk] = at32(tau_g, l); wv[kk] = at32(ssa_g, l); gv[kk] = at32(gasy_g, l);
+                    }
+                    else
+                    {
+                        tv[kk] = ld_nt(tau_g, l); wv[kk] = ld_nt(ssa_g, l); gv[kk] = ld_nt(gasy_g, l);
+                    }
                 }
 #pragma unroll
             for (int kk = 0; kk < K; ++kk)
@@ -663,17 +704,17 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
     St S = beam.dir * (active ? St(alb_dir[ia]) : St(0));
     {
         const St dir = beam.dir;
-        const St dn = (D + R_up * S) * rcp_den(St(1) - R_up * A);
-        const St up = A * dn + S;
+        const St dn = fma_of(R_up, S, D) * rcp_den(fma_of(-R_up, A, St(1)));
+        const St up = fma_of(A, dn, S);
         if (active && up_g)
         {
             const uint32_t o = ucol + uncol * lev_of(nlay);
-            at32(up_g, o) = Real(up); at32(dn_g, o) = Real(dn + dir); at32(dir_g, o) = Real(dir);
+            at32(up_g, o) = Real(up); at32(dn_g, o) = Real(add_alone(dn, dir)); at32(dir_g, o) = Real(dir);
         }
         if (reduce)
         {
             red[((K * NCH + 0) * GP + w) * SB_COLS + lane] = Real(up);
-            red[((K * NCH + 1) * GP + w) * SB_COLS + lane] = Real(dn + dir);
+            red[((K * NCH + 1) * GP + w) * SB_COLS + lane] = Real(add_alone(dn, dir));
             red[((K * NCH + 2) * GP + w) * SB_COLS + lane] = Real(dir);
         }
         up_below = up;
@@ -715,29 +756,31 @@ void sw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1,
                 if (kk < nk)
                 {
                     const St R = sR[kk], T = sT[kk];
-                    const St den = rcp_den(St(1) - R * A);
-                    S = St(sSU[kk]) + T * (S + A * St(sSD[kk])) * den;
-                    A = R + T * T * A * den;
+                    const St den = rcp_den(fma_of(-R, A, St(1)));
+                    S = fma_of(T * fma_of(A, St(sSD[kk]), S), den, St(sSU[kk]));
+                    A = fma_of(T * T * A, den, R);
                     const St ru = sRup[kk];
-                    const St dn = (St(sD[kk]) + ru * S) * rcp_den(St(1) - ru * A);
-                    const St up = A * dn + S;
+                    const St dn = fma_of(ru, S, St(sD[kk])) * rcp_den(fma_of(-ru, A, St(1)));
+                    const St up = fma_of(A, dn, S);
                     const St dd = sDir[kk];
                     if (up_g)
                     {
                         const uint32_t o = ucol + uncol * lev_of(j0 + kk);
-                        at32(up_g, o) = Real(up); at32(dn_g, o) = Real(dn + dd); at32(dir_g, o) = Real(dd);
+                        at32(up_g, o) = Real(up); at32(dn_g, o) = Real(add_alone(dn, dd)); at32(dir_g, o) = Real(dd);
                     }
                     if (reduce)
                     {
                         red[((kk * NCH + 0) * GP + w) * SB_COLS + lane] = Real(up);
-                        red[((kk * NCH + 1) * GP + w) * SB_COLS + lane] = Real(dn + dd);
+                        red[((kk * NCH + 1) * GP + w) * SB_COLS + lane] = Real(add_alone(dn, dd));
                         red[((kk * NCH + 2) * GP + w) * SB_COLS + lane] = Real(dd);
                     }
                     if constexpr (HR)
                     {
-                        const St ab = (dn + up_below) * St(sAb[kk]) + dd * St(sOmTn[kk]) - St(sSU[kk]) -
-                                      St(sSD[kk]);
-                        red[((kk * NCH + NC) * GP + w) * SB_COLS + lane] = Real(ab);
+                        const St ab = add_alone(add_alone(fma_of(add_alone(dn, up_below), St(sAb[kk]),
+                                                                 dd * St(sOmTn[kk])), -St(sSU[kk])), -St(sSD[kk]));
+                        if constexpr (SUMS) red[((kk * NCH + NC) * GP + w) * SB_COLS + lane] = Real(ab);
+                        else
+                            at32(reinterpret_cast<Real*>(absorbed) + lslab, ucol + uncol * lay_of(j0 + kk)) = Real(ab);
                         up_below = up;
                     }
                 }
@@ -813,10 +856,9 @@ __global__ void group_sums_kernel(int64_t ncv, GroupSums<Real> q)
     if (bb) bb[i] = first ? band : total + band;
 }
 
-// The sums that some output wants, in one launch.
+// The sums that some output wants.
 template<typename Real>
-int group_sums(int64_t ncv, const Groups& grp, int n, const Real* const* gf, Real* const* bnd, Real* const* bb,
-               hipStream_t s)
+GroupSums<Real> wanted_sums(const Groups& grp, int n, const Real* const* gf, Real* const* bnd, Real* const* bb)
 {
     GroupSums<Real> q{};
     for (int c = 0; c < n; ++c)
@@ -825,13 +867,131 @@ int group_sums(int64_t ncv, const Groups& grp, int n, const Real* const* gf, Rea
         q.gf[q.n] = gf[c]; q.bnd[q.n] = bnd[c]; q.bb[q.n] = bb[c];
         ++q.n;
     }
-    if (q.n == 0) return RRTMGP_OK;
     q.ngroups = grp.n;
     for (int g = 0; g < grp.n; ++g)
         if (g == 0 || grp.band[g] != grp.band[g - 1]) q.begins[g / 64] |= uint64_t(1) << (g % 64);
+    return q;
+}
+
+template<typename Real>
+int group_sums(int64_t ncv, const Groups& grp, int n, const Real* const* gf, Real* const* bnd, Real* const* bb,
+               hipStream_t s)
+{
+    const GroupSums<Real> q = wanted_sums<Real>(grp, n, gf, bnd, bb);
+    if (q.n == 0) return RRTMGP_OK;
     RRTMGP_TIMED("group_sums_kernel", s);
     hipLaunchKernelGGL(group_sums_kernel<Real>, dim3(grid1(ncv, 256), unsigned(q.n)), dim3(256), 0, s, ncv, q);
     RRTMGP_LAUNCHED("group_sums_kernel");
+    return RRTMGP_OK;
+}
+
+// The same sums from the fluxes of every g-point, and heating rates from their absorbed fluxes (blockIdx.y: the
+// flux components, then the heating rate): g-points in order within each group of up to 16, then as
+// group_sums_kernel and absorbed_heating_rate_kernel do, so that a call gives the same bits whether its
+// work-groups were cut or not.  A work-group takes 64 (column, level) pairs, 16 groups at a time with a thread
+// each.
+template<typename Real>
+struct GPointSums
+{
+    GroupSums<Real> f;                     // gf: g-point fluxes (ncol, nlev, ngpt)
+    const Real* absorbed;                  // (ncol, nlay, ngpt, nparts), or NULL
+    const Real* plev;
+    Real* hr;
+    int nparts;
+};
+
+template<typename Real>
+__global__ __launch_bounds__(SB_COLS * 16)
+void g_point_sums_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, Groups grp, GPointSums<Real> q)
+{
+    __shared__ double s_abs[2][16][SB_COLS];
+    Real (*s_sum)[SB_COLS] = reinterpret_cast<Real (*)[SB_COLS]>(&s_abs[0][0][0]);
+    const int lane = threadIdx.x, y = threadIdx.y;
+    const int64_t i = int64_t(blockIdx.x) * SB_COLS + lane;
+    const bool heating = int(blockIdx.y) == q.f.n;         // uniform over the work-group, as is every count below
+    const int64_t n = ncol * (heating ? nlay : nlay + 1);
+    const Real* in = heating ? q.absorbed : q.f.gf[blockIdx.y];
+    Real* bnd = heating ? nullptr : q.f.bnd[blockIdx.y];
+    Real total = Real(0), band = Real(0);
+    double rate = 0.;
+    int64_t o = i;
+    bool first = true;
+    for (int g0 = 0; g0 < grp.n; g0 += 16)
+    {
+        if (i < n && g0 + y < grp.n)
+        {
+            const int count = grp.count[g0 + y];
+            const Real* p = in + i + n * grp.start[g0 + y];
+            for (int part = 0; part < (heating ? q.nparts : 1); ++part, p += n * ngpt)
+            {
+                Real v[16];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) v[k] = p[n * min(k, count - 1)];
+                if (heating)
+                {
+                    double s = double(v[0]);
+#pragma unroll
+                    for (int k = 1; k < 16; ++k)
+                        if (k < count) s += double(v[k]);
+                    s_abs[part][y][lane] = s;
+                }
+                else
+                {
+                    Real s = v[0];
+#pragma unroll
+                    for (int k = 1; k < 16; ++k)
+                        if (k < count) s += v[k];
+                    s_sum[y][lane] = s;
+                }
+            }
+        }
+        __syncthreads();
+        if (y == 0 && i < n)
+            for (int k = 0; k < 16 && g0 + k < grp.n; ++k)
+            {
+                const int g = g0 + k;
+                if (heating)
+                {
+                    for (int part = 0; part < q.nparts; ++part) rate += s_abs[part][k][lane];
+                    continue;
+                }
+                const Real v = s_sum[k][lane];
+                if (!(q.f.begins[g / 64] >> (g % 64) & 1)) { band = band + v; continue; }
+                if (g > 0)
+                {
+                    if (bnd) bnd[o] = band;
+                    o += n;
+                    total = first ? band : total + band;
+                    first = false;
+                }
+                band = v;
+            }
+        __syncthreads();
+    }
+    if (y != 0 || i >= n) return;
+    if (heating)
+    {
+        q.hr[i] = absorbed_rate(rate, q.plev[i], q.plev[i + ncol]);
+        return;
+    }
+    if (bnd) bnd[o] = band;
+    if (q.f.bb[blockIdx.y]) q.f.bb[blockIdx.y][i] = first ? band : total + band;
+}
+
+template<typename Real>
+int g_point_sums(int64_t ncol, int64_t nlay, int64_t ngpt, int64_t nbnd, const int* band_lims, int n,
+                 const Real* const* gf, Real* const* bnd, Real* const* bb, const Real* absorbed, int nparts,
+                 const Real* plev, Real* hr, hipStream_t s)
+{
+    Groups grp;
+    RRTMGP_TRY(make_groups(ngpt, nbnd, band_lims, grp));
+    GPointSums<Real> q{};
+    q.f = wanted_sums<Real>(grp, n, gf, bnd, bb);
+    q.absorbed = absorbed; q.plev = plev; q.hr = hr; q.nparts = nparts;
+    RRTMGP_TIMED("g_point_sums_kernel", s);
+    hipLaunchKernelGGL(g_point_sums_kernel<Real>, dim3(grid1(ncol * (nlay + 1), SB_COLS), unsigned(q.f.n + (hr ? 1 : 0))),
+                       dim3(SB_COLS, 16), 0, s, ncol, nlay, ngpt, grp, q);
+    RRTMGP_LAUNCHED("g_point_sums_kernel");
     return RRTMGP_OK;
 }
 
@@ -904,15 +1064,23 @@ int lw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t nm
     hipStream_t s = as_stream(stream);
     Groups grp;
     int gpts = SB_GPTS;
-    RRTMGP_TRY(make_groups_for(grid1(ncol, SB_COLS), ngpt, band_lims ? nbnd : 1, band_lims, grp, gpts));
+    if (do_jac) RRTMGP_TRY(make_groups(ngpt, band_lims ? nbnd : 1, band_lims, grp));
+    else RRTMGP_TRY(make_groups_for(grid1(ncol, SB_COLS), ngpt, band_lims ? nbnd : 1, band_lims, grp, gpts));
+    const bool small = gpts <= SMALL_GPTS;                 // leaves g-point fluxes for g_point_sums
     const int64_t ncv = ncol * (nlay + 1);
-    const bool direct = bnd_up != nullptr && grp.n == int(nbnd);
+    const bool direct = !small && bnd_up != nullptr && grp.n == int(nbnd);
     const dim3 grid(grid1(ncol, SB_COLS), unsigned(grp.n));
     const dim3 block(SB_COLS, unsigned(gpts));
 
     Real *g_up = nullptr, *g_dn = nullptr, *g_jac = nullptr, *scratch = nullptr;
     double* absorbed = nullptr;
-    if (!spectral)
+    if (!spectral && small)
+    {
+        RRTMGP_TRY(scratch_alloc(&scratch, size_t(ncv * ngpt * 2), s));
+        flux_up = scratch;
+        flux_dn = scratch + ncv * ngpt;
+    }
+    else if (!spectral)
     {
         const int64_t nbuf = (direct ? 0 : 2) + (do_jac ? 1 : 0);
         RRTMGP_TRY(scratch_alloc(&scratch, size_t(ncv * grp.n * nbuf), s));
@@ -923,7 +1091,10 @@ int lw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t nm
     if (heating_rate)
     {
         // Per-group absorbed fluxes of the down and the up sweep, FP64, every element written.
-        const int rc0 = scratch_alloc(&absorbed, size_t(ncol * nlay * grp.n * 2), s);
+        // (Small work-groups: of every g-point, in the build's precision.)
+        const size_t n_abs = small ? (size_t(ncol * nlay * ngpt * 2) * sizeof(Real) + 7) / 8
+                                   : size_t(ncol * nlay * grp.n * 2);
+        const int rc0 = scratch_alloc(&absorbed, n_abs, s);
         if (rc0 != RRTMGP_OK) { scratch_free(scratch, s); return rc0; }
     }
     int rc = RRTMGP_OK;
@@ -938,8 +1109,8 @@ int lw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t nm
         auto choose = [&](auto gp) {
             constexpr int GP = decltype(gp)::value;
             if (do_jac)
-                launch(nmus == 1 ? lw_solver_kernel<GP, Real, true, 1, false> : lw_solver_kernel<GP, Real, true, 4, false>,
-                       sfc_src_jac, g_jac);
+                launch(nmus == 1 ? lw_solver_kernel<SB_GPTS, Real, true, 1, false>
+                                 : lw_solver_kernel<SB_GPTS, Real, true, 4, false>, sfc_src_jac, g_jac);
             else if (heating_rate && factored)
                 launch(nmus == 1 ? lw_solver_kernel<GP, Real, false, 1, true, true>
                                  : lw_solver_kernel<GP, Real, false, 4, true, true>, nullptr, nullptr);
@@ -957,14 +1128,22 @@ int lw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, int64_t nm
         else choose(std::integral_constant<int, SB_GPTS>());
         rc = check_hip(hipGetLastError(), "lw_solver_kernel");
     }
-    if (rc == RRTMGP_OK && !spectral)
+    if (rc == RRTMGP_OK && !spectral && small)
+    {
+        const Real* const gf[2] = {flux_up, flux_dn};
+        Real* const bo[2] = {bnd_up, bnd_dn};
+        Real* const bbo[2] = {bb_up, bb_dn};
+        rc = g_point_sums<Real>(ncol, nlay, ngpt, band_lims ? nbnd : 1, band_lims, 2, gf, bo, bbo,
+                                reinterpret_cast<const Real*>(absorbed), 2, plev, heating_rate, s);
+    }
+    else if (rc == RRTMGP_OK && !spectral)
     {
         const Real* const gf[3] = {g_up, g_dn, g_jac};
         Real* const bo[3] = {direct ? nullptr : bnd_up, direct ? nullptr : bnd_dn, nullptr};
         Real* const bbo[3] = {bb_up, bb_dn, do_jac ? flux_up_jac : nullptr};
         rc = group_sums<Real>(ncv, grp, 3, gf, bo, bbo, s);
     }
-    if (rc == RRTMGP_OK && heating_rate)
+    if (rc == RRTMGP_OK && heating_rate && !small)
         rc = absorbed_heating_rate<Real>(ncol, nlay, grp.n, 2, absorbed, plev, heating_rate, s);
     scratch_free(absorbed, s);
     scratch_free(scratch, s);
@@ -1014,7 +1193,7 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
         return arg_error("sw_solver: heating rates need plev and summed (not g-point) flux outputs");
     if (by_band && (!band_lims || nbnd < 1)) return arg_error("sw_solver: band surface inputs need band limits");
     // 32-bit lane offsets within one g-point's slab of levels or of checkpoints.
-    int K = sw_seg_k(sizeof(Real) == 4, coalbedo, heating_rate != nullptr, SB_GPTS);
+    int K = sw_seg_k(sizeof(Real) == 4, SB_GPTS);
     if (ncol * std::max<int64_t>(nlay + 1, 3 * ((nlay + K - 1) / K)) * int64_t(sizeof(Real)) >= (int64_t(1) << 32))
         return arg_error("sw_solver: ncol * (nlay + 1) values of one g-point must stay below 4 GiB");
     if (!tau || !ssa || !g || !mu0 || !alb_dir || !alb_dif || !inc_dir) return arg_error("sw_solver: NULL input");
@@ -1030,7 +1209,7 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
     Groups grp;
     int gpts = SB_GPTS;
     RRTMGP_TRY(make_groups_for(grid1(ncol, SB_COLS), ngpt, band_lims ? nbnd : 1, band_lims, grp, gpts));
-    if (gpts <= SMALL_GPTS) K = SEG8;
+    if (gpts <= SMALL_GPTS) K = sw_seg_k(sizeof(Real) == 4, SMALL_GPTS);
     const int64_t ncv = ncol * (nlay + 1);
 
     // Every element of the checkpoints, group partials and heating-rate parts is written by the
@@ -1038,22 +1217,30 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
     Real *ckpt = nullptr, *scratch = nullptr;
     double* absorbed = nullptr;
     const auto checkpoints = [&] { return size_t((nlay + K - 1) / K * 3 * ngpt * ncol); };
-    const auto is_direct = [&] { return want_bnd && grp.n == int(nbnd); };
-    const auto parts = [&] { return (!spectral && !is_direct()) ? size_t(ncv * grp.n * 3) : size_t(0); };
-    const auto abs_parts = [&] { return heating_rate ? size_t(ncol * nlay * grp.n) : size_t(0); };
+    // Small work-groups leave the fluxes of every g-point (and their absorbed fluxes, in the build's precision)
+    // for g_point_sums, the others sums over groups.
+    const auto is_small = [&] { return gpts <= SMALL_GPTS; };
+    const auto is_direct = [&] { return !is_small() && want_bnd && grp.n == int(nbnd); };
+    const auto parts = [&] {
+        return (!spectral && !is_direct()) ? size_t(ncv * (is_small() ? ngpt : grp.n) * 3) : size_t(0);
+    };
+    const auto abs_parts = [&] {
+        if (!heating_rate) return size_t(0);
+        return is_small() ? (size_t(ncol * nlay * ngpt) * sizeof(Real) + 7) / 8 : size_t(ncol * nlay * grp.n);
+    };
     auto round256 = [](size_t b) { return (b + 255) & ~size_t(255); };
     const auto needed = [&] {
         return round256(checkpoints() * sizeof(Real)) + round256(parts() * sizeof(Real)) +
                round256(abs_parts() * sizeof(double));
     };
-    // Smaller groups have more partial sums: where a fixed workspace does not hold them, whole ones.
+    // Where a fixed workspace does not hold every g-point's fluxes, whole groups.
     if (workspace && gpts < SB_GPTS && needed() > workspace_bytes)
     {
         gpts = SB_GPTS;
-        K = sw_seg_k(sizeof(Real) == 4, coalbedo, heating_rate != nullptr, SB_GPTS);
+        K = sw_seg_k(sizeof(Real) == 4, SB_GPTS);
         RRTMGP_TRY(make_groups(ngpt, band_lims ? nbnd : 1, band_lims, grp));
     }
-    const bool direct = is_direct();
+    const bool direct = is_direct(), small = is_small();
     const size_t n_ck = checkpoints(), n_part = parts(), n_abs = abs_parts();
     const dim3 grid(grid1(ncol, SB_COLS), unsigned(grp.n));
     const dim3 block(SB_COLS, unsigned(gpts));
@@ -1087,7 +1274,10 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
     Real* gf[3] = {nullptr, nullptr, nullptr};
     Real* const bo[3] = {bnd_up, bnd_dn, bnd_dir};
     Real* const bbo[3] = {bb_up, bb_dn, bb_dir};
-    if (!spectral)
+    Real* sf[3] = {flux_up, flux_dn, flux_dir};
+    if (!spectral && small)
+        for (int c = 0; c < 3; ++c) sf[c] = scratch + ncv * ngpt * c;
+    else if (!spectral)
         for (int c = 0; c < 3; ++c) gf[c] = direct ? bo[c] : scratch + ncv * grp.n * c;
     int rc = RRTMGP_OK;
     {
@@ -1098,19 +1288,22 @@ int sw_solver(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, const Real
                 ? (coalbedo ? sw_solver_kernel<GP, Real, true, true> : sw_solver_kernel<GP, Real, true, false>)
                 : (coalbedo ? sw_solver_kernel<GP, Real, false, true> : sw_solver_kernel<GP, Real, false, false>);
             hipLaunchKernelGGL(kernel, grid, block, 0, s, ncol, nlay, ngpt, top_at_1, tau, ssa, g, mu0, alb_dir,
-                               alb_dif, inc_dir, has_dif_bc ? inc_dif : nullptr, flux_up, flux_dn, flux_dir, ckpt, grp,
+                               alb_dif, inc_dir, has_dif_bc ? inc_dif : nullptr, sf[0], sf[1], sf[2], ckpt, grp,
                                gf[0], gf[1], gf[2], by_band ? nbnd : int64_t(0), absorbed);
         };
         if (gpts <= SMALL_GPTS) choose(std::integral_constant<int, SMALL_GPTS>());
         else choose(std::integral_constant<int, SB_GPTS>());
         rc = check_hip(hipGetLastError(), "sw_solver_kernel");
     }
-    if (rc == RRTMGP_OK && !spectral)
+    if (rc == RRTMGP_OK && !spectral && small)
+        rc = g_point_sums<Real>(ncol, nlay, ngpt, band_lims ? nbnd : 1, band_lims, 3, sf, bo, bbo,
+                                reinterpret_cast<const Real*>(absorbed), 1, plev, heating_rate, s);
+    else if (rc == RRTMGP_OK && !spectral)
     {
         Real* const none[3] = {nullptr, nullptr, nullptr};
         rc = group_sums<Real>(ncv, grp, 3, gf, direct ? none : bo, bbo, s);
     }
-    if (rc == RRTMGP_OK && heating_rate)
+    if (rc == RRTMGP_OK && heating_rate && !small)
         rc = absorbed_heating_rate<Real>(ncol, nlay, grp.n, 1, absorbed, plev, heating_rate, s);
     if (!workspace)
     {

@@ -57,8 +57,8 @@ inline int make_groups(int64_t ngpt, int64_t nbnd, const int* band_lims, Groups&
 // for.  A layer step of 16 wavefronts takes a compute unit four times as long as one of 4, one per SIMD: the
 // solvers are bound by the issue rate there.  So where the work-groups of 16 would leave compute units idle,
 // the bands are cut into halves or quarters as long as the chip holds the work-groups at once.  64 columns x
-// 60 layers FP32: SW 125 us in groups of 16, 69 us in groups of 4; LW 80 and 37 us; 250 x 60 FP64: 269 and 110, 165
-// and 64 us.
+// 60 layers FP32: SW 125 us in groups of 16, 66 us in groups of 4; LW 80 and 37 us; 250 x 60 FP64: 269 and 110, 165
+// and 64 us.  The small work-groups leave g-point fluxes, which are then added in the order of groups of 16.
 inline int make_groups_for(int64_t tiles, int64_t ngpt, int64_t nbnd, const int* band_lims, Groups& g, int& gpts)
 {
     gpts = SB_GPTS;

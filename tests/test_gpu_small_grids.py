@@ -1,10 +1,6 @@
 """Calls too small to fill the chip cut the bands over more work-groups (solvers: 8 or 4 g-points each; gas
-optics: fewer bands each).  The same columns as part of a call that is not cut give the same fluxes up to the
-order of the g-point sums, and the same gas optics exactly; column counts around the tile and split edges,
-with the ragged bands (1 to 33 g-points) of the gas-optics tests.
-
-Bar: sums of n = 91 positive terms in another order differ by less than n eps of the sum (heating rates: of
-the largest absolute rate, whose terms have both signs).
+optics: fewer bands each).  The same columns as part of a call that is not cut give the same bits; column
+counts around the tile and split edges, with the ragged bands (1 to 33 g-points) of the gas-optics tests.
 """
 import numpy as np
 import pytest
@@ -30,7 +26,6 @@ def test_split_matches_whole(G, syn, precision, ncol):
     small = syn.subset_columns(big, np.arange(ncol))
     kl = G.KDist(ragged(syn.make_kdist(True, 11)), AVAILABLE, precision)
     ks = G.KDist(ragged(syn.make_kdist(False, 12)), AVAILABLE, precision)
-    tol = 91 * np.finfo(G.real_dtype(precision)).eps
 
     def run(atm):
         n = atm.p_lay.shape[0]
@@ -48,10 +43,4 @@ def test_split_matches_whole(G, syn, precision, ncol):
     whole, part = run(big), run(small)
     assert whole.keys() == part.keys()
     for k in whole:
-        w = whole[k][:ncol]
-        if k.startswith("gas"):
-            assert np.array_equal(part[k], w), k
-        elif "heating" in k or "net" in k:
-            assert np.abs(part[k] - w).max() <= 2 * tol * np.abs(whole[k]).max(), k
-        else:
-            assert np.abs(part[k] - w).max() <= tol * np.abs(whole[k]).max(), k
+        assert np.array_equal(part[k], whole[k][:ncol]), k
