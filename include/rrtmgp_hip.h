@@ -230,7 +230,13 @@ RRTMGP_DECLARE_BOTH(RRTMGP_DECL_GAS_OPTICS_SW)
     int rrtmgp_hip_gas_optics_sw_coalbedo_##S(const rrtmgp_kdist_dev* kd, int64_t ncol,        \
         int64_t nlay, const T* play, const T* tlay, const T* col_dry,                            \
         const rrtmgp_gas_vmr* gases, const T* cloud_tau, const T* cloud_coalbedo,               \
-        const T* cloud_g, T* tau, T* coalbedo, T* g, void* stream);
+        const T* cloud_g, T* tau, T* coalbedo, T* g, void* stream);                             \
+    /* and with a second set of band properties, added after the clouds (which may be NULL) */  \
+    int rrtmgp_hip_gas_optics_sw_coalbedo_aerosol_##S(const rrtmgp_kdist_dev* kd, int64_t ncol, \
+        int64_t nlay, const T* play, const T* tlay, const T* col_dry,                            \
+        const rrtmgp_gas_vmr* gases, const T* cloud_tau, const T* cloud_coalbedo,               \
+        const T* cloud_g, const T* aerosol_tau, const T* aerosol_coalbedo, const T* aerosol_g,  \
+        T* tau, T* coalbedo, T* g, void* stream);
 RRTMGP_DECLARE_BOTH(RRTMGP_DECL_GAS_OPTICS_SW_CO)
 
 /* The fused gas optics restricted to listed (64-column tile, layer) pairs: tiles[i] =         */

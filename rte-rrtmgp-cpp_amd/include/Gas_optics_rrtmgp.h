@@ -136,6 +136,7 @@ class Gas_optics_rrtmgp_gpu : public Gas_optics_gpu
         // the gas-optics write).  cloud may be nullptr.  The shortwave one with coalbedo writes
         // the co-albedo 1 - ssa in place of ssa, and reads the cloud's as co-albedo too
         // (rrtmgp_hip_gas_optics_sw_coalbedo_*; plain gas optics only, not with a surrogate).
+        // With coalbedo, aerosol is a second set of band properties, added after the cloud's.
         // top_at_1, when given, receives play(1, 1) < play(1, nlay), read with the range checks.
         void gas_optics_with_clouds(
                 const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev,
@@ -149,7 +150,8 @@ class Gas_optics_rrtmgp_gpu : public Gas_optics_gpu
                 const Array_gpu<Float,2>& tlay, const Gas_concs_gpu& gas_desc,
                 Optical_props_arry_gpu& optical_props, Array_gpu<Float,2>& toa_src,
                 const Array_gpu<Float,2>& col_dry, const Optical_props_arry_gpu* cloud,
-                bool coalbedo = false, Bool* top_at_1 = nullptr);
+                bool coalbedo = false, Bool* top_at_1 = nullptr,
+                const Optical_props_arry_gpu* aerosol = nullptr);
 
         // gas concentrations as the rrtmgp_gas_vmr descriptor of the kernels, in this
         // k-distribution's gas order

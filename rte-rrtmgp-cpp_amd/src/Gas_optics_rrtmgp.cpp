@@ -617,10 +617,14 @@ void Gas_optics_rrtmgp_gpu::gas_optics_with_clouds(
 void Gas_optics_rrtmgp_gpu::gas_optics_with_clouds(
         const Array_gpu<Float,2>& play, const Array_gpu<Float,2>& plev, const Array_gpu<Float,2>& tlay,
         const Gas_concs_gpu& gas_desc, Optical_props_arry_gpu& props, Array_gpu<Float,2>& toa_src,
-        const Array_gpu<Float,2>& col_dry, const Optical_props_arry_gpu* cloud, bool coalbedo, Bool* top_at_1)
+        const Array_gpu<Float,2>& col_dry, const Optical_props_arry_gpu* cloud, bool coalbedo, Bool* top_at_1,
+        const Optical_props_arry_gpu* aerosol)
 {
     if (krayl.size() == 0) throw std::runtime_error("shortwave gas_optics called on a longwave k-distribution");
     if (coalbedo && use_mlp) throw std::invalid_argument("co-albedo gas optics with a surrogate set");
+    if (aerosol && !coalbedo) throw std::invalid_argument("aerosols are added here in the co-albedo form only");
+    if (aerosol && aerosol->get_ngpt() != get_nband())
+        throw std::runtime_error("add_to_coalbedo: the input must be band-resolved on the output's bands");
     const int ncol = play.dim(1), nlay = play.dim(2);
     (void)check_inputs(play, plev, tlay, col_dry, nullptr, nullptr, top_at_1);
     rrtmgp_gas_vmr v;
@@ -644,6 +648,11 @@ void Gas_optics_rrtmgp_gpu::gas_optics_with_clouds(
                                                     props.get_tau().ptr(), props.get_ssa().ptr(),
                                                     props.get_g().ptr(), stream()));
     }
+    else if (aerosol)
+        hip_check(K<Float>::gas_optics_sw_coalbedo_aerosol(
+                &dev, ncol, nlay, play.ptr(), tlay.ptr(), col_dry.ptr(), &v, ct, cs, cg, aerosol->get_tau().ptr(),
+                aerosol->get_ssa().ptr(), aerosol->get_g().ptr(), props.get_tau().ptr(), props.get_ssa().ptr(),
+                props.get_g().ptr(), stream()));
     else if (coalbedo)
         hip_check(K<Float>::gas_optics_sw_coalbedo(&dev, ncol, nlay, play.ptr(), tlay.ptr(), col_dry.ptr(), &v, ct,
                                                    cs, cg, props.get_tau().ptr(), props.get_ssa().ptr(),

@@ -344,8 +344,6 @@ void Radiation_solver_shortwave_gpu::solve_gpu(
             else cloud_optics->cloud_optics(a, b, c, d, *cloud_props);
             cloud = cloud_props.get();
         }
-        kdist->gas_optics_with_clouds(pl, pv, tl, gc, *optical_props, toa_src, cd, cloud, co,
-                                      c0 == 0 ? &top_at_1 : nullptr);
         if (switch_aerosol_optics)
         {
             std::unique_ptr<Aerosol_concs_gpu> asub;
@@ -353,10 +351,13 @@ void Radiation_solver_shortwave_gpu::solve_gpu(
             Array_gpu<Float,2> rhb = block_of(rh, c0, n, ws.rh);
             const Aerosol_concs_gpu& ac = whole ? aerosol_concs : *asub;
             aerosol_optics->compute(ac, rhb, pv, switch_delta_aerosol, *aerosol_props, co);
-            auto& ops = dynamic_cast<Optical_props_2str_gpu&>(*optical_props);
-            if (co) add_to_coalbedo(ops, *aerosol_props);
-            else add_to(ops, *aerosol_props);
         }
+        // The gas optics adds clouds and, in the co-albedo form, aerosols as it writes.
+        kdist->gas_optics_with_clouds(pl, pv, tl, gc, *optical_props, toa_src, cd, cloud, co,
+                                      c0 == 0 ? &top_at_1 : nullptr,
+                                      switch_aerosol_optics && co ? aerosol_props.get() : nullptr);
+        if (switch_aerosol_optics && !co)
+            add_to(dynamic_cast<Optical_props_2str_gpu&>(*optical_props), *aerosol_props);
         // TSI scaling of the incoming flux (src_test/Radiation_solver.cpp:739-743).
         hip_check(K<Float>::scale_by_col(n, ngpt, toa_src.ptr(), tsi.ptr(), stream()));
 

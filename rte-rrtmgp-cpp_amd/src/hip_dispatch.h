@@ -25,6 +25,7 @@ template<typename T> struct K;
     static constexpr auto gpt_to_band = rrtmgp_hip_gpt_to_band_##S; \
     static constexpr auto gas_optics_sw = rrtmgp_hip_gas_optics_sw_##S;  \
     static constexpr auto gas_optics_sw_coalbedo = rrtmgp_hip_gas_optics_sw_coalbedo_##S; \
+    static constexpr auto gas_optics_sw_coalbedo_aerosol = rrtmgp_hip_gas_optics_sw_coalbedo_aerosol_##S; \
     static constexpr auto interpolation = rrtmgp_hip_interpolation_##S;  \
     static constexpr auto compute_tau_absorption = rrtmgp_hip_compute_tau_absorption_##S; \
     static constexpr auto compute_tau_rayleigh = rrtmgp_hip_compute_tau_rayleigh_##S;     \
