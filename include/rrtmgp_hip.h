@@ -259,8 +259,8 @@ RRTMGP_DECLARE_BOTH(RRTMGP_DECL_GAS_OPTICS_TILES)
 /* The fused entries above restricted to bands band_start .. band_start+band_count-1 (0-based):*/
 /* the output g-point dimension is that range's g-points only (ngpt_range, counted from the    */
 /* first g-point of band_start); cloud arrays stay (ncol, nlay, nbnd).  No counterpart in the  */
-/* reference (whose gas optics always covers every band); used by the adjoint driver to        */
-/* recompute gas optics band by band.                                                           */
+/* reference (whose gas optics always covers every band).  The adjoint drivers use the forms    */
+/* of a band range further below.                                                               */
 #define RRTMGP_DECL_GAS_OPTICS_BANDS(S, T)                                                     \
     int rrtmgp_hip_gas_optics_lw_bands_##S(const rrtmgp_kdist_dev* kd, int64_t band_start,     \
         int64_t band_count, int64_t ncol, int64_t nlay, const T* play, const T* tlay,          \

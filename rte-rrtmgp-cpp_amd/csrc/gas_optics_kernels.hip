@@ -1216,8 +1216,10 @@ constexpr int ga_arrays() { return MODE == GA_LW3 ? 4 : MODE == GA_SW3 ? 3 : 2; 
 // At 16384 columns x 128 layers in FP32 both spectral ranges take 14.5 ms (two shortwave and four longwave
 // bands a launch); with one band a launch, phases 1 and 3 on one wavefront reading and writing memory, and
 // every table node of a pair live at once they took 25.5 ms.
+// GA_LW3 holds three more cotangents a g-point and their Planck terms: at the others' occupancy it spills 67
+// registers (a band of 16 g-points at 8192 x 64 FP64: 909 us, 577 us with the registers it asks for).
 template<typename Real, int MODE>
-__global__ __launch_bounds__(GO_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 4 : 2)))
+__global__ __launch_bounds__(GO_THREADS) __attribute__((amdgpu_waves_per_eu(MODE == GA_LW3 ? (sizeof(Real) == 4 ? 3 : 1) : sizeof(Real) == 4 ? 4 : 2)))
 void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t nlay, GoGrid grid,
                                const Real* __restrict__ play, const Real* __restrict__ tlay,
                                const Real* __restrict__ tlev, const Real* __restrict__ tsfc,
