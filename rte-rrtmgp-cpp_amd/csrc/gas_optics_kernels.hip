@@ -1219,7 +1219,8 @@ constexpr int ga_arrays() { return MODE == GA_LW3 ? 4 : MODE == GA_SW3 ? 3 : 2; 
 // GA_LW3 holds three more cotangents a g-point and their Planck terms: at the others' occupancy it spills 67
 // registers (a band of 16 g-points at 8192 x 64 FP64: 909 us, 577 us with the registers it asks for).
 template<typename Real, int MODE>
-__global__ __launch_bounds__(GO_THREADS) __attribute__((amdgpu_waves_per_eu(MODE == GA_LW3 ? (sizeof(Real) == 4 ? 3 : 1) : sizeof(Real) == 4 ? 4 : 2)))
+__global__ __launch_bounds__(GO_THREADS)
+__attribute__((amdgpu_waves_per_eu(MODE == GA_LW3 ? (sizeof(Real) == 4 ? 3 : 1) : sizeof(Real) == 4 ? 4 : 2)))
 void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t nlay, GoGrid grid,
                                const Real* __restrict__ play, const Real* __restrict__ tlay,
                                const Real* __restrict__ tlev, const Real* __restrict__ tsfc,
@@ -2132,8 +2133,8 @@ int col_dry_adjoint(int64_t ncol, int64_t nlay, const Real* h2o, int64_t d1, int
     if (!((d1 == 1 || d1 == ncol) && (d2 == 1 || d2 == nlay))) return arg_error("col_dry_adjoint: bad h2o dims");
     const int64_t scol = d1 == 1 ? 0 : 1, slay = d2 == 1 ? 0 : d1;
     RRTMGP_TIMED("col_dry_adjoint_kernel", as_stream(stream));
-    hipLaunchKernelGGL(col_dry_adjoint_kernel<Real>, dim3(grid1(ncol * (nlay + 1), 256)), dim3(256), 0, as_stream(stream),
-                       ncol, nlay, h2o, scol, slay, plev, g_col_dry, d_h2o, d_plev);
+    hipLaunchKernelGGL(col_dry_adjoint_kernel<Real>, dim3(grid1(ncol * (nlay + 1), 256)), dim3(256), 0,
+                       as_stream(stream), ncol, nlay, h2o, scol, slay, plev, g_col_dry, d_h2o, d_plev);
     RRTMGP_LAUNCHED("col_dry_adjoint_kernel");
     return RRTMGP_OK;
 }
