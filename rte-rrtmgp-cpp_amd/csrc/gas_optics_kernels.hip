@@ -435,6 +435,20 @@ struct PairInLds
     __device__ Real t_sfc() const { return v(GO_IN_FIXED + ngas + 2); }
 };
 
+// The same with the gases in memory: for a single band, which reads few of them.
+template<typename Real>
+struct PairInMem : PairInLds<Real>
+{
+    const GasRef<Real>* sg;
+    int64_t icol, ilay;
+    __device__ Real col(int gas, Real cdv) const
+    {
+        if (gas == 0) return cdv;
+        const GasRef<Real>& g = sg[gas - 1];
+        return g.p[icol * g.scol + ilay * g.slay] * cdv;
+    }
+};
+
 template<bool LW>
 __host__ __device__ constexpr int go_in_rows(int ngas) { return GO_IN_FIXED + ngas + (LW ? 3 : 0); }
 
@@ -1034,10 +1048,9 @@ void gas_optics_sw_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t nlay,
 // staged once; per band the pair states (phase 1, spread over the wavefronts), per 16-g-point chunk the
 // dot products (phase 2, lane = (pair, quad of g-points), one table node live at a time), and the chain
 // through the interpolation (ftemp, fpress, eta -> fmajor/fminor, col_mix), the minor scalings and the
-// Planck interpolation (phase 3, lane = column, the parts on different wavefronts, each adding into
-// gradient rows of its own in LDS).  Phase 3 of a band and phase 1 of the next share a barrier interval.
-// The rows are summed, in a fixed order, and added to memory once per launch.  The integer indices are
-// piecewise constant.
+// Planck interpolation (phase 3, lane = column, the parts on different wavefronts, adding into gradient
+// rows in LDS in a fixed order).  Phase 3 of a band and phase 1 of the next share a barrier interval.
+// The rows are added to memory once per launch.  The integer indices are piecewise constant.
 
 // The cotangents a launch is given.
 enum GaMode
@@ -1090,20 +1103,28 @@ __device__ __forceinline__ Real dot4(const Real (&a)[4], const Real (&b)[4])
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
 }
 
-// One wavefront's gradient rows of the 64 columns in LDS: the column amounts (0 = dry air, 1 .. ngas the
-// gases, ngas + 1 the derivative with respect to col_dry at fixed mixing ratios, times col_dry), then T, ln p.
+// Gradient rows of the 64 columns in LDS: the column amounts of dry air (0) and the gases 1 .. ngas, then the
+// rows of GaSum.  One set of gas rows serves the work-group, so that its LDS, and with it the occupancy, hardly
+// depends on the number of gases.  With a set per wavefront a k-distribution of 19 gases ran half as many
+// work-groups a compute unit as one of 5 (8192 x 64, four bands a launch: LW FP32 530 and 913 us with 5 and 19
+// gases, now 439 and 464; SW FP64 765 and 1353, now 766 and 806).  Each row has one writer at a time: wavefronts
+// 1 and 3 add the minor gases of even and odd number, wavefront 0 the major gases in the next barrier interval.
 template<typename Real>
 struct GaRows
 {
     Real* r;
-    int lane, ngas;
-    __device__ void col(int gas, Real v) const { r[gas * GO_COLS + lane] += v; }
-    __device__ void dry(Real v) const { r[(ngas + 1) * GO_COLS + lane] += v; }
-    __device__ void t(Real v) const { r[(ngas + 2) * GO_COLS + lane] += v; }
-    __device__ void lnp(Real v) const { r[(ngas + 3) * GO_COLS + lane] += v; }
+    int lane;
+    __device__ void add(int gas, Real v) const { r[gas * GO_COLS + lane] += v; }
 };
 
-inline __host__ __device__ constexpr int ga_rows(int ngas) { return ngas + 4; }
+// Sums over the bands in rows of a wavefront's own (w 0, 1, 3 and, shortwave, 2), three each: the derivative
+// with respect to col_dry at fixed mixing ratios, times col_dry; ln p; and T (0) or what dry air and h2o have in
+// common (the others; the T part of 1 and 3 is that of ln p times -1 / T).
+enum GaSum { GA_DRY, GA_LNP, GA_T, GA_XH = GA_T };
+template<bool LW> __host__ __device__ constexpr int ga_sums() { return LW ? 9 : 12; }
+__device__ __forceinline__ int ga_sum_row(int w) { return w == 3 ? 6 : w == 2 ? 9 : 3 * w; }
+
+template<bool LW> inline __host__ __device__ constexpr int ga_rows(int ngas) { return ngas + 1 + ga_sums<LW>(); }
 
 // Phase 3, the major species: the cotangents of col_mix, fmajor and fminor carried to the two gases, T and
 // ln p.  The derivative at fixed mixing ratios: every column the gas optics reads is a vmr times col_dry,
@@ -1113,7 +1134,7 @@ inline __host__ __device__ constexpr int ga_rows(int ngas) { return ngas + 4; }
 // over gases but not in rounded arithmetic, do not enter.
 template<typename Real, typename In>
 __device__ __forceinline__ void ga_major_back(const Kd<Real>& k, const GoBand& bd, const CL<Real>& c, const In& in,
-                                              Real cd, const Real* acc, const GaRows<Real>& out)
+                                              Real cd, Real* acc, Real* major, const GaRows<Real>& sum)
 {
     const int s = c.itropo, gas1 = bd.gas[s][0], gas2 = bd.gas[s][1];
     const Real c1 = in.col(gas1, cd), c2 = in.col(gas2, cd);
@@ -1152,55 +1173,55 @@ __device__ __forceinline__ void ga_major_back(const Kd<Real>& k, const GoBand& b
             g_c2 -= g_eta * eta * r * icm;
         }
     }
-    out.col(gas1, g_c1);
-    out.col(gas2, g_c2);
-    out.dry(g_dry);
-    out.t(g_ftemp / k.temp_ref_delta);
-    out.lnp(g_fp / k.press_ref_log_delta);
+    major[0] = g_c1; major[1] = g_c2; major[2] = Real(gas1 + 64 * gas2);
+    sum.add(GA_DRY, g_dry);
+    sum.add(GA_T, g_ftemp / k.temp_ref_delta);
+    sum.add(GA_LNP, g_fp / k.press_ref_log_delta);
 }
 
-// Phase 3, the minor scalings of slots q0, q0 + dq, ... (.cu:388-420): sc = col(gas) [P F], P = 0.01 p / T,
-// F = X or 1 - X with X = col(scal) / (col_dry + col(h2o)).
+// Phase 3, the minor scalings (.cu:388-420): sc = col(gas) [P F], P = 0.01 p / T, F = X or 1 - X with
+// X = col(scal) / (col_dry + col(h2o)).  A wavefront adds what goes to rows of its parity; the sums of a slot go
+// with its gas.
 template<typename Real, typename In>
 __device__ __forceinline__ void ga_minor_back(const Kd<Real>& k, const GoBand& bd, int s, const In& in, Real pv, Real tv,
-                                              Real cd, const Real* acc, int q0, int dq, const GaRows<Real>& out)
+                                              Real cd, const Real* acc, int parity, const GaRows<Real>& out,
+                                              const GaRows<Real>& sum)
 {
     const int nq = bd.nq[s];
     const Real P = Real(0.01) * pv / tv;
-    Real g_dry = Real(0), g_PP = Real(0);
-    for (int q = q0; q < nq; q += dq)
+    Real g_dry = Real(0), g_PP = Real(0), g_x = Real(0);
+    for (int q = 0; q < nq; ++q)
     {
         const GoMinor md = bd.minor[s][q];
+        const bool scaled = md.dens && md.scal_gas > 0;
+        const bool own = (md.gas & 1) == parity, own_scal = scaled && (md.scal_gas & 1) == parity;
+        if (!own && !own_scal) continue;
         const Real g_sc = acc[GA_SC + q];
         const Real base = in.col(md.gas, cd);
-        if (!md.dens)
+        Real PF = md.dens ? P : Real(1);
+        if (scaled)
         {
-            out.col(md.gas, g_sc);
-            g_dry += g_sc * base;
-            continue;
+            const Real den = cd + in.col(k.idx_h2o, cd);
+            const Real X = in.col(md.scal_gas, cd) / den;
+            if (own_scal)
+            {
+                const Real g_X = (md.compl_ ? -g_sc : g_sc) * base * P;
+                out.add(md.scal_gas, g_X / den);
+                g_x -= g_X * X / den;
+            }
+            PF *= md.compl_ ? Real(1) - X : X;
         }
-        Real F = Real(1), X = Real(0), den = Real(1);
-        if (md.scal_gas > 0)
+        if (own)
         {
-            den = cd + in.col(k.idx_h2o, cd);
-            X = in.col(md.scal_gas, cd) / den;
-            F = md.compl_ ? Real(1) - X : X;
-        }
-        out.col(md.gas, g_sc * P * F);
-        const Real v = g_sc * base * P * F;
-        g_dry += v;
-        g_PP += v;
-        if (md.scal_gas > 0)
-        {
-            const Real g_X = (md.compl_ ? -g_sc : g_sc) * base * P;
-            out.col(md.scal_gas, g_X / den);
-            out.col(0, -g_X * X / den);
-            out.col(k.idx_h2o, -g_X * X / den);
+            out.add(md.gas, g_sc * PF);
+            const Real v = g_sc * base * PF;
+            g_dry += v;
+            if (md.dens) g_PP += v;
         }
     }
-    out.dry(g_dry);
-    out.t(-g_PP / tv);
-    out.lnp(g_PP);
+    sum.add(GA_DRY, g_dry);
+    sum.add(GA_LNP, g_PP);
+    sum.add(GA_XH, g_x);
 }
 
 // Slope of a Planck table at a position of interp1d_pos.
@@ -1213,14 +1234,15 @@ __device__ __forceinline__ Real interp1d_slope(const Real* table, int idx, Real 
 template<typename Real, int MODE>
 constexpr int ga_arrays() { return MODE == GA_LW3 ? 4 : MODE == GA_SW3 ? 3 : 2; }
 
-// At 16384 columns x 128 layers in FP32 both spectral ranges take 14.5 ms (two shortwave and four longwave
+// At 16384 columns x 128 layers in FP32 both spectral ranges take 12.4 ms (two shortwave and four longwave
 // bands a launch); with one band a launch, phases 1 and 3 on one wavefront reading and writing memory, and
-// every table node of a pair live at once they took 25.5 ms.
-// GA_LW3 holds three more cotangents a g-point and their Planck terms: at the others' occupancy it spills 67
-// registers (a band of 16 g-points at 8192 x 64 FP64: 909 us, 577 us with the registers it asks for).
+// every table node of a pair live at once they took 25.5 ms.  Bound by the gathers and LDS; the occupancy by LDS
+// (57 to 93 registers in FP32, 101 to 169 in FP64): the pair sums held in registers over a band's chunks, through
+// phases 1 and 3, took 113 to 128 and spilled (14.5 ms).
+// One band a launch (GA_LW3, GA_SW3), 8192 x 64, 16 g-points: LW 143 us in FP32 and 357 in FP64, SW 135 and 296,
+// within 30 us of these with 32 gases (one wavefront's phases through memory took 181, 534, 189 and 519).
 template<typename Real, int MODE>
-__global__ __launch_bounds__(GO_THREADS)
-__attribute__((amdgpu_waves_per_eu(MODE == GA_LW3 ? (sizeof(Real) == 4 ? 3 : 1) : sizeof(Real) == 4 ? 4 : 2)))
+__global__ __launch_bounds__(GO_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 4 : 2)))
 void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t nlay, GoGrid grid,
                                const Real* __restrict__ play, const Real* __restrict__ tlay,
                                const Real* __restrict__ tlev, const Real* __restrict__ tsfc,
@@ -1229,17 +1251,29 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
     static_assert(GO_GPTS == 16 && GO_THREADS == 4 * GO_COLS, "lane layout of phase 2");
     constexpr bool LW = MODE == GA_LW3 || MODE == GA_LWF;
     constexpr int NA = ga_arrays<Real, MODE>();
+    constexpr bool ONE = MODE == GA_LW3 || MODE == GA_SW3;   // one band a launch
+    // Where the major gases' gradients (and numbers) wait in s_acc until no other wavefront adds to the rows:
+    // entries that phase 2 of the next band does not write, or with one band any.
+    constexpr int MAJOR = ONE ? GA_CM : MODE == GA_LWF ? GA_X : GA_X + 1;
     __shared__ PairState<Real> sst[GO_COLS];
     __shared__ __align__(16) Real s_g[NA][GO_GPTS][GO_COLS];
     __shared__ Real s_acc[GO_COLS][GA_N + 1];
     __shared__ ColState<Real, LW> s_cs;
-    __shared__ Real s_lev[LW ? 3 : 1][GO_COLS];              // LW: gradients of T_lev below, above, T_sfc
-    // The gas pointers are read by the input staging only: they share the cotangents' LDS.
+    __shared__ Real s_lev[LW ? 2 : 1][GO_COLS];              // LW: gradients of T_lev below, above
+    // With several bands the gas pointers are read by the input staging only: they share the cotangents' LDS.
+    // One band reads its gases from memory.
     static_assert(sizeof(GasRef<Real>) * RRTMGP_MAX_GAS <= sizeof(Real) * GO_GPTS * GO_COLS, "sg in s_g");
-    GasRef<Real>* const sg = reinterpret_cast<GasRef<Real>*>(&s_g[0][0][0]);
+    __shared__ GasRef<Real> s_ref[ONE ? RRTMGP_MAX_GAS : 1];
+    GasRef<Real>* const sg = ONE ? s_ref : reinterpret_cast<GasRef<Real>*>(&s_g[0][0][0]);
+    const int nin = ONE ? 0 : k.ngas;                        // gases among the input rows
     extern __shared__ __align__(16) unsigned char go_dyn[];
     Real* const s_in = reinterpret_cast<Real*>(go_dyn);                        // input rows, then gradient rows
-    Real* const s_d = s_in + go_in_rows<LW>(k.ngas) * GO_COLS;
+    // With one band the gradient rows are in use when the cotangents no longer are.
+    static_assert(!ONE || NA * GO_GPTS >= ga_rows<LW>(RRTMGP_MAX_GAS), "gradient rows in s_g");
+    Real* const s_d = ONE ? &s_g[0][0][0] : s_in + go_in_rows<LW>(nin) * GO_COLS;
+    auto clear_rows = [&] {
+        for (int e = threadIdx.x; e < ga_rows<LW>(k.ngas) * GO_COLS; e += GO_THREADS) s_d[e] = Real(0);
+    };
     const int64_t u = xcd_remap(blockIdx.x, grid.ntl);
     if (u >= grid.ntl) return;                               // uniform over the work-group
     const GoTl tl = go_tl(grid, u);
@@ -1249,26 +1283,15 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
     const bool at_sfc = LW && (ilay == sfc_lay - 1);
 
     if (threadIdx.x == 0) stage_gases(g, k.ngas, sg);
-    for (int e = threadIdx.x; e < 4 * ga_rows(k.ngas) * GO_COLS; e += GO_THREADS) s_d[e] = Real(0);
-    if (LW && w < 3) s_lev[w][lane] = Real(0);
+    if (!ONE) clear_rows();
+    if (LW && w < 2) s_lev[w][lane] = Real(0);
+    if (LW && w == 2) s_acc[lane][GA_N] = Real(0);           // the band Planck values' part of the T gradient
     __syncthreads();
-    stage_pair_inputs<Real, LW>(sg, k.ngas, tl.col0, ilay, ncol, nlay, play, tlay, tlev, tsfc, col_dry_a, s_in);
+    stage_pair_inputs<Real, LW>(sg, nin, tl.col0, ilay, ncol, nlay, play, tlay, tlev, tsfc, col_dry_a, s_in);
     __syncthreads();
-    col_state<Real, LW>(k, PairInLds<Real>{s_in, lane, k.ngas}, w, lane, s_cs);
+    col_state<Real, LW>(k, PairInLds<Real>{s_in, lane, nin}, w, lane, s_cs);
     __syncthreads();
 
-    Real fm[2][4], cm[2], fn[2][2], x[4];                    // the lane's sums of the band's weight cotangents
-    auto clear = [&] {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-        {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) fm[i][c] = Real(0);
-            cm[i] = Real(0);
-            fn[i][0] = Real(0); fn[i][1] = Real(0); x[2 * i] = Real(0); x[2 * i + 1] = Real(0);
-        }
-    };
-    clear();
     int back = -1;                                           // band whose phase 3 is due
     int group = 0;                                           // its first g-point group
     const int nchunk = grid.nbnd * int(grid.cpb);
@@ -1284,27 +1307,39 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
         asm volatile("" : "+v"(ln));
         const int64_t icol = tl.col0 + ln, idx = icol + ncol * ilay;
         const bool valid = icol < ncol;
-        const PairInLds<Real> in{s_in, ln, k.ngas};
+        const auto in = [&] {
+            const PairInLds<Real> rows{s_in, ln, nin};
+            if constexpr (ONE) return PairInMem<Real>{rows, sg, min(icol, ncol - 1), ilay};
+            else return rows;
+        }();
         const int pi = w * 16 + ln / 4;                      // pair of phase 2
         const int gq = 4 * (ln % 4);                         // first g-point of the lane's quad in a chunk
+        const GaRows<Real> rows{s_d, ln}, sums{s_d + (k.ngas + 1 + ga_sum_row(w)) * GO_COLS, ln};
+        const bool finish = ONE ? cb == nchunk : back >= 0;
+        if (ONE && finish)
+        {
+            clear_rows();
+            __syncthreads();
+        }
 
-        if (back >= 0)                                       // phase 3 of the band just finished
+        if (finish)                                          // phase 3 of the band just finished
         {
             const GoBand& bd = k.bands[back];
-            const GaRows<Real> rows{s_d + w * ga_rows(k.ngas) * GO_COLS, ln, k.ngas};
             const Real pv = in.p(), tv = in.t(), cd = in.cd();
             const CL<Real> c{s_cs.ci[0][ln], s_cs.ci[1][ln], s_cs.ci[2][ln], s_cs.cf[0][ln], s_cs.cf[1][ln]};
-            const Real* acc = s_acc[ln];
-            if (w == 0) ga_major_back(k, bd, c, in, cd, acc, rows);
-            else if (w == 1) ga_minor_back(k, bd, c.itropo, in, pv, tv, cd, acc, 0, 2, rows);
-            else if (w == 3) ga_minor_back(k, bd, c.itropo, in, pv, tv, cd, acc, 1, 2, rows);
+            Real* const acc = s_acc[ln];
+            if (w == 0) ga_major_back(k, bd, c, in, cd, acc, acc + MAJOR, sums);
+            else if (w == 1 || w == 3) ga_minor_back(k, bd, c.itropo, in, pv, tv, cd, acc, w / 2, rows, sums);
             else if constexpr (LW)
             {
                 const Real* tab = k.totplnk + int64_t(back) * k.nplanck;
-                Real xl = acc[GA_X], xh = acc[GA_X + 1], xo = acc[GA_X + 2];
-                if constexpr (MODE == GA_LWF)
+                Real xl = Real(0), xh = Real(0), xo = Real(0);
+                if constexpr (MODE == GA_LW3)
                 {
-                    xl = Real(0); xh = Real(0); xo = Real(0);
+                    xl = acc[GA_X]; xh = acc[GA_X + 1]; xo = acc[GA_X + 2];
+                }
+                else
+                {
                     for (int q = 0; q < bd.ng; q += GO_GPTS)
                     {
                         const int64_t ob = idx + ncl * (group + q / GO_GPTS);
@@ -1312,7 +1347,7 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                         xl += ct.blay[ob]; xh += ct.bhi[ob]; xo += ct.blo[ob];
                     }
                 }
-                rows.t(xl * interp1d_slope(tab, s_cs.ci[3][ln], k.totplnk_delta));
+                s_acc[ln][GA_N] += xl * interp1d_slope(tab, s_cs.ci[3][ln], k.totplnk_delta);
                 s_lev[1][ln] += xh * interp1d_slope(tab, s_cs.ci[4][ln], k.totplnk_delta);
                 s_lev[0][ln] += xo * interp1d_slope(tab, s_cs.ci[5][ln], k.totplnk_delta);
                 if (at_sfc)
@@ -1320,21 +1355,31 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                     int is;
                     Real fs;
                     interp1d_pos(in.t_sfc(), k.temp_ref_min, k.totplnk_delta, k.nplanck, is, fs);
-                    s_lev[2][ln] += acc[GA_X + 3] * interp1d_slope(tab, is, k.totplnk_delta);
+                    if (valid) out.d_tsfc[icol] += acc[GA_X + 3] * interp1d_slope(tab, is, k.totplnk_delta);
                 }
             }
             else
             {
-                const Real xr = acc[GA_X], ray = in.col(k.idx_h2o, cd) + cd;
-                rows.col(k.idx_h2o, xr);                     // col_ray = col(h2o) + col_dry
-                rows.col(0, xr);
-                rows.dry(xr * ray);
+                const Real xr = acc[GA_X];
+                sums.add(GA_XH, xr);                         // col_ray = col(h2o) + col_dry
+                sums.add(GA_DRY, xr * (in.col(k.idx_h2o, cd) + cd));
             }
             group += (bd.ng + GO_GPTS - 1) / GO_GPTS;
             back = -1;
-            clear();                                         // here: the sums need no registers in phase 3
         }
-        if (cb == nchunk) break;
+        auto add_major = [&] {
+            if (!finish || w != 0) return;
+            const Real* m = s_acc[ln] + MAJOR;
+            const int gases = int(m[2]);
+            rows.add(gases % 64, m[0]);
+            rows.add(gases / 64, m[1]);
+        };
+        if (cb == nchunk)
+        {
+            __syncthreads();
+            add_major();
+            break;
+        }
 
         const GoBand& bd = k.bands[ibnd];
         const int gbase = bd.g0 - k.bands[grid.b0].g0 + c0;
@@ -1353,6 +1398,7 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                 }
         }
         __syncthreads();
+        add_major();
 
         // Phase 2.  Lanes past the chunk's g-points run on its first quad with zero cotangents, so the
         // lanes of a pair stay together.
@@ -1362,6 +1408,13 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
             const uint32_t gl = uint32_t(c0 + (on ? gq : 0));
             const uint32_t gp = bd.gp, sE = uint32_t(k.npres + 1) * gp, sP = gp;
             auto cot = [&](int a, int e) { return s_g[a][gq + e][go_swz(gq + e, pi)]; };
+            // The pair's sum of a weight's cotangent over the band's chunks.  Each goes to LDS as soon as it is
+            // complete, so that no more registers are held through phase 1 and the minor slots than need be.
+            auto put = [&](int q, Real lanes) {
+                const Real v = quad_sum(lanes);
+                if (ln % 4 == 0) s_acc[pi][q] = c0 == 0 ? v : s_acc[pi][q] + v;
+            };
+            Real fm[2][4] = {}, fn[2][2] = {};
             Real gabs[4], gray[4];
             if constexpr (MODE == GA_SW3)
             {
@@ -1407,15 +1460,15 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                 load4(k.kmajor_p, o, n0); load4(k.kmajor_p, o + sE, n1);
                 load4(k.kmajor_p, o + sP, n2); load4(k.kmajor_p, o + sP + sE, n3);
                 const Real d0 = dot4(gabs, n0), d1 = dot4(gabs, n1), d2 = dot4(gabs, n2), d3 = dot4(gabs, n3);
-                cm[i] += st.fmajor[i][0] * d0 + st.fmajor[i][1] * d1 + st.fmajor[i][2] * d2 + st.fmajor[i][3] * d3;
+                put(GA_CM + i, st.fmajor[i][0] * d0 + st.fmajor[i][1] * d1 + st.fmajor[i][2] * d2 + st.fmajor[i][3] * d3);
                 const Real mix = st.col_mix[i];
-                fm[i][0] += mix * d0; fm[i][1] += mix * d1; fm[i][2] += mix * d2; fm[i][3] += mix * d3;
+                fm[i][0] = mix * d0; fm[i][1] = mix * d1; fm[i][2] = mix * d2; fm[i][3] = mix * d3;
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (LW)
             {
                 // Planck fractions: their cotangent, and (GA_LW3) the band Planck values'.
-                Real gpf[4];
+                Real gpf[4], pf[4] = {};
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     gpf[e] = MODE == GA_LWF ? cot(1, e)
@@ -1423,10 +1476,11 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                 auto node = [&](int i, int c, Real (&n)[4]) {
                     load4(k.planck_frac_p, kb + uint32_t(st.om[i]) + (c & 1 ? sE : 0u) + (c & 2 ? sP : 0u), n);
                 };
+                Real x3 = Real(0);
                 if (at_sfc)
                 {
                     // The surface source of the lowest layer (one layer of the launch: rolled loops).
-                    Real gs[4], xs = Real(0);
+                    Real gs[4];
                     const int64_t sc = tl.col0 + pi;
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -1439,10 +1493,10 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                     {
                         Real n[4];
                         node(ic >> 2, ic & 3, n);
-                        xs += st.fmajor[ic >> 2][ic & 3] * dot4(gs, n);
+                        x3 += st.fmajor[ic >> 2][ic & 3] * dot4(gs, n);
                     }
-                    x[3] += xs;
                 }
+                put(GA_X + 3, x3);
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
                 {
@@ -1455,20 +1509,26 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                         if constexpr (MODE == GA_LW3)
                         {
 #pragma unroll
-                            for (int q = 0; q < 3; ++q)
-                            {
-                                const Real gb[4] = {cot(q + 1, 0), cot(q + 1, 1), cot(q + 1, 2), cot(q + 1, 3)};
-                                x[q] += st.fmajor[i][c] * dot4(gb, n);
-                            }
+                            for (int e = 0; e < 4; ++e) pf[e] += st.fmajor[i][c] * n[e];
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
+                }
+                if constexpr (MODE == GA_LW3)
+                {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                    {
+                        const Real gb[4] = {cot(q + 1, 0), cot(q + 1, 1), cot(q + 1, 2), cot(q + 1, 3)};
+                        put(GA_X + q, dot4(gb, pf));
+                    }
                 }
             }
             else
             {
                 const uint32_t rb = uint32_t(bd.roff) + gl;
                 const Real ray = st.aux[0];
+                Real x0 = Real(0);
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1477,12 +1537,17 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                         Real n[4];
                         load4(k.krayl_p, rb + uint32_t(st.ry[i]) + (c ? gp : 0u), n);
                         const Real d = dot4(gray, n);
-                        x[0] += st.fminor[i][c] * d;
-                        fn[i][c] += ray * d;
+                        x0 += st.fminor[i][c] * d;
+                        fn[i][c] = ray * d;
                     }
+                put(GA_X, x0);
             }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) put(GA_FM + 4 * i + c, fm[i][c]);
             __builtin_amdgcn_sched_barrier(0);
-            // Minor absorption, one slot at a time; the first lane of the pair keeps the slot's sum.
+            // Minor absorption, one slot at a time.
             const int nslot = bd.nslot;
             const uint32_t sQ = uint32_t(nslot) * gp;
             const uint32_t mb = uint32_t(bd.moff) + gl;
@@ -1497,63 +1562,40 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
                 const Real d0 = dot4(gabs, n0), d1 = dot4(gabs, n1), d2 = dot4(gabs, n2), d3 = dot4(gabs, n3);
                 const Real sc = st.scaling[q];
                 fn[0][0] += sc * d0; fn[0][1] += sc * d1; fn[1][0] += sc * d2; fn[1][1] += sc * d3;
-                const Real tq = quad_sum(st.fminor[0][0] * d0 + st.fminor[0][1] * d1 + st.fminor[1][0] * d2 +
-                                         st.fminor[1][1] * d3);
-                if (ln % 4 == 0) s_acc[pi][GA_SC + q] = c0 == 0 ? tq : s_acc[pi][GA_SC + q] + tq;
+                put(GA_SC + q, st.fminor[0][0] * d0 + st.fminor[0][1] * d1 + st.fminor[1][0] * d2 + st.fminor[1][1] * d3);
             }
-            if (c0 + GO_GPTS >= bd.ng)
-            {
-                // The band's last chunk: the pair's totals.
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-                {
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                    {
-                        const Real f = quad_sum(fm[i][c]);
-                        if (ln % 4 == 0) s_acc[pi][GA_FM + 4 * i + c] = f;
-                    }
-                    const Real m = quad_sum(cm[i]);
-                    const Real f0 = quad_sum(fn[i][0]), f1 = quad_sum(fn[i][1]);
-                    if (ln % 4 == 0)
-                    {
-                        s_acc[pi][GA_CM + i] = m;
-                        s_acc[pi][GA_FN + 2 * i] = f0;
-                        s_acc[pi][GA_FN + 2 * i + 1] = f1;
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                {
-                    if (!LW && q > 0) break;
-                    const Real v = quad_sum(x[q]);
-                    if (ln % 4 == 0) s_acc[pi][GA_X + q] = v;
-                }
-                back = ibnd;
-            }
+                for (int c = 0; c < 2; ++c) put(GA_FN + 2 * i + c, fn[i][c]);
+            if (c0 + GO_GPTS >= bd.ng) back = ibnd;          // the band's last chunk
         }
         __syncthreads();
     }
     __syncthreads();
 
-    // The wavefronts' rows summed and added to memory.
+    // The rows and sums added to memory.
     const int64_t icol = tl.col0 + lane, idx = icol + ncol * ilay;
-    const Real cd = s_in[2 * GO_COLS + lane];
-    const int nr = ga_rows(k.ngas);
-    auto total = [&](int r) {
-        Real v = Real(0);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) v += s_d[(p * nr + r) * GO_COLS + lane];
-        return v;
-    };
     if (icol >= ncol) return;
-    for (int r = w; r < k.ngas + 2; r += 4)
+    auto sum = [&](int wave, int q) { return s_d[(k.ngas + 1 + ga_sum_row(wave) + q) * GO_COLS + lane]; };
+    for (int r = w; r <= k.ngas; r += 4)
     {
-        const Real v = total(r);
-        out.d_col[idx + ncl * r] += r == k.ngas + 1 ? v / cd : v;
+        Real v = s_d[r * GO_COLS + lane];
+        if (r == 0 || r == k.idx_h2o) v += LW ? sum(1, GA_XH) + sum(3, GA_XH) : (sum(1, GA_XH) + sum(2, GA_XH)) + sum(3, GA_XH);
+        if (__any(v != Real(0))) out.d_col[idx + ncl * r] += v;      // rows of gases that no band of the launch reads
     }
-    if (w == 0) out.d_tlay[idx] += total(k.ngas + 2);
-    else if (w == 1) out.d_lnp[idx] += total(k.ngas + 3);
+    const Real minor_lnp = sum(1, GA_LNP) + sum(3, GA_LNP);
+    if (w == 3)
+    {
+        const Real v = (sum(0, GA_DRY) + sum(1, GA_DRY)) + sum(3, GA_DRY);
+        out.d_col[idx + ncl * (k.ngas + 1)] += (LW ? v : v + sum(2, GA_DRY)) / s_in[2 * GO_COLS + lane];
+    }
+    else if (w == 0)
+    {
+        const Real v = sum(0, GA_T) - minor_lnp / s_in[GO_COLS + lane];
+        out.d_tlay[idx] += LW ? v + s_acc[lane][GA_N] : v;
+    }
+    else if (w == 1) out.d_lnp[idx] += sum(0, GA_LNP) + minor_lnp;
     if constexpr (LW)
     {
         if (w == 2)
@@ -1561,7 +1603,6 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
             out.d_tlev_lo[idx] += s_lev[0][lane];
             out.d_tlev_hi[idx] += s_lev[1][lane];
         }
-        else if (w == 3 && at_sfc) out.d_tsfc[icol] += s_lev[2][lane];
     }
 }
 
@@ -2084,7 +2125,9 @@ int gas_optics_adjoint(const rrtmgp_kdist_dev* kd, int64_t b0, int64_t nb, int64
     const Kd<Real> k = make_kd<Real>(*kd);
     const GoGrid grid = make_go_grid(ncol, nlay, b0, nb, kd->max_band_gpts);
     if (grid.ntl >= (int64_t(1) << 31)) return arg_error("gas_optics_adjoint: too many column tiles x layers");
-    const size_t dyn = size_t(go_in_rows<LW>(kd->ngas) + 4 * ga_rows(kd->ngas)) * GO_COLS * sizeof(Real);
+    constexpr bool ONE = MODE == GA_LW3 || MODE == GA_SW3;       // gradient rows in the cotangents' place
+    const size_t dyn = size_t(ONE ? go_in_rows<LW>(0) : go_in_rows<LW>(kd->ngas) + ga_rows<LW>(kd->ngas)) *
+                       GO_COLS * sizeof(Real);
     RRTMGP_TIMED("gas_optics_adjoint_kernel", as_stream(stream));
     hipLaunchKernelGGL((gas_optics_adjoint_kernel<Real, MODE>), dim3(xcd_grid(grid.ntl)), dim3(GO_THREADS), dyn,
                        as_stream(stream), k, g, ncol, nlay, grid, play, tlay, tlev, tsfc, col_dry, sfc_lay, ct, out);
