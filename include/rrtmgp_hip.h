@@ -628,6 +628,8 @@ RRTMGP_DECLARE_BOTH(RRTMGP_DECL_GO_ADJOINT)
 /* group of up to 16 consecutive g-points of a band: (ncol, nlay, groups).                       */
 /* sw_adjoint_gases: rrtmgp_hip_sw_solver_2stream_adjoint_* with the cotangents of tau, ssa and   */
 /* g carried on to the gases' absorption and Rayleigh optical depths (any band cloud held fixed). */
+/* Both may write over the optical properties they read: d_tau and d_planck_frac may be tau and    */
+/* planck_frac, d_tau_abs and d_tau_ray tau and ssa.                                              */
 /* gas_optics_{lw,sw}_adjoint_bands: rrtmgp_hip_gas_optics_{lw,sw}_adjoint_* for the range, from   */
 /* those cotangents.                                                                             */
 #define RRTMGP_DECL_ADJ_BANDS(S, T)                                                            \

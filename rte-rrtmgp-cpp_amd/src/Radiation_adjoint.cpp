@@ -39,19 +39,22 @@ Array_gpu<Float,2> expand(const Gas_optics_rrtmgp_gpu& kd, const Array_gpu<Float
 }
 
 // Bands processed together: consecutive bands whose per-g-point scratch (`arrays` values per column, layer
-// and g-point) stays below 2.25 GiB, at least one.  One launch per kernel then covers them: at a few
-// thousand columns and fewer a single band's work-groups leave most of the GPU idle (250 x 60 columns and
-// layers: 4 tiles x 16 g-points), at 16384 x 128 in FP32 two shortwave and four longwave bands share the
-// staging of the gas-optics inputs, with the peak scratch of one band's former 12-state store.
+// and g-point) stays below `bytes`, at least one.  One launch per kernel then covers them: at a few thousand
+// columns and fewer a single band's work-groups leave most of the GPU idle (250 x 60 columns and layers: 4 tiles
+// x 16 g-points), at 16384 x 128 in FP32 two shortwave and four longwave bands share the staging of the
+// gas-optics inputs.  Cotangents are written over the optical properties they belong to, so that both drivers
+// together take 2.6 GB of scratch there (one band at a time with 12 stored shortwave states took 3.1 GB).
+constexpr double GiB = 1024. * 1024. * 1024.;
+
 struct Batch
 {
     int b0, nb, g0, ng;              // bands, first g-point (0-based), g-points
     std::vector<int> lims;           // (2, nb) band limits, 1-based within the batch
 };
 
-std::vector<Batch> make_batches(const Gas_optics_rrtmgp_gpu& kd, int64_t ncl, double arrays)
+std::vector<Batch> make_batches(const Gas_optics_rrtmgp_gpu& kd, int64_t ncl, double arrays, double bytes)
 {
-    const double most = 2.25 * 1024. * 1024. * 1024. / (arrays * double(sizeof(Float)) * double(ncl));
+    const double most = bytes / (arrays * double(sizeof(Float)) * double(ncl));
     const Array<int,2>& bl = kd.get_band_lims_gpoint();
     std::vector<Batch> out;
     for (int b = 0; b < kd.get_nband(); ++b)
@@ -66,6 +69,21 @@ std::vector<Batch> make_batches(const Gas_optics_rrtmgp_gpu& kd, int64_t ncl, do
     }
     return out;
 }
+
+// A block of the library's caching allocator on the driver's stream.
+struct Scratch
+{
+    Float* ptr = nullptr;
+    explicit Scratch(int64_t n)
+    {
+        void* p = nullptr;
+        hip_check(rrtmgp_hip_cache_malloc(&p, size_t(n) * sizeof(Float), stream()));
+        ptr = static_cast<Float*>(p);
+    }
+    ~Scratch() { (void)rrtmgp_hip_cache_free(ptr, stream()); }
+    Scratch(const Scratch&) = delete;
+    Scratch& operator=(const Scratch&) = delete;
+};
 
 template<typename F>
 int most_of(const std::vector<Batch>& v, F f)
@@ -144,8 +162,9 @@ void lw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
     Array_gpu<Float,2> d_lo({ncol, nlay}), d_hi({ncol, nlay}), d_col_dry({ncol, nlay}), d_emis_gpt({ncol, ngpt});
     zero(d_col); zero(d_lo); zero(d_hi); zero(out.d_t_lay); zero(out.d_t_sfc); zero(out.d_lnp_lay); zero(out.d_p_lev);
 
-    // Factored sources, as the forward driver: per g-point only tau, the Planck fractions and their cotangents.
-    const std::vector<Batch> batches = make_batches(kdist, ncl, 4.5);
+    // Factored sources, as the forward driver: per g-point only tau and the Planck fractions, with their cotangents
+    // in the same place, and the solver's checkpoints (two values in four layers).
+    const std::vector<Batch> batches = make_batches(kdist, ncl, 2.5, 1.25 * GiB);
     const int mg = most_of(batches, [](const Batch& t) { return t.ng; });
     const int mb = most_of(batches, [](const Batch& t) { return t.nb; });
     const int mq = most_of(batches, [](const Batch& t) {
@@ -153,26 +172,31 @@ void lw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
         for (int i = 0; i < t.nb; ++i) n += (t.lims[2 * i + 1] - t.lims[2 * i] + 16) / 16;   // groups of 16 g-points
         return n;
     });
-    Array_gpu<Float,3> tau({ncol, nlay, mg}), pf({ncol, nlay, mg}), dtau({ncol, nlay, mg}), dpf({ncol, nlay, mg});
-    Array_gpu<Float,3> blay({ncol, nlay, mb}), blev({ncol, nlev, mb});
-    Array_gpu<Float,3> dblay({ncol, nlay, mq}), dblo({ncol, nlay, mq}), dbhi({ncol, nlay, mq});
-    Array_gpu<Float,2> sfc({ncol, mg}), sfcj({ncol, mg}), dsfc({ncol, mg});
+    // One block for all, so that the shortwave driver finds it large enough for its level states.
+    const int64_t sizes[] = {ncl * mg, ncl * mg, ncl * mb, int64_t(ncol) * nlev * mb, ncl * mq, ncl * mq, ncl * mq,
+                             int64_t(ncol) * mg, int64_t(ncol) * mg, int64_t(ncol) * mg};
+    int64_t total = 0;
+    for (const int64_t n : sizes) total += (n + 63) / 64 * 64;
+    Scratch block(total);
+    Float* part[10];
+    Float* next = block.ptr;
+    for (int i = 0; i < 10; ++i) { part[i] = next; next += (sizes[i] + 63) / 64 * 64; }
+    const auto [tau, pf, blay, blev, dblay, dblo, dbhi, sfc, sfcj, dsfc] = part;
     const Float* ctau = cl ? cl->get_tau().ptr() : nullptr;
     for (const Batch& t : batches)
     {
         hip_check(K<Float>::gas_optics_lw_bands_factored(
                 &kd, t.b0, t.nb, ncol, nlay, p_lay.ptr(), t_lay.ptr(), t_lev.ptr(), t_sfc.ptr(), col_dry.ptr(), &vmr,
-                sfc_lay, ctau, tau.ptr(), pf.ptr(), blay.ptr(), blev.ptr(), sfc.ptr(), sfcj.ptr(), stream()));
+                sfc_lay, ctau, tau, pf, blay, blev, sfc, sfcj, stream()));
         // One Gaussian angle, as the forward driver (src_test/Radiation_solver.cpp:533): D = 1.66, w = 0.5.
         hip_check(K<Float>::lw_adjoint_factored(
-                ncol, nlay, t.ng, top_at_1, 1.66, 0.5, tau.ptr(), pf.ptr(), blay.ptr(), blev.ptr(), t.nb,
-                t.lims.data(), emis_sfc.ptr() + t.b0, nbnd, sfc.ptr(), g_flux_up.ptr(), g_flux_dn.ptr(), dtau.ptr(),
-                dpf.ptr(), dblay.ptr(), dblo.ptr(), dbhi.ptr(), dsfc.ptr(),
+                ncol, nlay, t.ng, top_at_1, 1.66, 0.5, tau, pf, blay, blev, t.nb, t.lims.data(),
+                emis_sfc.ptr() + t.b0, nbnd, sfc, g_flux_up.ptr(), g_flux_dn.ptr(), tau, pf, dblay, dblo, dbhi, dsfc,
                 d_emis_gpt.ptr() + int64_t(ncol) * t.g0, stream()));
         hip_check(K<Float>::gas_optics_lw_adjoint_bands(
                 &kd, t.b0, t.nb, ncol, nlay, p_lay.ptr(), t_lay.ptr(), t_lev.ptr(), t_sfc.ptr(), col_dry.ptr(), &vmr,
-                sfc_lay, dtau.ptr(), dpf.ptr(), dblay.ptr(), dblo.ptr(), dbhi.ptr(), dsfc.ptr(), d_col.ptr(),
-                out.d_t_lay.ptr(), out.d_lnp_lay.ptr(), d_lo.ptr(), d_hi.ptr(), out.d_t_sfc.ptr(), stream()));
+                sfc_lay, tau, pf, dblay, dblo, dbhi, dsfc, d_col.ptr(), out.d_t_lay.ptr(), out.d_lnp_lay.ptr(),
+                d_lo.ptr(), d_hi.ptr(), out.d_t_sfc.ptr(), stream()));
     }
     hip_check(K<Float>::adjoint_levels(ncol, nlay, d_lo.ptr(), d_hi.ptr(), out.d_t_lev.ptr(), stream()));
     hip_check(K<Float>::adjoint_col_chain(ncol, nlay, &vmr, col_dry.ptr(), d_col.ptr(), out.d_vmr.ptr(),
@@ -231,10 +255,10 @@ void sw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
     Array_gpu<Float,2> d_col_dry({ncol, nlay}), d_ad({ncol, ngpt}), d_af({ncol, ngpt});
     zero(d_col); zero(out.d_t_lay); zero(out.d_lnp_lay); zero(out.d_p_lev);
 
-    const std::vector<Batch> batches = make_batches(kdist, ncl, 9.);     // 5 arrays and the solver's 4 level states
+    // Three arrays, two of which receive the cotangents, and the solver's four level states.
+    const std::vector<Batch> batches = make_batches(kdist, ncl, 7., 1.75 * GiB);
     const int mg = most_of(batches, [](const Batch& t) { return t.ng; });
     Array_gpu<Float,3> tau({ncol, nlay, mg}), ssa({ncol, nlay, mg}), g({ncol, nlay, mg});
-    Array_gpu<Float,3> dabs({ncol, nlay, mg}), dray({ncol, nlay, mg});
     const Float* ct = cl ? cl->get_tau().ptr() : nullptr;
     const Float* cs = cl ? cl->get_ssa().ptr() : nullptr;
     const Float* cg = cl ? cl->get_g().ptr() : nullptr;
@@ -246,9 +270,9 @@ void sw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
         hip_check(K<Float>::sw_adjoint_gases(
                 ncol, nlay, t.ng, top_at_1, tau.ptr(), ssa.ptr(), g.ptr(), mu0.ptr(), ad_gpt.ptr() + o,
                 af_gpt.ptr() + o, toa.ptr() + o, nullptr, g_flux_up.ptr(), g_flux_dn.ptr(), g_flux_dir.ptr(),
-                dabs.ptr(), dray.ptr(), d_ad.ptr() + o, d_af.ptr() + o, stream()));
+                tau.ptr(), ssa.ptr(), d_ad.ptr() + o, d_af.ptr() + o, stream()));
         hip_check(K<Float>::gas_optics_sw_adjoint_bands(&kd, t.b0, t.nb, ncol, nlay, p_lay.ptr(), t_lay.ptr(),
-                                                        col_dry.ptr(), &vmr, dabs.ptr(), dray.ptr(), d_col.ptr(),
+                                                        col_dry.ptr(), &vmr, tau.ptr(), ssa.ptr(), d_col.ptr(),
                                                         out.d_t_lay.ptr(), out.d_lnp_lay.ptr(), stream()));
     }
     hip_check(K<Float>::adjoint_col_chain(ncol, nlay, &vmr, col_dry.ptr(), d_col.ptr(), out.d_vmr.ptr(),
