@@ -179,6 +179,32 @@ __global__ void absorbed_heating_rate_kernel(int64_t ncol, int64_t nlay, int ngr
 }
 
 // ---------------------------------------------------------------------------------------------
+// A layer at one angle: its transmittance, the emission that leaves it at the far side, and for the heating rate
+// 1 - T and the part of the emission beyond (1 - T) B of the far level.
+template<typename Real>
+struct LayerLW { Real T, S, omT, B; };
+
+template<bool HR, typename Real>
+__device__ __forceinline__ LayerLW<Real> lw_emission(Real tau, Real D, Real lay, Real lev)
+{
+#pragma clang fp contract(off)
+    LayerLW<Real> L;
+    Real fact;
+    const Real t = tau * D;
+    lw_layer(t, L.T, fact);
+    L.B = Real(2) * fact * (lay - lev);
+    L.S = fma_of(Real(1) - L.T, lev, L.B);
+    L.omT = HR ? one_minus_T(t, L.T) : Real(0);
+    return L;
+}
+
+// The flux that the layer absorbs of an intensity I, less what it emits: added to ab with its sign.
+template<typename Real>
+__device__ __forceinline__ Real lw_absorbed(const LayerLW<Real>& L, Real lev, Real I, Real fac, Real ab)
+{
+    return fma_of(-fac, fma_of(L.omT, add_alone(lev, -I), L.B), ab);
+}
+
 // Longwave: no scattering, linear-in-tau source, nmus <= NMU Gaussian angles.  The layer inputs
 // of the next K-level segment are read while the current segment is computed.
 template<int GP, typename Real, bool JAC, int NMU, bool FACT, bool HR = false>
@@ -305,22 +331,11 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
             if (s0 + K <= nlay) fetch(s0 + K, lev_g, lsh, layer_of, up);
             // Small work-groups have one or two wavefronts per SIMD: the levels' transmittances and sources,
             // which do not depend on each other, are evaluated side by side before the recurrence.
-            Real pT[AHEAD ? K : 1], pS[AHEAD ? K : 1], pA[AHEAD && HR ? K : 1], pB[AHEAD && HR ? K : 1];
+            LayerLW<Real> ahead[AHEAD ? K : 1];
             if constexpr (AHEAD)
             {
 #pragma unroll
-                for (int kk = 0; kk < K; ++kk)
-                {
-                    Real fact;
-                    const Real t = ct[kk] * D[0];
-                    lw_layer(t, pT[kk], fact);
-                    pS[kk] = (Real(1) - pT[kk]) * cx[kk] + Real(2) * fact * (cl[kk] - cx[kk]);
-                    if constexpr (HR)
-                    {
-                        pA[kk] = one_minus_T(t, pT[kk]);
-                        pB[kk] = Real(2) * fact * (cl[kk] - cx[kk]);
-                    }
-                }
+                for (int kk = 0; kk < K; ++kk) ahead[kk] = lw_emission<HR>(ct[kk], D[0], cl[kk], cx[kk]);
             }
 #pragma unroll
             for (int kk = 0; kk < K; ++kk)
@@ -329,37 +344,25 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
                 Real f = Real(0), fj = Real(0), ab = Real(0);
                 if (active && j <= nlay)
                 {
-                    if constexpr (AHEAD)
-                    {
-                        if (j > 0)
-                        {
-                            if constexpr (HR) ab -= fac[0] * (pA[kk] * (cx[kk] - I[0]) + pB[kk]);
-                            I[0] = pT[kk] * I[0] + pS[kk];
-                            if (JAC && up) Ij[0] = pT[kk] * Ij[0];
-                        }
-                    }
-                    else if (j > 0)
+                    if (j > 0)
                     {
 #pragma unroll
                         for (int mu = 0; mu < NMU; ++mu)
                             if (mu < nmus)
                             {
-                                Real T, fact;
-                                const Real t = ct[kk] * D[mu];
-                                lw_layer(t, T, fact);
-                                if constexpr (HR)
-                                    ab -= fac[mu] * (one_minus_T(t, T) * (cx[kk] - I[mu]) +
-                                                     Real(2) * fact * (cl[kk] - cx[kk]));
-                                I[mu] = T * I[mu] + ((Real(1) - T) * cx[kk] + Real(2) * fact * (cl[kk] - cx[kk]));
-                                if (JAC && up) Ij[mu] = T * Ij[mu];
+                                const LayerLW<Real> L = AHEAD ? ahead[AHEAD ? kk : 0]
+                                                              : lw_emission<HR>(ct[kk], D[mu], cl[kk], cx[kk]);
+                                if constexpr (HR) ab = lw_absorbed(L, cx[kk], I[mu], fac[mu], ab);
+                                I[mu] = fma_of(L.T, I[mu], L.S);
+                                if (JAC && up) Ij[mu] = L.T * Ij[mu];
                             }
                     }
 #pragma unroll
                     for (int mu = 0; mu < NMU; ++mu)
                         if (mu < nmus)
                         {
-                            f = (mu == 0) ? fac[0] * I[0] : f + fac[mu] * I[mu];
-                            if (JAC && up) fj = (mu == 0) ? fac[0] * Ij[0] : fj + fac[mu] * Ij[mu];
+                            f = (mu == 0) ? fac[0] * I[0] : fma_of(fac[mu], I[mu], f);
+                            if (JAC && up) fj = (mu == 0) ? fac[0] * Ij[0] : fma_of(fac[mu], Ij[mu], fj);
                         }
                     if (flux_g) at32(flux_g, ucol + uncol * uint32_t(lev_out(j))) = f;
                     if constexpr (HR && !SUMS)
@@ -421,7 +424,7 @@ void lw_solver_kernel(int64_t ncol, int64_t nlay, int64_t ngpt, int top_at_1, in
 #pragma unroll
         for (int mu = 0; mu < NMU; ++mu)
         {
-            I[mu] = I[mu] * (Real(1) - e) + e * ss;
+            I[mu] = fma_of(I[mu], Real(1) - e, e * ss);
             Ij[mu] = e * sj;
         }
     }
@@ -537,18 +540,6 @@ __device__ __forceinline__ LayerSW<St> sw_layer(Real tau, Real w_in, Real g, Rea
 // Reciprocal of an adding denominator 1 - R A in (0, 1].
 __device__ __forceinline__ double rcp_den(double x) { return rcp_f64(x); }
 __device__ __forceinline__ float rcp_den(float x) { return rcp_f32(x); }
-
-// a + b as its own rounding, and a b + c in one.  Whether the compiler contracts an addition with the product
-// before it depends on the code around it, and the same columns have to give the same bits in every variant of
-// the kernel: the adding recurrences are written with these.
-__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
-template<typename St>
-__device__ __forceinline__ St add_alone(St a, St b)
-{
-#pragma clang fp contract(off)
-    return a + b;
-}
 
 // Column above the next level from the column above this one and the layer between.
 template<typename St>

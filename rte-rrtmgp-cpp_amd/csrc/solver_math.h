@@ -7,6 +7,18 @@
 
 namespace rrtmgp_hip
 {
+// a b + c in one rounding, and a + b as its own.  Whether the compiler contracts an addition with the product
+// before it depends on the code around it, and the same columns have to give the same bits in every variant of
+// a solver kernel: what the variants share is written with these.
+__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template<typename St>
+__device__ __forceinline__ St add_alone(St a, St b)
+{
+#pragma clang fp contract(off)
+    return a + b;
+}
+
 __device__ __forceinline__ float rcp_f32(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // e^{-y} for y >= 0 through 2^x.
@@ -15,12 +27,13 @@ __device__ __forceinline__ float exp_neg_f32(float y) { return __builtin_amdgcn_
 // 1 - e^{-y} for 0 <= y < 0.25 from its series (truncation < y^8/8! relative).
 __device__ __forceinline__ float one_minus_exp_neg_series_f32(float y)
 {
-    float t = 1.f / 720.f - y * (1.f / 5040.f);
-    t = 1.f / 120.f - y * t;
-    t = 1.f / 24.f - y * t;
-    t = 1.f / 6.f - y * t;
-    t = .5f - y * t;
-    t = 1.f - y * t;
+#pragma clang fp contract(off)
+    float t = fma_of(-y, 1.f / 5040.f, 1.f / 720.f);
+    t = fma_of(-y, t, 1.f / 120.f);
+    t = fma_of(-y, t, 1.f / 24.f);
+    t = fma_of(-y, t, 1.f / 6.f);
+    t = fma_of(-y, t, .5f);
+    t = fma_of(-y, t, 1.f);
     return y * t;
 }
 
@@ -59,20 +72,22 @@ __device__ __forceinline__ Real ld_nt(const Real* base, uint32_t i)
 // which avoids the cancellation of (1 - T)/t - T, and uses the hardware exp2 and reciprocal.
 __device__ __forceinline__ void lw_layer(double t, double& T, double& fact)
 {
+#pragma clang fp contract(off)
     T = exp(-t);
-    fact = (t > sqrt(Limits<double>::eps)) ? (1. - T) / t - T : t * (.5 - (1. / 3.) * t);
+    fact = (t > sqrt(Limits<double>::eps)) ? (1. - T) / t - T : t * fma_of(-(1. / 3.), t, .5);
 }
 
 __device__ __forceinline__ void lw_layer(float t, float& T, float& fact)
 {
+#pragma clang fp contract(off)
     T = exp_neg_f32(t);
-    float q = 1.f / 840.f - t * (1.f / 5760.f);
-    q = 1.f / 144.f - t * q;
-    q = 1.f / 30.f - t * q;
-    q = 1.f / 8.f - t * q;
-    q = 1.f / 3.f - t * q;
-    q = .5f - t * q;
-    fact = (t < .25f) ? t * q : (1.f - T) * rcp_f32(t) - T;
+    float q = fma_of(-t, 1.f / 5760.f, 1.f / 840.f);
+    q = fma_of(-t, q, 1.f / 144.f);
+    q = fma_of(-t, q, 1.f / 30.f);
+    q = fma_of(-t, q, 1.f / 8.f);
+    q = fma_of(-t, q, 1.f / 3.f);
+    q = fma_of(-t, q, .5f);
+    fact = (t < .25f) ? t * q : fma_of(1.f - T, rcp_f32(t), -T);
 }
 
 // 1 - e^{-t} given T = e^{-t}, without the cancellation of 1 - T for small t.
