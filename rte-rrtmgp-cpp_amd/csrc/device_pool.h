@@ -32,9 +32,11 @@ struct PoolBlock
 class PoolPolicy
 {
     public:
-        // Allocation granularity: 512 B below 1 MiB, 2 MiB above (large mappings are cheaper whole).
+        // Allocation granularity: 512 B below 1 MiB, 2 MiB above (large mappings are cheaper whole).  Sizes that
+        // no device holds, and whose rounding (or an eighth more) could wrap around, stay as they are.
         static size_t round_block(size_t bytes)
         {
+            if (bytes > SIZE_MAX / 4) return bytes;
             const size_t q = bytes > (size_t(1) << 20) ? (size_t(2) << 20) : size_t(512);
             return (bytes + q - 1) / q * q;
         }
@@ -43,6 +45,7 @@ class PoolPolicy
         // smallest at all, with wait = true.  The block becomes live.
         bool take(int device, size_t bytes, PoolBlock& out, bool& wait)
         {
+            if (bytes > SIZE_MAX / 4) return false;
             const size_t most = bytes + (bytes >> 3);
             size_t best = free_.size();
             bool best_waits = true;

@@ -23,6 +23,15 @@ int main()
     CHECK(PoolPolicy::round_block(MiB) == MiB);
     CHECK(PoolPolicy::round_block(MiB + 1) == 2 * MiB);
 
+    // Sizes near the end of the range do not wrap around to small ones.
+    for (size_t less = 0; less < 4 * MiB; less += MiB / 2 + 1) CHECK(PoolPolicy::round_block(SIZE_MAX - less) >= SIZE_MAX - less);
+    {
+        PoolPolicy p;
+        p.add_live(mem[0], 512, 0);
+        CHECK(p.give(mem[0], MiB, out));
+        CHECK(!p.take(0, PoolPolicy::round_block(SIZE_MAX), b, wait) && !p.take(0, SIZE_MAX - 100, b, wait));
+    }
+
     // One wait covers every block freed before it began, none freed after.
     {
         PoolPolicy p;
