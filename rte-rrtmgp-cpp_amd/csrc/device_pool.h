@@ -29,6 +29,26 @@ struct PoolBlock
     uint64_t freed = 0;              // generation of the free
 };
 
+// Calls free_block for every block with its device current, by way of set_device, and leaves `current` so again.
+// An error (a value other than 0) of either ends nothing; the first one is returned.
+template<typename SetDevice, typename FreeBlock>
+int for_each_on_device(const std::vector<PoolBlock>& blocks, int current, SetDevice set_device, FreeBlock free_block)
+{
+    int first = 0, device = current;
+    const auto note = [&](int rc) { if (first == 0) first = rc; return rc == 0; };
+    for (const PoolBlock& b : blocks)
+    {
+        if (b.device != device)
+        {
+            if (!note(set_device(b.device))) continue;
+            device = b.device;
+        }
+        note(free_block(b));
+    }
+    if (device != current) note(set_device(current));
+    return first;
+}
+
 class PoolPolicy
 {
     public:

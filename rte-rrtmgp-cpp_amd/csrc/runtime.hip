@@ -248,19 +248,16 @@ size_t pool_bound(int dev)
     return b;
 }
 
-// Gives blocks back to the driver (hipFree waits for the device).
+// Gives blocks back to the driver (hipFree waits for the device).  Every block is tried, the current device
+// restored, and the first error returned.
 int pool_give_back(const std::vector<PoolBlock>& blocks)
 {
     if (blocks.empty()) return RRTMGP_OK;
     int cur = 0;
     RRTMGP_HIP(hipGetDevice(&cur));
-    for (const auto& b : blocks)
-    {
-        if (b.device != cur) RRTMGP_HIP(hipSetDevice(b.device));
-        RRTMGP_HIP(hipFree(b.ptr));
-        if (b.device != cur) RRTMGP_HIP(hipSetDevice(cur));
-    }
-    return RRTMGP_OK;
+    return for_each_on_device(blocks, cur,
+                              [](int device) { return check_hip(hipSetDevice(device), "hipSetDevice"); },
+                              [](const PoolBlock& b) { return check_hip(hipFree(b.ptr), "hipFree"); });
 }
 
 int pool_release()

@@ -99,6 +99,27 @@ int main()
         CHECK(!p.take(0, 4096, b, wait));
     }
 
+    // Blocks are given back whatever the others' frees return, and the device in use is restored.
+    {
+        std::vector<PoolBlock> v(5);
+        const int on[5] = {0, 2, 1, 1, 0};
+        for (int i = 0; i < 5; ++i) { v[i].ptr = mem[i]; v[i].device = on[i]; }
+        int device = 0;
+        std::vector<void*> freed;
+        const auto set = [&](int d) { if (d == 2) return 7; device = d; return 0; };
+        const auto drop = [&](const PoolBlock& k) {
+            if (k.device != device) return 9;
+            freed.push_back(k.ptr);
+            return k.ptr == mem[2] ? 8 : 0;
+        };
+        CHECK(rrtmgp_hip::for_each_on_device(v, 0, set, drop) == 7);
+        CHECK(freed.size() == 4 && freed[0] == mem[0] && freed[1] == mem[2] && freed[2] == mem[3] && freed[3] == mem[4]);
+        CHECK(device == 0);
+        v.pop_back();
+        v.erase(v.begin() + 1);
+        CHECK(rrtmgp_hip::for_each_on_device(v, 0, set, drop) == 8 && device == 0 && freed.size() == 7);
+    }
+
     std::printf("ok\n");
     return 0;
 }
