@@ -16,6 +16,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <deque>
+#include <map>
 #include <unordered_map>
 #include <vector>
 
@@ -66,26 +67,22 @@ class PoolPolicy
         bool take(int device, size_t bytes, PoolBlock& out, bool& wait)
         {
             if (bytes > SIZE_MAX / 4) return false;
-            const size_t most = bytes + (bytes >> 3);
-            size_t best = free_.size();
-            bool best_waits = true;
-            for (size_t i = 0; i < free_.size(); ++i)
-            {
-                const PoolBlock& b = free_[i];
-                if (b.device != device || b.bytes < bytes || b.bytes > most) continue;
-                const bool w = b.freed >= safe_[device];
-                if (best == free_.size() || (best_waits && !w) || (best_waits == w && b.bytes < free_[best].bytes))
-                {
-                    best = i;
-                    best_waits = w;
-                }
-            }
-            if (best == free_.size()) return false;
-            out = free_[best];
-            wait = best_waits;
-            free_.erase(free_.begin() + std::ptrdiff_t(best));
-            held_[device] -= out.bytes;
+            const auto at = devices_.find(device);
+            if (at == devices_.end()) return false;
+            Device& d = at->second;
+            // A size's oldest block is the one that a wait has most likely covered.
+            auto best = d.by_size.lower_bound(bytes);
+            const auto end = d.by_size.upper_bound(bytes + (bytes >> 3));
+            if (best == end) return false;
+            const auto waits = [&](const std::deque<uint64_t>& ages) { return d.by_age.at(ages.front()).freed >= d.safe; };
+            auto it = best;
+            while (it != end && waits(it->second)) ++it;
+            wait = it == end;
+            if (!wait) best = it;
+            const auto block = d.by_age.find(best->second.front());
+            out = block->second;
             live_[out.ptr] = out;
+            forget(d, block);
             return true;
         }
 
@@ -100,7 +97,7 @@ class PoolPolicy
         uint64_t start_wait() { return ++generation_; }
         void waited(int device, uint64_t number)
         {
-            uint64_t& s = safe_[device];
+            uint64_t& s = devices_[device].safe;
             if (number > s) s = number;
         }
 
@@ -108,51 +105,72 @@ class PoolPolicy
         // free (the block itself when it alone exceeds the bound).  False for a pointer that is not live.
         bool give(void* ptr, size_t bound, std::vector<PoolBlock>& out)
         {
-            auto it = live_.find(ptr);
+            const auto it = live_.find(ptr);
             if (it == live_.end()) return false;
             PoolBlock b = it->second;
-            live_.erase(it);
             b.freed = generation_;
-            if (b.bytes > bound)
+            if (b.bytes > bound) out.push_back(b);
+            else
             {
-                out.push_back(b);
-                return true;
+                Device& d = devices_[b.device];
+                while (d.held + b.bytes > bound)
+                {
+                    out.push_back(d.by_age.begin()->second);
+                    forget(d, d.by_age.begin());
+                }
+                d.by_size[b.bytes].push_back(age_);
+                d.by_age.emplace(age_++, b);
+                d.held += b.bytes;
             }
-            size_t& held = held_[b.device];
-            for (size_t i = 0; i < free_.size() && held + b.bytes > bound;)
-            {
-                if (free_[i].device != b.device) { ++i; continue; }
-                held -= free_[i].bytes;
-                out.push_back(free_[i]);
-                free_.erase(free_.begin() + std::ptrdiff_t(i));
-            }
-            held += b.bytes;
-            free_.push_back(b);
+            live_.erase(it);
             return true;
         }
 
         // Empties the free list of every device.
         std::vector<PoolBlock> drain()
         {
-            std::vector<PoolBlock> out(free_.begin(), free_.end());
-            free_.clear();
-            held_.clear();
+            std::vector<PoolBlock> out;
+            for (auto& d : devices_)
+            {
+                for (const auto& b : d.second.by_age) out.push_back(b.second);
+                d.second.by_age.clear();
+                d.second.by_size.clear();
+                d.second.held = 0;
+            }
             return out;
         }
 
         size_t held(int device) const
         {
-            auto it = held_.find(device);
-            return it == held_.end() ? 0 : it->second;
+            const auto it = devices_.find(device);
+            return it == devices_.end() ? 0 : it->second.held;
         }
         size_t n_live() const { return live_.size(); }
 
     private:
+        // A device's free blocks by their age (a running number) and, for each size, the ages oldest first: a
+        // request looks at the sizes within an eighth of it, not at every block.
+        struct Device
+        {
+            std::map<uint64_t, PoolBlock> by_age;
+            std::map<size_t, std::deque<uint64_t>> by_size;
+            size_t held = 0;
+            uint64_t safe = 0;
+        };
+
+        // Only a size's oldest block is ever taken out.
+        static void forget(Device& d, std::map<uint64_t, PoolBlock>::iterator block)
+        {
+            d.held -= block->second.bytes;
+            const auto s = d.by_size.find(block->second.bytes);
+            s->second.pop_front();
+            if (s->second.empty()) d.by_size.erase(s);
+            d.by_age.erase(block);
+        }
+
         // Generation 0 is never safe: the first reuse waits.
-        uint64_t generation_ = 0;
-        std::unordered_map<int, uint64_t> safe_;
-        std::unordered_map<int, size_t> held_;
-        std::deque<PoolBlock> free_;
+        uint64_t generation_ = 0, age_ = 0;
+        std::unordered_map<int, Device> devices_;
         std::unordered_map<void*, PoolBlock> live_;
 };
 }  // namespace rrtmgp_hip
