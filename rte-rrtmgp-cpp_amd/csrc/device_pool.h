@@ -81,7 +81,7 @@ class PoolPolicy
             if (!wait) best = it;
             const auto block = d.by_age.find(best->second.front());
             out = block->second;
-            live_[out.ptr] = out;
+            live_[out.ptr] = out;                        // before the block leaves the list: this may throw
             forget(d, block);
             return true;
         }
@@ -101,7 +101,7 @@ class PoolPolicy
             if (number > s) s = number;
         }
 
-        // Returns a live block to the free list; blocks that the bound pushes out go to `out` for the caller to
+        // Returns a live block to the free list (the block stays live if there is no host memory for that); blocks that the bound pushes out go to `out` for the caller to
         // free (the block itself when it alone exceeds the bound).  False for a pointer that is not live.
         bool give(void* ptr, size_t bound, std::vector<PoolBlock>& out)
         {
@@ -118,8 +118,10 @@ class PoolPolicy
                     out.push_back(d.by_age.begin()->second);
                     forget(d, d.by_age.begin());
                 }
-                d.by_size[b.bytes].push_back(age_);
-                d.by_age.emplace(age_++, b);
+                const auto block = d.by_age.emplace(age_, b).first;
+                try { d.by_size[b.bytes].push_back(age_); }
+                catch (...) { d.by_age.erase(block); throw; }
+                ++age_;
                 d.held += b.bytes;
             }
             live_.erase(it);
@@ -130,6 +132,9 @@ class PoolPolicy
         std::vector<PoolBlock> drain()
         {
             std::vector<PoolBlock> out;
+            size_t n = 0;
+            for (const auto& d : devices_) n += d.second.by_age.size();
+            out.reserve(n);
             for (auto& d : devices_)
             {
                 for (const auto& b : d.second.by_age) out.push_back(b.second);

@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -270,6 +271,16 @@ int pool_release()
     return pool_give_back(blocks);
 }
 
+// The pool's bookkeeping needs host memory: what its containers throw must not leave a C entry.
+template<typename F>
+int pool_entry(F f)
+{
+    try { return f(); }
+    catch (const std::exception&) {}
+    try { return check_hip(hipErrorOutOfMemory, "array pool (host memory)"); }
+    catch (const std::exception&) { return RRTMGP_ERR_HIP; }
+}
+
 int pool_malloc(void** p, size_t bytes)
 {
     bytes = PoolPolicy::round_block(std::max<size_t>(bytes, 1));
@@ -309,8 +320,17 @@ int pool_malloc(void** p, size_t bytes)
         e = hipMalloc(p, bytes);
     }
     RRTMGP_TRY(check_hip(e, "hipMalloc"));
-    std::lock_guard<std::mutex> lock(g_pool_mutex);
-    g_pool.add_live(*p, bytes, dev);
+    try
+    {
+        std::lock_guard<std::mutex> lock(g_pool_mutex);
+        g_pool.add_live(*p, bytes, dev);
+    }
+    catch (...)
+    {
+        (void)hipFree(*p);
+        *p = nullptr;
+        throw;
+    }
     return RRTMGP_OK;
 }
 
@@ -321,9 +341,15 @@ int pool_free(void* p)
     RRTMGP_HIP(hipGetDevice(&dev));
     const size_t bound = pool_bound(dev);
     std::vector<PoolBlock> out;
+    try
     {
         std::lock_guard<std::mutex> lock(g_pool_mutex);
         if (!g_pool.give(p, bound, out)) return arg_error("pool_free: pointer was not allocated by the pool");
+    }
+    catch (...)
+    {
+        (void)pool_give_back(out);
+        throw;
     }
     return pool_give_back(out);
 }
@@ -360,17 +386,19 @@ int rrtmgp_hip_cache_free(void* ptr, void* stream) { return cache_free(ptr, as_s
 
 int rrtmgp_hip_cache_release(void)
 {
-    RRTMGP_TRY(pool_release());
-    return release_free_blocks();
+    return pool_entry([] {
+        RRTMGP_TRY(pool_release());
+        return release_free_blocks();
+    });
 }
 
 int rrtmgp_hip_pool_malloc(void** ptr, size_t bytes)
 {
     if (!ptr) return arg_error("pool_malloc: NULL output");
-    return pool_malloc(ptr, bytes);
+    return pool_entry([=] { return pool_malloc(ptr, bytes); });
 }
 
-int rrtmgp_hip_pool_free(void* ptr) { return pool_free(ptr); }
+int rrtmgp_hip_pool_free(void* ptr) { return pool_entry([=] { return pool_free(ptr); }); }
 
 int rrtmgp_hip_cache_stats(size_t* live_bytes, size_t* cached_bytes)
 {

@@ -2,6 +2,8 @@
 // Pointers are opaque here; the checks print "ok" and return 0 when all hold.
 #include <chrono>
 #include <cstdio>
+#include <cstdlib>
+#include <new>
 
 #include "device_pool.h"
 
@@ -10,6 +12,18 @@ using rrtmgp_hip::PoolPolicy;
 
 #define CHECK(c)                                                                  \
     do { if (!(c)) { std::printf("FAILED line %d: %s\n", __LINE__, #c); return 1; } } while (0)
+
+// Allocations left before operator new fails (-1: all succeed).
+static int g_fail_after = -1;
+void* operator new(size_t n)
+{
+    if (g_fail_after == 0) throw std::bad_alloc();
+    if (g_fail_after > 0) --g_fail_after;
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 int main()
 {
@@ -147,6 +161,30 @@ int main()
         p.waited(0, p.start_wait());
         for (int i = 2; i < 4; ++i) CHECK(p.give(mem[i], MiB, out));
         for (int i = 0; i < 4; ++i) CHECK(p.take(0, 4096, b, wait) && b.ptr == mem[i] && wait == (i > 1));
+    }
+
+    // Without host memory for its books a call throws and leaves every block where it was.
+    for (int fail = 0; fail < 8; ++fail)
+    {
+        PoolPolicy p;
+        p.add_live(mem[0], 4096, 0);
+        p.add_live(mem[1], 4608, 0);
+        CHECK(p.give(mem[0], MiB, out));
+        bool threw = false;
+        g_fail_after = fail;
+        try { (void)p.give(mem[1], MiB, out); }
+        catch (const std::bad_alloc&) { threw = true; }
+        g_fail_after = -1;
+        CHECK(p.n_live() == (threw ? 1u : 0u) && p.held(0) == (threw ? 4096u : 4096u + 4608u));
+        if (threw) CHECK(p.give(mem[1], MiB, out));
+        threw = false;
+        g_fail_after = fail;
+        try { CHECK(p.take(0, 4608, b, wait)); }
+        catch (const std::bad_alloc&) { threw = true; }
+        g_fail_after = -1;
+        CHECK(p.n_live() == (threw ? 0u : 1u) && p.held(0) == (threw ? 4096u + 4608u : 4096u));
+        if (threw) CHECK(p.take(0, 4608, b, wait) && b.ptr == mem[1]);
+        CHECK(p.take(0, 4096, b, wait) && b.ptr == mem[0] && p.held(0) == 0 && out.empty());
     }
 
     std::printf("ok\n");
