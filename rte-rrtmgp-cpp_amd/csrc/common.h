@@ -81,6 +81,8 @@ inline unsigned grid1(int64_t n, int block)
 int cache_alloc(void** p, size_t bytes, hipStream_t stream);
 int cache_free(void* p, hipStream_t stream);
 int retain_pool_memory();
+// hipMalloc, tried again after the free blocks of the cache and of the array pool have gone back to the driver.
+int device_malloc(void** p, size_t bytes, const char* what);
 
 // Scratch of a launcher: taken from the cache, returned right after the launches that use it
 // are queued (stream order keeps a later reuse on the same stream behind them).

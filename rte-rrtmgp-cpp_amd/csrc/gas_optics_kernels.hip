@@ -1886,7 +1886,7 @@ int pack_d2h(std::vector<T>& out, const void* src, int64_t n, const char* what)
 template<typename T>
 int pack_h2d(void** dst, const std::vector<T>& v)
 {
-    RRTMGP_HIP(hipMalloc(dst, std::max<size_t>(v.size(), 1) * sizeof(T)));
+    RRTMGP_TRY(device_malloc(dst, std::max<size_t>(v.size(), 1) * sizeof(T), "hipMalloc (packed tables)"));
     if (!v.empty()) RRTMGP_HIP(hipMemcpy(*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
     return RRTMGP_OK;
 }

@@ -149,7 +149,24 @@ int fence_event(hipStream_t s, void** ev)
 }
 }  // namespace
 
-namespace { int pool_release(); }
+namespace
+{
+int pool_release();
+template<typename F> int pool_entry(F f);
+}
+
+int device_malloc(void** p, size_t bytes, const char* what)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory)
+    {
+        (void)hipGetLastError();
+        RRTMGP_TRY(release_free_blocks());
+        RRTMGP_TRY(pool_entry(pool_release));
+        e = hipMalloc(p, bytes);
+    }
+    return check_hip(e, what);
+}
 
 int cache_alloc(void** p, size_t bytes, hipStream_t stream)
 {
@@ -176,15 +193,7 @@ int cache_alloc(void** p, size_t bytes, hipStream_t stream)
         *p = b.ptr;
         return RRTMGP_OK;
     }
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory)
-    {
-        (void)hipGetLastError();
-        RRTMGP_TRY(release_free_blocks());
-        RRTMGP_TRY(pool_release());
-        e = hipMalloc(p, bytes);
-    }
-    RRTMGP_TRY(check_hip(e, "hipMalloc (cached scratch)"));
+    RRTMGP_TRY(device_malloc(p, bytes, "hipMalloc (cached scratch)"));
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     g_cache.add_live(*p, bytes, dev, stream);
     return RRTMGP_OK;
@@ -311,15 +320,7 @@ int pool_malloc(void** p, size_t bytes)
         *p = b.ptr;
         return RRTMGP_OK;
     }
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory)
-    {
-        (void)hipGetLastError();
-        RRTMGP_TRY(pool_release());
-        RRTMGP_TRY(release_free_blocks());
-        e = hipMalloc(p, bytes);
-    }
-    RRTMGP_TRY(check_hip(e, "hipMalloc"));
+    RRTMGP_TRY(device_malloc(p, bytes, "hipMalloc"));
     try
     {
         std::lock_guard<std::mutex> lock(g_pool_mutex);
@@ -482,8 +483,8 @@ int rrtmgp_hip_device_name(char* buf, int len)
 
 int rrtmgp_hip_malloc(void** ptr, size_t bytes)
 {
-    RRTMGP_HIP(hipMalloc(ptr, bytes));
-    return RRTMGP_OK;
+    if (!ptr) return check_hip(hipErrorInvalidValue, "hipMalloc(ptr, bytes)");
+    return device_malloc(ptr, bytes, "hipMalloc(ptr, bytes)");
 }
 
 int rrtmgp_hip_free(void* ptr)

@@ -87,3 +87,29 @@ def test_outputs_in_reused_memory(precision, ncol, nlay):
         assert np.isfinite(again[k]).all(), k
         np.testing.assert_allclose(again[k], fresh[k], rtol=1e-5 if precision == 4 else 1e-11,
                                    atol=1e-5 * np.abs(fresh[k]).max(initial=0.0), err_msg=k)
+
+
+@pytest.mark.gpu
+def test_held_blocks_go_back_when_memory_runs_out():
+    """What the pool holds is there for the library's other allocations: with 6 GiB of the device left, 4 of them
+    freed into the pool, another 5 GiB are found through each entry.  Nothing touches the memory."""
+    torch = pytest.importorskip("torch")
+    from rrtmgp_amd import _lib
+    L, gib = _lib.hip(), 1 << 30
+    new = lambda entry, n, *a: (lambda p: (getattr(L, entry)(C.byref(p), C.c_size_t(n), *a), p))(C.c_void_p())   # noqa: E731
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    _lib.check_hip(L.rrtmgp_hip_cache_release())
+    rc, rest = new("rrtmgp_hip_malloc", torch.cuda.mem_get_info()[0] - 6 * gib)
+    assert rc == 0
+    try:
+        for entry, drop in (("rrtmgp_hip_malloc", L.rrtmgp_hip_free), ("rrtmgp_hip_pool_malloc", L.rrtmgp_hip_pool_free),
+                            ("rrtmgp_hip_cache_malloc", lambda p: L.rrtmgp_hip_cache_free(p, None))):
+            rc, p = new("rrtmgp_hip_pool_malloc", 4 * gib)
+            assert rc == 0 and L.rrtmgp_hip_pool_free(p) == 0
+            rc, p = new(entry, 5 * gib, *([None] if "cache" in entry else []))
+            assert rc == 0, entry
+            assert drop(p) == 0
+            _lib.check_hip(L.rrtmgp_hip_cache_release())
+    finally:
+        L.rrtmgp_hip_free(rest)
