@@ -136,6 +136,8 @@ def adjoint_measure(kl, ks, ll, ls, prec, ncol=16384, nlay=128, reps=3):
     device.synchronize()
     live1, cached1 = stats()
     peak_scratch = live1 + cached1 - live0
+    pool_live, pool_held = C.c_size_t(0), C.c_size_t(0)
+    _lib.check_hip(_lib.hip().rrtmgp_hip_pool_stats(C.byref(pool_live), C.byref(pool_held)))
     inputs = sum(a.nbytes for a in vars(da).values() if isinstance(a, device.DeviceArray))
     inputs += tsi.nbytes + sum(c.nbytes for c in cot)
     for name, fn in (("forward", fwd), ("adjoint", adj)):
@@ -151,6 +153,7 @@ def adjoint_measure(kl, ks, ll, ls, prec, ncol=16384, nlay=128, reps=3):
             "adjoint_over_forward": round(out["adjoint"] / out["forward"], 3),
             "adjoint_peak_scratch_bytes": int(peak_scratch),
             "adjoint_peak_bytes_with_inputs": int(peak_scratch + inputs),
+            "array_pool_bytes": {"in_use": int(pool_live.value), "held": int(pool_held.value)},
             "gradients": "T_lay, T_lev, T_sfc, ln p_lay, p_lev, vmr of every gas, emissivity, albedos"}
 
 

@@ -80,9 +80,12 @@ int rrtmgp_hip_cache_stats(size_t* live_bytes, size_t* cached_bytes);
 /* Pool for arrays that any stream or library may use: pool_malloc / pool_free stand in for    */
 /* rrtmgp_hip_malloc / _free.  A freed block is handed out again only after a device            */
 /* synchronisation that began after its free, so one wait covers all blocks freed before it.   */
-/* Per device the pool keeps at most a sixteenth of the memory; cache_release gives it back.   */
+/* Per device the pool keeps at most a sixteenth of the memory; cache_release gives it back, and */
+/* so does any allocation of the library that finds no memory.  pool_stats: bytes of arrays in   */
+/* use and of free blocks held, all devices (cache_stats covers the scratch cache only).         */
 int rrtmgp_hip_pool_malloc(void** ptr, size_t bytes);
 int rrtmgp_hip_pool_free(void* ptr);
+int rrtmgp_hip_pool_stats(size_t* live_bytes, size_t* held_bytes);
 
 /* Array_gpu element operations (reference include/Array.h): fill sets n elements of          */
 /* elem_size bytes (1, 2, 4 or 8) to *value (a host pointer), as Array_gpu::fill and fill_kernel*/

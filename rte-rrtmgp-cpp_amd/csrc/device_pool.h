@@ -150,7 +150,19 @@ class PoolPolicy
             const auto it = devices_.find(device);
             return it == devices_.end() ? 0 : it->second.held;
         }
+        size_t held() const
+        {
+            size_t n = 0;
+            for (const auto& d : devices_) n += d.second.held;
+            return n;
+        }
         size_t n_live() const { return live_.size(); }
+        size_t live_bytes() const
+        {
+            size_t n = 0;
+            for (const auto& b : live_) n += b.second.bytes;
+            return n;
+        }
 
     private:
         // A device's free blocks by their age (a running number) and, for each size, the ages oldest first: a

@@ -401,6 +401,14 @@ int rrtmgp_hip_pool_malloc(void** ptr, size_t bytes)
 
 int rrtmgp_hip_pool_free(void* ptr) { return pool_entry([=] { return pool_free(ptr); }); }
 
+int rrtmgp_hip_pool_stats(size_t* live_bytes, size_t* held_bytes)
+{
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    if (live_bytes) *live_bytes = g_pool.live_bytes();
+    if (held_bytes) *held_bytes = g_pool.held();
+    return RRTMGP_OK;
+}
+
 int rrtmgp_hip_cache_stats(size_t* live_bytes, size_t* cached_bytes)
 {
     std::lock_guard<std::mutex> lock(g_cache_mutex);

@@ -113,3 +113,29 @@ def test_held_blocks_go_back_when_memory_runs_out():
             _lib.check_hip(L.rrtmgp_hip_cache_release())
     finally:
         L.rrtmgp_hip_free(rest)
+
+
+@pytest.mark.gpu
+def test_stats():
+    import gc
+    from rrtmgp_amd import _lib
+    from rrtmgp_amd.device import DeviceArray
+    L = _lib.hip()
+
+    def stats():
+        live, held = C.c_size_t(0), C.c_size_t(0)
+        _lib.check_hip(L.rrtmgp_hip_pool_stats(C.byref(live), C.byref(held)))
+        return np.array([live.value, held.value], dtype=np.int64)
+
+    gc.collect()                                       # arrays that earlier tests left in reference cycles
+    _lib.check_hip(L.rrtmgp_hip_cache_release())
+    before, mib = stats(), 1 << 20
+    assert before[1] == 0
+    a = [DeviceArray((n,), np.uint8, zero=False) for n in (4 * mib, 1000)]
+    assert list(stats() - before) == [4 * mib + 1024, 0]
+    a[0].free()
+    assert list(stats() - before) == [1024, 4 * mib]
+    a[1].free()
+    assert list(stats() - before) == [0, 4 * mib + 1024]
+    _lib.check_hip(L.rrtmgp_hip_cache_release())
+    assert list(stats() - before) == [0, 0]
