@@ -781,6 +781,8 @@ int rrtmgp_hip_mlp_gas_optics_sw(const rrtmgp_mlp_net* net, int64_t ncol, int64_
 
 /* Training.  gemm_bf16: C[m sCm + n sCn] (+)= sum_k A[m sAm + k sAk] B[k sBk + n sBn], BF16      */
 /* operands, FP32 result (accumulate != 0 adds to C).  Row-major (rows, n) arrays below.        */
+/* These are the building blocks of a step by themselves; mlp_train_grads makes the gradients of   */
+/* this network's step in three launches.                                                        */
 int rrtmgp_hip_mlp_gemm_bf16(int64_t M, int64_t N, int64_t K, const void* A, int64_t sAm, int64_t sAk,
                              const void* B, int64_t sBk, int64_t sBn, float* C, int64_t sCm, int64_t sCn,
                              int accumulate, void* stream);

@@ -47,7 +47,6 @@ template<typename T> struct K;
     static constexpr auto lw_solver_noscat_bnd = rrtmgp_hip_lw_solver_noscat_bnd_##S; \
     static constexpr auto sw_solver_2stream_bnd = rrtmgp_hip_sw_solver_2stream_bnd_##S; \
     static constexpr auto sw_solver_2stream_bnd_coalbedo = rrtmgp_hip_sw_solver_2stream_bnd_coalbedo_##S; \
-    static constexpr auto sum_broadband = rrtmgp_hip_sum_broadband_##S;  \
     static constexpr auto net_broadband = rrtmgp_hip_net_broadband_##S;  \
     static constexpr auto sum_byband = rrtmgp_hip_sum_byband_##S;        \
     static constexpr auto net_byband_full = rrtmgp_hip_net_byband_full_##S; \
