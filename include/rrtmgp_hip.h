@@ -634,7 +634,8 @@ RRTMGP_DECLARE_BOTH(RRTMGP_DECL_GO_ADJOINT)
 /* Both may write over the optical properties they read: d_tau and d_planck_frac may be tau and    */
 /* planck_frac, d_tau_abs and d_tau_ray tau and ssa.                                              */
 /* gas_optics_{lw,sw}_adjoint_bands: rrtmgp_hip_gas_optics_{lw,sw}_adjoint_* for the range, from   */
-/* those cotangents.                                                                             */
+/* those cotangents.  (Shortwave: where the gases' optical depth is within the combine rule's     */
+/* cut-off of 2 eps, the one of the Rayleigh optical depth is replaced by that of absorption.)    */
 #define RRTMGP_DECL_ADJ_BANDS(S, T)                                                            \
     int rrtmgp_hip_gas_optics_lw_bands_factored_##S(const rrtmgp_kdist_dev* kd,                \
         int64_t band_start, int64_t band_count, int64_t ncol, int64_t nlay, const T* play,     \

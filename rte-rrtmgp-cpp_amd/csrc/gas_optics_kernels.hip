@@ -1058,7 +1058,7 @@ enum GaMode
     GA_LW3,        // tau, lay_src, lev_src_inc, lev_src_dec, sfc_src
     GA_LWF,        // tau, Planck fraction, sfc_src; band Planck values at the layer and its two levels
     GA_SW3,        // tau, ssa, g after the optional band cloud add_to
-    GA_SW2         // absorption and Rayleigh optical depths
+    GA_SW2         // absorption and Rayleigh optical depths, the latter as if the combine rule had no cut-off
 };
 
 // Rows of s_acc: the cotangents of a pair's weights for one band.
@@ -1224,6 +1224,35 @@ __device__ __forceinline__ void ga_minor_back(const Kd<Real>& k, const GoBand& b
     sum.add(GA_XH, g_x);
 }
 
+// The absorption optical depth of absorption4 added to tau, with one table node live at a time: for a path that
+// is rarely taken and must not add to the registers of the others.
+template<typename Real>
+__device__ __forceinline__ void add_absorption4_rolled(const Kd<Real>& k, const GoBand& bd, const PairState<Real>& st,
+                                                       uint32_t gl, Real (&tau)[4])
+{
+    const uint32_t gp = bd.gp, sE = uint32_t(k.npres + 1) * gp, sQ = uint32_t(bd.nslot) * gp;
+#pragma unroll 1
+    for (int ic = 0; ic < 8; ++ic)
+    {
+        const int i = ic >> 2, c = ic & 3;
+        Real n[4];
+        load4(k.kmajor_p, uint32_t(bd.koff) + gl + uint32_t(st.om[i]) + (c & 1 ? sE : 0u) + (c & 2 ? gp : 0u), n);
+        const Real f = st.col_mix[i] * st.fmajor[i][c];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tau[e] += f * n[e];
+    }
+#pragma unroll 1
+    for (int q = 0; q < 4 * bd.nslot; ++q)
+    {
+        const int slot = q >> 2, i = q >> 1 & 1, c = q & 1;
+        Real n[4];
+        load4(k.kminor_p, uint32_t(bd.moff) + gl + uint32_t(st.mn[i]) + uint32_t(slot) * gp + (c ? sQ : 0u), n);
+        const Real f = st.scaling[slot] * st.fminor[i][c];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tau[e] += f * n[e];
+    }
+}
+
 // Slope of a Planck table at a position of interp1d_pos.
 template<typename Real>
 __device__ __forceinline__ Real interp1d_slope(const Real* table, int idx, Real delta)
@@ -1237,7 +1266,7 @@ constexpr int ga_arrays() { return MODE == GA_LW3 ? 4 : MODE == GA_SW3 ? 3 : 2; 
 // At 16384 columns x 128 layers in FP32 both spectral ranges take 12.4 ms (two shortwave and four longwave
 // bands a launch); with one band a launch, phases 1 and 3 on one wavefront reading and writing memory, and
 // every table node of a pair live at once they took 25.5 ms.  Bound by the gathers and LDS; the occupancy by LDS
-// (57 to 93 registers in FP32, 101 to 169 in FP64): the pair sums held in registers over a band's chunks, through
+// (65 to 93 registers in FP32, 116 to 169 in FP64): the pair sums held in registers over a band's chunks, through
 // phases 1 and 3, took 113 to 128 and spilled (14.5 ms).
 // One band a launch (GA_LW3, GA_SW3), 8192 x 64, 16 g-points: LW 143 us in FP32 and 357 in FP64, SW 135 and 296,
 // within 30 us of these with 32 gases (one wavefront's phases through memory took 181, 534, 189 and 519).
@@ -1528,15 +1557,41 @@ void gas_optics_adjoint_kernel(Kd<Real> k, Gases<Real> g, int64_t ncol, int64_t 
             {
                 const uint32_t rb = uint32_t(bd.roff) + gl;
                 const Real ray = st.aux[0];
+                Real n[2][2][4];
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) load4(k.krayl_p, rb + uint32_t(st.ry[i]) + (c ? gp : 0u), n[i][c]);
+                if constexpr (MODE == GA_SW2)
+                {
+                    // Where the combine rule sets the gases' ssa to 0 (their optical depth up to 2 eps), Rayleigh
+                    // scattering is absorption to the fluxes.  The absorption is only looked at when some
+                    // Rayleigh optical depth of the wavefront does not exceed the cut-off by itself: at 1 Pa and
+                    // 1000 cm-1 it is about 1e-11.
+                    const Real eps2 = Real(2 * prop_eps);
+                    Real tr[4];
+                    bool thin = false;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                    {
+                        tr[e] = ray * (st.fminor[0][0] * n[0][0][e] + st.fminor[0][1] * n[0][1][e] +
+                                       st.fminor[1][0] * n[1][0][e] + st.fminor[1][1] * n[1][1][e]);
+                        thin = thin || (gq + e < ncg && tr[e] <= eps2);
+                    }
+                    if (__any(thin))
+                    {
+                        add_absorption4_rolled(k, bd, st, gl, tr);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) gray[e] = tr[e] > eps2 ? gray[e] : gabs[e];
+                    }
+                }
                 Real x0 = Real(0);
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int c = 0; c < 2; ++c)
                     {
-                        Real n[4];
-                        load4(k.krayl_p, rb + uint32_t(st.ry[i]) + (c ? gp : 0u), n);
-                        const Real d = dot4(gray, n);
+                        const Real d = dot4(gray, n[i][c]);
                         x0 += st.fminor[i][c] * d;
                         fn[i][c] = ray * d;
                     }

@@ -697,8 +697,9 @@ void sw_adjoint_down_kernel(SwAdjArgs<Real> a)
 // With CHAIN the cotangents of tau, ssa and g are carried on to the gases' absorption and Rayleigh optical
 // depths (d_tau and d_ssa receive those; the band cloud is held fixed): with the scattering optical depth
 // ts = ssa tau, tau = abs + ray + cloud and g a cloud quantity over ts,
-//     d_abs = d_tau - d_ssa ssa / tau,   d_ray = d_abs + d_ssa / tau - d_g g / ts,
-// and d_ray = d_abs where the combine rule sets ssa = 0 (tau <= 2 eps).
+//     d_abs = d_tau - d_ssa ssa / tau,   d_ray = d_abs + d_ssa / tau - d_g g / ts.
+// (The combine rule's cut-off is on the gases' optical depth, which the gas-optics adjoint knows: there
+// d_ray = d_abs where that is up to 2 eps.)
 // Bound by its FP64 arithmetic (153 VGPRs, 3 wavefronts per SIMD) next to 10 values of traffic a layer.
 // The pair of sweeps takes 3.4 + 5.4 ms for the 14 bands of 16384 columns x 128 layers in FP32; the four
 // it replaced (two forward and two reverse recursions through 12 stored states a level, the layer
@@ -759,7 +760,7 @@ void sw_adjoint_up_kernel(SwAdjArgs<Real> a)
             const double op_eps = 3. * double(Limits<Real>::tiny), ts = w0 * tau;
             const double it = tau > op_eps ? rcp_full(tau) : 0.;
             const double da = gt - gw * w0 * it;
-            const double dr = tau > 2. * prop_eps ? gw * it - (ts > op_eps ? gg * g * rcp_full(ts) : 0.) : 0.;
+            const double dr = gw * it - (ts > op_eps ? gg * g * rcp_full(ts) : 0.);
             a.d_tau[lo] = Real(da); a.d_ssa[lo] = Real(da + dr);
         }
         else

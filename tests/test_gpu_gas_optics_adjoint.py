@@ -301,3 +301,47 @@ def test_drivers_on_ragged_bands(G, O, syn, kd_lw, kd_sw, lut_lw, lut_sw, lw):
     fd = (loss(_perturbed(atm, v, h)) - loss(_perturbed(atm, v, -h))) / (2 * h)
     ad = _dot(G, grad, v, kd.gas_names, lw)
     assert abs(ad - fd) <= 1e-5 * abs(fd), (ad, fd)
+
+
+@pytest.mark.parametrize("thin", [False, True])
+def test_shortwave_chains_agree_in_cloud(G, syn, kd_sw, thin):
+    """Reverse mode of solver and gas optics through the gases' optical depths against the chain through tau, ssa
+    and g, with clouds in every layer.  Where a layer's gases are thinner than the combine rule's cut-off
+    (2 eps), Rayleigh scattering does not reach the fluxes, however thick the cloud.  Bar: both chains evaluate
+    the same derivatives in FP64, 1e-9 of a layer's largest."""
+    k = ragged(kd_sw)
+    c = Ctx(G, syn, k, G.KDist(k, AVAILABLE, 8), False, True)
+    if thin:
+        c.cd[::3, 1] = 1e3                       # molecules per cm2: optical depths of 1e-20 and less
+        c.cd[1::3, 2] = 1e9
+    nb, ng = len(SIZES), sum(SIZES)
+    full, lev, bnd = (c.n, c.nlay, ng), (c.n, c.nlay + 1), (c.n, ng)
+    a, keep = c.inputs(c.x)
+    i = C.c_int64
+    size, cl = [i(c.n), i(c.nlay)], [c.dev(v) for v in c.cloud]
+    opt = [c.new(*full) for _ in range(3)]
+    c.call("gas_optics_sw_bands", i(0), i(nb), *size, *a, *[v.ptr for v in cl], *[v.ptr for v in opt])
+    rng = np.random.default_rng(4)
+    mu0, alb, inc = c.dev(rng.uniform(0.2, 1, c.n)), c.dev(rng.uniform(0.1, 0.5, bnd)), c.dev(rng.uniform(1, 2, bnd))
+    cot = [c.dev(rng.normal(size=lev)) for _ in range(3)]
+    args = size + [i(ng), C.c_int(0)] + [v.ptr for v in (*opt, mu0, alb, alb, inc)] + [None] + [v.ptr for v in cot]
+    alb_out = [c.new(*bnd) for _ in range(2)]
+
+    def solver(name, out):
+        from rrtmgp_amd import _lib
+        _lib.check_hip(getattr(c.t.L, f"rrtmgp_hip_{name}_f64")(*args, *[v.ptr for v in out + alb_out], None))
+
+    d3, d2 = [c.new(*full) for _ in range(3)], [c.new(*full) for _ in range(2)]
+    solver("sw_solver_2stream_adjoint", d3)
+    solver("sw_adjoint_gases", d2)
+    one, two = c.outputs(), c.outputs()
+    g0 = 0
+    for b, n in enumerate(SIZES):
+        part = [c.dev(_host(v)[:, :, g0:g0 + n]) for v in d3]
+        c.call("gas_optics_sw_adjoint", i(b), *size, *a, *[v.ptr for v in cl], *[v.ptr for v in part], *[o.ptr for o in one])
+        g0 += n
+    c.call("gas_optics_sw_adjoint_bands", i(0), i(nb), *size, *a, *[v.ptr for v in d2], *[o.ptr for o in two])
+    for name, x, y in zip(("d_col", "d_t", "d_lnp"), one, two):
+        x, y = (_host(v).reshape(c.n, c.nlay, -1) for v in (x, y))
+        scale = np.abs(x).max(axis=0)            # per layer and gas: gradients of a thin layer are of another size
+        assert (np.abs(x - y) <= 1e-9 * scale).all(), (name, (np.abs(x - y) / np.maximum(scale, 1e-300)).max())
