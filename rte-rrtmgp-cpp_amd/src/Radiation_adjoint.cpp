@@ -42,13 +42,15 @@ Array_gpu<Float,2> expand(const Gas_optics_rrtmgp_gpu& kd, const Array_gpu<Float
 // and g-point) stays below `bytes`, at least one.  One launch per kernel then covers them: at a few thousand
 // columns and fewer a single band's work-groups leave most of the GPU idle (250 x 60 columns and layers: 4 tiles
 // x 16 g-points), at 16384 x 128 in FP32 two shortwave and four longwave bands share the staging of the
-// gas-optics inputs.  Cotangents are written over the optical properties they belong to, so that both drivers
+// gas-optics inputs.  A batch has at most 256 groups of 16 g-points of a band, which is what the longwave solver
+// adjoint takes.  Cotangents are written over the optical properties they belong to, so that both drivers
 // together take 2.6 GB of scratch there (one band at a time with 12 stored shortwave states took 3.1 GB).
 constexpr double GiB = 1024. * 1024. * 1024.;
 
 struct Batch
 {
     int b0, nb, g0, ng;              // bands, first g-point (0-based), g-points
+    int groups;                      // groups of up to 16 g-points of a band
     std::vector<int> lims;           // (2, nb) band limits, 1-based within the batch
 };
 
@@ -59,9 +61,11 @@ std::vector<Batch> make_batches(const Gas_optics_rrtmgp_gpu& kd, int64_t ncl, do
     std::vector<Batch> out;
     for (int b = 0; b < kd.get_nband(); ++b)
     {
-        const int s = bl({1, b + 1}), e = bl({2, b + 1});
-        if (out.empty() || double(out.back().ng + e - s + 1) > most) out.push_back({b, 0, s - 1, 0, {}});
+        const int s = bl({1, b + 1}), e = bl({2, b + 1}), groups = (e - s + 16) / 16;
+        if (out.empty() || double(out.back().ng + e - s + 1) > most || out.back().groups + groups > 256)
+            out.push_back({b, 0, s - 1, 0, 0, {}});
         Batch& t = out.back();
+        t.groups += groups;
         t.lims.push_back(s - t.g0);
         t.lims.push_back(e - t.g0);
         ++t.nb;
@@ -167,11 +171,7 @@ void lw_adjoint_gpu(Gas_optics_rrtmgp_gpu& kdist, Cloud_optics_gpu* cloud_optics
     const std::vector<Batch> batches = make_batches(kdist, ncl, 2.5, 1.25 * GiB);
     const int mg = most_of(batches, [](const Batch& t) { return t.ng; });
     const int mb = most_of(batches, [](const Batch& t) { return t.nb; });
-    const int mq = most_of(batches, [](const Batch& t) {
-        int n = 0;
-        for (int i = 0; i < t.nb; ++i) n += (t.lims[2 * i + 1] - t.lims[2 * i] + 16) / 16;   // groups of 16 g-points
-        return n;
-    });
+    const int mq = most_of(batches, [](const Batch& t) { return t.groups; });
     // One block for all, so that the shortwave driver finds it large enough for its level states.
     const int64_t sizes[] = {ncl * mg, ncl * mg, ncl * mb, int64_t(ncol) * nlev * mb, ncl * mq, ncl * mq, ncl * mq,
                              int64_t(ncol) * mg, int64_t(ncol) * mg, int64_t(ncol) * mg};
