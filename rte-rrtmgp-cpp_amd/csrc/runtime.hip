@@ -235,9 +235,9 @@ namespace
 {
 // Device-array pool: the reuse rules are those of PoolPolicy (device_pool.h).  It replaced a hipMalloc, a
 // clear and a hipFree per output array, each free a wait for the device and, for large arrays, an unmapping:
-// the LW gas optics through the class API at 4096 x 72 x 256 FP32 (four outputs of 302 MB) took 47 ms a call
-// for 1.7 ms of kernels, and takes 1.85 ms.  Of an eighth of waste at most, a repeated call with the same or
-// nearly the same sizes finds its blocks again.
+// the LW gas optics through the class API at 4096 x 72 x 256 FP32 (four outputs of 302 MB, 1.7 ms of kernels)
+// took 2.6 ms a call at best and 47 ms where every call mapped and unmapped its outputs, and takes 1.85 ms.  Of
+// an eighth of waste at most, a repeated call with the same or nearly the same sizes finds its blocks again.
 std::mutex g_pool_mutex;
 PoolPolicy g_pool;
 
