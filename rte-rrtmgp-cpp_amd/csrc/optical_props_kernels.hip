@@ -246,17 +246,24 @@ enum IncMode { INC_1SCL = 0, INC_2STR = 1, INC_COALB = 2 };
 // element, with a 64-bit division and a per-lane scan of the limits, ran at half the copy rate: at 4096 x 72
 // FP32 the LW and the 2-stream SW increment (256 and 224 g-points) took 938 us together and take 413 us
 // (5.3 TB/s); the FP64 co-albedo increment at 1000 x 72 x 224 took 157 us and takes 148 us (5.2 TB/s).
-template<typename Real, int MODE, int NV>
+//
+// FLAT gives a thread an element of the whole array instead: in FP64 the two-stream increments of slices that do
+// not start on 16 bytes then keep every wavefront's accesses on whole lines (4095 x 63 x 224: 518 us against 548;
+// 1001 x 59: 120 and 129; 301 x 137: 72 and 69).  In FP32, and for tau alone, the division costs more (337 us
+// without, 360 with; 302 and 334).
+template<typename Real, int MODE, int NV, bool FLAT = false>
 __global__ void inc_bybnd_kernel(int64_t ncl, int64_t ngpt, Real* __restrict__ tau1, Real* __restrict__ ssa1,
                                  Real* __restrict__ g1, const Real* __restrict__ tau2,
                                  const Real* __restrict__ ssa2, const Real* __restrict__ g2, int64_t nbnd,
                                  const int* __restrict__ band_lims)
 {
     using V = Vec<Real, NV>;
-    const int64_t cl = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) * NV;
-    if (cl >= ncl) return;
+    static_assert(!FLAT || NV == 1, "an element a thread");
+    const int64_t e = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) * NV;
+    const int64_t cl = FLAT ? e % ncl : e;
+    if (!FLAT && cl >= ncl) return;
     const Real eps = Real(3) * Limits<Real>::tiny;
-    for (int64_t gpt = blockIdx.y; gpt < ngpt; gpt += gridDim.y)
+    for (int64_t gpt = FLAT ? e / ncl : int64_t(blockIdx.y); gpt < ngpt; gpt += FLAT ? ngpt : int64_t(gridDim.y))
     {
         const int64_t i = cl + ncl * gpt;
         for (int64_t b = 0; b < nbnd; ++b)
@@ -319,6 +326,10 @@ void launch_inc_bybnd(int64_t ncl, int64_t ngpt, Real* tau1, Real* ssa1, Real* g
     if (ncl % NV == 0 && bits % 16 == 0)
         hipLaunchKernelGGL((inc_bybnd_kernel<Real, MODE, NV>), dim3(grid1(ncl / NV, 256), gy), dim3(256), 0, stream,
                            ncl, ngpt, tau1, ssa1, g1, tau2, ssa2, g2, nbnd, band_lims);
+    else if (sizeof(Real) == 8 && MODE != INC_1SCL && ncl >= 48 * 1024 && (ncl * ngpt + 255) / 256 < (int64_t(1) << 31))
+        hipLaunchKernelGGL((inc_bybnd_kernel<Real, MODE, 1, sizeof(Real) == 8 && MODE != INC_1SCL>),
+                           dim3(grid1(ncl * ngpt, 256)), dim3(256), 0, stream, ncl, ngpt, tau1, ssa1, g1, tau2, ssa2, g2,
+                           nbnd, band_lims);
     else
         hipLaunchKernelGGL((inc_bybnd_kernel<Real, MODE, 1>), dim3(grid1(ncl, 256), gy), dim3(256), 0, stream,
                            ncl, ngpt, tau1, ssa1, g1, tau2, ssa2, g2, nbnd, band_lims);

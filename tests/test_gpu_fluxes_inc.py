@@ -6,6 +6,7 @@ Sums are compared bit for bit with sums in g-point order in the same type.  Each
 of two products over a sum, a few roundings each, of positive terms: 8 eps.
 """
 import copy
+import ctypes as C
 
 import numpy as np
 import pytest
@@ -84,3 +85,30 @@ def test_increment_by_band(G, syn, precision, ncol, nlay):
     np.testing.assert_allclose(_host(d), a + x, rtol=tol)
     np.testing.assert_allclose(_host(ds), (a * b + x * y) / (a + x), rtol=tol)
     np.testing.assert_allclose(_host(dg), (a * b * c + x * y * z) / (a * b + x * y), rtol=tol)
+
+
+@pytest.mark.parametrize("ncol,nlay", [(1639, 31), (1, 49151), (49153, 1)])
+def test_increment_of_large_odd_slices(G, syn, ncol, nlay):
+    """FP64 two-stream increments beyond the size from which a thread takes an element of the whole array, with
+    bands that leave g-points out and overlap; bit for bit what a slice of fewer elements gives."""
+    from rrtmgp_amd import _lib
+    dt, ng = np.float64, 9
+    lims = np.array([[1, 3], [3, 4], [6, 9]], dtype=np.int32)
+    rng = np.random.default_rng(ncol)
+    n = ncol * nlay
+    a = [rng.uniform(0, 1, (n, ng)) for _ in range(3)]
+    b = [rng.uniform(0, 1, (n, len(lims))) for _ in range(3)]
+    dev = lambda x, t=dt: G.DeviceArray.from_host(np.asfortranarray(x), t)               # noqa: E731
+    for name in ("inc_bybnd", "inc_bybnd_coalbedo"):
+        def run(part):
+            x, y = [dev(v[part]) for v in a], [dev(v[part]) for v in b]
+            m, lim = len(a[0][part]), dev(lims.ravel(), np.int32)
+            _lib.check_hip(getattr(_lib.hip(), f"rrtmgp_hip_{name}_f64")(
+                C.c_int64(m), C.c_int64(1), C.c_int64(ng), *[v.ptr for v in x + y], C.c_int64(len(lims)), lim.ptr, None))
+            return [_host(v) for v in x]
+
+        whole = run(slice(None))
+        for s in (slice(0, 999), slice(n - 999, n)):
+            for w, p in zip(whole, run(s)):
+                assert np.array_equal(w[s], p), name
+        assert np.array_equal(whole[0][:, 4], a[0][:, 4])                # of no band
